@@ -28,14 +28,23 @@ namespace mlens
 /* Deflect one point per lane. Lanes that share a leaf are evaluated together
    with the leaf index made wave-uniform. cache_* hold the lane's last leaf and
    a box slightly inside it; a point inside that box needs no new descent. */
+// the argument block of a kernel whose first parameter it is, where the launch put it
+__device__ __forceinline__ const ShootArgs* kernarg_block()
+{
+	return reinterpret_cast<const ShootArgs*>((const void*)__builtin_amdgcn_kernarg_segment_ptr());
+}
+
 struct LeafCache
 {
 	int node = -1;
 	double x0 = 1, x1 = -1, y0 = 1, y1 = -1;
 };
 
-template <int PREC, bool MU>
-__device__ __forceinline__ Deflection deflect(const ShootArgs& a, double zx, double zy, LeafCache& c)
+/* cold: the argument block in memory, read only for points outside the root
+   box. Read from `a` instead, its tree pointers (16 scalar registers) would be
+   loaded ahead of the shooting loop and spilled. */
+template <int PREC, bool MU, bool LIN>
+__device__ __forceinline__ Deflection deflect(const ShootArgs& a, const ShootArgs* cold, double zx, double zy, LeafCache& c)
 {
 	if (!(zx > c.x0 && zx < c.x1 && zy > c.y0 && zy < c.y1))
 	{
@@ -74,14 +83,15 @@ __device__ __forceinline__ Deflection deflect(const ShootArgs& a, double zx, dou
 			asm volatile("" : "+v"(same));
 			if (same)
 			{
-				d = deflect_leaf<PREC, MU>(a, u, zx, zy);
+				d = deflect_leaf<PREC, MU, LIN>(a, u, zx, zy);
 				pending = false;
 			}
 		}
 	}
 	else
 	{
-		d = deflect_node<MU>(a, c.node, zx, zy);
+		asm volatile("" : "+s"(cold));   // keeps the loads here
+		d = deflect_node<MU, LIN>(*cold, c.node, zx, zy);
 	}
 	return d;
 }
@@ -759,8 +769,8 @@ static inline int ipm_tile_rows(long long ntx, long long rows, int num_cus)
 
 // One tile: this wave's 63 cells of lattice columns tile_x * 63 WAVES + wave * 63 + [0, 63),
 // cell rows [J0, J1). Every lane of the wave must call it.
-template <int PREC, bool PARITY, bool TILED, int WAVES, class Q>
-__device__ __forceinline__ void ipm_tile(const ShootArgs& a, Q& q, long long tile_x, long long J0, long long J1)
+template <int PREC, bool PARITY, bool TILED, int WAVES, bool LIN, class Q>
+__device__ __forceinline__ void ipm_tile(const ShootArgs& a, const ShootArgs* cold, Q& q, long long tile_x, long long J0, long long J1)
 {
 	const int lane = threadIdx.x & 63;
 	const int wave = threadIdx.x >> 6;
@@ -775,7 +785,7 @@ __device__ __forceinline__ void ipm_tile(const ShootArgs& a, Q& q, long long til
 
 	auto corner = [&](long long J, double& px, double& py) {
 		double zy = lattice_at(a.y0, a.stepy, J);
-		Deflection d = deflect<PREC, false>(a, zx, zy, cache);
+		Deflection d = deflect<PREC, false, LIN>(a, cold, zx, zy, cache);
 		// ipm_functions.cuh:159-165 and array_functions.cuh:70-75
 		px = ((d.wx - a.cyx) + a.h1) * a.s1;
 		py = double(a.n2) - ((d.wy - a.cyy) + a.h2) * a.s2;
@@ -815,12 +825,13 @@ __device__ __forceinline__ void ipm_tile(const ShootArgs& a, Q& q, long long til
 	acc_flush<MapT, PARITY>(a, acc);
 }
 
-// Three waves per SIMD: 136 VGPRs without spills, and 12.7 KB of LDS per wave for a
-// 100-entry queue and a 128-slot merge table. Four waves (128 VGPRs, about 25
+// Compiled for linear smooth matter (LIN) the kernel needs 114 VGPRs and spills no scalar
+// register; with the general sheet's code in it, 136 VGPRs hold 130 spilled scalars as well.
+// Three waves per SIMD, and 12.7 KB of LDS per wave for a 100-entry queue and a 128-slot merge table. Four waves (128 VGPRs, about 25
 // spilled) ran as fast with a 64-slot table and a 79-entry queue, the most that
 // fit in 10 KB, and gained nothing from a larger table (10000^2 map: 1.698 s at
 // three waves against 1.745 s at four)
-template <int PREC, bool PARITY>
+template <int PREC, bool PARITY, bool LIN>
 __global__ __launch_bounds__(64 * IPM_WAVES, 3) void k_ipm_fast(ShootArgs a, long long row0, long long row1,
 	MLENS_TABLE_PARAMS, void* __restrict__ map, void* __restrict__ mmin, void* __restrict__ msad,
 	void* __restrict__ span, void* __restrict__ span_sad, int tile_h)
@@ -835,7 +846,7 @@ __global__ __launch_bounds__(64 * IPM_WAVES, 3) void k_ipm_fast(ShootArgs a, lon
 	if (J0 >= row1) return;
 	const long long J1 = min(J0 + tile_h, row1);
 	__shared__ TriQueue<IPM_QCAP> queues[IPM_WAVES];
-	ipm_tile<PREC, PARITY, true, IPM_WAVES>(a, queues[threadIdx.x >> 6], blockIdx.x, J0, J1);
+	ipm_tile<PREC, PARITY, true, IPM_WAVES, LIN>(a, kernarg_block(), queues[threadIdx.x >> 6], blockIdx.x, J0, J1);
 }
 
 /*
@@ -848,14 +859,16 @@ row and 63-cell tile that holds such a cell: (row, first column, mask of the
 tile's cells). count ends as the number of records; those beyond cap are not
 written.
 */
+constexpr int WINDOW_TILE_H = 64;   // lattice rows a wave walks
+
 __global__ __launch_bounds__(64 * IPM_WAVES) void k_window_cells(ShootArgs a, long long row0, long long row1,
 	MLENS_TABLE_PARAMS, double wx0, double wx1, double wy0, double wy1, long long* __restrict__ rec, long long cap,
 	unsigned long long* __restrict__ count)
 {
 	MLENS_TABLE_REBIND(a)
-	const long long J0 = row0 + (long long)blockIdx.y * IPM_TILE_H;
+	const long long J0 = row0 + (long long)blockIdx.y * WINDOW_TILE_H;
 	if (J0 >= row1) return;
-	const long long J1 = min(J0 + IPM_TILE_H, row1);
+	const long long J1 = min(J0 + WINDOW_TILE_H, row1);
 	const int lane = threadIdx.x & 63;
 	const int wave = threadIdx.x >> 6;
 	const long long Ibase = (long long)blockIdx.x * IPM_TILE_W + wave * 63;
@@ -866,7 +879,7 @@ __global__ __launch_bounds__(64 * IPM_WAVES) void k_window_cells(ShootArgs a, lo
 	LeafCache cache;
 	auto corner = [&](long long J, double& px, double& py) {
 		double zy = lattice_at(a.y0, a.stepy, J);
-		Deflection d = deflect<PREC_MIXED, false>(a, zx, zy, cache);
+		Deflection d = deflect<PREC_MIXED, false, false>(a, kernarg_block(), zx, zy, cache);
 		px = ((d.wx - a.cyx) + a.h1) * a.s1;
 		py = double(a.n2) - ((d.wy - a.cyy) + a.h2) * a.s2;
 	};
@@ -912,7 +925,7 @@ long long Engine::window_cells(const LensParams& lens, const GridParams& g, int 
 	DeviceBuffer<unsigned long long> dcount;
 	dcount.alloc(1);
 	MLENS_HIP_CHECK(hipMemsetAsync(dcount.ptr, 0, sizeof(unsigned long long), stream_));
-	dim3 grid(unsigned((a.N1 + IPM_TILE_W - 1) / IPM_TILE_W), unsigned((a.N2 + IPM_TILE_H - 1) / IPM_TILE_H));
+	dim3 grid(unsigned((a.N1 + IPM_TILE_W - 1) / IPM_TILE_W), unsigned((a.N2 + WINDOW_TILE_H - 1) / WINDOW_TILE_H));
 	k_window_cells<<<grid, 64 * IPM_WAVES, 0, stream_>>>(a, 0, a.N2, MLENS_TABLE_ARGS(a), wx0 - margin, wx0 + ww + margin,
 		wy0 - margin, wy0 + wh + margin, drec.ptr, cap, dcount.ptr);
 	MLENS_HIP_CHECK(hipGetLastError());
@@ -941,10 +954,12 @@ struct BatchMap
 	int n1, n2, tiles_x;
 };
 
-// Three waves per SIMD (141 VGPRs, no spills): the batch's maps of 0.25-16 MB
-// stay in the caches, and at four waves (128 VGPRs) the spills cost more than
-// the fourth wave hides (256 maps: 1.669 s at 12 blocks per CU, 1.890 s at 16).
-// Blocks take tiles from a global counter and never wait for each other.
+// Three waves per SIMD: the batch's maps of 0.25-16 MB stay in the caches. Blocks take tiles
+// from a global counter and never wait for each other. The instance's arguments and, through
+// them, its leaf tables come in by scalar loads; read as ordinary memory, which the maps'
+// atomics might change, they took 24 maps of 256-512 pixels from 8.1 to 10.6 ms. LIN: every
+// instance's smooth matter is linear (117 VGPRs against 139).
+template <bool LIN>
 __global__ __launch_bounds__(64 * IPM_BATCH_WAVES, 3) void k_ipm_batch(const ShootArgs* __restrict__ args,
 	const long long* __restrict__ tile_start, int ninst, int tile_h, long long total, long long stride,
 	unsigned long long* __restrict__ counter)
@@ -967,12 +982,14 @@ __global__ __launch_bounds__(64 * IPM_BATCH_WAVES, 3) void k_ipm_batch(const Sho
 			else
 				hi = mid - 1;
 		}
-		const ShootArgs a = args[lo];
+		// one instance per block: its arguments are read once, into scalar registers
+		lo = __builtin_amdgcn_readfirstlane(lo);
+		const ShootArgs a = load_const(args + lo);
 		const long long local = t - tile_start[lo];
 		const long long ntx = (a.N1 + IPM_BATCH_TILE_W - 1) / IPM_BATCH_TILE_W;
 		const long long ty = local / ntx, tx = local - ty * ntx;
 		const long long J0 = ty * tile_h, J1 = min(J0 + (long long)tile_h, a.N2);
-		ipm_tile<PREC_MIXED, false, true, IPM_BATCH_WAVES>(a, queues[threadIdx.x >> 6], tx, J0, J1);
+		ipm_tile<PREC_MIXED, false, true, IPM_BATCH_WAVES, LIN>(a, args + lo, queues[threadIdx.x >> 6], tx, J0, J1);
 	}
 }
 
@@ -1347,16 +1364,32 @@ struct IrsWindow
 	int x0, y0;
 };
 
-__device__ __forceinline__ void irs_count(const ShootArgs& a, const IrsWindow& win, int px, int py, int v)
+/*
+With parities a count goes to the minima or the saddles map and the total is
+their sum (add_parity_maps), so only those two are counted. The window keeps
+both: minima in the low half of each word, saddles in the high half. A block
+flushes it every IRS_PARITY_ROWS rows, before 64 rays a row can fill a half.
+*/
+constexpr int IRS_PARITY_ROWS = 512;
+static_assert(64 * IRS_PARITY_ROWS < 65536, "a half word of the parity window counts every ray of its rows");
+
+template <bool PARITY>
+__device__ __forceinline__ void irs_count(const ShootArgs& a, const IrsWindow& win, int px, int key_y, int v)
 {
+	const int py = PARITY ? key_y >> 1 : key_y;
 	const int dx = px - win.x0, dy = py - win.y0;
 	if (dx >= 0 && dx < IRS_WX && dy >= 0 && dy < IRS_WY)
-		atomicAdd(win.w + dy * IRS_WX + dx, v);
+		atomicAdd(win.w + dy * IRS_WX + dx, PARITY && (key_y & 1) ? v << 16 : v);
 	else
-		atomicAdd(reinterpret_cast<int*>(a.map) + ((long long)py * a.n1 + px), v);
+		atomicAdd(reinterpret_cast<int*>(PARITY ? ((key_y & 1) ? a.msad : a.mmin) : a.map) + ((long long)py * a.n1 + px), v);
 }
 
-template <int PREC, bool PARITY>
+// LIN (linear smooth matter) takes the mixed kernel from 116 to 85 VGPRs and its 90 spilled scalar
+// registers to 2, hence from four waves per SIMD to five: 1.04e9 rays in 8.2 ms against 9.5 ms.
+// With parities (FP64 positions and magnifications; 1.6e9 rays) the shot took 118 ms with a second
+// pass over the leaf's tables for the magnification and parity counts sent straight to the maps,
+// and takes 40 ms.
+template <int PREC, bool PARITY, bool LIN>
 __global__ __launch_bounds__(IRS_THREADS) void k_irs_fast(ShootArgs a, long long row0, long long row1,
 	unsigned long long* __restrict__ received, MLENS_TABLE_PARAMS, void* __restrict__ map, void* __restrict__ mmin,
 	void* __restrict__ msad, int tile_h)
@@ -1375,77 +1408,92 @@ __global__ __launch_bounds__(IRS_THREADS) void k_irs_fast(ShootArgs a, long long
 	const double zx = lattice_at(a.x0, a.stepx, ok ? i : a.N1 - 1);
 	LeafCache cache;
 	unsigned long long got = 0;
-	for (int k = threadIdx.x; k < IRS_WX * IRS_WY; k += IRS_THREADS) win_counts[k] = 0;
-	__syncthreads();
-
-	// register cache: (x, y) of the two most recent pixels and their counts
-	int kx0 = -1, ky0 = -1, c0 = 0, kx1 = -1, ky1 = -1, c1 = 0;
-	PixelAcc<int> par;
-	IrsWindow win{win_counts, 0, 0};
-	for (long long j = J0; j < J1; j++)
+	// the window's rows of rays: the whole tile without parities
+	for (long long Ja = J0; Ja < J1; Ja = PARITY ? Ja + IRS_PARITY_ROWS : J1)
 	{
-		double zy = lattice_at(a.y0, a.stepy, j);
-		Deflection d = deflect<PREC, PARITY>(a, zx, zy, cache);
-		int px = 0, py = 0;
-		const bool hit = ok && !isnan(d.wx) && !isnan(d.wy) && irs_pixel(a, d.wx, d.wy, px, py);
-		if (j == J0)
+		const long long Jb = PARITY ? min(Ja + IRS_PARITY_ROWS, J1) : J1;
+		for (int k = threadIdx.x; k < IRS_WX * IRS_WY; k += IRS_THREADS) win_counts[k] = 0;
+		__syncthreads();
+
+		// register cache: (x, y) of the two most recent pixels and their counts; with
+		// parities the row is doubled and its low bit tells minima (0) from saddles (1)
+		int kx0 = -1, ky0 = -1, c0 = 0, kx1 = -1, ky1 = -1, c1 = 0;
+		IrsWindow win{win_counts, 0, 0};
+		for (long long j = Ja; j < Jb; j++)
 		{
-			// window centred on the bounding box of the block's (the wave's) first row
-			int mnx = hit ? px : 0x7fffffff, mny = hit ? py : 0x7fffffff;
-			int mxx = hit ? px : -0x7fffffff, mxy = hit ? py : -0x7fffffff;
-			for (int off = 32; off > 0; off >>= 1)
+			double zy = lattice_at(a.y0, a.stepy, j);
+			Deflection d = deflect<PREC, PARITY, LIN>(a, kernarg_block(), zx, zy, cache);
+			int px = 0, py = 0;
+			const bool hit = ok && !isnan(d.wx) && !isnan(d.wy) && irs_pixel(a, d.wx, d.wy, px, py);
+			if (j == Ja)
 			{
-				mnx = min(mnx, __shfl_xor(mnx, off));
-				mny = min(mny, __shfl_xor(mny, off));
-				mxx = max(mxx, __shfl_xor(mxx, off));
-				mxy = max(mxy, __shfl_xor(mxy, off));
+				// window centred on the bounding box of the block's (the wave's) first row
+				int mnx = hit ? px : 0x7fffffff, mny = hit ? py : 0x7fffffff;
+				int mxx = hit ? px : -0x7fffffff, mxy = hit ? py : -0x7fffffff;
+				for (int off = 32; off > 0; off >>= 1)
+				{
+					mnx = min(mnx, __shfl_xor(mnx, off));
+					mny = min(mny, __shfl_xor(mny, off));
+					mxx = max(mxx, __shfl_xor(mxx, off));
+					mxy = max(mxy, __shfl_xor(mxy, off));
+				}
+				if (mnx <= mxx)
+				{
+					win.x0 = (mnx + mxx) / 2 - IRS_WX / 2;
+					win.y0 = (mny + mxy) / 2 - IRS_WY / 2;
+				}
+				else
+				{
+					win.x0 = win.y0 = -0x3fffffff;   // no ray of the first row landed: no window
+				}
 			}
-			if (mnx <= mxx)
+			if (!hit) continue;
+			if (PARITY) py = 2 * py + (d.mu >= 0 ? 0 : 1);
+			if (px == kx0 && py == ky0)
 			{
-				win.x0 = (mnx + mxx) / 2 - IRS_WX / 2;
-				win.y0 = (mny + mxy) / 2 - IRS_WY / 2;
+				c0++;
+			}
+			else if (px == kx1 && py == ky1)
+			{
+				const int t = c1 + 1;
+				kx1 = kx0;
+				ky1 = ky0;
+				c1 = c0;
+				kx0 = px;
+				ky0 = py;
+				c0 = t;
 			}
 			else
 			{
-				win.x0 = win.y0 = -0x3fffffff;   // no ray of the first row landed: no window
+				if (c1) irs_count<PARITY>(a, win, kx1, ky1, c1);
+				kx1 = kx0;
+				ky1 = ky0;
+				c1 = c0;
+				kx0 = px;
+				ky0 = py;
+				c0 = 1;
+			}
+			got++;
+		}
+		if (c0) irs_count<PARITY>(a, win, kx0, ky0, c0);
+		if (c1) irs_count<PARITY>(a, win, kx1, ky1, c1);
+		__syncthreads();
+		for (int k = threadIdx.x; k < IRS_WX * IRS_WY; k += IRS_THREADS)
+		{
+			const int v = win_counts[k];
+			const long long pix = (long long)(win.y0 + k / IRS_WX) * a.n1 + (win.x0 + k % IRS_WX);
+			if (!PARITY)
+			{
+				if (v) atomicAdd(reinterpret_cast<int*>(a.map) + pix, v);
+			}
+			else
+			{
+				const int mn = v & 0xffff, sd = int(unsigned(v) >> 16);
+				if (mn) atomicAdd(reinterpret_cast<int*>(a.mmin) + pix, mn);
+				if (sd) atomicAdd(reinterpret_cast<int*>(a.msad) + pix, sd);
 			}
 		}
-		if (!hit) continue;
-		if (PARITY) acc_add<int, true>(a, par, ((long long)py * a.n1 + px) * 2 + (d.mu >= 0 ? 0 : 1), 1);
-		if (px == kx0 && py == ky0)
-		{
-			c0++;
-		}
-		else if (px == kx1 && py == ky1)
-		{
-			const int t = c1 + 1;
-			kx1 = kx0;
-			ky1 = ky0;
-			c1 = c0;
-			kx0 = px;
-			ky0 = py;
-			c0 = t;
-		}
-		else
-		{
-			if (c1) irs_count(a, win, kx1, ky1, c1);
-			kx1 = kx0;
-			ky1 = ky0;
-			c1 = c0;
-			kx0 = px;
-			ky0 = py;
-			c0 = 1;
-		}
-		got++;
-	}
-	if (c0) irs_count(a, win, kx0, ky0, c0);
-	if (c1) irs_count(a, win, kx1, ky1, c1);
-	if (PARITY) acc_flush<int, true>(a, par);
-	__syncthreads();
-	for (int k = threadIdx.x; k < IRS_WX * IRS_WY; k += IRS_THREADS)
-	{
-		const int v = win_counts[k];
-		if (v) atomicAdd(reinterpret_cast<int*>(a.map) + ((long long)(win.y0 + k / IRS_WX) * a.n1 + (win.x0 + k % IRS_WX)), v);
+		if (PARITY) __syncthreads();
 	}
 	// wave reduction, one 64-bit atomic per wave
 	for (int off = 32; off > 0; off >>= 1) got += __shfl_down(got, off);
@@ -1460,7 +1508,7 @@ __global__ void k_irs_positions(ShootArgs a, long long row, double* w, long long
 	double zx = lattice_at(a.x0, a.stepx, ok ? i : a.N1 - 1);
 	double zy = lattice_at(a.y0, a.stepy, row);
 	LeafCache cache;
-	Deflection d = deflect<PREC, false>(a, zx, zy, cache);
+	Deflection d = deflect<PREC, false, false>(a, kernarg_block(), zx, zy, cache);
 	if (!ok) return;
 	w[2 * i] = d.wx;
 	w[2 * i + 1] = d.wy;
@@ -1474,7 +1522,7 @@ __global__ void k_deflect_points(ShootArgs a, const double* z, int n, double* w,
 	bool ok = i < n;
 	double zx = ok ? z[2 * i] : 0, zy = ok ? z[2 * i + 1] : 0;
 	LeafCache cache;
-	Deflection d = deflect<PREC, MU>(a, zx, zy, cache);
+	Deflection d = deflect<PREC, MU, false>(a, kernarg_block(), zx, zy, cache);
 	if (!ok) return;
 	w[2 * i] = d.wx;
 	w[2 * i + 1] = d.wy;
@@ -1626,19 +1674,20 @@ ShootStats Engine::shoot_ipm(const LensParams& lens, const GridParams& g, Precis
 		if ((row1 - row0 + th - 1) / th > 65535) throw HipError("too many tiles of this height for one launch", __FILE__, __LINE__);
 		dim3 grid(unsigned(ntx), unsigned((row1 - row0 + th - 1) / th));
 		dim3 block(64 * IPM_WAVES);
+		// the instantiation for this precision, with or without parities, linear or general smooth matter
+		auto launch = [&](auto kernel) {
+			kernel<<<grid, block, 0, stream_>>>(a, row0, row1, MLENS_TABLE_ARGS(a), a.map, a.mmin, a.msad, a.span, a.span_sad, th);
+		};
+		const bool lin = a.smooth_linear != 0;
 		if (prec == PREC_FP64)
 		{
-			if (parities_) k_ipm_fast<PREC_FP64, true><<<grid, block, 0, stream_>>>(a, row0, row1, MLENS_TABLE_ARGS(a), a.map, a.mmin, a.msad,
-				a.span, a.span_sad, th);
-			else k_ipm_fast<PREC_FP64, false><<<grid, block, 0, stream_>>>(a, row0, row1, MLENS_TABLE_ARGS(a), a.map, a.mmin, a.msad,
-				a.span, a.span_sad, th);
+			if (parities_) launch(lin ? k_ipm_fast<PREC_FP64, true, true> : k_ipm_fast<PREC_FP64, true, false>);
+			else launch(lin ? k_ipm_fast<PREC_FP64, false, true> : k_ipm_fast<PREC_FP64, false, false>);
 		}
 		else
 		{
-			if (parities_) k_ipm_fast<PREC_MIXED, true><<<grid, block, 0, stream_>>>(a, row0, row1, MLENS_TABLE_ARGS(a), a.map, a.mmin, a.msad,
-				a.span, a.span_sad, th);
-			else k_ipm_fast<PREC_MIXED, false><<<grid, block, 0, stream_>>>(a, row0, row1, MLENS_TABLE_ARGS(a), a.map, a.mmin, a.msad,
-				a.span, a.span_sad, th);
+			if (parities_) launch(lin ? k_ipm_fast<PREC_MIXED, true, true> : k_ipm_fast<PREC_MIXED, true, false>);
+			else launch(lin ? k_ipm_fast<PREC_MIXED, false, true> : k_ipm_fast<PREC_MIXED, false, false>);
 		}
 		MLENS_HIP_CHECK(hipGetLastError());
 		fold_tiled_maps();
@@ -1674,15 +1723,19 @@ ShootStats Engine::shoot_irs(const LensParams& lens, const GridParams& g, Precis
 	if ((row1 - row0 + th - 1) / th > 65535) throw HipError("too many tiles of this height for one launch", __FILE__, __LINE__);
 	dim3 grid(unsigned(ntx), unsigned((row1 - row0 + th - 1) / th));
 	MLENS_HIP_CHECK(hipEventRecord(ev0_, stream_));
+	auto launch = [&](auto kernel) {
+		kernel<<<grid, IRS_THREADS, 0, stream_>>>(a, row0, row1, rec, MLENS_TABLE_ARGS(a), a.map, a.mmin, a.msad, th);
+	};
+	const bool lin = a.smooth_linear != 0;
 	if (prec == PREC_FP64)
 	{
-		if (parities_) k_irs_fast<PREC_FP64, true><<<grid, IRS_THREADS, 0, stream_>>>(a, row0, row1, rec, MLENS_TABLE_ARGS(a), a.map, a.mmin, a.msad, th);
-		else k_irs_fast<PREC_FP64, false><<<grid, IRS_THREADS, 0, stream_>>>(a, row0, row1, rec, MLENS_TABLE_ARGS(a), a.map, a.mmin, a.msad, th);
+		if (parities_) launch(lin ? k_irs_fast<PREC_FP64, true, true> : k_irs_fast<PREC_FP64, true, false>);
+		else launch(lin ? k_irs_fast<PREC_FP64, false, true> : k_irs_fast<PREC_FP64, false, false>);
 	}
 	else
 	{
-		if (parities_) k_irs_fast<PREC_MIXED, true><<<grid, IRS_THREADS, 0, stream_>>>(a, row0, row1, rec, MLENS_TABLE_ARGS(a), a.map, a.mmin, a.msad, th);
-		else k_irs_fast<PREC_MIXED, false><<<grid, IRS_THREADS, 0, stream_>>>(a, row0, row1, rec, MLENS_TABLE_ARGS(a), a.map, a.mmin, a.msad, th);
+		if (parities_) launch(lin ? k_irs_fast<PREC_MIXED, true, true> : k_irs_fast<PREC_MIXED, true, false>);
+		else launch(lin ? k_irs_fast<PREC_MIXED, false, true> : k_irs_fast<PREC_MIXED, false, false>);
 	}
 	MLENS_HIP_CHECK(hipGetLastError());
 	MLENS_HIP_CHECK(hipEventRecord(ev1_, stream_));
@@ -2054,7 +2107,10 @@ struct BatchShooter::Impl
 	void launch_shoot(int h, int blocks_per_cu, long long stride)
 	{
 		const unsigned blocks = unsigned(ncu * blocks_per_cu);
-		k_ipm_batch<<<blocks, 64 * IPM_BATCH_WAVES, 0, stream>>>(reinterpret_cast<const ShootArgs*>(d_args.ptr), d_start.ptr,
+		bool lin = true;
+		for (const ShootArgs& a : args) lin = lin && a.smooth_linear;
+		auto kernel = lin ? k_ipm_batch<true> : k_ipm_batch<false>;
+		kernel<<<blocks, 64 * IPM_BATCH_WAVES, 0, stream>>>(reinterpret_cast<const ShootArgs*>(d_args.ptr), d_start.ptr,
 			int(args.size()), h, total, stride, d_counter.ptr);
 		MLENS_HIP_CHECK(hipGetLastError());
 	}

@@ -108,43 +108,86 @@ __device__ __forceinline__ int find_node(const ShootArgs& a, double x, double y)
 	}
 }
 
+/* Leaf tables as constant memory: nothing writes them while a shooting kernel
+   runs, so reads at a wave-uniform index become scalar loads also where their
+   pointer came out of memory (the batch kernel's argument blocks), which the
+   compiler cannot tell from the maps it adds to. */
+template <typename T>
+using const_mem = const T __attribute__((address_space(4)))*;
+
+template <typename T>
+__device__ __forceinline__ const_mem<T> as_const(const T* p)
+{
+	return (const_mem<T>)(uintptr_t)p;
+}
+
+// a whole structure read that way
+template <typename T>
+__device__ __forceinline__ T load_const(const T* p)
+{
+	static_assert(sizeof(T) % 8 == 0, "read in words of eight bytes");
+	T v;
+	const auto q = as_const(reinterpret_cast<const unsigned long long*>(p));
+#pragma unroll
+	for (size_t i = 0; i < sizeof(T) / 8; i++) reinterpret_cast<unsigned long long*>(&v)[i] = q[i];
+	return v;
+}
+
 struct Deflection
 {
 	double wx, wy, mu;
 };
 
-/* lens equation at a leaf (leaf index L is wave-uniform) */
-template <int PREC, bool MU>
+/* lens equation at a leaf (leaf index L is wave-uniform). LIN: the smooth matter's deflection is
+   linear (the approximate circular sheet, folded into lin_x and lin_y), known at compile time: the
+   general sheet's logarithms and their constants then take no registers from the kernel. */
+template <int PREC, bool MU, bool LIN = false>
 __device__ __forceinline__ Deflection deflect_leaf(const ShootArgs& a, int L, double zx, double zy)
 {
-	const double* g = a.leaf_geom + 4 * (long long)L;
+	const auto g = as_const(a.leaf_geom + 4 * (long long)L);
 	const double cx = g[0], cy = g[1], ih = g[3];
-	const int packed = a.leaf_near_n[L];   // near stars (padded to 4) | FP32 entries to skip << 16
+	const int packed = *as_const(a.leaf_near_n + L);   // near stars (padded to 4) | FP32 entries to skip << 16
 	const int nn = packed & 0xffff;
 	const int p = a.p;
 	const double dzx = (zx - cx) * ih, dzy = (zy - cy) * ih;
 	double ax = 0, ay = 0, px = 0, py = 0;
+	double sx = 0, sy = 0, lx = 0, ly = 0;   // MU: sum m / (z - z_i)^2 and dP / d(dz)
 	if (PREC == PREC_FP64 || MU)
 	{
-		const double* s = a.near_d + (long long)L * MAX_NUM_STARS_DIRECT * 3;
+		const auto s = as_const(a.near_d + (long long)L * MAX_NUM_STARS_DIRECT * 3);
 		for (int k0 = 0; k0 < nn; k0 += 4)
 		{
 #pragma unroll
 			for (int k = k0; k < k0 + 4; k++)
 			{
 				double dx = zx - s[3 * k], dy = zy - s[3 * k + 1];
-				double f = s[3 * k + 2] * dev::rcp64(dx * dx + dy * dy);
+				double ir2 = dev::rcp64(dx * dx + dy * dy);
+				double f = s[3 * k + 2] * ir2;
 				ax = fma(f, dx, ax);
 				ay = fma(f, dy, ay);
+				if (MU)
+				{
+					// m / (z - z_i)^2 = m conj(d)^2 / |d|^4 from the reciprocal the deflection has taken
+					const double g = f * ir2;
+					sx = fma(g, fma(dx, dx, -dy * dy), sx);
+					sy = fma(g, -2 * dx * dy, sy);
+				}
 			}
 		}
 		const int SD = poly_stride_d(p);
-		const double* A = a.poly_d + (long long)L * SD * 2;
+		const auto A = as_const(a.poly_d + (long long)L * SD * 2);
 		for (int j0 = 0; j0 < SD; j0 += 4)
 		{
 #pragma unroll
 			for (int j = j0; j < j0 + 4; j++)
 			{
+				if (MU)
+				{
+					const double mx = fma(lx, dzx, fma(-ly, dzy, px));
+					const double my = fma(lx, dzy, fma(ly, dzx, py));
+					lx = mx;
+					ly = my;
+				}
 				double nx = fma(px, dzx, fma(-py, dzy, A[2 * j]));
 				double ny = fma(px, dzy, fma(py, dzx, A[2 * j + 1]));
 				px = nx;
@@ -156,16 +199,15 @@ __device__ __forceinline__ Deflection deflect_leaf(const ShootArgs& a, int L, do
 	{
 		// FP32 in leaf-relative coordinates; the leaf-constant term A_1 stays FP64
 		const float zrx = float(zx - cx), zry = float(zy - cy);
-		const float4* s = reinterpret_cast<const float4*>(a.near_f) + (long long)L * MAX_NUM_STARS_DIRECT;
+		const auto s = as_const(a.near_f + (long long)L * MAX_NUM_STARS_DIRECT * 4);
 		// The leaf's tables are read with scalar loads, and a wave waits for each batch before using it.
 		// Eight entries per trip instead of four halve those waits; the remainder of four (lists and
 		// polynomials are padded to fours) keeps the order of summation. Deflection alone on the
 		// 10000^2 map: 0.632 -> 0.610 s.
 		float fx = 0, fy = 0;
 		auto star = [&](int k) {
-			const float4 v = s[k];
-			const float dx = zrx - v.x, dy = zry - v.y;
-			const float f = v.z * dev::rcp32(dx * dx + dy * dy);
+			const float dx = zrx - s[4 * k], dy = zry - s[4 * k + 1];
+			const float f = s[4 * k + 2] * dev::rcp32(dx * dx + dy * dy);
 			fx = fmaf(f, dx, fx);
 			fy = fmaf(f, dy, fy);
 		};
@@ -184,7 +226,7 @@ __device__ __forceinline__ Deflection deflect_leaf(const ShootArgs& a, int L, do
 		ay = fy;
 		float qx = 0, qy = 0;
 		const int SF = poly_stride_f(p);
-		const float* A = a.poly_f + (long long)L * SF * 2;
+		const auto A = as_const(a.poly_f + (long long)L * SF * 2);
 		const float fdx = float(dzx), fdy = float(dzy);
 		auto term = [&](int j) {
 			const float nx = fmaf(qx, fdx, fmaf(-qy, fdy, A[2 * j]));
@@ -207,7 +249,7 @@ __device__ __forceinline__ Deflection deflect_leaf(const ShootArgs& a, int L, do
 		if (p >= 1)
 		{
 			const int SD = poly_stride_d(p);
-			const double* A1 = a.poly_d + ((long long)L * SD + SD - 1) * 2;   // A_1
+			const auto A1 = as_const(a.poly_d + ((long long)L * SD + SD - 1) * 2);   // A_1
 			px = A1[0] + (dzx * double(qx) - dzy * double(qy));
 			py = A1[1] + (dzx * double(qy) + dzy * double(qx));
 		}
@@ -216,7 +258,7 @@ __device__ __forceinline__ Deflection deflect_leaf(const ShootArgs& a, int L, do
 	d.wx = a.lin_x * zx - a.theta2 * ax - px;
 	d.wy = a.lin_y * zy - a.theta2 * ay + py;
 	d.mu = 0;
-	if (!a.smooth_linear)
+	if (!LIN && !a.smooth_linear)
 	{
 		dcx sm = dev::alpha_smooth(dcx{zx, zy}, a.kappastar, a.rectangular, a.approx, a.taylor_smooth, dcx{a.corner_re, a.corner_im});
 		d.wx -= sm.re;
@@ -224,39 +266,30 @@ __device__ __forceinline__ Deflection deflect_leaf(const ShootArgs& a, int L, do
 	}
 	if (MU)
 	{
-		// ipm_functions.cuh:67-82 with alpha_star.cuh:54-77 and alpha_local.cuh:51-69
-		const double* s = a.near_d + (long long)L * MAX_NUM_STARS_DIRECT * 3;
-		double sx = 0, sy = 0;   // sum m / (z - z_i)^2
-		for (int k = 0; k < nn; k++)
+		// ipm_functions.cuh:67-82 with alpha_star.cuh:54-77 and alpha_local.cuh:51-69. Both sums come
+		// from the deflection's own passes over the leaf's tables: a second pass took one division and
+		// one wait for a scalar load per star and order (IRS with parities, 1.6e9 rays: 118 ms with it).
+		if (isnan(sx) || isnan(sy))
 		{
-			double dx = zx - s[3 * k], dy = zy - s[3 * k + 1];
-			double r2 = dx * dx + dy * dy;
-			double ir4 = s[3 * k + 2] == 0 ? 0.0 : 1.0 / (r2 * r2);
-			double m = s[3 * k + 2];
-			sx += m * (dx * dx - dy * dy) * ir4;
-			sy += m * (-2 * dx * dy) * ir4;
+			// a point on a star: a massless one adds nothing
+			const auto s = as_const(a.near_d + (long long)L * MAX_NUM_STARS_DIRECT * 3);
+			sx = sy = 0;
+			for (int k = 0; k < nn; k++)
+			{
+				const double dx = zx - s[3 * k], dy = zy - s[3 * k + 1], m = s[3 * k + 2];
+				const double r2 = dx * dx + dy * dy, ir4 = m == 0 ? 0.0 : 1.0 / (r2 * r2);
+				sx += m * (dx * dx - dy * dy) * ir4;
+				sy += m * (-2 * dx * dy) * ir4;
+			}
 		}
 		// d alpha_star / d zbar = conj(-theta^2 * S)
 		double dsx = -a.theta2 * sx, dsy = a.theta2 * sy;
 		// d alpha_local / d zbar = conj( (1/h) dP/d(dz) ), P(dz) = sum_{i>=1} A_i dz^(i-1)
-		double lx = 0, ly = 0;
-		{
-			const int SD = poly_stride_d(p);
-			const double* A = a.poly_d + (long long)L * SD * 2;
-			for (int j = 0; j < SD - 1; j++)
-			{
-				double deg = double(SD - 1 - j);
-				double nx = lx * dzx - ly * dzy + deg * A[2 * j];
-				double ny = lx * dzy + ly * dzx + deg * A[2 * j + 1];
-				lx = nx;
-				ly = ny;
-			}
-			lx *= ih;
-			ly *= -ih;
-		}
-		double ddz;
-		dcx ddzb;
-		dev::d_alpha_smooth(dcx{zx, zy}, a.kappastar, a.rectangular, a.approx, a.taylor_smooth, dcx{a.corner_re, a.corner_im}, ddz, ddzb);
+		lx *= ih;
+		ly *= -ih;
+		double ddz = -a.kappastar;
+		dcx ddzb = {0, 0};
+		if (!LIN) dev::d_alpha_smooth(dcx{zx, zy}, a.kappastar, a.rectangular, a.approx, a.taylor_smooth, dcx{a.corner_re, a.corner_im}, ddz, ddzb);
 		double dwdz = (1 - a.kappa) - ddz;
 		double bx = a.gamma - dsx - lx - ddzb.re;
 		double by = -dsy - ly - ddzb.im;
@@ -269,7 +302,7 @@ __device__ __forceinline__ Deflection deflect_leaf(const ShootArgs& a, int L, do
 /* lens equation at a node that is not a leaf (a point outside the root box,
    tree_node.cuh:535-540): the node's own stars and neighbours' stars directly,
    plus its local expansion, all in FP64 */
-template <bool MU>
+template <bool MU, bool LIN = false>
 __device__ Deflection deflect_node(const ShootArgs& a, int node, double zx, double zy)
 {
 	double ax = 0, ay = 0, sx = 0, sy = 0;
@@ -312,7 +345,7 @@ __device__ Deflection deflect_node(const ShootArgs& a, int node, double zx, doub
 	d.wx = a.lin_x * zx - a.theta2 * ax - px;
 	d.wy = a.lin_y * zy - a.theta2 * ay + py;
 	d.mu = 0;
-	if (!a.smooth_linear)
+	if (!LIN && !a.smooth_linear)
 	{
 		dcx s = dev::alpha_smooth(dcx{zx, zy}, a.kappastar, a.rectangular, a.approx, a.taylor_smooth, dcx{a.corner_re, a.corner_im});
 		d.wx -= s.re;
@@ -330,9 +363,9 @@ __device__ Deflection deflect_node(const ShootArgs& a, int node, double zx, doub
 		lx *= a.theta2 / (h * h);
 		ly *= -a.theta2 / (h * h);
 		double dsx = -a.theta2 * sx, dsy = a.theta2 * sy;
-		double ddz;
-		dcx ddzb;
-		dev::d_alpha_smooth(dcx{zx, zy}, a.kappastar, a.rectangular, a.approx, a.taylor_smooth, dcx{a.corner_re, a.corner_im}, ddz, ddzb);
+		double ddz = -a.kappastar;
+		dcx ddzb = {0, 0};
+		if (!LIN) dev::d_alpha_smooth(dcx{zx, zy}, a.kappastar, a.rectangular, a.approx, a.taylor_smooth, dcx{a.corner_re, a.corner_im}, ddz, ddzb);
 		double dwdz = (1 - a.kappa) - ddz;
 		double bx = a.gamma - dsx - lx - ddzb.re;
 		double by = -dsy - ly - ddzb.im;
