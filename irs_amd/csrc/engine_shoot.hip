@@ -273,13 +273,12 @@ image of a demagnified region near a star then no longer stalls the other 63
 (those images are a tenth of the general triangles and four fifths of their
 pixels).
 */
-// Entries per wave: 100 (12.7 KB with the ring and the mark array) for the
-// single-map kernel, whose flushes then fill their passes better (10000^2 map:
-// 1.695 s against 1.710 s with 79); 79 (10.7 KB) for the persistent batch
-// kernel, whose 12 blocks per CU must all be resident at once (256 maps:
-// 1.664 s with 79 entries, 1.866 s with 100)
-constexpr int IPM_QCAP = 100;
-constexpr int IPM_BATCH_QCAP = 79;
+// Entries per wave: 74, with the ring and the mark array 10,176 bytes, so that 16 one-wave
+// blocks (four waves per SIMD) share a CU's 160 KB in the 1,280-byte granules LDS comes in.
+// A larger queue fills the passes of a flush better but costs waves: the 10000^2 map at four
+// rays a pixel took 1.145 s with 100 entries (12 blocks), 1.130 s with 88 (14) and 1.126 s
+// with 74; 24 batched maps 8.1 ms with 79 entries at 12 blocks, 7.2 ms with 74 at 16.
+constexpr int IPM_QCAP = 74;
 
 template <int CAP>
 struct TriQueue
@@ -749,16 +748,20 @@ constexpr int IPM_WAVES = 1;
 constexpr int IPM_TILE_W = 63 * IPM_WAVES;
 constexpr int IPM_BATCH_WAVES = 1;
 constexpr int IPM_BATCH_TILE_W = 63 * IPM_BATCH_WAVES;
-constexpr int IPM_RESIDENT_WAVES_PER_CU = 12;   // 3 per SIMD: up to 168 VGPRs and a 12.7 KB wave queue
-constexpr int IPM_TILE_H = 64;       // lattice rows a wave walks: the shortest tile
+constexpr int IPM_RESIDENT_WAVES_PER_CU = 16;   // four per SIMD: up to 128 VGPRs and a 10 KB wave queue
+constexpr int IPM_TILE_H = 8;         // lattice rows a wave walks: the shortest tile
 constexpr int IPM_TILE_H_MAX = 1024;  // and the tallest
 
 /* Rows per tile for a launch of ntx tile columns over `rows` lattice rows: the
    tallest power of two in [IPM_TILE_H, IPM_TILE_H_MAX] that still gives at
    least eight blocks per resident block slot. A tall tile deflects
    its first row once per 1024 rows instead of once per 64 and flushes its
-   queue less often (10000^2 map: 2.475 s at 64 rows, 2.428 s at 1024); a short
-   one keeps a small lattice spread over the whole device. */
+   queue less often (10000^2 map: 2.475 s at 64 rows, 2.428 s at 1024). A short
+   one keeps a small lattice spread over the whole device and its longest tile
+   short: the demagnified images around one star are the work of thousands of
+   other cells, and the launch ends with the tile that holds them. A 256^2 map
+   (2048 x 6144 cells) took 2.24 ms at 64 rows, 1.08 ms at 16, 0.64 ms at 8 and
+   the same at 4 or 2; a 1000^2 map (4288 x 10716) 6.1, 3.4, 3.3 and 3.3 ms. */
 static inline int ipm_tile_rows(long long ntx, long long rows, int num_cus)
 {
 	const long long want = 8LL * (IPM_RESIDENT_WAVES_PER_CU / IPM_WAVES) * (num_cus > 0 ? num_cus : 256);
@@ -826,13 +829,10 @@ __device__ __forceinline__ void ipm_tile(const ShootArgs& a, const ShootArgs* co
 }
 
 // Compiled for linear smooth matter (LIN) the kernel needs 114 VGPRs and spills no scalar
-// register; with the general sheet's code in it, 136 VGPRs hold 130 spilled scalars as well.
-// Three waves per SIMD, and 12.7 KB of LDS per wave for a 100-entry queue and a 128-slot merge table. Four waves (128 VGPRs, about 25
-// spilled) ran as fast with a 64-slot table and a 79-entry queue, the most that
-// fit in 10 KB, and gained nothing from a larger table (10000^2 map: 1.698 s at
-// three waves against 1.745 s at four)
+// register: four waves per SIMD. With the general sheet's code in it, 136 VGPRs hold 130
+// spilled scalars as well, and it runs at three.
 template <int PREC, bool PARITY, bool LIN>
-__global__ __launch_bounds__(64 * IPM_WAVES, 3) void k_ipm_fast(ShootArgs a, long long row0, long long row1,
+__global__ __launch_bounds__(64 * IPM_WAVES, LIN ? 4 : 3) void k_ipm_fast(ShootArgs a, long long row0, long long row1,
 	MLENS_TABLE_PARAMS, void* __restrict__ map, void* __restrict__ mmin, void* __restrict__ msad,
 	void* __restrict__ span, void* __restrict__ span_sad, int tile_h)
 {
@@ -940,7 +940,10 @@ long long Engine::window_cells(const LensParams& lens, const GridParams& g, int 
 /* ---------------------------------------------------------------------------
 Many maps in one launch. A persistent grid takes (instance, tile) work items
 from a global counter: item t covers tile t * stride of the concatenation of
-every instance's tiles (stride > 1 samples the batch for the autotuner). The
+every instance's tiles (stride > 1 samples the batch for the autotuner). Tiles
+from `whole` on are handed out in pieces of BATCH_PIECE_H rows: a tile that
+holds a star takes several times the average one, and whole tiles at the end
+leave the device waiting for the last of them. The
 instance of a tile comes from a binary search over the running tile counts;
 its arguments, including its own tables and map, are read from device memory.
 --------------------------------------------------------------------------- */
@@ -954,24 +957,38 @@ struct BatchMap
 	int n1, n2, tiles_x;
 };
 
-// Three waves per SIMD: the batch's maps of 0.25-16 MB stay in the caches. Blocks take tiles
+// Four waves per SIMD (three with general smooth matter). Blocks take tiles
 // from a global counter and never wait for each other. The instance's arguments and, through
 // them, its leaf tables come in by scalar loads; read as ordinary memory, which the maps'
 // atomics might change, they took 24 maps of 256-512 pixels from 8.1 to 10.6 ms. LIN: every
 // instance's smooth matter is linear (117 VGPRs against 139).
+constexpr int BATCH_PIECE_H = 8;        // rows of a piece, as the shortest tile of a single map
+// tiles per resident block that go out in pieces (24 maps of 256-512 pixels, tiles of 64 rows,
+// 12 blocks per CU: 9.0 ms with none, 8.2 with two, 7.8 with four, 8.1 with eight)
+constexpr int BATCH_WHOLE_ROUNDS = 4;
+
 template <bool LIN>
-__global__ __launch_bounds__(64 * IPM_BATCH_WAVES, 3) void k_ipm_batch(const ShootArgs* __restrict__ args,
-	const long long* __restrict__ tile_start, int ninst, int tile_h, long long total, long long stride,
+__global__ __launch_bounds__(64 * IPM_BATCH_WAVES, LIN ? 4 : 3) void k_ipm_batch(const ShootArgs* __restrict__ args,
+	const long long* __restrict__ tile_start, int ninst, int tile_h, long long total, long long stride, long long whole,
 	unsigned long long* __restrict__ counter)
 {
-	__shared__ TriQueue<IPM_BATCH_QCAP> queues[IPM_BATCH_WAVES];
+	__shared__ TriQueue<IPM_QCAP> queues[IPM_BATCH_WAVES];
 	__shared__ long long next;
 	for (;;)
 	{
 		__syncthreads();   // every thread has read the previous item
 		if (threadIdx.x == 0) next = (long long)atomicAdd(counter, 1ull) * stride;
 		__syncthreads();
-		const long long t = next;
+		long long t = next;
+		int piece = 0, rows = tile_h;
+		if (t >= whole)
+		{
+			const int pieces = (tile_h + BATCH_PIECE_H - 1) / BATCH_PIECE_H;
+			const long long k = (t - whole) / pieces;
+			piece = int(t - whole - k * pieces);
+			rows = BATCH_PIECE_H;
+			t = whole + k;
+		}
 		if (t >= total) break;
 		int lo = 0, hi = ninst - 1;
 		while (lo < hi)
@@ -988,7 +1005,9 @@ __global__ __launch_bounds__(64 * IPM_BATCH_WAVES, 3) void k_ipm_batch(const Sho
 		const long long local = t - tile_start[lo];
 		const long long ntx = (a.N1 + IPM_BATCH_TILE_W - 1) / IPM_BATCH_TILE_W;
 		const long long ty = local / ntx, tx = local - ty * ntx;
-		const long long J0 = ty * tile_h, J1 = min(J0 + (long long)tile_h, a.N2);
+		const long long J0 = ty * tile_h + piece * BATCH_PIECE_H;
+		const long long J1 = min(min(J0 + (long long)rows, (ty + 1) * tile_h), a.N2);
+		if (J0 >= J1) continue;
 		ipm_tile<PREC_MIXED, false, true, IPM_BATCH_WAVES, LIN>(a, args + lo, queues[threadIdx.x >> 6], tx, J0, J1);
 	}
 }
@@ -2050,7 +2069,7 @@ struct BatchShooter::Impl
 	std::vector<long long> tiles_x;   // per instance: column tiles
 	std::vector<std::unique_ptr<DeviceBuffer<char>>> tiled;   // per instance: tiled accumulation and span maps
 	bool dirty = true;
-	int tile_h = IPM_TILE_H, bpc = 12, ncu = 0;
+	int tile_h = 64, bpc = 12, ncu = 0;
 	double tune_ms = 0;
 	bool tuned = false;
 	hipStream_t stream = nullptr;
@@ -2109,9 +2128,11 @@ struct BatchShooter::Impl
 		const unsigned blocks = unsigned(ncu * blocks_per_cu);
 		bool lin = true;
 		for (const ShootArgs& a : args) lin = lin && a.smooth_linear;
+		// a sampled launch takes whole tiles only, and its stride leaves the last ones out
+		const long long whole = stride > 1 ? total : std::max(0LL, total - (long long)BATCH_WHOLE_ROUNDS * blocks);
 		auto kernel = lin ? k_ipm_batch<true> : k_ipm_batch<false>;
 		kernel<<<blocks, 64 * IPM_BATCH_WAVES, 0, stream>>>(reinterpret_cast<const ShootArgs*>(d_args.ptr), d_start.ptr,
-			int(args.size()), h, total, stride, d_counter.ptr);
+			int(args.size()), h, total, stride, whole, d_counter.ptr);
 		MLENS_HIP_CHECK(hipGetLastError());
 	}
 
@@ -2143,8 +2164,8 @@ struct BatchShooter::Impl
 	{
 		// about an eighth of the tiles, spread over every instance
 		const long long stride = 8;
-		const int heights[3] = {32, 64, 128};
-		const int resident[3] = {8, 10, 12};   // one-wave blocks; 12 fill a CU at 3 waves per SIMD
+		const int heights[3] = {16, 32, 64};
+		const int resident[3] = {10, 13, 16};   // one-wave blocks; 16 fill a CU at 4 waves per SIMD
 		float best = -1;
 		auto t0 = std::chrono::steady_clock::now();
 		for (int h : heights)

@@ -82,7 +82,7 @@ class IPMBatch:
 
     def set_tuning(self, tile_h, blocks_per_cu):
         """Use these tiles instead of autotuning: tile_h lattice rows per tile and
-        blocks_per_cu resident blocks of one wave each per CU (12 fill a CU)."""
+        blocks_per_cu resident blocks of one wave each per CU (16 fill a CU)."""
         if not self.lib.ipm_batch_set_tuning(self.obj, int(tile_h), int(blocks_per_cu)):
             raise ValueError("invalid batch tuning")
 

@@ -43,3 +43,37 @@ def test_irs_parity_windows(oracle, rect, tmp_path):
         for got, want in zip((m.num_rays, m.num_rays_minima, m.num_rays_saddles), ref):
             assert np.abs(got.astype(np.int64) - want).sum() <= 2
         m.close()
+
+
+@pytest.mark.parametrize("general", [False, True])
+def test_batch_tiles_and_pieces(general):
+    """The last tiles of a batch go out in pieces of eight rows: tile heights below
+    a piece, one piece, and with a remainder, at few and many resident blocks, for
+    batches of linear smooth matter and with one general instance, against the
+    instances' single maps (FP32 summation order only, the bound of the batched
+    parity test)."""
+    from irs_amd.microlensing.IPM.batch import IPMBatch, draw_instances
+    from irs_amd.microlensing.IPM.ipm import IPM
+    params = draw_instances(3, seed=5, sides=(64, 96), star_range=(1.5e3, 3.0e3), num_rays_y=3)
+    if general:
+        params[1]["rectangular"] = True
+    objs, refs = [], []
+    for p in params:
+        m = IPM(**p)
+        m.run()
+        refs.append(m.magnifications.astype(np.float64))
+        objs.append(m)
+    for tile_h, blocks in ((1, 1), (8, 16), (20, 12), (63, 2), (300, 16)):
+        say(f"[batch pieces] general {general}, tile_h {tile_h}, blocks/CU {blocks}")
+        batch = IPMBatch()
+        batch.set_tuning(tile_h, blocks)
+        for m in objs:
+            batch.add(m)
+        h = batch.run()
+        for m, ref, counts in zip(objs, refs, h):
+            e = np.abs(m.magnifications - ref) / np.maximum(ref, 1e-3 * ref.max())
+            assert np.max(e) < 2e-5
+            assert counts.sum() == ref.size
+        batch.close()
+    for m in objs:
+        m.close()
