@@ -168,7 +168,7 @@ private:
 	void ensure_node_capacity(int n);
 	void build_leaf_tables(const LensParams& lens);
 	void m2l_prepare(int p, bool f32);
-	void m2l_level(int lev, int p, bool f32, hipEvent_t e0, hipEvent_t e1);
+	void m2l_all(int p, bool f32);
 
 	hipStream_t stream_ = nullptr;
 	int num_cus_ = 0;   // compute units of the current device
@@ -179,6 +179,7 @@ private:
 	int nstars_ = 0;
 	DeviceBuffer<double> sx_, sy_, sm_, tx_, ty_, tm_;
 	DeviceBuffer<int> star_node_, star_node_tmp_;
+	DeviceBuffer<int> node_flag_, node_rank_, level_count_;   // of the level being split
 
 	int levels_ = 0;
 	int num_nodes_ = 0;
@@ -192,8 +193,7 @@ private:
 	DeviceBuffer<double> binom_;
 	DeviceBuffer<double> mult_, local_;   // interleaved re, im
 
-	// MFMA M2L: the 40 offset matrices (real-stacked, transposed, padded),
-	// per-level source tables and real-stacked multipoles
+	// MFMA M2L: the 40 offset matrices (real-stacked, transposed, padded)
 	int m2l_mode_ = M2L_DIRECT;
 	double m2l_ms_ = 0;
 	long long m2l_pairs_ = 0;
@@ -202,13 +202,10 @@ private:
 	bool m2l_ready_f32_ = false;
 	DeviceBuffer<float> m2l_af_;
 	DeviceBuffer<double> m2l_ad_;
-	DeviceBuffer<int> m2l_src_;
-	DeviceBuffer<float> mstack_f_;
-	DeviceBuffer<double> mstack_d_;
 	DeviceBuffer<unsigned long long> m2l_count_;
-	std::vector<hipEvent_t> m2l_ev_;
+	hipEvent_t m2l_ev0_ = nullptr, m2l_ev1_ = nullptr;
 
-	int num_leaves_ = 0;
+	int num_leaves_ = 0;   // entries of the leaf tables: one per node, those of inner nodes empty
 	DeviceBuffer<int> leaf_of_node_;
 	DeviceBuffer<double> leaf_geom_;      // cx, cy, hl, 1/hl per leaf
 	DeviceBuffer<int> leaf_near_n_;       // padded to a multiple of 4; FP32 polynomial entries to skip << 16

@@ -56,7 +56,8 @@ Engine::~Engine()
 	if (stream_) (void)hipStreamSynchronize(stream_);
 	if (ev0_) (void)hipEventDestroy(ev0_);
 	if (ev1_) (void)hipEventDestroy(ev1_);
-	for (hipEvent_t e : m2l_ev_) (void)hipEventDestroy(e);
+	if (m2l_ev0_) (void)hipEventDestroy(m2l_ev0_);
+	if (m2l_ev1_) (void)hipEventDestroy(m2l_ev1_);
 	if (stream_) (void)hipStreamDestroy(stream_);
 }
 
@@ -293,50 +294,211 @@ __device__ __forceinline__ int quadrant(double x, double y, double cx, double cy
 	return (x < cx) ? 2 : 3;
 }
 
-// tree_node.cuh:321-345: stars in a node plus its neighbours decide subdivision
-__global__ void k_near_count(TreeView t, int l0, int l1, I4* flags, int* maxcnt)
+// what the host reads after each level: nodes that split, and the stars of the largest of them
+struct LevelCount
 {
-	int i = l0 + blockIdx.x * blockDim.x + threadIdx.x;
-	if (i >= l1) return;
-	int c = t.count[i];
-	for (int j = 0; j < t.nnbr[i]; j++) c += t.count[t.nbr[8 * i + j]];
-	flags[i - l0] = I4{c > MAX_NUM_STARS_DIRECT ? 1 : 0, 0, 0, 0};
-	atomicMax(maxcnt, c);
+	int split, largest;
+};
+
+// The root (ipm.cuh:746-773): it splits when it holds more stars than a leaf may sum directly
+// (tree_node.cuh:321-345).
+__global__ void k_make_root(TreeView t, double half_length, int n, int* flags, int* rank, LevelCount* counts)
+{
+	t.cx[0] = 0;
+	t.cy[0] = 0;
+	t.hl[0] = half_length;
+	t.level[0] = 0;
+	t.parent[0] = -1;
+	t.child0[0] = -1;
+	t.begin[0] = 0;
+	t.count[0] = n;
+	t.nnbr[0] = 0;
+	t.nm2l[0] = 0;
+	t.np2l[0] = 0;
+	flags[0] = n > MAX_NUM_STARS_DIRECT ? 1 : 0;
+	rank[0] = 0;
+	counts->split = flags[0];
+	counts->largest = n;
 }
 
-// tree_node.cuh:151-177: four children, offsets (+,+), (-,+), (-,-), (+,-)
-__global__ void k_make_children(TreeView t, int l0, int l1, const I4* flags, const I4* rank, int base)
+// rank[i] = nodes before i that split; one block, for levels of at most RANK_MAX nodes. Clears
+// nothing: k_set_neighbors left the largest count in counts.
+constexpr int RANK_THREADS = 1024;
+constexpr int RANK_MAX = 32768;
+
+__global__ __launch_bounds__(RANK_THREADS) void k_rank(const int* __restrict__ flags, int* __restrict__ rank, int nl, LevelCount* counts)
 {
-	int i = l0 + blockIdx.x * blockDim.x + threadIdx.x;
-	if (i >= l1 || !flags[i - l0].x) return;
-	int c0 = base + 4 * rank[i - l0].x;
-	t.child0[i] = c0;
-	double nh = t.hl[i] / 2;
-	const double ox[4] = {1, -1, -1, 1};
-	const double oy[4] = {1, 1, -1, -1};
-	for (int q = 0; q < 4; q++)
+	__shared__ int part[RANK_THREADS / 64];
+	const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+	int carry = 0;
+	for (int base = 0; base < nl; base += RANK_THREADS)
 	{
-		int c = c0 + q;
-		t.cx[c] = t.cx[i] + nh * ox[q];
-		t.cy[c] = t.cy[i] + nh * oy[q];
-		t.hl[c] = nh;
-		t.level[c] = t.level[i] + 1;
-		t.parent[c] = i;
-		t.child0[c] = -1;
-		t.nnbr[c] = 0;
-		t.nm2l[c] = 0;
-		t.np2l[c] = 0;
+		const int i = base + threadIdx.x;
+		const int f = i < nl ? flags[i] : 0;
+		const unsigned long long m = __ballot(f);
+		if (lane == 0) part[wave] = __popcll(m);
+		__syncthreads();
+		int before = carry;
+		for (int w = 0; w < RANK_THREADS / 64; w++)
+		{
+			if (w < wave) before += part[w];
+			carry += part[w];
+		}
+		if (i < nl) rank[i] = before + int(__popcll(m & ((1ull << lane) - 1)));
+		__syncthreads();
+	}
+	if (threadIdx.x == 0) counts->split = carry;
+}
+
+__global__ void k_flags_to_i4(const int* flags, I4* out, int nl)
+{
+	const int i = blockIdx.x * blockDim.x + threadIdx.x;
+	if (i < nl) out[i] = I4{flags[i], 0, 0, 0};
+}
+
+__global__ void k_i4_to_rank(const I4* in, int* rank, int nl, LevelCount* counts)
+{
+	const int i = blockIdx.x * blockDim.x + threadIdx.x;
+	if (i < nl) rank[i] = in[i].x;
+	if (i == nl) counts->split = in[nl].x;
+}
+
+// child q of node i (tree_node.cuh:151-177: offsets (+,+), (-,+), (-,-), (+,-))
+__device__ __forceinline__ void make_child(TreeView t, int i, int c0, int q)
+{
+	const double nh = t.hl[i] / 2;
+	const double ox = (q == 0 || q == 3) ? 1 : -1, oy = q < 2 ? 1 : -1;
+	const int c = c0 + q;
+	t.cx[c] = t.cx[i] + nh * ox;
+	t.cy[c] = t.cy[i] + nh * oy;
+	t.hl[c] = nh;
+	t.level[c] = t.level[i] + 1;
+	t.parent[c] = i;
+	t.child0[c] = -1;
+}
+
+/*
+A level's splits, one block per node: its four children, and a stable partition of its stars into
+them (sort_stars_kernel, tree_node.cuh:392-501) by way of the scratch arrays. One launch per level
+where the device-wide partition below takes seven; that one is kept for nodes of more than
+SPLIT_MAX stars, whose passes a single block would walk alone.
+*/
+constexpr int SPLIT_MAX = 16384;
+
+template <int THREADS>
+__global__ __launch_bounds__(THREADS) void k_split_nodes(TreeView t, int l0, const int* __restrict__ flags, const int* __restrict__ rank,
+	int base, double* sx, double* sy, double* sm, double* tx, double* ty, double* tm)
+{
+	constexpr int WAVES = THREADS / 64;
+	__shared__ int part[4][WAVES];
+	const int i = l0 + blockIdx.x;
+	if (!flags[blockIdx.x]) return;
+	const int c0 = base + 4 * rank[blockIdx.x];
+	const int b = t.begin[i], n = t.count[i];
+	const double cx = t.cx[i], cy = t.cy[i];
+	const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+	// quadrant sizes
+	int mine[4] = {0, 0, 0, 0};
+	for (int s = threadIdx.x; s < n; s += THREADS)
+	{
+		const int q = quadrant(sx[b + s], sy[b + s], cx, cy);
+#pragma unroll
+		for (int k = 0; k < 4; k++) mine[k] += q == k;
+	}
+#pragma unroll
+	for (int k = 0; k < 4; k++)
+	{
+		for (int off = 32; off > 0; off >>= 1) mine[k] += __shfl_xor(mine[k], off);
+		if (lane == 0) part[k][wave] = mine[k];
+	}
+	__syncthreads();
+	int start[4], total = 0;
+#pragma unroll
+	for (int k = 0; k < 4; k++)
+	{
+		int c = 0;
+		for (int w = 0; w < WAVES; w++) c += part[k][w];
+		start[k] = b + total;
+		total += c;
+		mine[k] = c;
+	}
+	if (threadIdx.x == 0) t.child0[i] = c0;
+	if (threadIdx.x < 4)
+	{
+		const int q = threadIdx.x;
+		make_child(t, i, c0, q);
+		t.begin[c0 + q] = q == 0 ? start[0] : (q == 1 ? start[1] : (q == 2 ? start[2] : start[3]));
+		t.count[c0 + q] = q == 0 ? mine[0] : (q == 1 ? mine[1] : (q == 2 ? mine[2] : mine[3]));
+	}
+	// stable placement, THREADS stars at a time
+	for (int s0 = 0; s0 < n; s0 += THREADS)
+	{
+		__syncthreads();
+		const int s = s0 + threadIdx.x;
+		double x = 0, y = 0, m = 0;
+		int q = 4;
+		if (s < n)
+		{
+			x = sx[b + s];
+			y = sy[b + s];
+			m = sm[b + s];
+			q = quadrant(x, y, cx, cy);
+		}
+		int before = 0;
+#pragma unroll
+		for (int k = 0; k < 4; k++)
+		{
+			const unsigned long long mk = __ballot(q == k);
+			if (lane == 0) part[k][wave] = __popcll(mk);
+			if (q == k) before = __popcll(mk & ((1ull << lane) - 1));
+		}
+		__syncthreads();
+#pragma unroll
+		for (int k = 0; k < 4; k++)
+		{
+			int all = 0, ahead = 0;
+			for (int w = 0; w < WAVES; w++)
+			{
+				if (w < wave) ahead += part[k][w];
+				all += part[k][w];
+			}
+			if (q == k)
+			{
+				const int dst = start[k] + ahead + before;
+				tx[dst] = x;
+				ty[dst] = y;
+				tm[dst] = m;
+			}
+			start[k] += all;
+		}
+	}
+	__syncthreads();
+	for (int s = threadIdx.x; s < n; s += THREADS)
+	{
+		sx[b + s] = tx[b + s];
+		sy[b + s] = ty[b + s];
+		sm[b + s] = tm[b + s];
 	}
 }
 
+// the device-wide partition of a level (k_split_nodes takes the levels whose nodes are small)
+__global__ void k_make_children(TreeView t, int l0, int l1, const int* flags, const int* rank, int base)
+{
+	int i = l0 + blockIdx.x * blockDim.x + threadIdx.x;
+	if (i >= l1 || !flags[i - l0]) return;
+	int c0 = base + 4 * rank[i - l0];
+	t.child0[i] = c0;
+	for (int q = 0; q < 4; q++) make_child(t, i, c0, q);
+}
+
 __global__ void k_star_onehot(TreeView t, const double* sx, const double* sy, const int* star_node, int l0,
-	const I4* flags, I4* onehot, int n)
+	const int* flags, I4* onehot, int n)
 {
 	int s = blockIdx.x * blockDim.x + threadIdx.x;
 	if (s >= n) return;
 	int node = star_node[s];
 	I4 v{0, 0, 0, 0};
-	if (node >= 0 && flags[node - l0].x)
+	if (node >= 0 && flags[node - l0])
 	{
 		int q = quadrant(sx[s], sy[s], t.cx[node], t.cy[node]);
 		v.x = q == 0;
@@ -347,10 +509,10 @@ __global__ void k_star_onehot(TreeView t, const double* sx, const double* sy, co
 	onehot[s] = v;
 }
 
-__global__ void k_child_ranges(TreeView t, int l0, int l1, const I4* flags, const I4* pre)
+__global__ void k_child_ranges(TreeView t, int l0, int l1, const int* flags, const I4* pre)
 {
 	int i = l0 + blockIdx.x * blockDim.x + threadIdx.x;
-	if (i >= l1 || !flags[i - l0].x) return;
+	if (i >= l1 || !flags[i - l0]) return;
 	int b = t.begin[i];
 	I4 c = pre[b + t.count[i]] - pre[b];
 	int c0 = t.child0[i];
@@ -366,12 +528,12 @@ __global__ void k_child_ranges(TreeView t, int l0, int l1, const I4* flags, cons
 
 // stable partition of each split node's stars into its four children (sort_stars_kernel, tree_node.cuh:392-501)
 __global__ void k_star_scatter(TreeView t, const double* sx, const double* sy, const double* sm, double* tx, double* ty,
-	double* tm, const int* star_node, int* star_node_out, int l0, const I4* flags, const I4* pre, int n)
+	double* tm, const int* star_node, int* star_node_out, int l0, const int* flags, const I4* pre, int n)
 {
 	int s = blockIdx.x * blockDim.x + threadIdx.x;
 	if (s >= n) return;
 	int node = star_node[s];
-	if (node >= 0 && flags[node - l0].x)
+	if (node >= 0 && flags[node - l0])
 	{
 		int q = quadrant(sx[s], sy[s], t.cx[node], t.cy[node]);
 		int b = t.begin[node];
@@ -392,49 +554,69 @@ __global__ void k_star_scatter(TreeView t, const double* sx, const double* sy, c
 	}
 }
 
-// tree_node.cuh:183-267
-__global__ void k_set_neighbors(TreeView t, int n0, int n1)
+/*
+The lists of a level's nodes (tree_node.cuh:183-267) and the nodes that split next (the stars of a
+node and its neighbours, 321-345). One wave per node, one candidate per lane: the four siblings, then
+the four children of each neighbour of the parent (or that neighbour itself, where it is a leaf), in
+the order the lists keep. A lane's place in its list is the number of lanes before it that chose the
+same list. Walked by one lane per node, the candidates' dependent loads took 17 us a level.
+*/
+__global__ __launch_bounds__(256) void k_set_neighbors(TreeView t, int n0, int n1, int* flags, LevelCount* counts)
 {
-	int i = n0 + blockIdx.x * blockDim.x + threadIdx.x;
+	const int i = n0 + blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
 	if (i >= n1) return;
-	int par = t.parent[i];
-	double cx = t.cx[i], cy = t.cy[i], h = t.hl[i];
-	int nn = 0, nm = 0, np = 0;
-	int pc0 = t.child0[par];
-	for (int q = 0; q < 4; q++)
+	const int par = t.parent[i];
+	const double cx = t.cx[i], cy = t.cy[i], h = t.hl[i];
+	enum
 	{
-		int c = pc0 + q;
-		if (t.count[c] == 0 || c == i) continue;
-		t.nbr[8 * i + nn++] = c;
+		NONE,
+		NEAR,
+		M2L,
+		P2L
+	};
+	int kind = NONE, c = -1, count = 0;
+	if (lane < 4)
+	{
+		c = t.child0[par] + lane;
+		count = t.count[c];
+		if (count != 0 && c != i) kind = NEAR;
 	}
-	for (int j = 0; j < t.nnbr[par]; j++)
+	else if (lane < 4 + 4 * MAX_NUM_NEIGHBORS)
 	{
-		int nb = t.nbr[8 * par + j];
-		if (t.count[nb] == 0) continue;
-		if (t.child0[nb] < 0)
+		const int j = (lane - 4) >> 2, q = lane & 3;
+		if (j < t.nnbr[par])
 		{
-			if (fabs(t.cx[nb] - cx) < 3.5 * h && fabs(t.cy[nb] - cy) < 3.5 * h)
-				t.nbr[8 * i + nn++] = nb;
-			else
-				t.p2l[5 * i + np++] = nb;
-		}
-		else
-		{
-			int c0 = t.child0[nb];
-			for (int q = 0; q < 4; q++)
+			const int nb = t.nbr[8 * par + j];
+			const int c0 = t.child0[nb];
+			const bool leaf = c0 < 0;
+			c = leaf ? nb : c0 + q;
+			count = t.count[c];
+			if (leaf)
 			{
-				int c = c0 + q;
-				if (t.count[c] == 0) continue;
-				if (fabs(t.cx[c] - cx) < 3 * h && fabs(t.cy[c] - cy) < 3 * h)
-					t.nbr[8 * i + nn++] = c;
-				else
-					t.m2l[27 * i + nm++] = c;
+				if (q == 0 && count != 0) kind = (fabs(t.cx[c] - cx) < 3.5 * h && fabs(t.cy[c] - cy) < 3.5 * h) ? NEAR : P2L;
 			}
+			else if (count != 0)
+				kind = (fabs(t.cx[c] - cx) < 3 * h && fabs(t.cy[c] - cy) < 3 * h) ? NEAR : M2L;
 		}
 	}
-	t.nnbr[i] = nn;
-	t.nm2l[i] = nm;
-	t.np2l[i] = np;
+	const unsigned long long below = (1ull << lane) - 1;
+	const unsigned long long near = __ballot(kind == NEAR), m2l = __ballot(kind == M2L), p2l = __ballot(kind == P2L);
+	if (kind == NEAR) t.nbr[8 * (long long)i + __popcll(near & below)] = c;
+	if (kind == M2L) t.m2l[27 * (long long)i + __popcll(m2l & below)] = c;
+	if (kind == P2L) t.p2l[5 * (long long)i + __popcll(p2l & below)] = c;
+	int stars = kind == NEAR ? count : 0;
+	for (int off = 32; off > 0; off >>= 1) stars += __shfl_xor(stars, off);
+	if (lane == 0)
+	{
+		t.nnbr[i] = __popcll(near);
+		t.nm2l[i] = __popcll(m2l);
+		t.np2l[i] = __popcll(p2l);
+		const int own = t.count[i];
+		const bool split = stars + own > MAX_NUM_STARS_DIRECT;
+		flags[i - n0] = split;
+		// few nodes raise the maximum: most need no atomic on the one address
+		if (split && own > *static_cast<volatile int*>(&counts->largest)) atomicMax(&counts->largest, own);
+	}
 }
 
 template <typename T>
@@ -486,88 +668,95 @@ void Engine::build_tree(double root_half_length)
 	level_start_.assign({0, 1});
 	levels_ = 0;
 
-	// root (ipm.cuh:746-773)
-	{
-		double g[3] = {0.0, 0.0, root_half_length};
-		int iv[11] = {0, -1, -1, 0, n, 0, 0, 0};
-		MLENS_HIP_CHECK(hipMemcpy(ncx_.ptr, &g[0], sizeof(double), hipMemcpyHostToDevice));
-		MLENS_HIP_CHECK(hipMemcpy(ncy_.ptr, &g[1], sizeof(double), hipMemcpyHostToDevice));
-		MLENS_HIP_CHECK(hipMemcpy(nhl_.ptr, &g[2], sizeof(double), hipMemcpyHostToDevice));
-		MLENS_HIP_CHECK(hipMemcpy(nlevel_.ptr, &iv[0], sizeof(int), hipMemcpyHostToDevice));
-		MLENS_HIP_CHECK(hipMemcpy(nparent_.ptr, &iv[1], sizeof(int), hipMemcpyHostToDevice));
-		MLENS_HIP_CHECK(hipMemcpy(nchild0_.ptr, &iv[2], sizeof(int), hipMemcpyHostToDevice));
-		MLENS_HIP_CHECK(hipMemcpy(nbegin_.ptr, &iv[3], sizeof(int), hipMemcpyHostToDevice));
-		MLENS_HIP_CHECK(hipMemcpy(ncount_.ptr, &iv[4], sizeof(int), hipMemcpyHostToDevice));
-		MLENS_HIP_CHECK(hipMemcpy(nnnbr_.ptr, &iv[5], sizeof(int), hipMemcpyHostToDevice));
-		MLENS_HIP_CHECK(hipMemcpy(nnm2l_.ptr, &iv[6], sizeof(int), hipMemcpyHostToDevice));
-		MLENS_HIP_CHECK(hipMemcpy(nnp2l_.ptr, &iv[7], sizeof(int), hipMemcpyHostToDevice));
-	}
 	num_nodes_ = 1;
-
-	star_node_.alloc(std::max(n, 1));
-	star_node_tmp_.alloc(std::max(n, 1));
-	tx_.alloc(std::max(n, 1));
-	ty_.alloc(std::max(n, 1));
-	tm_.alloc(std::max(n, 1));
-	MLENS_HIP_CHECK(hipMemsetAsync(star_node_.ptr, 0, std::max(n, 1) * sizeof(int), stream_));
-
-	DeviceBuffer<int> maxcnt;
-	maxcnt.alloc(1);
-	// scratch: flags/rank for nodes, onehot/pre for stars, tiles
+	const size_t ns = size_t(std::max(n, 1));
+	tx_.alloc(ns);
+	ty_.alloc(ns);
+	tm_.alloc(ns);
+	level_count_.alloc(2);
+	LevelCount* counts = reinterpret_cast<LevelCount*>(level_count_.ptr);
+	auto tree = [&]() {
+		return view(ncx_, ncy_, nhl_, nlevel_, nparent_, nchild0_, nbegin_, ncount_, nnnbr_, nnm2l_, nnp2l_, nnbr_, nm2l_, np2l_);
+	};
+	node_flag_.alloc(node_cap_);
+	node_rank_.alloc(node_cap_);
+	k_make_root<<<1, 1, 0, stream_>>>(tree(), root_half_length, n, node_flag_.ptr, node_rank_.ptr, counts);
+	MLENS_HIP_CHECK(hipGetLastError());
+	// the device-wide partition's scratch, taken only if a level needs it
 	DeviceBuffer<char> sbuf;
-
+	bool star_nodes = false;   // star_node_ holds every star's node of this level (-1: in a leaf)
 	while (true)
 	{
-		int l0 = level_start_[levels_];
-		int l1 = level_start_[levels_ + 1];
-		int nl = l1 - l0;
-		size_t need = sizeof(I4) * (size_t(nl) + size_t(nl) + 1 + size_t(n) + size_t(n) + 1 +
-			2 * (size_t(std::max(n, nl)) / SCAN_TILE + 4));
-		sbuf.alloc(need);
-		I4* flags = reinterpret_cast<I4*>(sbuf.ptr);
-		I4* rank = flags + nl;
-		I4* onehot = rank + nl + 1;
-		I4* pre = onehot + n;
-		I4* tiles = pre + n + 1;
-
-		TreeView t = view(ncx_, ncy_, nhl_, nlevel_, nparent_, nchild0_, nbegin_, ncount_, nnnbr_, nnm2l_, nnp2l_, nnbr_, nm2l_, np2l_);
-		MLENS_HIP_CHECK(hipMemsetAsync(maxcnt.ptr, 0, sizeof(int), stream_));
-		k_near_count<<<blocks_for(nl, 256), 256, 0, stream_>>>(t, l0, l1, flags, maxcnt.ptr);
+		const int l0 = level_start_[levels_], l1 = level_start_[levels_ + 1], nl = l1 - l0;
+		const size_t tiles_n = 2 * (size_t(std::max(n, nl)) / SCAN_TILE + 4);
+		if (nl > RANK_MAX)
+		{
+			sbuf.alloc(sizeof(I4) * (2 * size_t(nl) + 1 + tiles_n));
+			I4* f = reinterpret_cast<I4*>(sbuf.ptr);
+			I4* r = f + nl;
+			k_flags_to_i4<<<blocks_for(nl, 256), 256, 0, stream_>>>(node_flag_.ptr, f, nl);
+			scan_i4(f, r, r + nl + 1, nl, stream_);
+			k_i4_to_rank<<<blocks_for(nl + 1, 256), 256, 0, stream_>>>(r, node_rank_.ptr, nl, counts);
+		}
+		else if (levels_ > 0)
+			k_rank<<<1, RANK_THREADS, 0, stream_>>>(node_flag_.ptr, node_rank_.ptr, nl, counts);
 		MLENS_HIP_CHECK(hipGetLastError());
-		int hmax = 0;
-		MLENS_HIP_CHECK(hipMemcpyAsync(&hmax, maxcnt.ptr, sizeof(int), hipMemcpyDeviceToHost, stream_));
+		LevelCount lc;
+		MLENS_HIP_CHECK(hipMemcpyAsync(&lc, counts, sizeof(lc), hipMemcpyDeviceToHost, stream_));
 		MLENS_HIP_CHECK(hipStreamSynchronize(stream_));
-		if (hmax <= MAX_NUM_STARS_DIRECT) break;
-
-		scan_i4(flags, rank, tiles, nl, stream_);
-		I4 tot;
-		MLENS_HIP_CHECK(hipMemcpyAsync(&tot, rank + nl, sizeof(I4), hipMemcpyDeviceToHost, stream_));
-		MLENS_HIP_CHECK(hipStreamSynchronize(stream_));
-		int nsplit = tot.x;
-		int base = l1;
-		ensure_node_capacity(base + 4 * nsplit);
-		t = view(ncx_, ncy_, nhl_, nlevel_, nparent_, nchild0_, nbegin_, ncount_, nnnbr_, nnm2l_, nnp2l_, nnbr_, nm2l_, np2l_);
-
-		k_make_children<<<blocks_for(nl, 256), 256, 0, stream_>>>(t, l0, l1, flags, rank, base);
-		k_star_onehot<<<blocks_for(n, 256), 256, 0, stream_>>>(t, sx_.ptr, sy_.ptr, star_node_.ptr, l0, flags, onehot, n);
-		MLENS_HIP_CHECK(hipGetLastError());
-		scan_i4(onehot, pre, tiles, n, stream_);
-		k_child_ranges<<<blocks_for(nl, 256), 256, 0, stream_>>>(t, l0, l1, flags, pre);
-		k_star_scatter<<<blocks_for(n, 256), 256, 0, stream_>>>(t, sx_.ptr, sy_.ptr, sm_.ptr, tx_.ptr, ty_.ptr, tm_.ptr,
-			star_node_.ptr, star_node_tmp_.ptr, l0, flags, pre, n);
-		MLENS_HIP_CHECK(hipGetLastError());
-		std::swap(sx_.ptr, tx_.ptr);
-		std::swap(sy_.ptr, ty_.ptr);
-		std::swap(sm_.ptr, tm_.ptr);
-		std::swap(star_node_.ptr, star_node_tmp_.ptr);
-
-		num_nodes_ = base + 4 * nsplit;
+		if (lc.split == 0) break;
+		const int base = l1;
+		ensure_node_capacity(base + 4 * lc.split);
+		const TreeView t = tree();
+		if (lc.largest > SPLIT_MAX)
+		{
+			sbuf.alloc(sizeof(I4) * (2 * size_t(n) + 1 + tiles_n));
+			I4* onehot = reinterpret_cast<I4*>(sbuf.ptr);
+			I4* pre = onehot + n;
+			I4* tiles = pre + n + 1;
+			star_node_.alloc(ns);
+			star_node_tmp_.alloc(ns);
+			if (!star_nodes) MLENS_HIP_CHECK(hipMemsetAsync(star_node_.ptr, 0, ns * sizeof(int), stream_));
+			star_nodes = true;
+			k_make_children<<<blocks_for(nl, 256), 256, 0, stream_>>>(t, l0, l1, node_flag_.ptr, node_rank_.ptr, base);
+			k_star_onehot<<<blocks_for(n, 256), 256, 0, stream_>>>(t, sx_.ptr, sy_.ptr, star_node_.ptr, l0, node_flag_.ptr, onehot, n);
+			MLENS_HIP_CHECK(hipGetLastError());
+			scan_i4(onehot, pre, tiles, n, stream_);
+			k_child_ranges<<<blocks_for(nl, 256), 256, 0, stream_>>>(t, l0, l1, node_flag_.ptr, pre);
+			k_star_scatter<<<blocks_for(n, 256), 256, 0, stream_>>>(t, sx_.ptr, sy_.ptr, sm_.ptr, tx_.ptr, ty_.ptr, tm_.ptr,
+				star_node_.ptr, star_node_tmp_.ptr, l0, node_flag_.ptr, pre, n);
+			MLENS_HIP_CHECK(hipGetLastError());
+			std::swap(sx_.ptr, tx_.ptr);
+			std::swap(sy_.ptr, ty_.ptr);
+			std::swap(sm_.ptr, tm_.ptr);
+			std::swap(sx_.count, tx_.count);
+			std::swap(sy_.count, ty_.count);
+			std::swap(sm_.count, tm_.count);
+			std::swap(star_node_.ptr, star_node_tmp_.ptr);
+			std::swap(star_node_.count, star_node_tmp_.count);
+		}
+		else
+		{
+			// a block per node, as wide as its largest node can use (children never hold more stars than
+			// their parent, so the device-wide partition is not needed again)
+			auto split = [&](auto kernel, int threads) {
+				kernel<<<nl, threads, 0, stream_>>>(t, l0, node_flag_.ptr, node_rank_.ptr, base, sx_.ptr, sy_.ptr, sm_.ptr, tx_.ptr,
+					ty_.ptr, tm_.ptr);
+			};
+			if (lc.largest <= 256) split(k_split_nodes<64>, 64);
+			else if (lc.largest <= 2048) split(k_split_nodes<256>, 256);
+			else split(k_split_nodes<1024>, 1024);
+			MLENS_HIP_CHECK(hipGetLastError());
+		}
+		num_nodes_ = base + 4 * lc.split;
 		levels_++;
 		level_start_.push_back(num_nodes_);
-		k_set_neighbors<<<blocks_for(4 * nsplit, 256), 256, 0, stream_>>>(t, base, num_nodes_);
+		node_flag_.alloc(4 * size_t(lc.split));
+		node_rank_.alloc(4 * size_t(lc.split));
+		MLENS_HIP_CHECK(hipMemsetAsync(counts, 0, sizeof(LevelCount), stream_));
+		k_set_neighbors<<<blocks_for(4 * lc.split, 4), 256, 0, stream_>>>(t, base, num_nodes_, node_flag_.ptr, counts);
 		MLENS_HIP_CHECK(hipGetLastError());
 	}
-	MLENS_HIP_CHECK(hipStreamSynchronize(stream_));
 }
 
 void Engine::export_tree(double* geom, int* info, int* lists) const
@@ -633,14 +822,14 @@ __device__ __forceinline__ void st(double* a, long long i, dcx v)
 	a[2 * i + 1] = v.im;
 }
 
-// P2M at leaves holding stars (fmm.cuh:21-98)
-__global__ void k_p2m(TreeView t, int l0, int l1, int p, const double* sx, const double* sy, const double* sm, double* mult)
+// P2M at every leaf, zero where it holds no stars (fmm.cuh:21-98); M2M writes the other nodes
+__global__ void k_p2m(TreeView t, int nn, int p, const double* sx, const double* sy, const double* sm, double* mult)
 {
 	long long g = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-	int i = l0 + int(g / (p + 1));
+	int i = int(g / (p + 1));
 	int k = int(g % (p + 1));
-	if (i >= l1) return;
-	if (t.child0[i] >= 0 || t.count[i] == 0) return;
+	if (i >= nn) return;
+	if (t.child0[i] >= 0) return;
 	double cx = t.cx[i], cy = t.cy[i], h = t.hl[i];
 	int b = t.begin[i], n = t.count[i];
 	dcx r = {0, 0};
@@ -661,56 +850,86 @@ __global__ void k_p2m(TreeView t, int l0, int l1, int p, const double* sx, const
 	st(mult, (long long)i * (p + 1) + k, r);
 }
 
-// M2M, children to parent (fmm.cuh:109-192)
-__global__ void k_m2m(TreeView t, int l0, int l1, int p, const double* B, double* mult)
+/*
+M2M, children to parent (fmm.cuh:109-192): one thread per (child, order), the four children of a
+parent summed in order. Blocks hold whole sibling groups, FMM_THREADS / (p + 1) children rounded down
+to groups; their multipoles and the binomials come from LDS, since every order's chain of steps
+reads all of them (a level took 16 us with one thread per parent and order and the operands in L2).
+*/
+constexpr int FMM_THREADS = 256;
+constexpr int FMM_BINOMIALS = (MAX_EXPANSION_ORDER + 1) * (MAX_EXPANSION_ORDER + 2) / 2;   // rows 0..p
+
+__host__ __device__ inline int fmm_nodes_per_block(int p) { return FMM_THREADS / (p + 1) / 4 * 4; }
+
+__global__ __launch_bounds__(FMM_THREADS) void k_m2m(TreeView t, int c0, int c1, int p, const double* __restrict__ B, double* mult)
 {
-	long long g = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-	int i = l0 + int(g / (p + 1));
-	int l = int(g % (p + 1));
-	if (i >= l1 || t.child0[i] < 0) return;
-	dcx acc = {0, 0};
-	for (int c = t.child0[i]; c < t.child0[i] + 4; c++)
+	__shared__ dcx m[FMM_THREADS], part[FMM_THREADS];
+	__shared__ double b[FMM_BINOMIALS];
+	const int P = p + 1, per = fmm_nodes_per_block(p);
+	const int first = c0 + blockIdx.x * per, n = min(per, c1 - first);
+	const int x = threadIdx.x, ci = x / P, l = x - ci * P;
+	for (int i = x; i < p * (p + 1) / 2; i += FMM_THREADS) b[i] = B[i];
+	const bool on = ci < n;
+	if (on) m[x] = ld(mult, (long long)first * P + x);
+	__syncthreads();
+	const int c = first + ci;
+	int par = 0;
+	if (on)
 	{
-		const long long cb = (long long)c * (p + 1);
-		if (l == 0)
+		par = t.parent[c];
+		const dcx* mc = m + ci * P;
+		dcx r = mc[0];
+		if (l > 0)
 		{
-			acc = dev::add(acc, ld(mult, cb));
-			continue;
+			dcx dz = dcx{(t.cx[c] - t.cx[par]) / t.hl[c], (t.cy[c] - t.cy[par]) / t.hl[c]};
+			dcx idz = dev::cdiv(dcx{1, 0}, dz);
+			r = dcx{0, 0};
+			const double* row = b + (l - 1) * l / 2;   // C(l - 1, .)
+			for (int k = l; k >= 1; k--)
+			{
+				r = dev::add(r, dev::scale(mc[k], row[k - 1]));
+				r = dev::mul(r, idz);
+			}
+			r = dev::sub(r, dev::scale(mc[0], 1.0 / l));
+			r = dev::mul(r, dev::cpow(dz, l));
+			r = dev::scale(r, ldexp(1.0, -l));
 		}
-		dcx dz = dcx{(t.cx[c] - t.cx[i]) / t.hl[c], (t.cy[c] - t.cy[i]) / t.hl[c]};
-		dcx idz = dev::cdiv(dcx{1, 0}, dz);
-		dcx r = {0, 0};
-		for (int k = l; k >= 1; k--)
-		{
-			r = dev::add(r, dev::scale(ld(mult, cb + k), binom(B, l - 1, k - 1)));
-			r = dev::mul(r, idz);
-		}
-		r = dev::sub(r, dev::scale(ld(mult, cb), 1.0 / l));
-		r = dev::mul(r, dev::cpow(dz, l));
-		r = dev::scale(r, ldexp(1.0, -l));
-		acc = dev::add(acc, r);
+		part[x] = r;
 	}
-	st(mult, (long long)i * (p + 1) + l, acc);
+	__syncthreads();
+	if (!on || (ci & 3) != 0) return;
+	dcx acc = {0, 0};
+	for (int q = 0; q < 4; q++) acc = dev::add(acc, part[x + q * P]);
+	st(mult, (long long)par * P + l, acc);
 }
 
-// L2L (overwrite), M2L and P2L for one level (fmm.cuh:204-464)
-__global__ void k_local(TreeView t, int l0, int l1, int p, const double* B, const double* mult, double* local,
-	const double* sx, const double* sy, const double* sm, int do_m2l)
+// L2L, M2L and P2L for one level (fmm.cuh:204-464). The M2L sums are recurrences here (do_m2l) or
+// were left in local by k_m2l.
+// Blocks as in k_m2m, their parents' expansions and the binomials in LDS.
+__global__ __launch_bounds__(FMM_THREADS) void k_local(TreeView t, int l0, int l1, int p, const double* __restrict__ B,
+	const double* __restrict__ mult, double* local, const double* __restrict__ sx, const double* __restrict__ sy,
+	const double* __restrict__ sm, int do_m2l)
 {
-	long long g = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-	int i = l0 + int(g / (p + 1));
-	int l = int(g % (p + 1));
-	if (i >= l1) return;
+	__shared__ dcx pl[FMM_THREADS / 4];
+	__shared__ double b[FMM_BINOMIALS];
+	const int P = p + 1, per = fmm_nodes_per_block(p);
+	const int first = l0 + blockIdx.x * per, n = min(per, l1 - first);
+	const int x = threadIdx.x, ci = x / P, l = x - ci * P;
+	for (int k = x; k < P * (P + 1) / 2; k += FMM_THREADS) b[k] = B[k];
+	if (x < n / 4 * P) pl[x] = ld(local, (long long)t.parent[first + 4 * (x / P)] * P + x % P);
+	__syncthreads();
+	if (ci >= n) return;
+	const int i = first + ci;
 	const double cx = t.cx[i], cy = t.cy[i], h = t.hl[i];
 	dcx acc;
 	{
 		int par = t.parent[i];
-		const long long pb = (long long)par * (p + 1);
+		const dcx* lp = pl + (ci >> 2) * P;
 		dcx dz = dcx{(cx - t.cx[par]) / t.hl[par], (cy - t.cy[par]) / t.hl[par]};
 		dcx r = {0, 0};
 		for (int k = p; k >= 1; k--)
 		{
-			r = dev::add(r, dev::scale(ld(local, pb + k), binom(B, k, l)));
+			r = dev::add(r, dev::scale(lp[k], k < l ? 0.0 : b[k * (k + 1) / 2 + l]));
 			r = dev::mul(r, dz);
 		}
 		r = dev::cdiv(r, dev::cpow(dz, l));
@@ -758,14 +977,8 @@ __global__ void k_local(TreeView t, int l0, int l1, int p, const double* B, cons
 			}
 		}
 	}
+	if (!do_m2l) acc = dev::add(acc, ld(local, (long long)i * (p + 1) + l));
 	st(local, (long long)i * (p + 1) + l, acc);
-}
-
-// leaf flags for compaction
-__global__ void k_leaf_flags(const int* child0, int nn, I4* flags)
-{
-	int i = blockIdx.x * blockDim.x + threadIdx.x;
-	if (i < nn) flags[i] = I4{child0[i] < 0 ? 1 : 0, 0, 0, 0};
 }
 
 /*
@@ -773,101 +986,109 @@ Leaf tables for shooting: geometry, the near-field star list (own stars then
 each neighbour's, alpha_star.cuh:26-37) and the deflection polynomial
 A_i = (theta^2/h) i c_i of alpha_local.cuh:18-36, so that
 alpha_local(z) = conj( sum_{i=1..p} A_i dz^(i-1) ), dz = (z - c)/h.
+A leaf's tables stand at its node's index (inner nodes leave theirs unused, a
+quarter of them): no scan over the nodes and no wait for its total. 32 lanes per
+leaf, a near star and a polynomial entry each: one lane per leaf wrote 2 KB in
+24-byte steps (2.0 ms for the 1.28e6-star tree).
 */
-__global__ void k_leaf_tables(TreeView t, int nn, const I4* pre, int p, double theta2, const double* sx, const double* sy,
-	const double* sm, const double* local, int* leaf_of_node, double* geom, int* near_n, int* near_true, double* near_d,
-	float* near_f, double* poly_d, float* poly_f)
+__global__ __launch_bounds__(256) void k_leaf_tables(TreeView t, int nn, int p, double theta2, const double* __restrict__ sx,
+	const double* __restrict__ sy, const double* __restrict__ sm, const double* __restrict__ local, int* leaf_of_node, double* geom,
+	int* near_n, int* near_true, double* near_d, float* near_f, double* poly_d, float* poly_f)
 {
-	int i = blockIdx.x * blockDim.x + threadIdx.x;
-	if (i >= nn) return;
-	if (t.child0[i] >= 0)
+	constexpr int LANES = 32;   // per leaf
+	static_assert(MAX_NUM_STARS_DIRECT == LANES, "a lane per near star");
+	static_assert((MAX_EXPANSION_ORDER + 3) / 4 * 4 <= LANES, "a lane per polynomial entry");
+	__shared__ double lead_s[256 / LANES][LANES];
+	const int lane = threadIdx.x % LANES, slot = threadIdx.x / LANES;
+	const int i = blockIdx.x * (256 / LANES) + slot;
+	const bool node = i < nn, leaf = node && t.child0[i] < 0;
+	if (node && lane == 0) leaf_of_node[i] = leaf ? i : -1;
+	const long long L = i;
+	if (node && !leaf && lane == 0)
 	{
-		leaf_of_node[i] = -1;
-		return;
+		// an inner node's entry: no area and no stars
+		for (int k = 0; k < 4; k++) geom[4 * L + k] = 0;
+		near_n[L] = 0;
+		near_true[L] = 0;
 	}
-	int L = pre[i].x;
-	leaf_of_node[i] = L;
-	double cx = t.cx[i], cy = t.cy[i], h = t.hl[i];
-	geom[4 * (long long)L] = cx;
-	geom[4 * (long long)L + 1] = cy;
-	geom[4 * (long long)L + 2] = h;
-	geom[4 * (long long)L + 3] = 1.0 / h;
-	int k = 0;
-	auto put = [&](int b, int n) {
-		for (int s = b; s < b + n && k < MAX_NUM_STARS_DIRECT; s++, k++)
-		{
-			long long o = ((long long)L * MAX_NUM_STARS_DIRECT + k) * 3;
-			near_d[o] = sx[s];
-			near_d[o + 1] = sy[s];
-			near_d[o + 2] = sm[s];
-			long long of = ((long long)L * MAX_NUM_STARS_DIRECT + k) * 4;
-			near_f[of] = float(sx[s] - cx);
-			near_f[of + 1] = float(sy[s] - cy);
-			near_f[of + 2] = float(sm[s]);
-			near_f[of + 3] = 0.0f;
-		}
-	};
-	put(t.begin[i], t.count[i]);
-	for (int j = 0; j < t.nnbr[i]; j++)
-	{
-		int nb = t.nbr[8 * i + j];
-		put(t.begin[nb], t.count[nb]);
-	}
-	near_true[L] = k;
-	// pad to a multiple of 4 with massless stars far away (their terms are exactly 0)
-	for (; (k & 3) != 0; k++)
-	{
-		long long o = ((long long)L * MAX_NUM_STARS_DIRECT + k) * 3;
-		near_d[o] = 1e150;
-		near_d[o + 1] = 1e150;
-		near_d[o + 2] = 0.0;
-		long long of = ((long long)L * MAX_NUM_STARS_DIRECT + k) * 4;
-		near_f[of] = 1e18f;
-		near_f[of + 1] = 1e18f;
-		near_f[of + 2] = 0.0f;
-		near_f[of + 3] = 0.0f;
-	}
-	// polynomial tables in descending degree, zero-padded at the top to a
-	// multiple of 4: entry j of the FP64 table is the coefficient of
-	// dz^(SD-1-j) in P(dz) = sum_{i=1..p} A_i dz^(i-1); entry j of the FP32
-	// table is the coefficient of dz^(SF-1-j) in Q(dz) = sum_{i=2..p} A_i dz^(i-2)
+	double cx = 0, cy = 0, h = 1, scale_l1 = 0, lead = 0;
+	int total = 0, padded = 0;
 	const int SD = poly_stride_d(p), SF = poly_stride_f(p);
-	static_assert((MAX_EXPANSION_ORDER - 1 + 3) / 4 * 4 <= 32, "FP32 polynomial longer than its bound table");
-	const long long lb = (long long)i * (p + 1);
-	for (int j = 0; j < SD; j++)
+	if (leaf)
 	{
-		int q = SD - j;   // A_q
-		dcx a = (q <= p) ? dev::scale(ld(local, lb + q), theta2 / h * q) : dcx{0, 0};
-		poly_d[2 * ((long long)L * SD + j)] = a.re;
-		poly_d[2 * ((long long)L * SD + j) + 1] = a.im;
+		cx = t.cx[i];
+		cy = t.cy[i];
+		h = t.hl[i];
+		if (lane < 4) geom[4 * L + lane] = lane == 0 ? cx : (lane == 1 ? cy : (lane == 2 ? h : 1.0 / h));
+		// near star `lane`: own stars, then each neighbour's, at most MAX_NUM_STARS_DIRECT
+		int star = -1;
+		const int nb = t.nnbr[i];
+		for (int j = -1; j < nb; j++)
+		{
+			const int f = j < 0 ? i : t.nbr[8 * (long long)i + j];
+			const int c = t.count[f];
+			if (lane >= total && lane < total + c) star = t.begin[f] + (lane - total);
+			total += c;
+		}
+		total = min(total, MAX_NUM_STARS_DIRECT);
+		padded = (total + 3) & ~3;
+		if (lane < padded)
+		{
+			// padding: massless stars far away (their terms are exactly 0)
+			const bool real = lane < total;
+			const double x = real ? sx[star] : 1e150, y = real ? sy[star] : 1e150, m = real ? sm[star] : 0.0;
+			double* d = near_d + (L * MAX_NUM_STARS_DIRECT + lane) * 3;
+			d[0] = x;
+			d[1] = y;
+			d[2] = m;
+			float4 f = make_float4(1e18f, 1e18f, 0.0f, 0.0f);
+			if (real) f = make_float4(float(x - cx), float(y - cy), float(m), 0.0f);
+			reinterpret_cast<float4*>(near_f)[L * MAX_NUM_STARS_DIRECT + lane] = f;
+		}
+		// polynomial tables in descending degree, zero-padded at the top to a
+		// multiple of 4: entry j of the FP64 table is the coefficient of
+		// dz^(SD-1-j) in P(dz) = sum_{i=1..p} A_i dz^(i-1); entry j of the FP32
+		// table is the coefficient of dz^(SF-1-j) in Q(dz) = sum_{i=2..p} A_i dz^(i-2)
+		const long long lb = (long long)i * (p + 1);
+		if (lane < SD)
+		{
+			const int q = SD - lane;   // A_q
+			const dcx a = (q <= p) ? dev::scale(ld(local, lb + q), theta2 / h * q) : dcx{0, 0};
+			poly_d[2 * (L * SD + lane)] = a.re;
+			poly_d[2 * (L * SD + lane) + 1] = a.im;
+		}
+		// the FP32 evaluation skips its leading groups of 4 entries while their
+		// terms together stay below 2^-28 of the scale of all terms, bounded over
+		// the leaf (|dz| <= sqrt(2) in units of the half-size): an eighth of one
+		// rounding of the FP32 sum, which carries about SF such roundings already.
+		// On the 10000^2 map (p = 30) this leaves the mixed map's error against FP64
+		// as it was (median 2.1e-6, max 6.9e-4) and takes 1% off the shot; at 2^-25
+		// single pixels moved by 3e-3.
+		scale_l1 = dev::cabs(dev::scale(ld(local, lb + 1), theta2 / h));
+		if (lane < SF)
+		{
+			const int q = SF - lane + 1;   // A_q
+			const dcx a = (q <= p && q >= 2) ? dev::scale(ld(local, lb + q), theta2 / h * q) : dcx{0, 0};
+			poly_f[2 * (L * SF + lane)] = float(a.re);
+			poly_f[2 * (L * SF + lane) + 1] = float(a.im);
+			lead = dev::cabs(a) * pow(1.4143, double(q - 1));   // bound of A_q dz^(q-1) over the leaf
+		}
 	}
-	// the FP32 evaluation skips its leading groups of 4 entries while their
-	// terms together stay below 2^-28 of the scale of all terms, bounded over
-	// the leaf (|dz| <= sqrt(2) in units of the half-size): an eighth of one
-	// rounding of the FP32 sum, which carries about SF such roundings already.
-	// On the 10000^2 map (p = 30) this leaves the mixed map's error against FP64
-	// as it was (median 2.1e-6, max 6.9e-4) and takes 1% off the shot; at 2^-25
-	// single pixels moved by 3e-3.
-	const double R = 1.4143;
-	double S = dev::cabs(dev::scale(ld(local, lb + 1), theta2 / h)), lead[32];   // SF <= 32 up to MAX_EXPANSION_ORDER
-	for (int j = 0; j < SF; j++)
-	{
-		int q = SF - j + 1;   // A_q
-		dcx a = (q <= p && q >= 2) ? dev::scale(ld(local, lb + q), theta2 / h * q) : dcx{0, 0};
-		poly_f[2 * ((long long)L * SF + j)] = float(a.re);
-		poly_f[2 * ((long long)L * SF + j) + 1] = float(a.im);
-		lead[j] = dev::cabs(a) * pow(R, double(q - 1));   // bound of A_q dz^(q-1) over the leaf
-		S += lead[j];
-	}
+	lead_s[slot][lane] = lead;
+	__syncthreads();
+	if (!leaf || lane != 0) return;
+	near_true[L] = total;
+	double S = scale_l1, tail = 0;
+	for (int j = 0; j < SF; j++) S += lead_s[slot][j];
 	int skip = 0;
-	double tail = 0;
 	for (int j0 = 0; j0 + 4 <= SF; j0 += 4)
 	{
-		tail += lead[j0] + lead[j0 + 1] + lead[j0 + 2] + lead[j0 + 3];
+		const double* l = lead_s[slot] + j0;
+		tail += l[0] + l[1] + l[2] + l[3];
 		if (!(tail <= 0x1p-28 * S)) break;
 		skip = j0 + 4;
 	}
-	near_n[L] = k | (skip << 16);
+	near_n[L] = padded | (skip << 16);
 }
 
 void Engine::fmm(int p, const LensParams& lens)
@@ -890,17 +1111,18 @@ void Engine::fmm(int p, const LensParams& lens)
 	const size_t nc = size_t(num_nodes_) * (p + 1) * 2;
 	mult_.alloc(nc);
 	local_.alloc(nc);
-	MLENS_HIP_CHECK(hipMemsetAsync(mult_.ptr, 0, nc * sizeof(double), stream_));
-	MLENS_HIP_CHECK(hipMemsetAsync(local_.ptr, 0, nc * sizeof(double), stream_));
+	// levels 0 and 1 have no far field; k_m2l or k_local writes the others
+	const int far = levels_ >= 2 ? level_start_[2] : num_nodes_;
+	MLENS_HIP_CHECK(hipMemsetAsync(local_.ptr, 0, size_t(far) * (p + 1) * 2 * sizeof(double), stream_));
 	TreeView t = view(ncx_, ncy_, nhl_, nlevel_, nparent_, nchild0_, nbegin_, ncount_, nnnbr_, nnm2l_, nnp2l_, nnbr_, nm2l_, np2l_);
-	for (int lev = levels_; lev >= 0; lev--)
+	k_p2m<<<blocks_for((long long)num_nodes_ * (p + 1), 256), 256, 0, stream_>>>(t, num_nodes_, p, sx_.ptr, sy_.ptr, sm_.ptr, mult_.ptr);
+	const int per = fmm_nodes_per_block(p);
+	for (int lev = levels_ - 1; lev >= 0; lev--)
 	{
-		int l0 = level_start_[lev], l1 = level_start_[lev + 1];
-		long long work = (long long)(l1 - l0) * (p + 1);
-		k_p2m<<<blocks_for(work, 256), 256, 0, stream_>>>(t, l0, l1, p, sx_.ptr, sy_.ptr, sm_.ptr, mult_.ptr);
-		k_m2m<<<blocks_for(work, 256), 256, 0, stream_>>>(t, l0, l1, p, binom_.ptr, mult_.ptr);
-		MLENS_HIP_CHECK(hipGetLastError());
+		const int c0 = level_start_[lev + 1], c1 = level_start_[lev + 2];
+		k_m2m<<<blocks_for(c1 - c0, per), FMM_THREADS, 0, stream_>>>(t, c0, c1, p, binom_.ptr, mult_.ptr);
 	}
+	MLENS_HIP_CHECK(hipGetLastError());
 	// M2L: FP64 recurrences inside k_local, or batched GEMMs on MFMA after it
 	const bool mfma = m2l_mode_ != M2L_DIRECT;
 	const bool f32 = m2l_mode_ == M2L_MFMA_F32 || (m2l_mode_ == M2L_MFMA && p <= 20);
@@ -909,21 +1131,18 @@ void Engine::fmm(int p, const LensParams& lens)
 		m2l_prepare(p, f32);
 		if (m2l_count_.count < 2) m2l_count_.alloc(2);
 		MLENS_HIP_CHECK(hipMemsetAsync(m2l_count_.ptr, 0, 2 * sizeof(unsigned long long), stream_));
-		while (m2l_ev_.size() < size_t(2 * (levels_ + 1)))
-		{
-			hipEvent_t e;
-			MLENS_HIP_CHECK(hipEventCreate(&e));
-			m2l_ev_.push_back(e);
-		}
+		if (!m2l_ev0_) MLENS_HIP_CHECK(hipEventCreate(&m2l_ev0_));
+		if (!m2l_ev1_) MLENS_HIP_CHECK(hipEventCreate(&m2l_ev1_));
+		MLENS_HIP_CHECK(hipEventRecord(m2l_ev0_, stream_));
+		if (levels_ >= 2) m2l_all(p, f32);
+		MLENS_HIP_CHECK(hipEventRecord(m2l_ev1_, stream_));
 	}
 	for (int lev = 2; lev <= levels_; lev++)
 	{
 		int l0 = level_start_[lev], l1 = level_start_[lev + 1];
-		long long work = (long long)(l1 - l0) * (p + 1);
-		k_local<<<blocks_for(work, 256), 256, 0, stream_>>>(t, l0, l1, p, binom_.ptr, mult_.ptr, local_.ptr, sx_.ptr,
+		k_local<<<blocks_for(l1 - l0, per), FMM_THREADS, 0, stream_>>>(t, l0, l1, p, binom_.ptr, mult_.ptr, local_.ptr, sx_.ptr,
 			sy_.ptr, sm_.ptr, mfma ? 0 : 1);
 		MLENS_HIP_CHECK(hipGetLastError());
-		if (mfma) m2l_level(lev, p, f32, m2l_ev_[2 * lev], m2l_ev_[2 * lev + 1]);
 	}
 	build_leaf_tables(lens);
 	MLENS_HIP_CHECK(hipStreamSynchronize(stream_));
@@ -932,12 +1151,9 @@ void Engine::fmm(int p, const LensParams& lens)
 	m2l_f32_ = mfma && f32;
 	if (mfma)
 	{
-		for (int lev = 2; lev <= levels_; lev++)
-		{
-			float ms = 0;
-			MLENS_HIP_CHECK(hipEventElapsedTime(&ms, m2l_ev_[2 * lev], m2l_ev_[2 * lev + 1]));
-			m2l_ms_ += ms;
-		}
+		float ms = 0;
+		MLENS_HIP_CHECK(hipEventElapsedTime(&ms, m2l_ev0_, m2l_ev1_));
+		m2l_ms_ = ms;
 		unsigned long long h[2];
 		MLENS_HIP_CHECK(hipMemcpy(h, m2l_count_.ptr, sizeof(h), hipMemcpyDeviceToHost));
 		m2l_pairs_ = (long long)h[0];
@@ -948,17 +1164,7 @@ void Engine::fmm(int p, const LensParams& lens)
 void Engine::build_leaf_tables(const LensParams& lens)
 {
 	const int nn = num_nodes_;
-	DeviceBuffer<char> sbuf;
-	sbuf.alloc(sizeof(I4) * (2 * size_t(nn) + 1 + 2 * (size_t(nn) / SCAN_TILE + 4)));
-	I4* flags = reinterpret_cast<I4*>(sbuf.ptr);
-	I4* pre = flags + nn;
-	I4* tiles = pre + nn + 1;
-	k_leaf_flags<<<blocks_for(nn, 256), 256, 0, stream_>>>(nchild0_.ptr, nn, flags);
-	scan_i4(flags, pre, tiles, nn, stream_);
-	I4 tot;
-	MLENS_HIP_CHECK(hipMemcpyAsync(&tot, pre + nn, sizeof(I4), hipMemcpyDeviceToHost, stream_));
-	MLENS_HIP_CHECK(hipStreamSynchronize(stream_));
-	num_leaves_ = tot.x;
+	num_leaves_ = nn;   // entries: one per node
 	const int SD = poly_stride_d(p_), SF = poly_stride_f(p_);
 	leaf_of_node_.alloc(nn);
 	leaf_geom_.alloc(size_t(num_leaves_) * 4);
@@ -969,12 +1175,11 @@ void Engine::build_leaf_tables(const LensParams& lens)
 	leaf_poly_d_.alloc(size_t(std::max(num_leaves_, 1)) * SD * 2);
 	leaf_poly_f_.alloc(size_t(std::max(num_leaves_, 1)) * std::max(SF, 1) * 2);
 	TreeView t = view(ncx_, ncy_, nhl_, nlevel_, nparent_, nchild0_, nbegin_, ncount_, nnnbr_, nnm2l_, nnp2l_, nnbr_, nm2l_, np2l_);
-	k_leaf_tables<<<blocks_for(nn, 256), 256, 0, stream_>>>(t, nn, pre, p_, lens.theta * lens.theta, sx_.ptr, sy_.ptr,
+	k_leaf_tables<<<blocks_for(nn, 8), 256, 0, stream_>>>(t, nn, p_, lens.theta * lens.theta, sx_.ptr, sy_.ptr,
 		sm_.ptr, local_.ptr, leaf_of_node_.ptr, leaf_geom_.ptr, leaf_near_n_.ptr, leaf_near_true_.ptr, leaf_near_d_.ptr,
 		leaf_near_f_.ptr,
 		leaf_poly_d_.ptr, leaf_poly_f_.ptr);
 	MLENS_HIP_CHECK(hipGetLastError());
-	MLENS_HIP_CHECK(hipStreamSynchronize(stream_));
 }
 
 void Engine::export_coeffs(int which, double* out) const

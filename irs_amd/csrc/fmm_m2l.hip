@@ -13,12 +13,23 @@
 // level-dependent b_0 log h term. Complex products run as real products of
 // the stacked form [Mr -Mi; Mi Mr] [b_re; b_im], padded to a multiple of 16.
 //
-// One wave owns 16 targets (the columns of a 16 x 16 output tile); for each
-// offset it gathers the 16 source multipoles at that offset (zero where a
-// target has none) and accumulates M_o b over all offsets in its registers,
-// so no target is written by two waves and no atomics are needed. The block's
-// four waves share each offset matrix through LDS. The MFMA shape is
-// 16 x 16 x 4 in FP32 (v_mfma_f32_16x16x4_f32) or FP64
+// Sources sit at their target's level and the matrices do not depend on it, so
+// one launch translates every level. A block takes 16 (or 32) sibling groups
+// (the four children of a node, consecutive) and one of the four quadrants:
+// targets of the same quadrant share the 27 offsets their M2L lists can hold,
+// where a mixed block would step through all 40. Wave w owns row tile w of the
+// block's targets (the columns of a 16 x 16 output tile): for each offset that
+// some target has, it accumulates M_o b in registers, offsets ascending, so no
+// target row is written by two waves and no atomics are needed. The block
+// gathers each offset's sources into LDS once for all its waves (two buffers,
+// one barrier an offset), each wave its rows of the matrix into registers, both
+// an offset ahead. The offset matrices (1.3 MB) stay in L2. 1.28e6 stars at
+// p = 30 (2.2e7 pairs): 5.1 ms, 43% of the FP64 MFMA time of the padded
+// products; 13.0 ms with one launch per level, mixed quadrants and every wave
+// computing all row tiles of its own targets, 10 ms with the sources gathered
+// by each wave. 7e3 stars at p = 20, where the chain of offsets is the time:
+// 54 us against six launches of 265 us.
+// The MFMA shape is 16 x 16 x 4 in FP32 (v_mfma_f32_16x16x4_f32) or FP64
 // (v_mfma_f64_16x16x4_f64); both take A[i][k] from lane i + 16 k and B[k][j]
 // from lane j + 16 k. Lane l gets back D[4 (l / 16) + r][l % 16] in FP32 and
 // D[(l / 16) + 4 r][l % 16] in FP64, r = 0..3 (checked on the device).
@@ -35,8 +46,7 @@ namespace
 {
 
 constexpr int M2L_OFFSETS = 40;
-constexpr int M2L_WAVES = 4;
-constexpr int M2L_TARGETS_PER_WAVE = 16;
+constexpr int M2L_LIST = 27;   // longest M2L list (tree_node.cuh:41-49)
 
 inline int m2l_kp(int p) { return (2 * (p + 1) + 15) / 16 * 16; }
 
@@ -71,114 +81,178 @@ struct MfmaVec<double>
 	static __device__ __forceinline__ int row(int kq, int r) { return kq + 4 * r; }
 };
 
-// src[o * n + (t - l0)] = the M2L source of target t at offset o, else -1
-__global__ void k_m2l_table(const double* cx, const double* cy, const double* hl, const int* nm2l, const int* m2l, int l0,
-	int n, int* src, unsigned long long* pairs, int* bad)
+/*
+out[node][2 row + c] = row `row` (real c = 0, imaginary 1) of the M2L sum of nodes
+first + 4 g + q, g < groups. KP: stacked size (2 (p + 1) rounded up to 16), KP / 16
+waves per block; NT: column tiles (16 targets each) per block. The four quadrants of
+the same groups, which share most of their sources, are consecutive pieces of work, and
+each XCD (blocks go to the eight in turn) takes a contiguous run of them, so that its
+L2 holds the multipoles that they read over and over.
+count[0] collects the list entries, the low bit of count[1] a source that is not at
+one of the 40 offsets.
+*/
+template <typename T, int KP, int NT>
+__global__ __launch_bounds__(KP * 4) void k_m2l(const T* __restrict__ At, const double* __restrict__ mult, double* __restrict__ out,
+	const double* __restrict__ cx, const double* __restrict__ cy, const double* __restrict__ hl, const int* __restrict__ nm2l,
+	const int* __restrict__ m2l, int first, int groups, int p, unsigned long long* __restrict__ count)
 {
-	int t = blockIdx.x * blockDim.x + threadIdx.x;
-	if (t >= n) return;
-	const int i = l0 + t;
-	const double h2 = 2 * hl[i];
-	const int cnt = nm2l[i];
-	for (int j = 0; j < cnt; j++)
+	using V = typename MfmaVec<T>::v4;
+	constexpr int KS = KP / 4, TARGETS = 16 * NT, THREADS = KP * 4, STAGE = TARGETS * KP / THREADS;
+	// 2 modulo 32 eight-byte banks: the 16 targets and two rows a half-wave reads fall on 32 of them
+	constexpr int STRIDE = (KP + 31) / 32 * 32 + 2;
+	__shared__ T gathered[2][TARGETS * STRIDE];
+	__shared__ int src[M2L_OFFSETS][TARGETS];   // the source of each target at each offset, or -1
+	__shared__ unsigned active[2];              // offsets that some target has
+	__shared__ unsigned found;
+	const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+	const int col = lane & 15, kq = lane >> 4;
+	const int run = int(gridDim.x) / 8;   // pieces per XCD (the grid is a multiple of 8)
+	const int piece = int(blockIdx.x % 8) * run + int(blockIdx.x / 8);
+	const int g0 = (piece >> 2) * TARGETS, q = piece & 3;
+	if (g0 >= groups) return;
+	for (int i = threadIdx.x; i < M2L_OFFSETS * TARGETS; i += blockDim.x) src[i / TARGETS][i % TARGETS] = -1;
+	for (int i = threadIdx.x; i < 2 * TARGETS * STRIDE; i += blockDim.x) gathered[0][i] = T(0);
+	if (threadIdx.x == 0) active[0] = active[1] = found = 0;
+	__syncthreads();
+	for (int i = threadIdx.x; i < M2L_LIST * TARGETS; i += blockDim.x)
 	{
-		const int f = m2l[27 * i + j];
-		const int a = int(lrint((cx[f] - cx[i]) / h2)), b = int(lrint((cy[f] - cy[i]) / h2));
-		const int o = m2l_offset_index(a, b);
-		if (o < 0 || f < l0 || f >= l0 + n)
+		const int c = i / M2L_LIST, j = i - c * M2L_LIST;
+		if (g0 + c >= groups) continue;
+		const int t = first + 4 * (g0 + c) + q;
+		if (j >= nm2l[t]) continue;
+		const int f = m2l[M2L_LIST * (long long)t + j];
+		const double h2 = 2 * hl[t];
+		const int o = m2l_offset_index(int(lrint((cx[f] - cx[t]) / h2)), int(lrint((cy[f] - cy[t]) / h2)));
+		atomicAdd(&found, 1u);
+		if (o < 0 || hl[f] != hl[t])
 		{
-			atomicOr(bad, 1);
+			atomicOr(reinterpret_cast<unsigned*>(count + 1), 1u);
 			continue;
 		}
-		src[(long long)o * n + t] = f - l0;
+		src[o][c] = f;
+		atomicOr(&active[o >> 5], 1u << (o & 31));
 	}
-	if (cnt > 0) atomicAdd(pairs, (unsigned long long)cnt);
-}
-
-__global__ void k_fill_int(int* a, long long n, int v)
-{
-	long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-	if (i < n) a[i] = v;
-}
-
-// real-stacked multipoles of the level's nodes: row k = Re b_k, row P + k = Im b_k
-template <typename T>
-__global__ void k_mstack(const double* mult, int l0, int n, int p, int kp, T* ms)
-{
-	long long g = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-	if (g >= (long long)n * kp) return;
-	const int t = int(g / kp), r = int(g % kp), P = p + 1;
-	const double* b = mult + (long long)(l0 + t) * P * 2;
-	T v = 0;
-	if (r < P)
-		v = T(b[2 * r]);
-	else if (r < 2 * P)
-		v = T(b[2 * (r - P) + 1]);
-	ms[g] = v;
-}
-
-template <typename T>
-__global__ __launch_bounds__(64 * M2L_WAVES) void k_m2l_mfma(const T* __restrict__ At, const int* __restrict__ src,
-	const T* __restrict__ ms, const double* __restrict__ mult, double* local, const double* hl, int l0, int n, int p, int kp)
-{
-	extern __shared__ char smem_raw[];
-	T* As = reinterpret_cast<T*>(smem_raw);   // kp x kp, transposed: As[k * kp + row]
-	using V = typename MfmaVec<T>::v4;
-	const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-	const int t0 = (blockIdx.x * M2L_WAVES + wave) * M2L_TARGETS_PER_WAVE;
-	const int col = lane & 15, kq = lane >> 4;
-	const int t = t0 + col;
-	const int ntile = kp / 16;   // row tiles (<= 4)
-	V acc[4];
-#pragma unroll
-	for (int r = 0; r < 4; r++) acc[r] = V{0, 0, 0, 0};
-	for (int o = 0; o < M2L_OFFSETS; o++)
-	{
-		__syncthreads();
-		const T* Ao = At + (long long)o * kp * kp;
-		for (int i = threadIdx.x; i < kp * kp; i += blockDim.x) As[i] = Ao[i];
-		__syncthreads();
-		const int s = (t < n) ? src[(long long)o * n + t] : -1;
-		if (__ballot(s >= 0) == 0) continue;
-		const T* bs = ms + (long long)(s >= 0 ? s : 0) * kp;
-		for (int ks = 0; ks < kp / 4; ks++)
-		{
-			const int k = ks * 4 + kq;
-			const T b = s >= 0 ? bs[k] : T(0);
-#pragma unroll
-			for (int rt = 0; rt < 4; rt++)
-				if (rt < ntile) acc[rt] = MfmaVec<T>::mfma(As[k * kp + rt * 16 + col], b, acc[rt]);
-		}
-	}
-	if (t >= n) return;
+	__syncthreads();
+	if (threadIdx.x == 0 && found) atomicAdd(count, (unsigned long long)found);
+	unsigned long long todo = ((unsigned long long)__builtin_amdgcn_readfirstlane(active[1]) << 32) |
+		(unsigned)__builtin_amdgcn_readfirstlane(active[0]);
 	const int P = p + 1;
-	// b_0 log h in FP64 from the FP64 multipoles, added with row 0 (real) and
-	// row P (imaginary) by the lanes that own those rows
-	const double lh = log(hl[l0 + t]);
-	double sre = 0, sim = 0;
-	for (int o = 0; o < M2L_OFFSETS; o++)
-	{
-		const int sidx = src[(long long)o * n + t];
-		if (sidx >= 0)
-		{
-			sre += mult[(long long)(l0 + sidx) * P * 2];
-			sim += mult[(long long)(l0 + sidx) * P * 2 + 1];
-		}
-	}
-	double* c = local + (long long)(l0 + t) * P * 2;
+	V acc[NT];
+	double sum0[NT];   // sum of the sources' b_0, for the b_0 log h term (its lanes: row 0)
 #pragma unroll
-	for (int rt = 0; rt < 4; rt++)
+	for (int n = 0; n < NT; n++)
 	{
-		if (rt >= ntile) break;
+		acc[n] = V{0, 0, 0, 0};
+		sum0[n] = 0;
+	}
+	// the operands of one offset: this wave's rows of the matrix, and this thread's
+	// share of the sources' multipoles
+	struct Operands
+	{
+		T a[KS];
+		T b[STAGE];
+		double b0[NT];
+	};
+	auto load = [&](int o, Operands& x) {
+		const T* Ao = At + ((long long)o * KP + kq) * KP + wave * 16 + col;
+#pragma unroll
+		for (int ks = 0; ks < KS; ks++) x.a[ks] = Ao[(long long)ks * 4 * KP];
+#pragma unroll
+		for (int r = 0; r < STAGE; r++)
+		{
+			const int e = threadIdx.x + r * THREADS, c = e / KP, j = e % KP;
+			const int s = src[o][c];
+			x.b[r] = (s >= 0 && j < 2 * P) ? T(mult[(long long)s * P * 2 + j]) : T(0);
+		}
+#pragma unroll
+		for (int n = 0; n < NT; n++)
+		{
+			const int s = wave == 0 ? src[o][n * 16 + col] : -1;
+			x.b0[n] = s >= 0 ? mult[(long long)s * P * 2] : 0.0;
+		}
+	};
+	// row k < P of a stacked multipole is Re b_k, then Im b_(k - P); rows past 2 P stay zero
+	auto stage = [&](const Operands& x, T* to) {
+#pragma unroll
+		for (int r = 0; r < STAGE; r++)
+		{
+			const int e = threadIdx.x + r * THREADS, c = e / KP, j = e % KP;
+			if (j < 2 * P) to[c * STRIDE + ((j & 1) ? P + (j >> 1) : (j >> 1))] = x.b[r];
+		}
+	};
+	auto multiply = [&](const Operands& x, const T* from) {
+#pragma unroll
+		for (int ks = 0; ks < KS; ks++)
+#pragma unroll
+			for (int n = 0; n < NT; n++)
+				acc[n] = MfmaVec<T>::mfma(x.a[ks], from[(n * 16 + col) * STRIDE + ks * 4 + kq], acc[n]);
+#pragma unroll
+		for (int n = 0; n < NT; n++) sum0[n] += x.b0[n];
+	};
+	auto next = [&]() {
+		const int o = __builtin_ctzll(todo);
+		todo &= todo - 1;
+		return o;
+	};
+	Operands x, y;
+	bool have = todo != 0;
+	if (have) load(next(), x);
+	while (have)
+	{
+		// each buffer is written two barriers after its last readers passed one
+		stage(x, gathered[0]);
+		__syncthreads();
+		bool more = todo != 0;
+		if (more) load(next(), y);
+		multiply(x, gathered[0]);
+		if (!more) break;
+		stage(y, gathered[1]);
+		__syncthreads();
+		have = todo != 0;
+		if (have) load(next(), x);
+		multiply(y, gathered[1]);
+	}
+#pragma unroll
+	for (int n = 0; n < NT; n++)
+	{
+		const int g = g0 + n * 16 + col;
+		if (g >= groups) continue;
+		const int t = first + 4 * g + q;
+		double* c = out + (long long)t * P * 2;
+		// the b_0 log h term in FP64 from the FP64 multipoles (b_0 is real), added after the product
+		double extra;
+		{
+#pragma clang fp contract(off)
+			extra = sum0[n] * log(hl[t]);
+		}
 #pragma unroll
 		for (int r = 0; r < 4; r++)
 		{
-			const int row = rt * 16 + MfmaVec<T>::row(kq, r);
+			const int row = wave * 16 + MfmaVec<T>::row(kq, r);
+			const double v = double(acc[n][r]) + (row == 0 ? extra : 0.0);
 			if (row < P)
-				c[2 * row] += double(acc[rt][r]) + (row == 0 ? sre * lh : 0.0);
+				c[2 * row] = v;
 			else if (row < 2 * P)
-				c[2 * (row - P) + 1] += double(acc[rt][r]) + (row == P ? sim * lh : 0.0);
+				c[2 * (row - P) + 1] = v;
 		}
+	}
+}
+
+// launches the instantiation for kp; wide: two column tiles per block
+template <typename T>
+void launch_m2l(int kp, bool wide, hipStream_t st, const T* At, const double* mult, double* out, const double* cx,
+	const double* cy, const double* hl, const int* nm2l, const int* m2l, int first, int groups, int p, unsigned long long* count)
+{
+	auto go = [&](auto kernel, int targets) {
+		kernel<<<unsigned((4 * ((groups + targets - 1) / targets) + 7) / 8 * 8), kp * 4, 0, st>>>(At, mult, out, cx, cy, hl, nm2l, m2l, first,
+			groups, p, count);
+	};
+	switch (kp)
+	{
+	case 16: wide ? go(k_m2l<T, 16, 2>, 32) : go(k_m2l<T, 16, 1>, 16); break;
+	case 32: wide ? go(k_m2l<T, 32, 2>, 32) : go(k_m2l<T, 32, 1>, 16); break;
+	case 48: wide ? go(k_m2l<T, 48, 2>, 32) : go(k_m2l<T, 48, 1>, 16); break;
+	default: wide ? go(k_m2l<T, 64, 2>, 32) : go(k_m2l<T, 64, 1>, 16); break;
 	}
 }
 
@@ -242,42 +316,19 @@ void Engine::m2l_prepare(int p, bool f32)
 	m2l_ready_f32_ = f32;
 }
 
-void Engine::m2l_level(int lev, int p, bool f32, hipEvent_t e0, hipEvent_t e1)
+// the M2L sums of every node at level 2 and below, into local_ (k_local adds the rest)
+void Engine::m2l_all(int p, bool f32)
 {
-	const int l0 = level_start_[lev], n = level_start_[lev + 1] - l0;
-	if (n <= 0)
-	{
-		MLENS_HIP_CHECK(hipEventRecord(e0, stream_));
-		MLENS_HIP_CHECK(hipEventRecord(e1, stream_));
-		return;
-	}
-	const int kp = m2l_kp(p);
-	const long long nsrc = (long long)M2L_OFFSETS * n;
-	if ((long long)m2l_src_.count < nsrc) m2l_src_.alloc(size_t(nsrc));
-	k_fill_int<<<unsigned((nsrc + 255) / 256), 256, 0, stream_>>>(m2l_src_.ptr, nsrc, -1);
-	int* bad = reinterpret_cast<int*>(m2l_count_.ptr + 1);
-	k_m2l_table<<<unsigned((n + 255) / 256), 256, 0, stream_>>>(ncx_.ptr, ncy_.ptr, nhl_.ptr, nnm2l_.ptr, nm2l_.ptr, l0, n,
-		m2l_src_.ptr, m2l_count_.ptr, bad);
-	const long long nms = (long long)n * kp;
-	const unsigned blocks = unsigned((n + M2L_WAVES * M2L_TARGETS_PER_WAVE - 1) / (M2L_WAVES * M2L_TARGETS_PER_WAVE));
+	const int first = level_start_[2], groups = (num_nodes_ - first) / 4;
+	if (groups <= 0) return;
+	// two column tiles halve the matrix traffic once one tile per block fills the device
+	const bool wide = groups >= 16 * num_cus_;
 	if (f32)
-	{
-		if ((long long)mstack_f_.count < nms) mstack_f_.alloc(size_t(nms));
-		k_mstack<float><<<unsigned((nms + 255) / 256), 256, 0, stream_>>>(mult_.ptr, l0, n, p, kp, mstack_f_.ptr);
-		MLENS_HIP_CHECK(hipEventRecord(e0, stream_));
-		k_m2l_mfma<float><<<blocks, 64 * M2L_WAVES, size_t(kp) * kp * sizeof(float), stream_>>>(m2l_af_.ptr, m2l_src_.ptr,
-			mstack_f_.ptr, mult_.ptr, local_.ptr, nhl_.ptr, l0, n, p, kp);
-		MLENS_HIP_CHECK(hipEventRecord(e1, stream_));
-	}
+		launch_m2l<float>(m2l_kp(p), wide, stream_, m2l_af_.ptr, mult_.ptr, local_.ptr, ncx_.ptr, ncy_.ptr, nhl_.ptr, nnm2l_.ptr,
+			nm2l_.ptr, first, groups, p, m2l_count_.ptr);
 	else
-	{
-		if ((long long)mstack_d_.count < nms) mstack_d_.alloc(size_t(nms));
-		k_mstack<double><<<unsigned((nms + 255) / 256), 256, 0, stream_>>>(mult_.ptr, l0, n, p, kp, mstack_d_.ptr);
-		MLENS_HIP_CHECK(hipEventRecord(e0, stream_));
-		k_m2l_mfma<double><<<blocks, 64 * M2L_WAVES, size_t(kp) * kp * sizeof(double), stream_>>>(m2l_ad_.ptr, m2l_src_.ptr,
-			mstack_d_.ptr, mult_.ptr, local_.ptr, nhl_.ptr, l0, n, p, kp);
-		MLENS_HIP_CHECK(hipEventRecord(e1, stream_));
-	}
+		launch_m2l<double>(m2l_kp(p), wide, stream_, m2l_ad_.ptr, mult_.ptr, local_.ptr, ncx_.ptr, ncy_.ptr, nhl_.ptr, nnm2l_.ptr,
+			nm2l_.ptr, first, groups, p, m2l_count_.ptr);
 	MLENS_HIP_CHECK(hipGetLastError());
 }
 

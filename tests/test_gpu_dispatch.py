@@ -77,3 +77,76 @@ def test_batch_tiles_and_pieces(general):
         batch.close()
     for m in objs:
         m.close()
+
+
+def write_field(path, stars, radius):
+    with open(path, "wb") as fh:
+        np.array([len(stars), 0], dtype=np.int32).tofile(fh)
+        np.array([radius, 0.0, 1.0]).tofile(fh)
+        np.ascontiguousarray(stars, dtype=np.float64).tofile(fh)
+
+
+def disk(rng, n, radius, centre=(0.0, 0.0)):
+    r, t = radius * np.sqrt(rng.random(n)), 2 * np.pi * rng.random(n)
+    return np.stack([centre[0] + r * np.cos(t), centre[1] + r * np.sin(t)], axis=1)
+
+
+def built(path, stars, order, mode=3):
+    """A built double-precision object over `stars` in a disk of radius 40."""
+    from irs_amd.microlensing.IPM.ipm import IPM
+    write_field(path, stars, 40.0)
+    m = IPM(kappa_tot=0.3, shear=0.3, light_loss=0.01, starfile=str(path), half_length_y1=0.5, half_length_y2=0.5,
+            num_pixels_y1=16, num_pixels_y2=16, is_double=True, expansion_order=order, m2l_mode=mode)
+    m.prepare()
+    m.build()
+    return m
+
+
+def coefficient_errors(m, tree):
+    for which in ("multipole", "local"):
+        g, o = m.export_coeffs(which), tree.coeffs(which)
+        yield which, np.max(np.abs(g - o) / np.maximum(np.max(np.abs(o), axis=1, keepdims=True), 1e-300))
+
+
+@pytest.mark.parametrize("n,cluster", [(1, 0), (32, 0), (33, 0), (300, 0), (3000, 0), (16384, 0), (16385, 0), (60000, 0),
+                                       (250000, 0), (2000, 1500), (2000, 20000)])
+def test_trees_of_every_split_path(oracle, tmp_path, n, cluster):
+    """A level is split by one block per node of 64, 256 or 1024 threads, or device-wide
+    above 16384 stars in a node, its nodes ranked by one block or, above 32768 of them,
+    by a device-wide scan; M2L runs one or two column tiles per block. Even fields and
+    fields with a cluster a few thousandths wide: the oracle's tree bit for bit, its
+    coefficients to FP64 rounding (the bound of the parity tests)."""
+    rng = np.random.default_rng(n + cluster)
+    xy = np.concatenate([disk(rng, n, 39.0), disk(rng, cluster, 2e-3, (3.1, -7.3))])
+    stars = np.concatenate([xy, np.full((len(xy), 1), 16.0 / len(xy))], axis=1)
+    say(f"[tree] {n} stars, {cluster} in a cluster")
+    m = built(tmp_path / "stars.bin", stars, 12)
+    tree = oracle.Tree(stars, m.root_half_length)
+    for got, want in zip(m.export_tree(), tree.export()):
+        np.testing.assert_array_equal(got, want)
+    np.testing.assert_array_equal(m.stars, tree.stars())
+    tree.fmm(12)
+    for which, err in coefficient_errors(m, tree):
+        say(f"[tree] {which}: {err:.1e}")
+        assert err < 1e-11, which
+    m.close()
+
+
+@pytest.mark.parametrize("order", [1, 3, 7, 8, 15, 16, 23, 24, 31])
+def test_fmm_at_the_edges_of_its_matrix_sizes(oracle, tmp_path, order):
+    """The stacked M2L matrices are padded to 16, 32, 48 or 64: the first and last order
+    of each, by recurrences, FP64 and FP32 MFMA, and with two column tiles per block.
+    FP64 to rounding; FP32 to single precision of the products (the parity tests' bounds)."""
+    rng = np.random.default_rng(order)
+    for n, modes in ((3000, (0, 3, 2)), (60000, (3,))):
+        stars = np.concatenate([disk(rng, n, 39.0), np.full((n, 1), 16.0 / n)], axis=1)
+        tree = None
+        for mode in modes:
+            m = built(tmp_path / "stars.bin", stars, order, mode)
+            if tree is None:
+                tree = oracle.Tree(stars, m.root_half_length)
+                tree.fmm(order)
+            for which, err in coefficient_errors(m, tree):
+                say(f"[fmm] {n} stars, order {order}, m2l_mode {mode}, {which}: {err:.1e}")
+                assert err < (2e-5 if mode == 2 else 1e-11)
+            m.close()
