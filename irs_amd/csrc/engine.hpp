@@ -71,6 +71,12 @@ struct CCFResult
 	bool has_nan = false;   // some error bound is not finite
 };
 
+struct MapExtremes
+{
+	double min, max;
+	double positive_min;   // smallest positive value, +infinity if there is none
+};
+
 struct ShootStats
 {
 	double ms = 0;                 // kernel time (HIP events)
@@ -128,9 +134,12 @@ public:
 	int last_tile_rows() const { return last_tile_rows_; }   // the height of the last shooting launch
 	void add_parity_maps();
 	void download_map(int which, void* host) const;   // 0 = total, 1 = minima, 2 = saddles
-	void map_minmax(int which, double* mn, double* mx);
-	void map_histogram(int which, bool log10_of_value, int factor, long long hist_min, long long length,
-		long long* host_hist);
+	/* of the first nmaps of total, minima, saddles (which must exist) */
+	void map_extremes(int nmaps, MapExtremes* out);
+	/* counts of round(value * factor - hist_min) in [0, length) and, with log_length > 0, of log10(value)
+	   likewise over the positive pixels: length + log_length counts per map */
+	void map_histograms(int nmaps, int factor, long long hist_min, long long length, long long log_min,
+		long long log_length, long long* host_hist);
 
 	/* critical curves (ccf_functions.cuh, ccf.cuh): refine nroots roots per phase for
 	   nphi + nb phases (nb branches of nphi / nb + 1 phases), starting from init_roots
@@ -229,9 +238,12 @@ private:
 	void ensure_tiled_maps();
 	void fold_tiled_maps();
 
+	template <typename F>
+	void with_maps(F f) const;
+
 	DeviceBuffer<int> scratch_i_;
 	DeviceBuffer<double> scratch_d_;
-	DeviceBuffer<long long> scratch_ll_;
+	DeviceBuffer<long long> scratch_ll_, hist_;
 };
 
 /*

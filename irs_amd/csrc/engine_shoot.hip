@@ -1944,102 +1944,155 @@ void Engine::download_map(int which, void* host) const
 	MLENS_HIP_CHECK(hipMemcpy(host, b.ptr, size_t(npix_[0]) * npix_[1] * elem, hipMemcpyDeviceToHost));
 }
 
+// the maps of a shot: the total, then minima and saddles
 template <typename V>
-__global__ void k_minmax(const V* v, long long n, double* out)
+struct MapSet
 {
-	__shared__ double slo[256], shi[256];
-	double lo = 1e308, hi = -1e308;
-	for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (long long)gridDim.x * blockDim.x)
+	const V* map[3];
+};
+
+// minimum, maximum and smallest positive value of a map in n partials per map (blockIdx.y = map), then of the
+// partials of every map (k_extremes_of_partials, one block per map)
+struct Extremes
+{
+	double lo, hi, pos;
+	__device__ void take(double l, double h, double p)
 	{
-		double x = double(v[i]);
-		lo = fmin(lo, x);
-		hi = fmax(hi, x);
+		lo = fmin(lo, l);
+		hi = fmax(hi, h);
+		pos = fmin(pos, p);
 	}
-	slo[threadIdx.x] = lo;
-	shi[threadIdx.x] = hi;
+};
+
+__device__ inline void block_extremes(Extremes e, Extremes* out)
+{
+	__shared__ Extremes part[4];
+	for (int off = 32; off > 0; off >>= 1) e.take(__shfl_xor(e.lo, off), __shfl_xor(e.hi, off), __shfl_xor(e.pos, off));
+	if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = e;
 	__syncthreads();
-	for (int off = blockDim.x / 2; off > 0; off >>= 1)
-	{
-		if ((int)threadIdx.x < off)
-		{
-			slo[threadIdx.x] = fmin(slo[threadIdx.x], slo[threadIdx.x + off]);
-			shi[threadIdx.x] = fmax(shi[threadIdx.x], shi[threadIdx.x + off]);
-		}
-		__syncthreads();
-	}
-	if (threadIdx.x == 0)
-	{
-		out[2 * blockIdx.x] = slo[0];
-		out[2 * blockIdx.x + 1] = shi[0];
-	}
+	if (threadIdx.x != 0) return;
+	for (int w = 1; w < 4; w++) e.take(part[w].lo, part[w].hi, part[w].pos);
+	*out = e;
 }
 
-void Engine::map_minmax(int which, double* mn, double* mx)
-{
-	const DeviceBuffer<char>& b = which == 0 ? map_ : (which == 1 ? map_min_ : map_sad_);
-	long long n = (long long)npix_[0] * npix_[1];
-	const int nb = 1024;
-	scratch_d_.alloc(2 * nb);
-	if (map_int_)
-		k_minmax<int><<<nb, 256, 0, stream_>>>((const int*)b.ptr, n, scratch_d_.ptr);
-	else if (map_fp32_)
-		k_minmax<float><<<nb, 256, 0, stream_>>>((const float*)b.ptr, n, scratch_d_.ptr);
-	else
-		k_minmax<double><<<nb, 256, 0, stream_>>>((const double*)b.ptr, n, scratch_d_.ptr);
-	MLENS_HIP_CHECK(hipGetLastError());
-	std::vector<double> h(2 * nb);
-	MLENS_HIP_CHECK(hipMemcpyAsync(h.data(), scratch_d_.ptr, h.size() * sizeof(double), hipMemcpyDeviceToHost, stream_));
-	MLENS_HIP_CHECK(hipStreamSynchronize(stream_));
-	double lo = 1e308, hi = -1e308;
-	for (int i = 0; i < nb; i++)
-	{
-		lo = std::min(lo, h[2 * i]);
-		hi = std::max(hi, h[2 * i + 1]);
-	}
-	*mn = lo;
-	*mx = hi;
-}
-
-// array_functions.cuh:114-160: index = round(value * factor - min), or of log10(value)
 template <typename V>
-__global__ void k_histogram(const V* v, long long n, int log_mode, int factor, long long hmin, long long len,
-	unsigned long long* hist)
+__global__ __launch_bounds__(256) void k_extremes(MapSet<V> maps, long long n, Extremes* partials)
 {
+	const V* v = maps.map[blockIdx.y];
+	Extremes e{1e308, -1e308, HUGE_VAL};
 	for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (long long)gridDim.x * blockDim.x)
 	{
-		double x = double(v[i]);
-		long long idx;
-		if (log_mode)
+		const double x = double(v[i]);
+		e.take(x, x, x > 0 ? x : HUGE_VAL);
+	}
+	block_extremes(e, partials + (long long)blockIdx.y * gridDim.x + blockIdx.x);
+}
+
+__global__ __launch_bounds__(256) void k_extremes_of_partials(const Extremes* partials, int n, Extremes* out)
+{
+	Extremes e{1e308, -1e308, HUGE_VAL};
+	for (int i = threadIdx.x; i < n; i += 256)
+	{
+		const Extremes p = partials[(long long)blockIdx.x * n + i];
+		e.take(p.lo, p.hi, p.pos);
+	}
+	block_extremes(e, out + blockIdx.x);
+}
+
+constexpr int EXTREMES_BLOCKS = 512;
+constexpr int HIST_WINDOW = 8192;       // bins of each histogram that a block counts in LDS (32 KB)
+constexpr int HIST_THREADS = 1024;
+constexpr int HIST_PIXELS = 16384;      // pixels a block takes at least
+constexpr int HIST_BLOCKS_MAX = 512;    // two blocks fill a CU's LDS
+
+/*
+Histograms of every map (blockIdx.y), array_functions.cuh:114-160: index = round(value * factor - min),
+and with log_len > 0 the same of log10(value) over the positive pixels, in one pass. Each block counts the
+first HIST_WINDOW bins in LDS and adds them to the 64-bit counts once; the few pixels past the window go
+straight to them. A block takes HIST_PIXELS pixels or more, so that it meets a bin several times over: with a
+global atomic per pixel, a 1000^2 map took 270 us for each of its two histograms (a ray-count map 826 us),
+since a few thousand hot bins serialise. hist: [map][len + log_len].
+*/
+template <typename V>
+__global__ __launch_bounds__(HIST_THREADS) void k_histograms(MapSet<V> maps, long long n, int factor, long long hmin, long long len,
+	long long log_min, long long log_len, unsigned long long* hist)
+{
+	__shared__ unsigned bins[2][HIST_WINDOW];
+	for (int i = threadIdx.x; i < 2 * HIST_WINDOW; i += HIST_THREADS) bins[0][i] = 0;
+	__syncthreads();
+	unsigned long long* lin = hist + blockIdx.y * (len + log_len);
+	unsigned long long* lg = lin + len;
+	const V* v = maps.map[blockIdx.y];
+	for (long long i = (long long)blockIdx.x * HIST_THREADS + threadIdx.x; i < n; i += (long long)gridDim.x * HIST_THREADS)
+	{
+		const double x = double(v[i]);
+		const long long idx = llround(1.0 * x * factor - double(hmin));
+		if (idx >= 0 && idx < len)
 		{
-			if (!(x > 0)) continue;
-			idx = llround(log10(x) * factor - double(hmin));
+			if (idx < HIST_WINDOW) atomicAdd(&bins[0][idx], 1u);
+			else atomicAdd(&lin[idx], 1ull);
 		}
-		else
+		if (log_len > 0 && x > 0)
 		{
-			idx = llround(1.0 * x * factor - double(hmin));
+			const long long k = llround(log10(x) * factor - double(log_min));
+			if (k >= 0 && k < log_len)
+			{
+				if (k < HIST_WINDOW) atomicAdd(&bins[1][k], 1u);
+				else atomicAdd(&lg[k], 1ull);
+			}
 		}
-		if (idx >= 0 && idx < len) atomicAdd(&hist[idx], 1ull);
+	}
+	__syncthreads();
+	for (int i = threadIdx.x; i < HIST_WINDOW; i += HIST_THREADS)
+	{
+		if (bins[0][i]) atomicAdd(&lin[i], (unsigned long long)bins[0][i]);
+		if (bins[1][i]) atomicAdd(&lg[i], (unsigned long long)bins[1][i]);
 	}
 }
 
-void Engine::map_histogram(int which, bool log_mode, int factor, long long hmin, long long len, long long* host_hist)
+// f(MapSet of the maps' type) for the total map and, with parities, minima and saddles
+template <typename F>
+void Engine::with_maps(F f) const
 {
-	const DeviceBuffer<char>& b = which == 0 ? map_ : (which == 1 ? map_min_ : map_sad_);
-	long long n = (long long)npix_[0] * npix_[1];
-	DeviceBuffer<long long> dh;
-	dh.alloc(std::max(len, 1LL));
-	MLENS_HIP_CHECK(hipMemsetAsync(dh.ptr, 0, sizeof(long long) * std::max(len, 1LL), stream_));
-	unsigned long long* hp = reinterpret_cast<unsigned long long*>(dh.ptr);
-	const int nb = 2048;
-	if (map_int_)
-		k_histogram<int><<<nb, 256, 0, stream_>>>((const int*)b.ptr, n, log_mode, factor, hmin, len, hp);
-	else if (map_fp32_)
-		k_histogram<float><<<nb, 256, 0, stream_>>>((const float*)b.ptr, n, log_mode, factor, hmin, len, hp);
-	else
-		k_histogram<double><<<nb, 256, 0, stream_>>>((const double*)b.ptr, n, log_mode, factor, hmin, len, hp);
+	auto set = [&](auto* zero) {
+		using V = std::remove_pointer_t<decltype(zero)>;
+		f(MapSet<V>{{(const V*)map_.ptr, (const V*)map_min_.ptr, (const V*)map_sad_.ptr}});
+	};
+	if (map_int_) set((int*)nullptr);
+	else if (map_fp32_) set((float*)nullptr);
+	else set((double*)nullptr);
+}
+
+void Engine::map_extremes(int nmaps, MapExtremes* out)
+{
+	static_assert(sizeof(Extremes) == sizeof(MapExtremes), "copied as they are");
+	const long long n = (long long)npix_[0] * npix_[1];
+	const unsigned nb = unsigned(std::min<long long>(EXTREMES_BLOCKS, (n + 1023) / 1024));
+	scratch_d_.alloc(3 * size_t(nmaps) * (EXTREMES_BLOCKS + 1));
+	Extremes* partials = reinterpret_cast<Extremes*>(scratch_d_.ptr);
+	Extremes* total = partials + nmaps * EXTREMES_BLOCKS;
+	with_maps([&](auto maps) { k_extremes<<<dim3(nb, nmaps), 256, 0, stream_>>>(maps, n, partials); });
+	k_extremes_of_partials<<<nmaps, 256, 0, stream_>>>(partials, int(nb), total);
 	MLENS_HIP_CHECK(hipGetLastError());
+	MLENS_HIP_CHECK(hipMemcpyAsync(out, total, nmaps * sizeof(Extremes), hipMemcpyDeviceToHost, stream_));
 	MLENS_HIP_CHECK(hipStreamSynchronize(stream_));
-	MLENS_HIP_CHECK(hipMemcpy(host_hist, dh.ptr, sizeof(long long) * len, hipMemcpyDeviceToHost));
+}
+
+void Engine::map_histograms(int nmaps, int factor, long long hmin, long long len, long long log_min, long long log_len,
+	long long* host_hist)
+{
+	const long long n = (long long)npix_[0] * npix_[1];
+	const size_t total = size_t(nmaps) * size_t(len + log_len);
+	hist_.alloc(total);
+	MLENS_HIP_CHECK(hipMemsetAsync(hist_.ptr, 0, sizeof(long long) * total, stream_));
+	unsigned long long* hp = reinterpret_cast<unsigned long long*>(hist_.ptr);
+	const unsigned nb = unsigned(std::min<long long>(HIST_BLOCKS_MAX, (n + HIST_PIXELS - 1) / HIST_PIXELS));
+	with_maps([&](auto maps) {
+		k_histograms<<<dim3(nb, nmaps), HIST_THREADS, 0, stream_>>>(maps, n, factor, hmin, len, log_min, log_len, hp);
+	});
+	MLENS_HIP_CHECK(hipGetLastError());
+	MLENS_HIP_CHECK(hipMemcpyAsync(host_hist, hist_.ptr, sizeof(long long) * total, hipMemcpyDeviceToHost, stream_));
+	MLENS_HIP_CHECK(hipStreamSynchronize(stream_));
 }
 
 }  // namespace mlens

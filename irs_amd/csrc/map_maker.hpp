@@ -732,11 +732,12 @@ private:
 		const int factor = IS_IPM ? 1000 : 1;
 		T mu_min_theory = 1 / ((1 - kappa_tot + kappa_star) * (1 - kappa_tot + kappa_star));
 		long long lo = std::numeric_limits<long long>::max(), hi = std::numeric_limits<long long>::min();
+		MapExtremes ext[3];
+		engine_->map_extremes(nmaps, ext);
 		for (int k = 0; k < nmaps; k++)
 		{
-			double mn, mx;
-			engine_->map_minmax(k, &mn, &mx);
-			// in double, as k_histogram bins every pixel (the reference rounds these two in T
+			const double mn = ext[k].min, mx = ext[k].max;
+			// in double, as k_histograms bins every pixel (the reference rounds these two in T
 			// and its pixels in double, ipm.cuh:972-973 and array_functions.cuh:127, so a float
 			// map's extreme pixel can fall outside its own histogram there)
 			long long a = IS_IPM ? std::llround(double(T(mn)) * factor) : (long long)mn;
@@ -755,57 +756,30 @@ private:
 		min_mag_ = lo;
 		max_mag_ = hi;
 		long long len = hi - lo + 1;
+		// log10 histogram over the positive pixels (a zero pixel has no log10)
+		long long llo = std::numeric_limits<long long>::max(), lhi = std::numeric_limits<long long>::min();
+		for (int k = 0; k < nmaps && IS_IPM; k++)
+		{
+			const double pos_min = ext[k].positive_min;
+			if (!std::isfinite(pos_min) || !(ext[k].max > 0)) continue;
+			llo = std::min(llo, (long long)std::llround(std::log10(double(T(pos_min))) * factor));
+			lhi = std::max(lhi, (long long)std::llround(std::log10(double(T(ext[k].max))) * factor));
+		}
+		const long long log_len = lhi >= llo ? lhi - llo + 1 : 0;
+		if (log_len > 0)
+		{
+			min_log_mag_ = llo;
+			max_log_mag_ = lhi;
+		}
+		std::vector<long long> counts(size_t(nmaps) * size_t(len + log_len));
+		engine_->map_histograms(nmaps, factor, lo, len, llo, log_len, counts.data());
 		for (int k = 0; k < nmaps; k++)
 		{
-			hist_[k].assign(len, 0);
-			engine_->map_histogram(k, false, factor, lo, len, hist_[k].data());
-		}
-		if (IS_IPM)
-		{
-			// log10 histogram over the positive pixels (a zero pixel has no log10)
-			long long llo = std::numeric_limits<long long>::max(), lhi = std::numeric_limits<long long>::min();
-			for (int k = 0; k < nmaps; k++)
-			{
-				double mn, mx;
-				engine_->map_minmax(k, &mn, &mx);
-				double pos_min = mn > 0 ? mn : positive_min(k);
-				if (!(pos_min > 0) || !(mx > 0)) continue;
-				llo = std::min(llo, (long long)std::llround(std::log10(double(T(pos_min))) * factor));
-				lhi = std::max(lhi, (long long)std::llround(std::log10(double(T(mx))) * factor));
-			}
-			if (lhi >= llo)
-			{
-				min_log_mag_ = llo;
-				max_log_mag_ = lhi;
-				for (int k = 0; k < nmaps; k++)
-				{
-					log_hist_[k].assign(lhi - llo + 1, 0);
-					engine_->map_histogram(k, true, factor, llo, lhi - llo + 1, log_hist_[k].data());
-				}
-			}
+			const auto first = counts.begin() + k * (len + log_len);
+			hist_[k].assign(first, first + len);
+			if (log_len > 0) log_hist_[k].assign(first + len, first + len + log_len);
 		}
 		return true;
-	}
-
-	double positive_min(int k)
-	{
-		// smallest positive pixel of map k, on the host copy of the map
-		size_t n = size_t(num_pixels_y.re) * num_pixels_y.im;
-		std::vector<double> v(n);
-		if (engine_->maps_are_fp32())
-		{
-			std::vector<float> f(n);
-			engine_->download_map(k, f.data());
-			for (size_t i = 0; i < n; i++) v[i] = f[i];
-		}
-		else
-		{
-			engine_->download_map(k, v.data());
-		}
-		double m = std::numeric_limits<double>::infinity();
-		for (double x : v)
-			if (x > 0 && x < m) m = x;
-		return m;
 	}
 
 	// the star field in tree order, as get_stars returns it

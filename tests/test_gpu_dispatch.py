@@ -150,3 +150,31 @@ def test_fmm_at_the_edges_of_its_matrix_sizes(oracle, tmp_path, order):
                 say(f"[fmm] {n} stars, order {order}, m2l_mode {mode}, {which}: {err:.1e}")
                 assert err < (2e-5 if mode == 2 else 1e-11)
             m.close()
+
+
+@pytest.mark.parametrize("irs,double", [(False, False), (False, True), (True, False)])
+@pytest.mark.parametrize("n1,n2", [(1, 1), (128, 128), (129, 127), (400, 300)])
+def test_histograms_inside_and_past_the_window(tmp_path, irs, double, n1, n2):
+    """Blocks of at least 16384 pixels count the first 8192 bins of both histograms in LDS:
+    maps of less than, exactly and several blocks, whose bright pixels and ray counts lie
+    past the window. Every bin of the files against numpy's count of the returned maps."""
+    prefix = str(tmp_path) + "/"
+    m = make(dict(kappa_tot=0.45, shear=0.45, kappa_star=0.36, mass_function="equal"), irs=irs, half_length_y1=0.02 * n1,
+             half_length_y2=0.02 * n2, num_pixels_y1=n1, num_pixels_y2=n2, num_rays_y=900 if irs else 4, light_loss=0.01,
+             random_seed=5, expansion_order=12, write_parities=True, write_histograms=True, outfile_prefix=prefix,
+             **({"is_double": double} if not irs else {}))
+    m.save()
+    maps = (m.num_rays, m.num_rays_minima, m.num_rays_saddles) if irs else (
+        m.magnifications, m.magnifications_minima, m.magnifications_saddles)
+    for suffix, mp in zip(("", "_minima", "_saddles"), maps):
+        v = np.asarray(mp, dtype=np.float64).ravel()
+        kinds = [("numrays_numpixels" if irs else "mags_numpixels", v if irs else 1000.0 * v)]
+        if not irs:
+            kinds.append(("log_mags_numpixels", 1000.0 * np.log10(v[v > 0])))
+        for kind, x in kinds:
+            t = np.trunc(x)
+            u, c = np.unique((t + np.where(np.abs(x - t) >= 0.5, np.sign(x), 0.0)).astype(np.int64), return_counts=True)
+            got = np.loadtxt(prefix + ("irs_" if irs else "ipm_") + kind + suffix + ".txt", dtype=np.int64, ndmin=2)
+            np.testing.assert_array_equal(got, np.column_stack([u, c]), err_msg=kind + suffix)
+            say(f"[hist] {kind}{suffix}: {len(u)} bins up to {u[-1]}")
+    m.close()
