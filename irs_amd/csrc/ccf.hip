@@ -8,13 +8,14 @@
 // from positions next to the stars, then stepping phi outwards in both
 // directions with the previous phase's roots as starting points.
 //
-// On this GPU eight lanes update one root, a block of 256 lanes 32 roots of one
-// phase. The sums over all roots and all stars of every update stream through
-// LDS tiles, split over the root's eight lanes, so a root update costs
-// O((roots + stars) / 8) arithmetic per lane with one global read per tile
-// element per block. Updates are simultaneous (Jacobi): an iteration reads one
-// copy of the roots and writes the other, so the result does not depend on
-// the order in which blocks run.
+// On this GPU a wave of 64 lanes updates one root: the sums over all roots and
+// all stars are split over its lanes, so a root update costs
+// O((roots + stars) / 64) arithmetic per lane. Updates are simultaneous
+// (Jacobi): an iteration reads one copy of the roots and writes the other, so
+// the result does not depend on the order in which blocks run. Each branch and
+// side is a chain of steps and iterations that only its own roots link; the
+// blocks of a chain stay resident and meet at a barrier after each iteration,
+// and leave a step as soon as every root has converged.
 #include "shoot_common.hpp"
 
 #include <algorithm>
@@ -27,7 +28,6 @@ namespace mlens
 namespace
 {
 
-constexpr int CCF_THREADS = 256;
 constexpr double CCF_PI = 3.14159265358979323846;
 
 // the derivative terms of the lens equation at z, in the node z falls in
@@ -42,6 +42,7 @@ struct CCTerms
 // alpha_star.cuh:55-114, alpha_local.cuh:52-108, alpha_smooth.cuh:142-316. With part < parts, only
 // the near stars whose position in the node's near list is part (mod parts) enter S1 and S2, and the
 // expansion and smooth terms are evaluated by part 0 only (zero elsewhere): the caller adds the parts.
+template <bool LIN = false>
 __device__ CCTerms cc_terms(const ShootArgs& a, int node, dcx z, bool second, int part = 0, int parts = 1)
 {
 	CCTerms t;
@@ -89,6 +90,11 @@ __device__ CCTerms cc_terms(const ShootArgs& a, int node, dcx z, bool second, in
 	}
 	t.L1 = dev::scale(l1, a.theta2 / (h * h));
 	t.L2 = dev::scale(l2, a.theta2 / (h * h * h));
+	if (LIN)
+	{
+		t.ddz = -a.kappastar;
+		return t;
+	}
 	const dcx corner = dcx{a.corner_re, a.corner_im};
 	dev::d_alpha_smooth(z, a.kappastar, a.rectangular, a.approx, a.taylor_smooth, corner, t.ddz, t.ddzb);
 	t.d2s = second ? dev::d2_alpha_smooth(z, a.kappastar, a.rectangular, a.approx, a.taylor_smooth, corner) : dcx{0, 0};
@@ -128,142 +134,339 @@ __device__ __forceinline__ CCRow cc_row(int c, int sgn, int j, int nphi, int nb)
 	return r;
 }
 
-/*
-One Aberth iteration of the roots at step j of every branch and side
-(ccf_functions.cuh:171-240, 309-386). Each root is updated by CCF_PARTS
-consecutive lanes, which share its sums over the other roots, the stars (the
-poles) and its near stars, and combine them with butterfly shuffles; the
-group's first lane evaluates the expansion and smooth terms and writes the
-root. Block (x, y): roots x * CCF_ROOTS + [0, CCF_ROOTS) of branch y / sides,
-side y % sides (side 0 steps phi down, side 1 up; at j = 0 there is one
-side). src and dst hold (nphi + nb) rows of nroots roots.
-*/
-constexpr int CCF_PARTS = 64;
-constexpr int CCF_ROOTS = CCF_THREADS / CCF_PARTS;
-
-__device__ __forceinline__ double group_sum(double v)
+__device__ __forceinline__ double wave_sum(double v)
 {
 #pragma unroll
-	for (int o = CCF_PARTS / 2; o > 0; o >>= 1) v += __shfl_xor(v, o);
+	for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
 	return v;
 }
 
-__global__ __launch_bounds__(CCF_THREADS) void k_ccf_iterate(ShootArgs a, const dcx* __restrict__ src, dcx* __restrict__ dst,
-	char* __restrict__ fin, int* __restrict__ leaf_cache, int nroots, int nstars, int circle_pole, int j, int nphi, int nb,
-	int sides)
+/*
+The derivative terms of cc_terms at z in leaf `node` (the same in every lane), with one near star per lane,
+S1 and S2 summed over the wave. Each lane fetches one near star (the leaf's table pads the list with massless
+ones) and one coefficient of the expansion at the start, so that nothing below waits for memory.
+*/
+struct CCLeaf
 {
-	__shared__ double tx[CCF_THREADS], ty[CCF_THREADS];
-	const int c = blockIdx.y / sides, b = blockIdx.y % sides;
-	const int sgn = (sides == 1) ? 0 : (b == 0 ? -1 : 1);
-	const CCRow R = cc_row(c, sgn == 0 ? 1 : sgn, sgn == 0 ? 0 : j, nphi, nb);
-	const dcx* row = src + (long long)R.row * nroots;
-	const int part = threadIdx.x % CCF_PARTS;
-	const int k = blockIdx.x * CCF_ROOTS + threadIdx.x / CCF_PARTS;
-	const bool mine = k < nroots;
-	const long long slot = ((long long)c * 2 + b) * nroots + k;
-	char* done = fin + slot;
-	const bool active = mine && !*done;
-	const dcx z = mine ? row[k] : dcx{0, 0};
-	// this lane's share of the sums over the other roots and over the poles (stars)
-	double rx = 0, ry = 0, px = 0, py = 0;
-	for (int t0 = 0; t0 < nroots; t0 += CCF_THREADS)
-	{
-		const int i = t0 + threadIdx.x;
-		tx[threadIdx.x] = i < nroots ? row[i].re : 0;
-		ty[threadIdx.x] = i < nroots ? row[i].im : 0;
-		__syncthreads();
-		if (active)
-		{
-			const int n = min(CCF_THREADS, nroots - t0);
-			for (int q = part; q < n; q += CCF_PARTS)
-			{
-				if (t0 + q == k) continue;
-				const double dx = z.re - tx[q], dy = z.im - ty[q];
-				const double ir2 = dev::rcp64(dx * dx + dy * dy);
-				rx += dx * ir2;
-				ry -= dy * ir2;
-			}
-		}
-		__syncthreads();
-	}
-	for (int t0 = 0; t0 < nstars; t0 += CCF_THREADS)
-	{
-		const int i = t0 + threadIdx.x;
-		tx[threadIdx.x] = i < nstars ? a.sx[i] : 0;
-		ty[threadIdx.x] = i < nstars ? a.sy[i] : 0;
-		__syncthreads();
-		if (active)
-		{
-			const int n = min(CCF_THREADS, nstars - t0);
-			for (int q = part; q < n; q += CCF_PARTS)
-			{
-				const double dx = z.re - tx[q], dy = z.im - ty[q];
-				const double ir2 = dev::rcp64(dx * dx + dy * dy);
-				px += dx * ir2;
-				py -= dy * ir2;
-			}
-		}
-		__syncthreads();
-	}
-	// the whole group follows the same branch: it shares its root and its done flag
-	if (!active)
-	{
-		if (mine && part == 0) dst[(long long)R.row * nroots + k] = z;
-		return;
-	}
-	// the root's leaf from the previous iteration while the root stays strictly inside
-	// it (there the tree descent would end in the same leaf), else a fresh descent
-	const int cached = leaf_cache[slot];
-	bool inside = false;
-	if (cached >= 0)
-	{
-		const double h = a.nhl[cached] * (1 - 1e-12);
-		inside = fabs(z.re - a.ncx[cached]) < h && fabs(z.im - a.ncy[cached]) < h;
-	}
-	const int node = inside ? cached : find_node(a, z.re, z.im);
-	if (!inside && part == 0) leaf_cache[slot] = a.nchild0[node] < 0 ? node : -1;
-	CCTerms t = cc_terms(a, node, z, true, part, CCF_PARTS);
-	rx = group_sum(rx);
-	ry = group_sum(ry);
-	px = group_sum(px);
-	py = group_sum(py);
-	t.S1.re = group_sum(t.S1.re);
-	t.S1.im = group_sum(t.S1.im);
-	t.S2.re = group_sum(t.S2.re);
-	t.S2.im = group_sum(t.S2.im);
-	if (part != 0) return;
-	dcx* out = dst + (long long)R.row * nroots + k;
-	const dcx f0 = cc_f0(a, t, R.phi);
-	if (cc_inv_mu_error(a, t, f0) < 1e-9)
-	{
-		// 1/mu is already below 1e-9 here (both bounds of ccf_functions.cuh:207-211)
-		*out = z;
-		*done = 1;
-		return;
-	}
-	const dcx f1 = dcx{-2 * a.theta2 * t.S2.re - t.L2.re - t.d2s.re, -2 * a.theta2 * t.S2.im - t.L2.im + t.d2s.im};
-	dcx psum = dcx{2 * px, 2 * py};
-	if (circle_pole)
-	{
-		const dcx iz = dev::cdiv(dcx{1, 0}, z);
-		psum = dev::add(psum, dev::scale(iz, 2));
-	}
-	const dcx den = dev::add(f1, dev::mul(f0, dcx{psum.re - rx, psum.im - ry}));
-	const dcx zn = dev::sub(z, dev::cdiv(f0, den));
-	*out = zn;
-	if (dev::cabs(dev::sub(zn, z)) / sqrt(a.theta2) < 1e-9) *done = 1;
+	double x, y, m;     // this lane's near star
+	double cre, cim;    // coefficient `lane` of the local expansion
+	double cx, cy, h;
+	int near;           // near stars in the table
+};
+
+__device__ __forceinline__ CCLeaf cc_load_leaf(const ShootArgs& a, int node)
+{
+	const int lane = threadIdx.x & 63;
+	const long long L = a.leaf_of_node[node];
+	CCLeaf f;
+	f.near = a.leaf_near_n[L] & 0xffff;
+	const double* s = a.near_d + (L * MAX_NUM_STARS_DIRECT + min(lane, MAX_NUM_STARS_DIRECT - 1)) * 3;
+	f.x = s[0];
+	f.y = s[1];
+	f.m = s[2];
+	const double* c = a.local + 2 * ((long long)node * (a.p + 1) + min(lane, a.p));
+	f.cre = c[0];
+	f.cim = c[1];
+	f.cx = a.ncx[node];
+	f.cy = a.ncy[node];
+	f.h = a.nhl[node];
+	return f;
 }
 
-// roots of step j start at those of step j - 1 on each side; clear the done flags
-__global__ void k_ccf_prepare(dcx* roots, char* fin, int nroots, int j, int nphi, int nb)
+__device__ __forceinline__ double lane_value(double v, int lane)
+{
+	const unsigned long long b = __builtin_bit_cast(unsigned long long, v);
+	const unsigned lo = __builtin_amdgcn_readlane(unsigned(b), lane), hi = __builtin_amdgcn_readlane(unsigned(b >> 32), lane);
+	return __builtin_bit_cast(double, (static_cast<unsigned long long>(hi) << 32) | lo);
+}
+
+template <bool LIN>
+__device__ __forceinline__ CCTerms cc_terms_leaf(const ShootArgs& a, const CCLeaf& f, dcx z)
+{
+	CCTerms t;
+	t.S1 = t.S2 = dcx{0, 0};
+	if (int(threadIdx.x & 63) < f.near)
+	{
+		const double dx = z.re - f.x, dy = z.im - f.y;
+		const double ir2 = dev::rcp64(dx * dx + dy * dy);
+		const double ux = dx * ir2, uy = -dy * ir2;
+		const double u2x = ux * ux - uy * uy, u2y = 2 * ux * uy;
+		t.S1.re += f.m * u2x;
+		t.S1.im += f.m * u2y;
+		t.S2.re += f.m * (u2x * ux - u2y * uy);
+		t.S2.im += f.m * (u2x * uy + u2y * ux);
+	}
+	const dcx dz = dcx{(z.re - f.cx) / f.h, (z.im - f.cy) / f.h};
+	dcx l1 = {0, 0}, l2 = {0, 0};
+	for (int i = a.p; i >= 2; i--)
+	{
+		const dcx c = dcx{lane_value(f.cre, i), lane_value(f.cim, i)};
+		l1 = dev::add(dev::mul(l1, dz), dev::scale(c, double(i) * (i - 1)));
+		if (i >= 3) l2 = dev::add(dev::mul(l2, dz), dev::scale(c, double(i) * (i - 1) * (i - 2)));
+	}
+	t.L1 = dev::scale(l1, a.theta2 / (f.h * f.h));
+	t.L2 = dev::scale(l2, a.theta2 / (f.h * f.h * f.h));
+	t.ddz = -a.kappastar;
+	t.ddzb = t.d2s = dcx{0, 0};
+	if (LIN) return t;
+	const dcx corner = dcx{a.corner_re, a.corner_im};
+	dev::d_alpha_smooth(z, a.kappastar, a.rectangular, a.approx, a.taylor_smooth, corner, t.ddz, t.ddzb);
+	t.d2s = dev::d2_alpha_smooth(z, a.kappastar, a.rectangular, a.approx, a.taylor_smooth, corner);
+	return t;
+}
+
+// Roots cross between the blocks of a chain through these: relaxed atomics of device scope, which the
+// per-XCD L2 caches do not hold back, so that nothing else cached (tree, stars) has to be invalidated.
+__device__ __forceinline__ double load_shared(const double* p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+__device__ __forceinline__ void store_shared(double* p, double v) { __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+
+/*
+The barrier after iteration `slot` of a chain of `blocks` blocks: each adds one to the low half of the slot's word
+and its count of unconverged roots to the high half. Returns the chain's total (final, and so the same in every
+block, once all have arrived), or -1 if some block waited CCF_SPINS polls in vain and set *failed. Every slot is
+used once and starts at zero.
+*/
+constexpr int CCF_THREADS = 512;
+constexpr int CCF_TILE = 2048;   // roots and stars staged in LDS at a time (32 KB each)
+constexpr long long CCF_SPINS = 1ll << 24;
+
+__device__ int chain_barrier(unsigned long long* slot, int blocks, int active, int* failed)
+{
+	__shared__ int result;
+	// this wave's stores have reached the coherence point; then every wave's have
+	asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+	__syncthreads();
+	if (threadIdx.x == 0)
+	{
+		unsigned long long v = __hip_atomic_fetch_add(slot, 1ull + ((unsigned long long)active << 32), __ATOMIC_RELAXED,
+			__HIP_MEMORY_SCOPE_AGENT);
+		long long spins = 0;
+		result = 0;
+		do
+		{
+			v = __hip_atomic_load(slot, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+			if (int(v & 0xffffffffu) == blocks) break;
+			if (++spins > CCF_SPINS || __hip_atomic_load(failed, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+			{
+				__hip_atomic_store(failed, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+				result = -1;
+				break;
+			}
+			__builtin_amdgcn_s_sleep(1);
+		} while (true);
+		if (result == 0) result = int(v >> 32);
+	}
+	__syncthreads();
+	const int r = result;
+	asm volatile("" ::: "memory");
+	return r;
+}
+
+/*
+Steps j0 .. j1 of chains first_chain + [0, gridDim.y) (ccf_functions.cuh:171-240, 309-386): chain c * sides + b is
+branch c, side b (side 0 steps phi down, side 1 up; at j = 0 there is one side). A step starts from the roots of
+the one before it and runs at most `iters` Aberth iterations; once every root of the chain has converged the rest
+would change nothing and is left out. Blocks of eight waves, a wave per root at a time, root by root round the
+chain's gridDim.x blocks. 137 stars (274 roots, 100 phases): 1.78 ms, against 5.20 ms with one launch per
+iteration and all 20 of them at every step; 1500 stars, 20 phases: 3.0 against 4.9 ms. A step takes about seven
+iterations of 5 us, most of which is the round trip through the barrier and the shared roots. Blocks of 256 or
+1024 threads took 1.74 and 2.37 ms, and 4.1 and 2.7 ms on the larger field. rows: (nphi + nb) rows of nroots roots, the result; work: two copies of each chain's
+roots; slots: iters words per step of each chain, zeroed. Every block of a chain must be resident (a cooperative
+launch), since it waits for the others.
+*/
+template <bool LIN>
+__global__ __launch_bounds__(CCF_THREADS) void k_ccf_chain(ShootArgs a, dcx* __restrict__ rows, double* work, char* __restrict__ fin,
+	int* __restrict__ leaf_cache, unsigned long long* slots, int* failed, int nroots, int nstars, int circle_pole, int j0, int j1,
+	int nphi, int nb, int sides, int iters, int first_chain)
+{
+	__shared__ double rx_s[CCF_TILE], ry_s[CCF_TILE], px_s[CCF_TILE], py_s[CCF_TILE];
+	__shared__ int active_s;
+	const int chain = first_chain + blockIdx.y;
+	const int c = chain / sides, b = chain % sides;
+	const int sgn = (sides == 1 || b == 1) ? 1 : -1;
+	const int lane = threadIdx.x & 63;
+	const int wave = __builtin_amdgcn_readfirstlane(int(blockIdx.x) * (CCF_THREADS / 64) + int(threadIdx.x >> 6));
+	const int waves = int(gridDim.x) * (CCF_THREADS / 64);
+	double* cur = work + 4ll * chain * nroots;   // (re, im) of every root, twice
+	double* nxt = cur + 2ll * nroots;
+	const bool stars_fit = nstars <= CCF_TILE;
+	if (stars_fit)
+		for (int i = threadIdx.x; i < nstars; i += CCF_THREADS)
+		{
+			px_s[i] = a.sx[i];
+			py_s[i] = a.sy[i];
+		}
+	unsigned long long* slot = slots + (long long)chain * (j1 - j0 + 1) * iters;
+	char* done = fin + ((long long)c * 2 + b) * nroots;
+	int* leaves = leaf_cache + ((long long)c * 2 + b) * nroots;
+	for (int j = j0; j <= j1; j++)
+	{
+		const CCRow R = cc_row(c, sgn, j, nphi, nb);
+		for (int k = wave; k < nroots; k += waves)
+			if (lane == 0) done[k] = 0;
+		for (int it = 0; it < iters; it++)
+		{
+			if (threadIdx.x == 0) active_s = 0;
+			// the loop runs once if the roots fit one tile; a wave then updates its roots in turn
+			const bool roots_fit = nroots <= CCF_TILE;
+			if (roots_fit)
+				for (int i = threadIdx.x; i < nroots; i += CCF_THREADS)
+				{
+					rx_s[i] = load_shared(cur + 2 * i);
+					ry_s[i] = load_shared(cur + 2 * i + 1);
+				}
+			__syncthreads();
+			// every wave takes as many turns as the first, since the tiles are shared by the block
+			const int turns = (nroots - (wave & ~(CCF_THREADS / 64 - 1)) + waves - 1) / waves;
+			for (int turn = 0; turn < turns; turn++)
+			{
+				const int k = wave + turn * waves;
+				const bool mine = k < nroots;
+				const bool active = mine && !done[k];
+				dcx z = {0, 0};
+				if (mine) z = roots_fit ? dcx{rx_s[k], ry_s[k]} : dcx{load_shared(cur + 2 * k), load_shared(cur + 2 * k + 1)};
+				// the root's leaf from the previous iteration while the root stays strictly inside
+				// it (there the tree descent would end in the same leaf), else a fresh descent
+				int node = 0;
+				bool leaf = false;
+				CCLeaf f;
+				if (active)
+				{
+					const int cached = __builtin_amdgcn_readfirstlane(leaves[k]);
+					bool inside = false;
+					if (cached >= 0)
+					{
+						const double h = a.nhl[cached] * (1 - 1e-12);
+						inside = fabs(z.re - a.ncx[cached]) < h && fabs(z.im - a.ncy[cached]) < h;
+					}
+					node = __builtin_amdgcn_readfirstlane(inside ? cached : find_node(a, z.re, z.im));
+					leaf = a.nchild0[node] < 0;
+					if (!inside && lane == 0) leaves[k] = leaf ? node : -1;
+					if (leaf) f = cc_load_leaf(a, node);
+				}
+				// this lane's share of the sums over the other roots and over the poles (stars)
+				double rx = 0, ry = 0, px = 0, py = 0;
+				for (int t0 = 0; t0 < nroots; t0 += CCF_TILE)
+				{
+					const int n = min(CCF_TILE, nroots - t0);
+					if (!roots_fit)
+					{
+						__syncthreads();
+						for (int i = threadIdx.x; i < n; i += CCF_THREADS)
+						{
+							rx_s[i] = load_shared(cur + 2 * (t0 + i));
+							ry_s[i] = load_shared(cur + 2 * (t0 + i) + 1);
+						}
+						__syncthreads();
+					}
+					if (active)
+						for (int q = lane; q < n; q += 64)
+						{
+							if (t0 + q == k) continue;
+							const double dx = z.re - rx_s[q], dy = z.im - ry_s[q];
+							const double ir2 = dev::rcp64(dx * dx + dy * dy);
+							rx += dx * ir2;
+							ry -= dy * ir2;
+						}
+				}
+				for (int t0 = 0; t0 < nstars; t0 += CCF_TILE)
+				{
+					const int n = min(CCF_TILE, nstars - t0);
+					if (!stars_fit)
+					{
+						__syncthreads();
+						for (int i = threadIdx.x; i < n; i += CCF_THREADS)
+						{
+							px_s[i] = a.sx[t0 + i];
+							py_s[i] = a.sy[t0 + i];
+						}
+						__syncthreads();
+					}
+					if (active)
+						for (int q = lane; q < n; q += 64)
+						{
+							const double dx = z.re - px_s[q], dy = z.im - py_s[q];
+							const double ir2 = dev::rcp64(dx * dx + dy * dy);
+							px += dx * ir2;
+							py -= dy * ir2;
+						}
+				}
+				if (!mine) continue;
+				if (!active)
+				{
+					if (lane == 0)
+					{
+						store_shared(nxt + 2 * k, z.re);
+						store_shared(nxt + 2 * k + 1, z.im);
+					}
+					continue;
+				}
+				CCTerms t;
+				if (leaf)
+					t = cc_terms_leaf<LIN>(a, f, z);
+				else
+				{
+					// outside the root box; the tree's pointers are read here only
+					const ShootArgs* cold = reinterpret_cast<const ShootArgs*>((const void*)__builtin_amdgcn_kernarg_segment_ptr());
+					asm volatile("" : "+s"(cold));
+					t = cc_terms<LIN>(*cold, node, z, true, lane, 64);
+				}
+				rx = wave_sum(rx);
+				ry = wave_sum(ry);
+				px = wave_sum(px);
+				py = wave_sum(py);
+				t.S1.re = wave_sum(t.S1.re);
+				t.S1.im = wave_sum(t.S1.im);
+				t.S2.re = wave_sum(t.S2.re);
+				t.S2.im = wave_sum(t.S2.im);
+				if (lane == 0)
+				{
+					const dcx f0 = cc_f0(a, t, R.phi);
+					dcx zn = z;
+					// 1/mu below 1e-9 (both bounds of ccf_functions.cuh:207-211): the root stays
+					bool fin_now = cc_inv_mu_error(a, t, f0) < 1e-9;
+					if (!fin_now)
+					{
+						const dcx f1 = dcx{-2 * a.theta2 * t.S2.re - t.L2.re - t.d2s.re, -2 * a.theta2 * t.S2.im - t.L2.im + t.d2s.im};
+						dcx psum = dcx{2 * px, 2 * py};
+						if (circle_pole)
+						{
+							const dcx iz = dev::cdiv(dcx{1, 0}, z);
+							psum = dev::add(psum, dev::scale(iz, 2));
+						}
+						const dcx den = dev::add(f1, dev::mul(f0, dcx{psum.re - rx, psum.im - ry}));
+						zn = dev::sub(z, dev::cdiv(f0, den));
+						fin_now = dev::cabs(dev::sub(zn, z)) / sqrt(a.theta2) < 1e-9;
+					}
+					store_shared(nxt + 2 * k, zn.re);
+					store_shared(nxt + 2 * k + 1, zn.im);
+					if (fin_now)
+						done[k] = 1;
+					else
+						atomicAdd(&active_s, 1);
+				}
+			}
+			__syncthreads();
+			const int left = chain_barrier(slot + (long long)(j - j0) * iters + it, int(gridDim.x), active_s, failed);
+			if (left < 0) return;
+			double* swap = cur;
+			cur = nxt;
+			nxt = swap;
+			if (left == 0) break;
+		}
+		for (int k = wave; k < nroots; k += waves)
+			if (lane < 2) reinterpret_cast<double*>(rows + (long long)R.row * nroots + k)[lane] = load_shared(cur + 2 * k + lane);
+	}
+}
+
+// every chain's working copy from the rows its first step starts from (step j)
+__global__ void k_ccf_start(const dcx* __restrict__ rows, dcx* work, int nroots, int j, int nphi, int nb, int sides)
 {
 	const int k = blockIdx.x * blockDim.x + threadIdx.x;
 	if (k >= nroots) return;
-	const int c = blockIdx.y / 2, b = blockIdx.y % 2;
-	const int sgn = b == 0 ? -1 : 1;
-	const CCRow to = cc_row(c, sgn, j, nphi, nb), from = cc_row(c, sgn, j - 1, nphi, nb);
-	roots[(long long)to.row * nroots + k] = roots[(long long)from.row * nroots + k];
-	fin[((long long)c * 2 + b) * nroots + k] = 0;
+	const int c = blockIdx.y / sides, b = blockIdx.y % sides;
+	const CCRow from = cc_row(c, (sides == 1 || b == 1) ? 1 : -1, j, nphi, nb);
+	work[2ll * blockIdx.y * nroots + k] = rows[(long long)from.row * nroots + k];
 }
 
 /*
@@ -329,87 +532,89 @@ CCFResult Engine::ccf_solve(const LensParams& lens, const double* init_roots, in
 	DeviceBuffer<double> Ab, Bb, Cb, Wb, M;
 	DeviceBuffer<char> fin;
 	DeviceBuffer<int> leaf_cache;
-	DeviceBuffer<unsigned long long> err;
-	DeviceBuffer<int> nanf;
+	DeviceBuffer<unsigned long long> err, slots;
+	DeviceBuffer<int> flags;   // a non-finite error; a barrier that timed out
 	Ab.alloc(2 * total);
-	Bb.alloc(2 * total);
+	Bb.alloc(2 * 4 * (size_t)nb * nroots);
 	Cb.alloc(2 * total);
 	if (caustics) Wb.alloc(2 * total);
 	if (mu_scales) M.alloc(total);
 	struct
 	{
 		dcx* ptr;
-	} A{reinterpret_cast<dcx*>(Ab.ptr)}, B{reinterpret_cast<dcx*>(Bb.ptr)}, C{reinterpret_cast<dcx*>(Cb.ptr)},
-		W{reinterpret_cast<dcx*>(Wb.ptr)};
+	} A{reinterpret_cast<dcx*>(Ab.ptr)}, C{reinterpret_cast<dcx*>(Cb.ptr)}, W{reinterpret_cast<dcx*>(Wb.ptr)};
 	fin.alloc(2 * (size_t)nb * nroots);
 	leaf_cache.alloc(2 * (size_t)nb * nroots);
 	err.alloc(1);
-	nanf.alloc(1);
+	flags.alloc(2);
+	const size_t nslots = std::max((size_t)nb * init_iters, 2 * (size_t)nb * J * step_iters);
+	slots.alloc(std::max<size_t>(nslots, 1));
 	MLENS_HIP_CHECK(hipMemsetAsync(A.ptr, 0, total * sizeof(dcx), stream_));
-	MLENS_HIP_CHECK(hipMemsetAsync(fin.ptr, 0, 2 * (size_t)nb * nroots, stream_));
 	MLENS_HIP_CHECK(hipMemsetAsync(leaf_cache.ptr, 0xff, 2 * (size_t)nb * nroots * sizeof(int), stream_));   // -1: none
 	MLENS_HIP_CHECK(hipMemsetAsync(err.ptr, 0, sizeof(unsigned long long), stream_));
-	MLENS_HIP_CHECK(hipMemsetAsync(nanf.ptr, 0, sizeof(int), stream_));
+	MLENS_HIP_CHECK(hipMemsetAsync(flags.ptr, 0, 2 * sizeof(int), stream_));
 	// starting roots at the centre row of each branch
 	for (int c = 0; c < nb; c++)
 		MLENS_HIP_CHECK(hipMemcpyAsync(A.ptr + (long long)(c * (2 * J + 1) + J) * nroots, init_roots + 2 * (long long)c * nroots,
 			nroots * sizeof(dcx), hipMemcpyHostToDevice, stream_));
-	const unsigned gx = unsigned((nroots + CCF_ROOTS - 1) / CCF_ROOTS);
-	// an even number of iterations leaves the roots in A
-	auto iterate = [&](int j, int sides, int iters) {
-		for (int it = 0; it < iters; it++)
+	// Steps j0 .. j1 of every chain. The blocks of a chain wait for each other, so all blocks of a launch must be
+	// resident: they share out evenly over the chains what the device holds, no more than a chain has roots for;
+	// chains beyond that go into further launches.
+	const void* kernel = a.smooth_linear ? (const void*)k_ccf_chain<true> : (const void*)k_ccf_chain<false>;
+	int per_cu = 0;
+	MLENS_HIP_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, CCF_THREADS, 0));
+	const int resident = num_cus_ * std::max(1, per_cu);
+	auto sweep = [&](int from, int j0, int j1, int sides, int iters) {
+		if (j1 < j0 || iters < 1) return;
+		const int chains = nb * sides, group = std::min(chains, resident);
+		MLENS_HIP_CHECK(hipMemsetAsync(slots.ptr, 0, (size_t)chains * (j1 - j0 + 1) * iters * sizeof(unsigned long long), stream_));
+		k_ccf_start<<<dim3(blocks_for(nroots, 256), unsigned(chains)), 256, 0, stream_>>>(A.ptr, reinterpret_cast<dcx*>(Bb.ptr), nroots,
+			from, nphi, nb, sides);
+		MLENS_HIP_CHECK(hipGetLastError());
+		const int waves = CCF_THREADS / 64;
+		for (int first = 0; first < chains; first += group)
 		{
-			const dcx* s = (it % 2 == 0) ? A.ptr : B.ptr;
-			dcx* d = (it % 2 == 0) ? B.ptr : A.ptr;
-			k_ccf_iterate<<<dim3(gx, unsigned(nb * sides)), CCF_THREADS, 0, stream_>>>(a, s, d, fin.ptr, leaf_cache.ptr,
-				nroots, nstars_, circle_pole ? 1 : 0, j, nphi, nb, sides);
-		}
-		if (iters % 2)
-		{
-			// copy the rows just refined back into A
-			for (int c = 0; c < nb; c++)
-				for (int b = 0; b < sides; b++)
-				{
-					const int row = c * (2 * J + 1) + J + (sides == 1 ? 0 : (b == 0 ? -j : j));
-					MLENS_HIP_CHECK(hipMemcpyAsync(A.ptr + (long long)row * nroots, B.ptr + (long long)row * nroots,
-						nroots * sizeof(dcx), hipMemcpyDeviceToDevice, stream_));
-				}
+			const int here = std::min(group, chains - first);
+			const int blocks = std::max(1, std::min((nroots + waves - 1) / waves, resident / here));
+			dcx* rows = A.ptr;
+			double* work = Bb.ptr;
+			char* fp = fin.ptr;
+			int *lp = leaf_cache.ptr, *bad = flags.ptr + 1, ns = nstars_, pole = circle_pole ? 1 : 0;
+			unsigned long long* sp = slots.ptr;
+			void* args[] = {&a, &rows, &work, &fp, &lp, &sp, &bad, &nroots, &ns, &pole, &j0, &j1, &nphi, &nb, &sides, &iters, &first};
+			MLENS_HIP_CHECK(hipLaunchCooperativeKernel(kernel, dim3(unsigned(blocks), unsigned(here)), dim3(CCF_THREADS),
+				args, 0, stream_));
 		}
 	};
 	CCFResult r;
 	MLENS_HIP_CHECK(hipEventRecord(ev0_, stream_));
-	iterate(0, 1, init_iters);
-	MLENS_HIP_CHECK(hipGetLastError());
+	sweep(0, 0, 0, 1, init_iters);
 	MLENS_HIP_CHECK(hipEventRecord(ev1_, stream_));
 	MLENS_HIP_CHECK(hipEventSynchronize(ev1_));
 	float ms = 0;
 	MLENS_HIP_CHECK(hipEventElapsedTime(&ms, ev0_, ev1_));
 	r.t_init_ms = ms;
 	MLENS_HIP_CHECK(hipEventRecord(ev0_, stream_));
-	for (int j = 1; j <= J; j++)
-	{
-		k_ccf_prepare<<<dim3(blocks_for(nroots, 256), unsigned(2 * nb)), 256, 0, stream_>>>(A.ptr, fin.ptr, nroots, j, nphi, nb);
-		iterate(j, 2, step_iters);
-	}
-	MLENS_HIP_CHECK(hipGetLastError());
+	if (step_iters > 0) sweep(0, 1, J, 2, step_iters);
 	MLENS_HIP_CHECK(hipEventRecord(ev1_, stream_));
 	MLENS_HIP_CHECK(hipEventSynchronize(ev1_));
 	MLENS_HIP_CHECK(hipEventElapsedTime(&ms, ev0_, ev1_));
 	r.t_ccs_ms = ms;
 	MLENS_HIP_CHECK(hipEventRecord(ev0_, stream_));
 	k_ccf_finish<<<blocks_for(total, 256), 256, 0, stream_>>>(a, A.ptr, nroots, nphi, nb, C.ptr, caustics ? W.ptr : nullptr,
-		mu_scales ? M.ptr : nullptr, err.ptr, nanf.ptr);
+		mu_scales ? M.ptr : nullptr, err.ptr, flags.ptr);
 	MLENS_HIP_CHECK(hipGetLastError());
 	MLENS_HIP_CHECK(hipEventRecord(ev1_, stream_));
 	MLENS_HIP_CHECK(hipEventSynchronize(ev1_));
 	MLENS_HIP_CHECK(hipEventElapsedTime(&ms, ev0_, ev1_));
 	r.t_caustics_ms = ms;
 	unsigned long long eb = 0;
-	int nf = 0;
+	int nf[2] = {0, 0};
 	MLENS_HIP_CHECK(hipMemcpy(&eb, err.ptr, sizeof(eb), hipMemcpyDeviceToHost));
-	MLENS_HIP_CHECK(hipMemcpy(&nf, nanf.ptr, sizeof(nf), hipMemcpyDeviceToHost));
+	MLENS_HIP_CHECK(hipMemcpy(nf, flags.ptr, sizeof(nf), hipMemcpyDeviceToHost));
+	if (nf[1]) throw HipError("the blocks of a critical-curve chain did not meet", __FILE__, __LINE__);
 	std::memcpy(&r.max_error, &eb, sizeof(double));
-	r.has_nan = nf != 0;
+	r.has_nan = nf[0] != 0;
 	MLENS_HIP_CHECK(hipMemcpy(ccs, C.ptr, total * sizeof(dcx), hipMemcpyDeviceToHost));
 	if (caustics) MLENS_HIP_CHECK(hipMemcpy(caustics, W.ptr, total * sizeof(dcx), hipMemcpyDeviceToHost));
 	if (mu_scales) MLENS_HIP_CHECK(hipMemcpy(mu_scales, M.ptr, total * sizeof(double), hipMemcpyDeviceToHost));

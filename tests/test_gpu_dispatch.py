@@ -178,3 +178,32 @@ def test_histograms_inside_and_past_the_window(tmp_path, irs, double, n1, n2):
             np.testing.assert_array_equal(got, np.column_stack([u, c]), err_msg=kind + suffix)
             say(f"[hist] {kind}{suffix}: {len(u)} bins up to {u[-1]}")
     m.close()
+
+
+@pytest.mark.parametrize("stars,phases,branches,exact", [(1, 4, 1, False), (2, 4, 2, True), (5, 600, 300, False),
+                                                         (1100, 2, 1, False), (2100, 2, 1, False)])
+def test_critical_curve_chains(stars, phases, branches, exact):
+    """Chains of one block and of many, more chains than the device holds at once (600),
+    roots past one LDS tile (2048) and stars past it, linear and general smooth matter:
+    every root solves the critical-curve equation by direct sums (1/mu below 1e-6, as in
+    the oracle tests) and the roots of a phase are distinct."""
+    from irs_amd.microlensing.CCF.ccf import CCF
+    from oracle import ccf as OC
+    from scipy.spatial import cKDTree
+    say(f"[ccf] {stars} stars, {phases} phases, {branches} branches, exact sheet {exact}")
+    # one star on one branch cannot leave the line its starting roots lie on: use two there
+    branches = max(branches, 2) if stars == 1 else branches
+    c = CCF(kappa_tot=0.3, shear=0.3, kappa_star=0.27, num_stars=stars, num_phi=phases, num_branches=branches, random_seed=7,
+            approx=not exact, write_stars=False)
+    c.run()
+    prob = OC.Problem(c.stars, 0.3, 0.3, 1.0, 0.27, c.corner, approx=int(not exact))
+    z = c.critical_curves[..., 0] + 1j * c.critical_curves[..., 1]
+    half = phases // (2 * branches)
+    phi = np.array([[np.pi / branches + 2 * np.pi * b / branches + (k - half) * 2 * np.pi / phases for k in range(2 * half + 1)]
+                    for b in range(branches)])
+    assert np.nanmax(prob.inv_mu_error(z, np.tile(phi, (c.num_roots, 1)))) < 1e-6
+    for b in range(0, branches, max(1, branches // 3)):
+        r = z[b::branches, 0]
+        d, _ = cKDTree(np.column_stack([r.real, r.imag])).query(np.column_stack([r.real, r.imag]), k=2)
+        assert d[:, 1].min() > 1e-8
+    c.close()
