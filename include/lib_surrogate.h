@@ -30,6 +30,8 @@ bool surrogate_set_params(SurrogateHandle* self, const float* params);   /* also
 bool surrogate_get_params(SurrogateHandle* self, float* params);
 bool surrogate_load_data(SurrogateHandle* self, const float* x, const float* t, int n);   /* device-resident training set */
 double surrogate_train_step(SurrogateHandle* self, const int* rows, int m, float lr, float wd);   /* mean loss; m % 16 == 0 */
+/* `steps` of them in one call: step k takes rows[k m .. (k + 1) m) at rate lr[k] and leaves its mean loss in losses[k] */
+bool surrogate_train(SurrogateHandle* self, const int* rows, int steps, int m, const float* lr, float wd, double* losses);
 double surrogate_gradients(SurrogateHandle* self, const float* x, const float* t, int n, float* grads);   /* loss; n % 16 == 0 */
 bool surrogate_predict(SurrogateHandle* self, const float* x, int n, float* probs);
 double surrogate_time_predict(SurrogateHandle* self, const float* x, int n, int reps);   /* seconds per histogram */

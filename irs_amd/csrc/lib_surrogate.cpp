@@ -45,6 +45,10 @@ double surrogate_train_step(SurrogateHandle* self, const int* rows, int m, float
 {
 	SURR_GUARD(return self->s.train_step(rows, m, lr, wd), return -1.0)
 }
+bool surrogate_train(SurrogateHandle* self, const int* rows, int steps, int m, const float* lr, float wd, double* losses)
+{
+	SURR_GUARD(self->s.train(rows, steps, m, lr, wd, losses); return true, return false)
+}
 double surrogate_gradients(SurrogateHandle* self, const float* x, const float* t, int n, float* grads)
 {
 	SURR_GUARD(return self->s.gradients(x, t, n, grads), return -1.0)

@@ -12,6 +12,15 @@ constexpr int SURR_HIDDEN = 256;
 constexpr int SURR_NOUT = 128;     // log10 magnification bins over [-2, 2]
 constexpr int SURR_LAYERS = 4;
 
+// where a training pass leaves what the weight gradients read: [feature][row], ld rows each
+struct NetTrace
+{
+	unsigned short* in[SURR_LAYERS];    // a layer's input: the batch, then the hidden activations
+	unsigned short* dz16[SURR_LAYERS];  // gradient of its pre-activations in BF16
+	float* dz32[SURR_LAYERS];           // and in FP32
+	int ld;
+};
+
 class Surrogate
 {
 public:
@@ -30,28 +39,27 @@ public:
 	void predict(const float* x, int n, float* probs);                // n x 128 softmax outputs
 	double time_predict(const float* x, int n, int reps);             // seconds per predicted histogram on the device
 
-private:
-	void gemm(int M, int N, int K, const unsigned short* A, long long sam, long long sak, const unsigned short* B,
-		long long sbk, long long sbn, float* C, int ldc, bool accumulate);
-	void forward(int M);
-	double backward(int M);
+	// `steps` of them: step k on rows[k m .. (k + 1) m) at rate lr[k]; losses[k] its mean loss
+	void train(const int* rows, int steps, int m, const float* lr, float wd, double* losses);
 
-	static const int dims_[SURR_LAYERS + 1];
+private:
+	NetTrace trace(int M);
+	void launch_predict(const unsigned short* x, int rows, float* probs);
+
+	static constexpr int PREDICT_SMALL = 256;   // rows of a request that goes through pinned memory
+	static constexpr int PREDICT_ROWS = 8192;   // rows at a time of a larger one
+
 	int max_batch_;
 	hipStream_t stream_ = nullptr;
 	size_t nparams_ = 0;
-	size_t w_off_[SURR_LAYERS], b_off_[SURR_LAYERS];
 	int step_ = 0;
 	int ndata_ = 0;
+	void* small_ = nullptr;   // pinned: a small request's inputs, then its outputs
 	DeviceBuffer<float> w_, g_, m_, v_;
-	DeviceBuffer<unsigned short> w16_;
-	DeviceBuffer<unsigned short> xall_, xb_;
-	DeviceBuffer<float> tall_, tb_;
+	DeviceBuffer<unsigned short> w16_, wt16_;   // BF16 weights [out x in] and [in x out]
+	DeviceBuffer<unsigned short> xall_, xb_, trace16_;
+	DeviceBuffer<float> tall_, p_, loss_, trace32_;
 	DeviceBuffer<int> idx_;
-	DeviceBuffer<float> z_[SURR_LAYERS];
-	DeviceBuffer<unsigned short> h_[SURR_LAYERS];
-	DeviceBuffer<float> c_, p_, loss_, d32_, dh_;
-	DeviceBuffer<unsigned short> d16_;
 };
 
 }  // namespace mlens

@@ -6,7 +6,7 @@ import os
 from ... import BIN_DIR
 
 SYMBOLS = ["surrogate_create", "surrogate_free", "surrogate_num_params", "surrogate_set_params", "surrogate_get_params",
-           "surrogate_load_data", "surrogate_train_step", "surrogate_gradients", "surrogate_predict",
+           "surrogate_load_data", "surrogate_train_step", "surrogate_train", "surrogate_gradients", "surrogate_predict",
            "surrogate_time_predict"]
 
 
@@ -31,6 +31,7 @@ def load(path=None):
     sig("surrogate_get_params", [v, F], b)
     sig("surrogate_load_data", [v, F, F, i], b)
     sig("surrogate_train_step", [v, I, i, ctypes.c_float, ctypes.c_float], d)
+    sig("surrogate_train", [v, I, i, i, F, ctypes.c_float, ctypes.POINTER(ctypes.c_double)], b)
     sig("surrogate_gradients", [v, F, F, i, F], d)
     sig("surrogate_predict", [v, F, i, F], b)
     sig("surrogate_time_predict", [v, F, i, i], d)

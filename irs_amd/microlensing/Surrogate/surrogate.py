@@ -120,16 +120,18 @@ class HistogramSurrogate:
         step = 0
         for ep in range(epochs):
             perm = rng.permutation(n).astype(np.int32)
-            tot = 0.0
-            for b0 in range(0, n - batch + 1, batch):
-                rows = np.ascontiguousarray(perm[b0:b0 + batch])
-                rate = lr * 0.5 * (1 + np.cos(np.pi * step / max(steps, 1)))
-                loss = lib.surrogate_train_step(self.obj, rows.ctypes.data_as(ctypes.POINTER(ctypes.c_int)), batch,
-                                                rate, wd)
-                if loss < 0:
-                    raise Exception("Error in a surrogate training step")
-                tot += loss
+            rates = []
+            for _ in range(n // batch):
+                rates.append(lr * 0.5 * (1 + np.cos(np.pi * step / max(steps, 1))))
                 step += 1
+            rates = np.array(rates, dtype=np.float32)
+            losses = np.zeros(len(rates))
+            if not lib.surrogate_train(self.obj, perm.ctypes.data_as(ctypes.POINTER(ctypes.c_int)), len(rates), batch,
+                                       rates.ctypes.data_as(F), wd, losses.ctypes.data_as(ctypes.POINTER(ctypes.c_double))):
+                raise Exception("Error in a surrogate training step")
+            tot = 0.0
+            for loss in losses:
+                tot += float(loss)
             self.losses.append(tot / max(n // batch, 1))
             if log and (ep % 10 == 0 or ep == epochs - 1):
                 log(f"[surrogate] epoch {ep}: loss {self.losses[-1]:.5f}")

@@ -207,3 +207,38 @@ def test_critical_curve_chains(stars, phases, branches, exact):
         d, _ = cKDTree(np.column_stack([r.real, r.imag])).query(np.column_stack([r.real, r.imag]), k=2)
         assert d[:, 1].min() > 1e-8
     c.close()
+
+
+@pytest.mark.parametrize("batch,n", [(16, 16), (48, 100), (240, 256)])
+def test_surrogate_batches_and_requests(batch, n):
+    """One block per 16 rows: batches of one, several and fifteen blocks, whose epochs
+    leave rows over, against an epoch made of single steps (the same kernels in the same
+    order: equal); and requests through pinned memory (up to 256 rows) and through device
+    buffers, padded or not, against the FP64 network (the bound of the gradient test)."""
+    import ctypes
+    from irs_amd.microlensing.Surrogate import surrogate as S
+    from oracle import mlp
+    rng = np.random.default_rng(batch)
+    x, t = rng.normal(size=(n, 6)), rng.random((n, 128)) + 0.1
+    s = S.HistogramSurrogate(max_batch=256, seed=4)
+    p0 = s.params()
+    losses = s.fit(x, t, epochs=2, batch=batch)
+    trained = s.params()
+    s.set_params(p0)
+    order, step, steps = np.random.default_rng(0), 0, 2 * (n // batch)
+    for ep in range(2):
+        perm, tot = order.permutation(n).astype(np.int32), 0.0
+        for b0 in range(0, n - batch + 1, batch):
+            rows = np.ascontiguousarray(perm[b0:b0 + batch])
+            tot += S.lib.surrogate_train_step(s.obj, rows.ctypes.data_as(ctypes.POINTER(ctypes.c_int)), batch,
+                                              2e-3 * 0.5 * (1 + np.cos(np.pi * step / steps)), 1e-4)
+            step += 1
+        assert tot / (n // batch) == losses[ep]
+    np.testing.assert_array_equal(s.params(), trained)
+    for rows in (1, 15, 16, 17, 255, 256, 257, 300):
+        q = rng.normal(size=(rows, 6))
+        got = s.predict(q)
+        want, _, _ = mlp.forward(s.params().astype(np.float64), s._inputs(q).astype(np.float64), bf16_ops=True)
+        say(f"[surrogate] batch {batch}, request of {rows}: {np.max(np.abs(got - want)):.1e}")
+        assert np.max(np.abs(got - want)) < 1e-4
+    s.close()
