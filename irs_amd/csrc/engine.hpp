@@ -243,6 +243,7 @@ private:
 
 	DeviceBuffer<int> scratch_i_;
 	DeviceBuffer<double> scratch_d_;
+	DeviceBuffer<double> points_;   // deflect_points: points, deflections, magnifications
 	DeviceBuffer<long long> scratch_ll_, hist_;
 };
 

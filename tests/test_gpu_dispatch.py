@@ -242,3 +242,35 @@ def test_surrogate_batches_and_requests(batch, n):
         say(f"[surrogate] batch {batch}, request of {rows}: {np.max(np.abs(got - want)):.1e}")
         assert np.max(np.abs(got - want)) < 1e-4
     s.close()
+
+
+@pytest.mark.parametrize("rect", [False, True])
+def test_deflections_of_mixed_waves(oracle, tmp_path, rect):
+    """A wave of points serves two shared leaves, then its other lanes one by one: waves
+    of one leaf, of two, of three and of 64, partial waves, and points outside the root
+    box, for linear and general smooth matter: the deflection and magnification of a point
+    do not depend on its neighbours, and match the oracle (the parity tests' bounds)."""
+    from irs_amd.microlensing.IPM.ipm import IPM
+    field = dict(C1_SMALL, rectangular=rect)
+    stars = write_starfile(oracle, tmp_path / "stars.bin", field, seed=9)
+    m = IPM(**from_starfile(field, tmp_path / "stars.bin"), is_double=True, expansion_order=16)
+    m.run()
+    tree = Mirror(oracle, m, stars=stars)
+    rng = np.random.default_rng(2)
+    far = 2.0 * m.root_half_length
+    spots = np.array([0.1 + 0.2j, 9.3 - 4.1j, -7.7 + 11.2j])
+    waves = [np.repeat(spots[:k], 64 // k + 1)[:64] + 1e-3 * (rng.random(64) + 1j * rng.random(64)) for k in (1, 2, 3)]
+    waves.append(20 * (rng.random(64) - 0.5) + 40j * (rng.random(64) - 0.5))
+    waves.append(np.where(np.arange(64) % 3 == 0, far * np.exp(2j * np.pi * rng.random(64)), waves[3]))
+    z = np.concatenate(waves)
+    w, mu = m.deflect(z, want_mu=True)
+    one = [m.deflect(z[k:k + 1], want_mu=True) for k in range(len(z))]
+    assert np.max(np.abs(w - np.array([o[0][0] for o in one]))) <= 1e-13 * np.max(np.abs(w))
+    np.testing.assert_allclose(mu, [o[1][0] for o in one], rtol=1e-9)
+    for n in (1, 63, 65, 127):
+        np.testing.assert_allclose(m.deflect(z[:n]), w[:n], rtol=0, atol=1e-13 * np.max(np.abs(w)))
+    inside = np.concatenate(waves[:4])
+    ref = tree.tree.deflect(tree.lens, inside)
+    ref = ref[0] if isinstance(ref, tuple) else ref
+    assert np.max(np.abs(w[:256] - ref)) < 1e-10
+    m.close()
