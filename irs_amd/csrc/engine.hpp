@@ -98,7 +98,9 @@ public:
 	void upload_stars(const double* aos, int n);
 	void generate_stars(int n, int rectangular, double c_re, double c_im, int mass_function, double m_lower,
 		double m_upper, double m_solar, uint32_t seed);
-	void download_stars(double* aos) const;   // AoS x1, x2, m in the current (tree) order
+	// AoS x1, x2, m in the current (tree) order, rounded to the caller's type on the device
+	void download_stars(double* aos);
+	void download_stars(float* aos);
 	StarStats star_stats();
 	int num_stars() const { return nstars_; }
 
@@ -148,6 +150,9 @@ public:
 	   real; caustics and mu_scales may be null. Needs build_tree and fmm first. */
 	CCFResult ccf_solve(const LensParams& lens, const double* init_roots, int nroots, int nphi, int nb, bool circle_pole,
 		double* ccs, double* caustics, double* mu_scales, int init_iters = 30, int step_iters = 20);
+
+	/* false: one iteration per launch, as when other work keeps the blocks of a chain from being resident at once */
+	void set_ccf_together(bool on) { ccf_together_ = on; }
 
 	/* thin test entry: lens equation at arbitrary points through the tree */
 	void deflect_points(const LensParams& lens, const double* z, int n, Precision prec, double* w, double* mu);
@@ -241,8 +246,13 @@ private:
 	template <typename F>
 	void with_maps(F f) const;
 
+	template <typename F>
+	void download_stars_as(F* aos);
+
 	DeviceBuffer<int> scratch_i_;
+	DeviceBuffer<char> stars_aos_;
 	DeviceBuffer<double> scratch_d_;
+	bool ccf_together_ = true;
 	DeviceBuffer<double> points_;   // deflect_points: points, deflections, magnifications
 	DeviceBuffer<long long> scratch_ll_, hist_;
 };

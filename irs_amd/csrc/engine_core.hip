@@ -121,20 +121,31 @@ void Engine::generate_stars(int n, int rectangular, double c_re, double c_im, in
 	MLENS_HIP_CHECK(hipStreamSynchronize(stream_));
 }
 
-void Engine::download_stars(double* aos) const
+template <typename F>
+__global__ void k_stars_aos(const double* sx, const double* sy, const double* sm, int n, F* out)
 {
-	int n = nstars_;
-	std::vector<double> a(n), b(n), c(n);
-	MLENS_HIP_CHECK(hipMemcpy(a.data(), sx_.ptr, n * sizeof(double), hipMemcpyDeviceToHost));
-	MLENS_HIP_CHECK(hipMemcpy(b.data(), sy_.ptr, n * sizeof(double), hipMemcpyDeviceToHost));
-	MLENS_HIP_CHECK(hipMemcpy(c.data(), sm_.ptr, n * sizeof(double), hipMemcpyDeviceToHost));
-	for (int i = 0; i < n; i++)
-	{
-		aos[3 * i] = a[i];
-		aos[3 * i + 1] = b[i];
-		aos[3 * i + 2] = c[i];
-	}
+	const int i = blockIdx.x * blockDim.x + threadIdx.x;
+	if (i >= n) return;
+	out[3 * (long long)i] = F(sx[i]);
+	out[3 * (long long)i + 1] = F(sy[i]);
+	out[3 * (long long)i + 2] = F(sm[i]);
 }
+
+template <typename F>
+void Engine::download_stars_as(F* aos)
+{
+	const int n = nstars_;
+	if (n <= 0) return;
+	stars_aos_.alloc(3 * sizeof(F) * size_t(n));
+	F* d = reinterpret_cast<F*>(stars_aos_.ptr);
+	k_stars_aos<F><<<blocks_for(n, 256), 256, 0, stream_>>>(sx_.ptr, sy_.ptr, sm_.ptr, n, d);
+	MLENS_HIP_CHECK(hipGetLastError());
+	MLENS_HIP_CHECK(hipMemcpyAsync(aos, d, 3 * sizeof(F) * size_t(n), hipMemcpyDeviceToHost, stream_));
+	MLENS_HIP_CHECK(hipStreamSynchronize(stream_));
+}
+
+void Engine::download_stars(double* aos) { download_stars_as(aos); }
+void Engine::download_stars(float* aos) { download_stars_as(aos); }
 
 // star.cuh:124-161: totals in FP64; one block reduces everything (N fits easily)
 __global__ void k_star_stats(const double* sm, int n, double* out)

@@ -1804,7 +1804,7 @@ void Engine::deflect_points(const LensParams& lens, const double* z, int n, Prec
 	g.num_pixels[0] = g.num_pixels[1] = 1;
 	ShootArgs a = ShootArgsBuilder::make(lens, g, false);
 	MLENS_TREE_ARGS(a)
-	if (n <= 0) return;
+	if (n < 1) throw HipError("a deflection call needs at least one point", __FILE__, __LINE__);
 	points_.alloc(size_t(5) * n);
 	double *dz = points_.ptr, *dw = dz + size_t(2) * n, *dmu = dw + size_t(2) * n;
 	MLENS_HIP_CHECK(hipMemcpyAsync(dz, z, sizeof(double) * 2 * n, hipMemcpyHostToDevice, stream_));

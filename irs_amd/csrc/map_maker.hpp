@@ -13,6 +13,7 @@
 
 #include "common.hpp"
 #include "engine.hpp"
+#include "host_array.hpp"
 #include "io.hpp"
 #include "mass_functions.hpp"
 
@@ -325,10 +326,10 @@ private:
 	long long num_rays_received_ = 0;
 	StarFileData file_stars_;
 
-	std::vector<T> stars_host_;
+	HostArray<T> stars_host_;
 	bool stars_stale_ = false;
-	std::vector<T> pix_, pix_min_, pix_sad_;
-	std::vector<int> ipix_, ipix_min_, ipix_sad_;
+	HostArray<T> pix_, pix_min_, pix_sad_;
+	HostArray<int> ipix_, ipix_min_, ipix_sad_;
 	long long min_mag_ = 0, max_mag_ = 0, min_log_mag_ = 0, max_log_mag_ = 0;
 	std::vector<long long> hist_[3], log_hist_[3];
 
@@ -785,16 +786,15 @@ private:
 	// the star field in tree order, as get_stars returns it
 	void download_stars()
 	{
-		std::vector<double> s(size_t(num_stars_) * 3);
-		engine_->download_stars(s.data());
-		stars_host_.assign(s.begin(), s.end());
+		stars_host_.resize(size_t(num_stars_) * 3);
+		engine_->download_stars(stars_host_.data());
 		stars_stale_ = false;
 	}
 
 	void download_results()
 	{
 		size_t n = size_t(num_pixels_y.re) * num_pixels_y.im;
-		auto fetch = [&](int which, std::vector<T>& dst) {
+		auto fetch = [&](int which, HostArray<T>& dst) {
 			dst.resize(n);
 			if (engine_->maps_are_fp32())
 			{

@@ -8,6 +8,7 @@
 #pragma once
 
 #include "common.hpp"
+#include "host_array.hpp"
 #include "io.hpp"
 #include "ncc.hpp"
 
@@ -73,7 +74,7 @@ private:
 	std::unique_ptr<NCCDevice> device_;
 	int num_rows_ = 0, num_cols_ = 0;
 	std::vector<double> caustics_;
-	std::vector<int> num_;
+	HostArray<int> num_;
 	std::vector<long long> histogram_;
 	int min_num_ = 0, max_num_ = 0;
 	double t_ncc_ = 0, t_reduce_ = 0;
@@ -158,7 +159,7 @@ private:
 		g.num_pixels_re = num_pixels_y.re;
 		g.num_pixels_im = num_pixels_y.im;
 		g.over_sample = over_sample;
-		num_.assign(size_t(num_pixels_y.re) * size_t(num_pixels_y.im), 0);
+		num_.resize(size_t(num_pixels_y.re) * size_t(num_pixels_y.im));
 		device_->count(caustics_.data(), num_rows_, num_cols_, g, num_.data(), stats_);
 		t_ncc_ = stats_.t_ncc_ms / 1000;
 		t_reduce_ = stats_.t_reduce_ms / 1000;

@@ -544,17 +544,16 @@ class IPM(object):
 
     def deflect(self, z, want_mu=False):
         """Lens equation w(z) through the built tree (FP64 output; mu if asked)."""
-        z = np.asarray(z, dtype=np.complex128).ravel()
-        zz = np.ascontiguousarray(np.column_stack([z.real, z.imag]))
-        w = np.zeros((len(z), 2))
-        mu = np.zeros(len(z)) if want_mu else None
+        # a complex array is its (re, im) pairs already, and the library fills the results in place
+        z = np.ascontiguousarray(np.asarray(z, dtype=np.complex128).ravel())
+        w = np.empty(len(z), dtype=np.complex128)
+        mu = np.empty(len(z)) if want_mu else None
         P = ctypes.POINTER(ctypes.c_double)
-        ok = self.lib.ipm_deflect(self.obj, zz.ctypes.data_as(P), len(z), w.ctypes.data_as(P),
+        ok = self.lib.ipm_deflect(self.obj, z.ctypes.data_as(P), len(z), w.ctypes.data_as(P),
                                   mu.ctypes.data_as(P) if want_mu else None)
         if not ok:
             raise Exception("Error deflecting points")
-        wc = w[:, 0] + 1j * w[:, 1]
-        return (wc, mu) if want_mu else wc
+        return (w, mu) if want_mu else w
 
     def window_cells(self, x0, y0, width, height, margin=1.0, capacity=1 << 22):
         """The lattice cells that can reach columns [x0, x0 + width) and rows
