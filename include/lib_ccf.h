@@ -83,6 +83,11 @@ int get_write_caustics(CCFHandle* self);
 int get_write_mu_length_scales(CCFHandle* self);
 const char* get_outfile_prefix(CCFHandle* self);
 
+/* extension: 0 launches every iteration by itself instead of keeping a branch's blocks on the device (default 1; the
+   solver does so by itself where other work keeps them from being there at once); the results are the same */
+void set_resident_chains(CCFHandle* self, int val);
+int get_resident_chains(CCFHandle* self);
+
 /* derived values and results, lib_ccf.cu:62-69 */
 int get_num_roots(CCFHandle* self);
 ccf_dtype get_corner_x1(CCFHandle* self);          /* (R, 0) for a circular field */

@@ -229,6 +229,42 @@ used once and starts at zero.
 constexpr int CCF_THREADS = 512;
 constexpr int CCF_TILE = 2048;   // roots and stars staged in LDS at a time (32 KB each)
 constexpr long long CCF_SPINS = 1ll << 24;
+constexpr long long CCF_MEET_TICKS = 500000;   // 5 ms of the 100 MHz clock
+
+/*
+Whether every block of the launch is on the device at once, which the barriers need: the last block to arrive
+decides that they are, a block that has waited 5 ms that they are not (other work holds the device), and all blocks
+follow the one decision. state: blocks arrived in the low half, the decision (1 go, 2 no) above; starts at zero.
+*/
+__device__ bool all_resident(unsigned long long* state)
+{
+	__shared__ int go;
+	if (threadIdx.x == 0)
+	{
+		constexpr unsigned long long GO = 1ull << 32, NO = 2ull << 32;
+		const unsigned long long all = (unsigned long long)gridDim.x * gridDim.y;
+		const long long t0 = wall_clock64();
+		unsigned long long v = __hip_atomic_fetch_add(state, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1;
+		for (;;)
+		{
+			if (v >> 32) break;
+			const bool here = v == all, late = wall_clock64() - t0 > CCF_MEET_TICKS;
+			if (here || late)
+			{
+				// decides unless the word has changed meanwhile; v is then its new value
+				const unsigned long long want = v | (here ? GO : NO);
+				if (__hip_atomic_compare_exchange_strong(state, &v, want, __ATOMIC_RELAXED, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+					v = want;
+				continue;
+			}
+			__builtin_amdgcn_s_sleep(1);
+			v = __hip_atomic_load(state, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+		}
+		go = (v >> 32) == 1;
+	}
+	__syncthreads();
+	return go;
+}
 
 __device__ int chain_barrier(unsigned long long* slot, int blocks, int active, int* failed)
 {
@@ -271,16 +307,24 @@ chain's gridDim.x blocks. 137 stars (274 roots, 100 phases): 1.78 ms, against 5.
 iteration and all 20 of them at every step; 1500 stars, 20 phases: 3.0 against 4.9 ms. A step takes about seven
 iterations of 5 us, most of which is the round trip through the barrier and the shared roots. Blocks of 256 or
 1024 threads took 1.74 and 2.37 ms, and 4.1 and 2.7 ms on the larger field. rows: (nphi + nb) rows of nroots roots, the result; work: two copies of each chain's
-roots; slots: iters words per step of each chain, zeroed. Every block of a chain must be resident (a cooperative
-launch), since it waits for the others.
+roots; slots: one word for the launch, then iters words per step of each chain, zeroed. The blocks meet first:
+if they are not all resident at once, the launch does nothing and failed[1] says so. (A cooperative launch would
+promise that they are, but the device grants those to one process at a time.) The same work then goes out one
+iteration per launch, `only` = its number (j0 = j1, flip: which copy is current), with no waiting.
 */
 template <bool LIN>
 __global__ __launch_bounds__(CCF_THREADS) void k_ccf_chain(ShootArgs a, dcx* __restrict__ rows, double* work, char* __restrict__ fin,
 	int* __restrict__ leaf_cache, unsigned long long* slots, int* failed, int nroots, int nstars, int circle_pole, int j0, int j1,
-	int nphi, int nb, int sides, int iters, int first_chain)
+	int nphi, int nb, int sides, int iters, int first_chain, int only, int flip)
 {
 	__shared__ double rx_s[CCF_TILE], ry_s[CCF_TILE], px_s[CCF_TILE], py_s[CCF_TILE];
 	__shared__ int active_s;
+	const bool together = only < 0;
+	if (together && !all_resident(slots + first_chain))
+	{
+		if (threadIdx.x == 0) __hip_atomic_store(failed + 1, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+		return;
+	}
 	const int chain = first_chain + blockIdx.y;
 	const int c = chain / sides, b = chain % sides;
 	const int sgn = (sides == 1 || b == 1) ? 1 : -1;
@@ -289,6 +333,12 @@ __global__ __launch_bounds__(CCF_THREADS) void k_ccf_chain(ShootArgs a, dcx* __r
 	const int waves = int(gridDim.x) * (CCF_THREADS / 64);
 	double* cur = work + 4ll * chain * nroots;   // (re, im) of every root, twice
 	double* nxt = cur + 2ll * nroots;
+	auto turn_over = [&]() {
+		double* t = cur;
+		cur = nxt;
+		nxt = t;
+	};
+	if (flip) turn_over();
 	const bool stars_fit = nstars <= CCF_TILE;
 	if (stars_fit)
 		for (int i = threadIdx.x; i < nstars; i += CCF_THREADS)
@@ -296,15 +346,17 @@ __global__ __launch_bounds__(CCF_THREADS) void k_ccf_chain(ShootArgs a, dcx* __r
 			px_s[i] = a.sx[i];
 			py_s[i] = a.sy[i];
 		}
-	unsigned long long* slot = slots + (long long)chain * (j1 - j0 + 1) * iters;
+	unsigned long long* slot = slots + nb * sides + (long long)chain * (j1 - j0 + 1) * iters;
 	char* done = fin + ((long long)c * 2 + b) * nroots;
 	int* leaves = leaf_cache + ((long long)c * 2 + b) * nroots;
 	for (int j = j0; j <= j1; j++)
 	{
 		const CCRow R = cc_row(c, sgn, j, nphi, nb);
-		for (int k = wave; k < nroots; k += waves)
-			if (lane == 0) done[k] = 0;
-		for (int it = 0; it < iters; it++)
+		const int it0 = together ? 0 : only, it1 = together ? iters : only + 1;
+		if (it0 == 0)
+			for (int k = wave; k < nroots; k += waves)
+				if (lane == 0) done[k] = 0;
+		for (int it = it0; it < it1; it++)
 		{
 			if (threadIdx.x == 0) active_s = 0;
 			// the loop runs once if the roots fit one tile; a wave then updates its roots in turn
@@ -447,13 +499,21 @@ __global__ __launch_bounds__(CCF_THREADS) void k_ccf_chain(ShootArgs a, dcx* __r
 				}
 			}
 			__syncthreads();
-			const int left = chain_barrier(slot + (long long)(j - j0) * iters + it, int(gridDim.x), active_s, failed);
-			if (left < 0) return;
-			double* swap = cur;
-			cur = nxt;
-			nxt = swap;
-			if (left == 0) break;
+			if (together)
+			{
+				const int left = chain_barrier(slot + (long long)(j - j0) * iters + it, int(gridDim.x), active_s, failed);
+				if (left < 0) return;
+				turn_over();
+				if (left == 0) break;
+			}
+			else
+			{
+				// the roots this wave has just written are the ones it stores below
+				asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+				turn_over();
+			}
 		}
+		if (!together && it1 < iters) continue;
 		for (int k = wave; k < nroots; k += waves)
 			if (lane < 2) reinterpret_cast<double*>(rows + (long long)R.row * nroots + k)[lane] = load_shared(cur + 2 * k + lane);
 	}
@@ -533,7 +593,7 @@ CCFResult Engine::ccf_solve(const LensParams& lens, const double* init_roots, in
 	DeviceBuffer<char> fin;
 	DeviceBuffer<int> leaf_cache;
 	DeviceBuffer<unsigned long long> err, slots;
-	DeviceBuffer<int> flags;   // a non-finite error; a barrier that timed out
+	DeviceBuffer<int> flags;   // a non-finite error; a barrier that timed out; blocks that did not meet
 	Ab.alloc(2 * total);
 	Bb.alloc(2 * 4 * (size_t)nb * nroots);
 	Cb.alloc(2 * total);
@@ -546,13 +606,13 @@ CCFResult Engine::ccf_solve(const LensParams& lens, const double* init_roots, in
 	fin.alloc(2 * (size_t)nb * nroots);
 	leaf_cache.alloc(2 * (size_t)nb * nroots);
 	err.alloc(1);
-	flags.alloc(2);
-	const size_t nslots = std::max((size_t)nb * init_iters, 2 * (size_t)nb * J * step_iters);
-	slots.alloc(std::max<size_t>(nslots, 1));
+	flags.alloc(3);
+	const size_t nslots = 2 * (size_t)nb + std::max((size_t)nb * init_iters, 2 * (size_t)nb * J * step_iters);
+	slots.alloc(nslots);
 	MLENS_HIP_CHECK(hipMemsetAsync(A.ptr, 0, total * sizeof(dcx), stream_));
 	MLENS_HIP_CHECK(hipMemsetAsync(leaf_cache.ptr, 0xff, 2 * (size_t)nb * nroots * sizeof(int), stream_));   // -1: none
 	MLENS_HIP_CHECK(hipMemsetAsync(err.ptr, 0, sizeof(unsigned long long), stream_));
-	MLENS_HIP_CHECK(hipMemsetAsync(flags.ptr, 0, 2 * sizeof(int), stream_));
+	MLENS_HIP_CHECK(hipMemsetAsync(flags.ptr, 0, 3 * sizeof(int), stream_));
 	// starting roots at the centre row of each branch
 	for (int c = 0; c < nb; c++)
 		MLENS_HIP_CHECK(hipMemcpyAsync(A.ptr + (long long)(c * (2 * J + 1) + J) * nroots, init_roots + 2 * (long long)c * nroots,
@@ -566,24 +626,37 @@ CCFResult Engine::ccf_solve(const LensParams& lens, const double* init_roots, in
 	const int resident = num_cus_ * std::max(1, per_cu);
 	auto sweep = [&](int from, int j0, int j1, int sides, int iters) {
 		if (j1 < j0 || iters < 1) return;
-		const int chains = nb * sides, group = std::min(chains, resident);
-		MLENS_HIP_CHECK(hipMemsetAsync(slots.ptr, 0, (size_t)chains * (j1 - j0 + 1) * iters * sizeof(unsigned long long), stream_));
-		k_ccf_start<<<dim3(blocks_for(nroots, 256), unsigned(chains)), 256, 0, stream_>>>(A.ptr, reinterpret_cast<dcx*>(Bb.ptr), nroots,
-			from, nphi, nb, sides);
+		const int chains = nb * sides, waves = CCF_THREADS / 64;
+		const unsigned row_blocks = blocks_for(nroots, 256);
+		dcx* work = reinterpret_cast<dcx*>(Bb.ptr);
+		int* bad = flags.ptr + 1;
+		const int ns = nstars_, pole = circle_pole ? 1 : 0;
+		auto launch = [&](int first, int here, int ja, int jb, int only, int flip) {
+			const int blocks = std::max(1, std::min((nroots + waves - 1) / waves, resident / here));
+			auto kernel = a.smooth_linear ? k_ccf_chain<true> : k_ccf_chain<false>;
+			kernel<<<dim3(unsigned(blocks), unsigned(here)), CCF_THREADS, 0, stream_>>>(a, A.ptr, Bb.ptr, fin.ptr, leaf_cache.ptr,
+				slots.ptr, bad, nroots, ns, pole, ja, jb, nphi, nb, sides, iters, first, only, flip);
+			MLENS_HIP_CHECK(hipGetLastError());
+		};
+		k_ccf_start<<<dim3(row_blocks, unsigned(chains)), 256, 0, stream_>>>(A.ptr, work, nroots, from, nphi, nb, sides);
 		MLENS_HIP_CHECK(hipGetLastError());
-		const int waves = CCF_THREADS / 64;
+		MLENS_HIP_CHECK(hipMemsetAsync(slots.ptr, 0, (chains + (size_t)chains * (j1 - j0 + 1) * iters) * sizeof(unsigned long long), stream_));
+		const int group = std::min(chains, resident);
 		for (int first = 0; first < chains; first += group)
 		{
 			const int here = std::min(group, chains - first);
-			const int blocks = std::max(1, std::min((nroots + waves - 1) / waves, resident / here));
-			dcx* rows = A.ptr;
-			double* work = Bb.ptr;
-			char* fp = fin.ptr;
-			int *lp = leaf_cache.ptr, *bad = flags.ptr + 1, ns = nstars_, pole = circle_pole ? 1 : 0;
-			unsigned long long* sp = slots.ptr;
-			void* args[] = {&a, &rows, &work, &fp, &lp, &sp, &bad, &nroots, &ns, &pole, &j0, &j1, &nphi, &nb, &sides, &iters, &first};
-			MLENS_HIP_CHECK(hipLaunchCooperativeKernel(kernel, dim3(unsigned(blocks), unsigned(here)), dim3(CCF_THREADS),
-				args, 0, stream_));
+			int nf[2] = {0, 1};
+			if (ccf_together_)
+			{
+				MLENS_HIP_CHECK(hipMemsetAsync(bad, 0, sizeof(nf), stream_));
+				launch(first, here, j0, j1, -1, 0);
+				MLENS_HIP_CHECK(hipMemcpyAsync(nf, bad, sizeof(nf), hipMemcpyDeviceToHost, stream_));
+				MLENS_HIP_CHECK(hipStreamSynchronize(stream_));
+			}
+			if (nf[0]) throw HipError("the blocks of a critical-curve chain lost each other", __FILE__, __LINE__);
+			if (!nf[1]) continue;
+			for (int j = j0, n = 0; j <= j1; j++)
+				for (int it = 0; it < iters; it++, n++) launch(first, here, j, j, it, n & 1);
 		}
 	};
 	CCFResult r;
@@ -609,12 +682,11 @@ CCFResult Engine::ccf_solve(const LensParams& lens, const double* init_roots, in
 	MLENS_HIP_CHECK(hipEventElapsedTime(&ms, ev0_, ev1_));
 	r.t_caustics_ms = ms;
 	unsigned long long eb = 0;
-	int nf[2] = {0, 0};
+	int nf = 0;
 	MLENS_HIP_CHECK(hipMemcpy(&eb, err.ptr, sizeof(eb), hipMemcpyDeviceToHost));
-	MLENS_HIP_CHECK(hipMemcpy(nf, flags.ptr, sizeof(nf), hipMemcpyDeviceToHost));
-	if (nf[1]) throw HipError("the blocks of a critical-curve chain did not meet", __FILE__, __LINE__);
+	MLENS_HIP_CHECK(hipMemcpy(&nf, flags.ptr, sizeof(nf), hipMemcpyDeviceToHost));
 	std::memcpy(&r.max_error, &eb, sizeof(double));
-	r.has_nan = nf[0] != 0;
+	r.has_nan = nf != 0;
 	MLENS_HIP_CHECK(hipMemcpy(ccs, C.ptr, total * sizeof(dcx), hipMemcpyDeviceToHost));
 	if (caustics) MLENS_HIP_CHECK(hipMemcpy(caustics, W.ptr, total * sizeof(dcx), hipMemcpyDeviceToHost));
 	if (mu_scales) MLENS_HIP_CHECK(hipMemcpy(mu_scales, M.ptr, total * sizeof(double), hipMemcpyDeviceToHost));

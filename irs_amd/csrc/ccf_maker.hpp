@@ -52,6 +52,9 @@ public:
 	int write_mu_length_scales = 0;
 	std::string outfile_prefix = "./";
 
+	/* extension: 0 sends every iteration out as a launch of its own (Engine::set_ccf_together) */
+	int resident_chains = 1;
+
 	/* ccf.cuh:1263-1280 */
 	bool run(int verbose)
 	{
@@ -425,6 +428,7 @@ private:
 		const size_t total = size_t(num_phi + num_branches) * num_roots_;
 		std::vector<double> ccs(2 * total), caust(write_caustics ? 2 * total : 0), mu(write_mu_length_scales ? total : 0);
 		MLENS_VERBOSE("Finding critical curve positions...\n", verbose, 1);
+		engine_->set_ccf_together(resident_chains != 0);
 		CCFResult r = engine_->ccf_solve(lens(), init.data(), num_roots_, num_phi, num_branches, !rectangular && !approx, ccs.data(),
 			write_caustics ? caust.data() : nullptr, write_mu_length_scales ? mu.data() : nullptr);
 		t_init_roots_ = r.t_init_ms / 1000.0;

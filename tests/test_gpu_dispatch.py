@@ -1,12 +1,16 @@
 """The kernel variants that a call's sizes and options choose, each at the edges of
 its range, against the FP64 oracle or the general path."""
 
+import os
+
 import numpy as np
 import pytest
 
 from common import C1_SMALL, Mirror, from_starfile, write_starfile
 
 pytestmark = pytest.mark.gpu
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 
 
 def say(msg):
@@ -180,6 +184,48 @@ def test_histograms_inside_and_past_the_window(tmp_path, irs, double, n1, n2):
     m.close()
 
 
+def test_critical_curves_beside_other_work(tmp_path):
+    """Chains of two objects and of two processes on the device at once, with a map being
+    shot beside them: blocks that are not all resident give way, and the roots stay the same."""
+    import subprocess
+    import sys
+    import threading
+    from irs_amd.microlensing.CCF.ccf import CCF
+    from irs_amd.microlensing.IPM.ipm import IPM
+    code = ("import sys; sys.path.insert(0, {root!r})\n"
+            "import numpy as np\n"
+            "from irs_amd.microlensing.CCF.ccf import CCF\n"
+            "for k in range(3):\n"
+            "    c = CCF(kappa_tot=0.3, shear=0.3, kappa_star=0.27, num_stars=600, num_phi=12, random_seed=3, write_stars=False)\n"
+            "    c.run()\n"
+            "np.save({out!r}, c.critical_curves)\n").format(root=ROOT, out=str(tmp_path / "other.npy"))
+
+    def curves():
+        c = CCF(kappa_tot=0.3, shear=0.3, kappa_star=0.27, num_stars=600, num_phi=12, random_seed=3, write_stars=False)
+        c.run()
+        out = c.critical_curves.copy()
+        c.close()
+        return out
+
+    alone = curves()
+    say("[ccf] beside another process, another object and a map")
+    other = subprocess.Popen([sys.executable, "-c", code])
+    results = []
+    threads = [threading.Thread(target=lambda: results.append(curves())) for _ in range(3)]
+    m = IPM(kappa_tot=0.45, shear=0.4, kappa_star=0.36, half_length_y1=5, half_length_y2=5, num_pixels_y1=1000,
+            num_pixels_y2=1000, num_rays_y=16, random_seed=2, write_histograms=False)
+    threads.append(threading.Thread(target=m.run))
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert other.wait(timeout=100) == 0
+    m.close()
+    for r in results + [np.load(tmp_path / "other.npy")]:
+        np.testing.assert_array_equal(r, alone)
+    assert len(results) == 3
+
+
 @pytest.mark.parametrize("stars,phases,branches,exact", [(1, 4, 1, False), (2, 4, 2, True), (5, 600, 300, False),
                                                          (1100, 2, 1, False), (2100, 2, 1, False)])
 def test_critical_curve_chains(stars, phases, branches, exact):
@@ -193,9 +239,15 @@ def test_critical_curve_chains(stars, phases, branches, exact):
     say(f"[ccf] {stars} stars, {phases} phases, {branches} branches, exact sheet {exact}")
     # one star on one branch cannot leave the line its starting roots lie on: use two there
     branches = max(branches, 2) if stars == 1 else branches
-    c = CCF(kappa_tot=0.3, shear=0.3, kappa_star=0.27, num_stars=stars, num_phi=phases, num_branches=branches, random_seed=7,
-            approx=not exact, write_stars=False)
+    kw = dict(kappa_tot=0.3, shear=0.3, kappa_star=0.27, num_stars=stars, num_phi=phases, num_branches=branches, random_seed=7,
+              approx=not exact, write_stars=False)
+    c, single = CCF(**kw), CCF(**kw)
     c.run()
+    # the path that a busy device takes, one iteration per launch: the same roots bit for bit
+    single.lib.set_resident_chains(single.obj, 0)
+    single.run()
+    np.testing.assert_array_equal(single.critical_curves, c.critical_curves)
+    single.close()
     prob = OC.Problem(c.stars, 0.3, 0.3, 1.0, 0.27, c.corner, approx=int(not exact))
     z = c.critical_curves[..., 0] + 1j * c.critical_curves[..., 1]
     half = phases // (2 * branches)
