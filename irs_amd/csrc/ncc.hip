@@ -5,14 +5,15 @@ weisluke/irs) on the MI355X.
 The reference gives each caustic segment a thread that, for every pixel row
 whose centre the segment crosses, adds +1 or -1 to every pixel left of the
 crossing: one global atomic per pixel, O(crossings x width). Here a crossing
-adds its +1 or -1 once, at the crossing's column of a row-difference grid;
-suffix sums along each row then give exactly the reference's counts (integer
-sums do not depend on their order). The over-sampled grid is reduced to the
-final one by the maximum over each 2^over_sample x 2^over_sample block, which
-is what the reference's repeated 2 x 2 reductions and shifts
-(ncc_functions.cuh:345-411) leave behind; one workgroup per final row does
-the sums and the maxima together, so the over-sampled counts never go back to
-memory.
+is recorded once, in the list of its sub-pixel row; a wave then spreads the
+row's list over the row's columns in LDS and takes suffix sums, which give exactly
+the reference's counts (integer sums do not depend on their order). The
+over-sampled grid is reduced to the final one by the maximum over each
+2^over_sample x 2^over_sample block, which is what the reference's repeated
+2 x 2 reductions and shifts (ncc_functions.cuh:345-411) leave behind. The
+over-sampled counts never exist in memory. Grids of more than NCC_LIST_COLS
+columns, and maps with a row whose list overflows, keep a row-difference grid
+in memory instead, to which a crossing adds its +1 or -1.
 
 Segment clipping and crossing positions follow ncc_functions.cuh:43-301 step
 by step in FP64. The reference evaluates the line intersection as
@@ -28,6 +29,7 @@ crossing bit for bit.
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <climits>
 #include <cmath>
 #include <stdexcept>
@@ -45,6 +47,23 @@ struct NCCArgs
 	double cx, cy;     // centre of the map
 	double hx, hy;     // half-lengths
 	int npx, npy;      // fine pixels per axis (final pixels << over_sample)
+};
+
+// what the host reads back: the map's extremes, the crossings made and those outside the grid, and whether a
+// row's list overflowed
+struct NCCMeta
+{
+	unsigned long long made, dropped;
+	int lo, hi, overflow, pad;
+};
+
+// the crossings of each sub-pixel row: count[row] of them (those past cap are not kept), each
+// column * 2 + (1 for an upward crossing)
+struct NCCLists
+{
+	int* count;
+	unsigned* entry;   // cap per row
+	int cap;
 };
 
 __device__ __forceinline__ double ncc_sgn(double v) { return v < 0 ? -1.0 : (v > 0 ? 1.0 : 0.0); }
@@ -105,16 +124,17 @@ __device__ __forceinline__ void corrected(double p1x, double p1y, double p2x, do
 The crossings (find_num_caustic_crossings_kernel, ncc_functions.cuh:170-301).
 A row crossed upwards (the caustics are traced clockwise) takes 1 from every
 pixel left of the crossing, a row crossed downwards adds 1: here at the
-crossing's column of the difference grid. Each lane clips one segment and
+crossing's column of the difference grid, or with LISTS an entry in the row's list. Each lane clips one segment and
 counts its crossings; the wave then deals all crossings of its 64 segments
 out to its lanes, 64 at a time, so that a long segment near a cusp (hundreds
 of rows) does not hold up the wave: a lane finds the segment of crossing c by
-a binary search over the lanes' first crossing indices. counters[0] counts the
-crossings, counters[1] those whose row is outside the grid (dropped, as the
+a binary search over the lanes' first crossing indices. meta counts the
+crossings and those whose row is outside the grid (dropped, as the
 reference's bounds check drops them). One wave per workgroup.
 */
+template <bool LISTS>
 __global__ __launch_bounds__(64) void k_ncc_crossings(const double* __restrict__ caus, int nrows, int ncols, NCCArgs g,
-	int* __restrict__ diff, unsigned long long* __restrict__ counters)
+	int* __restrict__ diff, NCCLists lists, NCCMeta* __restrict__ meta)
 {
 	const int lane = threadIdx.x & 63;
 	const long long nseg = (long long)nrows * (ncols - 1);
@@ -192,7 +212,16 @@ __global__ __launch_bounds__(64) void k_ncc_crossings(const double* __restrict__
 				dropped++;
 				continue;
 			}
-			atomicAdd(diff + row * g.npx + col, qup ? -1 : 1);
+			if (LISTS)
+			{
+				const int at = atomicAdd(lists.count + row, 1);
+				if (at < lists.cap)
+					lists.entry[row * lists.cap + at] = unsigned(col) * 2 + (qup ? 1 : 0);
+				else
+					meta->overflow = 1;
+			}
+			else
+				atomicAdd(diff + row * g.npx + col, qup ? -1 : 1);
 			made++;
 		}
 	}
@@ -204,8 +233,8 @@ __global__ __launch_bounds__(64) void k_ncc_crossings(const double* __restrict__
 	}
 	if (lane == 0 && (made | dropped))
 	{
-		atomicAdd(counters, made);
-		atomicAdd(counters + 1, dropped);
+		atomicAdd(&meta->made, made);
+		atomicAdd(&meta->dropped, dropped);
 	}
 }
 
@@ -263,6 +292,10 @@ one final pixel: they take their maximum by DPP and one of them merges it
 into LDS.
 */
 constexpr int NCC_FUSED_COLS = 8192;
+
+// orders this wave's LDS accesses: the compiler keeps them in program order
+// and the wave waits for its outstanding LDS operations
+__device__ __forceinline__ void wave_lds_sync() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
 
 __global__ __launch_bounds__(256) void k_ncc_rows_to_map(const int* __restrict__ diff, int* __restrict__ map, int np1,
 	int s, int* __restrict__ row_ext)
@@ -332,8 +365,123 @@ __global__ __launch_bounds__(256) void k_ncc_rows_to_map(const int* __restrict__
 	}
 }
 
+/*
+The final map from the rows' lists. A workgroup of WAVES waves owns WAVES / s final rows (at least one); a wave takes
+one sub-pixel row at a time: it clears the row's columns in LDS, adds the row's crossings to them, and sums from
+the right in tiles of 64 words, two columns a word in halves (an upward crossing's -1 borrows from the upper half,
+which reading the lower half as signed gives back; |difference| <= cap < 2^15). The s columns of a final pixel are
+s / 2 words of consecutive lanes, which take their maximum by DPP; one of them merges it into the final row in LDS.
+The over-sampled grid used to be zeroed, added to and read back in memory (64 MB at the defaults: 16 + 24 + 26 us,
+and 350 us to allocate and free); this takes no grid. Four waves share a workgroup up to 8192 columns, two up to
+16384 and one up to 32768, so that their rows fit in LDS.
+*/
+constexpr int NCC_LIST_COLS = 32768;
+
+template <int COLS, int WAVES>
+__global__ __launch_bounds__(64 * WAVES) void k_ncc_map_from_lists(NCCLists lists, int* __restrict__ map, int np1, int np2, int s,
+	int* __restrict__ row_ext)
+{
+	constexpr int THREADS = 64 * WAVES;
+	__shared__ unsigned words[WAVES][COLS / 2];
+	__shared__ int cmax[WAVES > 2 ? COLS : COLS / 2];   // the workgroup's final rows, s > 1
+	__shared__ int part[2][WAVES];
+	const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+	const int width = np1 * s, nw = (width + 1) / 2;
+	const int per = s >= WAVES ? 1 : WAVES / s;   // final rows of this workgroup
+	const int j0 = blockIdx.x * per;
+	unsigned* w = words[wave];
+	if (s > 1)
+	{
+		for (int c = threadIdx.x; c < per * np1; c += THREADS) cmax[c] = INT_MIN;
+		__syncthreads();
+	}
+	int lo = INT_MAX, hi = INT_MIN;   // s = 1: of this wave's row
+	for (int a = wave; a < per * s; a += WAVES)
+	{
+		const int j = j0 + a / s;
+		if (j >= np2) break;
+		const long long row = (long long)j0 * s + a;
+		for (int c = lane; c < nw; c += 64) w[c] = 0;
+		wave_lds_sync();
+		const int n = min(lists.count[row], lists.cap);
+		for (int e = lane; e < n; e += 64)
+		{
+			const unsigned v = lists.entry[row * lists.cap + e], col = v >> 1;
+			const unsigned one = (v & 1) ? ~0u : 1u;   // -1 for an upward crossing
+			atomicAdd(w + (col >> 1), (col & 1) ? one << 16 : one);
+		}
+		wave_lds_sync();
+		int carry = 0;
+		int* final_row = s > 1 ? cmax + (a / s) * np1 : nullptr;
+		int* out = map + (long long)j * np1;
+		for (int end = nw; end > 0; end -= 64)
+		{
+			const int c = end - 1 - lane;
+			const unsigned v = c >= 0 ? w[c] : 0;
+			const int left = int(short(v & 0xffffu)), right = int(v - unsigned(left)) >> 16;
+			const int sum = wave_prefix_sum(left + right) + carry;   // columns 2 c and up
+			carry = __builtin_amdgcn_readlane(sum, 63);
+			if (s == 1)
+			{
+				if (c >= 0)
+				{
+					const int r = sum - left;   // columns 2 c + 1 and up
+					out[2 * c] = sum;
+					lo = min(lo, sum);
+					hi = max(hi, sum);
+					if (2 * c + 1 < width)
+					{
+						out[2 * c + 1] = r;
+						lo = min(lo, r);
+						hi = max(hi, r);
+					}
+				}
+			}
+			else
+			{
+				const int g = min(s / 2, 64);
+				const int m = wave_group_max(c >= 0 ? max(sum, sum - left) : INT_MIN, g);
+				if (c >= 0 && (lane & (g - 1)) == 0) atomicMax(final_row + 2 * c / s, m);
+			}
+		}
+		wave_lds_sync();
+	}
+	if (s > 1)
+	{
+		// the final rows, and the extremes of all of them
+		__syncthreads();
+		for (int c = threadIdx.x; c < per * np1; c += THREADS)
+		{
+			if (j0 + c / np1 >= np2) break;
+			const int v = cmax[c];
+			map[(long long)j0 * np1 + c] = v;
+			lo = min(lo, v);
+			hi = max(hi, v);
+		}
+	}
+	for (int o = 32; o > 0; o >>= 1)
+	{
+		lo = min(lo, __shfl_xor(lo, o));
+		hi = max(hi, __shfl_xor(hi, o));
+	}
+	if (lane == 0)
+	{
+		part[0][wave] = lo;
+		part[1][wave] = hi;
+	}
+	__syncthreads();
+	if (threadIdx.x != 0) return;
+	for (int k = 1; k < WAVES; k++)
+	{
+		lo = min(lo, part[0][k]);
+		hi = max(hi, part[1][k]);
+	}
+	row_ext[2 * blockIdx.x] = lo;
+	row_ext[2 * blockIdx.x + 1] = hi;
+}
+
 // the map's extremes from the per-row ones: one workgroup
-__global__ __launch_bounds__(256) void k_ncc_row_extremes(const int* __restrict__ row_ext, int rows, int* __restrict__ ext)
+__global__ __launch_bounds__(256) void k_ncc_row_extremes(const int* __restrict__ row_ext, int rows, NCCMeta* __restrict__ meta)
 {
 	__shared__ int part[2][4];
 	int lo = INT_MAX, hi = INT_MIN;
@@ -360,25 +508,22 @@ __global__ __launch_bounds__(256) void k_ncc_row_extremes(const int* __restrict_
 			lo = min(lo, part[0][w]);
 			hi = max(hi, part[1][w]);
 		}
-		ext[0] = lo;
-		ext[1] = hi;
+		meta->lo = lo;
+		meta->hi = hi;
 	}
 }
 
-__global__ void k_ncc_init(int* ext, unsigned long long* counters)
+// clears meta and the first n list counts
+__global__ void k_ncc_init(NCCMeta* meta, int* count, int n)
 {
-	if (threadIdx.x == 0)
-	{
-		ext[0] = INT_MAX;
-		ext[1] = INT_MIN;
-		counters[0] = 0;
-		counters[1] = 0;
-	}
+	const int i = blockIdx.x * blockDim.x + threadIdx.x;
+	if (i == 0) *meta = NCCMeta{0, 0, INT_MAX, INT_MIN, 0, 0};
+	if (i < n) count[i] = 0;
 }
 
 // minimum and maximum of the map: one pair of atomics per workgroup (a few
 // dozen workgroups), not per wave, so they do not queue on two addresses
-__global__ __launch_bounds__(256) void k_ncc_extremes(const int* __restrict__ map, long long n, int* __restrict__ ext)
+__global__ __launch_bounds__(256) void k_ncc_extremes(const int* __restrict__ map, long long n, NCCMeta* __restrict__ meta)
 {
 	__shared__ int part[2][4];
 	int lo = INT_MAX, hi = INT_MIN;
@@ -405,15 +550,41 @@ __global__ __launch_bounds__(256) void k_ncc_extremes(const int* __restrict__ ma
 			lo = min(lo, part[0][w]);
 			hi = max(hi, part[1][w]);
 		}
-		atomicMin(ext, lo);
-		atomicMax(ext + 1, hi);
+		atomicMin(&meta->lo, lo);
+		atomicMax(&meta->hi, hi);
 	}
 }
 
 constexpr int NCC_LDS_BINS = 8192;
 
-// histogram_kernel (array_functions.cuh:115-131) with integer values: bins of
-// width 1 from vmin; per-workgroup counts in LDS when the range fits
+constexpr int NCC_FEW_BINS = 64;
+
+/* histogram_kernel (array_functions.cuh:115-131) with integer values: bins of width 1 from vmin, for ranges of at most
+   NCC_FEW_BINS values, the rule for crossing counts. Neighbouring pixels have equal counts, so a wave's atomics on
+   shared bins would queue on one or two addresses (30 us for 1000^2 pixels); here every lane counts in a column of
+   its own, and the columns are summed once. */
+__global__ __launch_bounds__(256) void k_ncc_histogram_few(const int* __restrict__ map, long long n, int vmin, int len,
+	unsigned long long* __restrict__ hist)
+{
+	__shared__ unsigned bins[NCC_FEW_BINS][64];
+	const int lane = threadIdx.x & 63;
+	for (int i = threadIdx.x; i < len * 64; i += 256) bins[i >> 6][i & 63] = 0;
+	__syncthreads();
+	for (long long q = (long long)blockIdx.x * 256 + threadIdx.x; q < n; q += (long long)gridDim.x * 256)
+	{
+		const int b = map[q] - vmin;
+		if (b >= 0 && b < len) atomicAdd(&bins[b][lane], 1u);   // values outside [vmin, vmax] are not counted
+	}
+	__syncthreads();
+	for (int b = threadIdx.x >> 6; b < len; b += 4)
+	{
+		unsigned v = bins[b][lane];
+		for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
+		if (lane == 0 && v) atomicAdd(hist + b, (unsigned long long)v);
+	}
+}
+
+// the same for any range; per-workgroup counts in LDS when the range fits
 template <bool LOCAL>
 __global__ __launch_bounds__(256) void k_ncc_histogram(const int* __restrict__ map, long long n, int vmin, int len,
 	unsigned long long* __restrict__ hist)
@@ -493,63 +664,87 @@ void NCCDevice::count(const double* caustics, int nrows, int ncols, const NCCGri
 
 	const size_t npts = size_t(nrows) * size_t(ncols);
 	if (caustics_.count < 2 * npts) caustics_.alloc(2 * npts);
-	const size_t nfine = size_t(npx) * size_t(npy);
-	if (fine_.count < nfine) fine_.alloc(nfine);
 	const long long npix = (long long)g.num_pixels_re * g.num_pixels_im;
 	if (map_.count < size_t(npix)) map_.alloc(size_t(npix));
-	if (extremes_.count < 2) extremes_.alloc(2);
-	if (counters_.count < 2) counters_.alloc(2);
 	map_pixels_ = npix;
-
+	if (row_ext_.count < size_t(2) * size_t(g.num_pixels_im)) row_ext_.alloc(size_t(2) * size_t(g.num_pixels_im));
+	if (meta_.count < sizeof(NCCMeta)) meta_.alloc(sizeof(NCCMeta));
+	NCCMeta* meta = reinterpret_cast<NCCMeta*>(meta_.ptr);
 	MLENS_HIP_CHECK(hipMemcpyAsync(caustics_.ptr, caustics, 2 * npts * sizeof(double), hipMemcpyHostToDevice, stream_));
-	MLENS_HIP_CHECK(hipMemsetAsync(fine_.ptr, 0, nfine * sizeof(int), stream_));
-	k_ncc_init<<<1, 64, 0, stream_>>>(extremes_.ptr, counters_.ptr);
-	MLENS_HIP_CHECK(hipGetLastError());
 
 	NCCArgs a{g.center_re, g.center_im, g.half_length_re, g.half_length_im, int(npx), int(npy)};
 	const long long nseg = (long long)nrows * (ncols - 1);
-	MLENS_HIP_CHECK(hipEventRecord(ev0_, stream_));
 	// one wave per workgroup: a few tens of thousands of segments still reach every CU
-	k_ncc_crossings<<<grid_for(nseg, 64, 1 << 16), 64, 0, stream_>>>(caustics_.ptr, nrows, ncols, a, fine_.ptr, counters_.ptr);
-	MLENS_HIP_CHECK(hipGetLastError());
-	MLENS_HIP_CHECK(hipEventRecord(ev1_, stream_));
-	const bool fused = g.num_pixels_re <= NCC_FUSED_COLS;
-	if (fused)
+	const unsigned seg_blocks = grid_for(nseg, 64, 1 << 16);
+	NCCMeta m;
+	auto finish = [&]() {
+		MLENS_HIP_CHECK(hipGetLastError());
+		MLENS_HIP_CHECK(hipMemcpyAsync(&m, meta, sizeof(m), hipMemcpyDeviceToHost, stream_));
+		MLENS_HIP_CHECK(hipMemcpyAsync(out, map_.ptr, size_t(npix) * sizeof(int), hipMemcpyDeviceToHost, stream_));
+		MLENS_HIP_CHECK(hipStreamSynchronize(stream_));
+	};
+	bool lists = npx <= NCC_LIST_COLS;
+	if (lists)
 	{
-		if (row_ext_.count < size_t(2) * size_t(g.num_pixels_im)) row_ext_.alloc(size_t(2) * size_t(g.num_pixels_im));
-		k_ncc_rows_to_map<<<unsigned(g.num_pixels_im), 256, 0, stream_>>>(fine_.ptr, map_.ptr, g.num_pixels_re, int(s),
-			row_ext_.ptr);
-		MLENS_HIP_CHECK(hipGetLastError());
+		// room for 512 crossings a row, more where rows are few; never more than the grid would take
+		NCCLists l;
+		l.cap = int(std::min<long long>(std::min<long long>(npx, 8192), std::max<long long>(512, (1 << 20) / npy)));
+		if (lists_.count < size_t(npy) * size_t(l.cap + 1)) lists_.alloc(size_t(npy) * size_t(l.cap + 1));
+		l.count = lists_.ptr;
+		l.entry = reinterpret_cast<unsigned*>(lists_.ptr + npy);
+		k_ncc_init<<<unsigned((npy + 255) / 256), 256, 0, stream_>>>(meta, l.count, int(npy));
+		MLENS_HIP_CHECK(hipEventRecord(ev0_, stream_));
+		k_ncc_crossings<true><<<seg_blocks, 64, 0, stream_>>>(caustics_.ptr, nrows, ncols, a, nullptr, l, meta);
+		MLENS_HIP_CHECK(hipEventRecord(ev1_, stream_));
+		unsigned blocks = 0;
+		auto rows_to_map = [&](auto kernel, int waves) {
+			const int per = s >= waves ? 1 : int(waves / s);
+			blocks = unsigned((g.num_pixels_im + per - 1) / per);
+			kernel<<<blocks, 64 * waves, 0, stream_>>>(l, map_.ptr, g.num_pixels_re, g.num_pixels_im, int(s), row_ext_.ptr);
+		};
+		if (npx <= 4096) rows_to_map(k_ncc_map_from_lists<4096, 4>, 4);
+		else if (npx <= 8192) rows_to_map(k_ncc_map_from_lists<8192, 4>, 4);
+		else if (npx <= 16384) rows_to_map(k_ncc_map_from_lists<16384, 2>, 2);
+		else rows_to_map(k_ncc_map_from_lists<32768, 1>, 1);
+		MLENS_HIP_CHECK(hipEventRecord(ev2_, stream_));
+		k_ncc_row_extremes<<<1, 256, 0, stream_>>>(row_ext_.ptr, int(blocks), meta);
+		finish();
+		lists = !m.overflow;
 	}
-	else
+	if (!lists)
 	{
-		k_ncc_row_sums<<<unsigned(npy), 256, 0, stream_>>>(fine_.ptr, int(npx));
-		MLENS_HIP_CHECK(hipGetLastError());
-		k_ncc_block_max<<<grid_for(npix), 256, 0, stream_>>>(fine_.ptr, map_.ptr, g.num_pixels_re, g.num_pixels_im, int(s));
-		MLENS_HIP_CHECK(hipGetLastError());
+		const size_t nfine = size_t(npx) * size_t(npy);
+		if (fine_.count < nfine) fine_.alloc(nfine);
+		MLENS_HIP_CHECK(hipMemsetAsync(fine_.ptr, 0, nfine * sizeof(int), stream_));
+		k_ncc_init<<<1, 64, 0, stream_>>>(meta, nullptr, 0);
+		MLENS_HIP_CHECK(hipEventRecord(ev0_, stream_));
+		k_ncc_crossings<false><<<seg_blocks, 64, 0, stream_>>>(caustics_.ptr, nrows, ncols, a, fine_.ptr, NCCLists{}, meta);
+		MLENS_HIP_CHECK(hipEventRecord(ev1_, stream_));
+		const bool fused = g.num_pixels_re <= NCC_FUSED_COLS;
+		if (fused)
+			k_ncc_rows_to_map<<<unsigned(g.num_pixels_im), 256, 0, stream_>>>(fine_.ptr, map_.ptr, g.num_pixels_re, int(s),
+				row_ext_.ptr);
+		else
+		{
+			k_ncc_row_sums<<<unsigned(npy), 256, 0, stream_>>>(fine_.ptr, int(npx));
+			k_ncc_block_max<<<grid_for(npix), 256, 0, stream_>>>(fine_.ptr, map_.ptr, g.num_pixels_re, g.num_pixels_im, int(s));
+		}
+		MLENS_HIP_CHECK(hipEventRecord(ev2_, stream_));
+		if (fused)
+			k_ncc_row_extremes<<<1, 256, 0, stream_>>>(row_ext_.ptr, g.num_pixels_im, meta);
+		else
+			k_ncc_extremes<<<grid_for(npix, 256, NCC_REDUCE_GRID), 256, 0, stream_>>>(map_.ptr, npix, meta);
+		finish();
 	}
-	MLENS_HIP_CHECK(hipEventRecord(ev2_, stream_));
-	if (fused)
-		k_ncc_row_extremes<<<1, 256, 0, stream_>>>(row_ext_.ptr, g.num_pixels_im, extremes_.ptr);
-	else
-		k_ncc_extremes<<<grid_for(npix, 256, NCC_REDUCE_GRID), 256, 0, stream_>>>(map_.ptr, npix, extremes_.ptr);
-	MLENS_HIP_CHECK(hipGetLastError());
-
-	MLENS_HIP_CHECK(hipMemcpyAsync(out, map_.ptr, size_t(npix) * sizeof(int), hipMemcpyDeviceToHost, stream_));
-	int ext[2];
-	unsigned long long cnt[2];
-	MLENS_HIP_CHECK(hipMemcpyAsync(ext, extremes_.ptr, sizeof(ext), hipMemcpyDeviceToHost, stream_));
-	MLENS_HIP_CHECK(hipMemcpyAsync(cnt, counters_.ptr, sizeof(cnt), hipMemcpyDeviceToHost, stream_));
-	MLENS_HIP_CHECK(hipStreamSynchronize(stream_));
 	float ms = 0;
 	MLENS_HIP_CHECK(hipEventElapsedTime(&ms, ev0_, ev1_));
 	st.t_ncc_ms = ms;
 	MLENS_HIP_CHECK(hipEventElapsedTime(&ms, ev1_, ev2_));
 	st.t_reduce_ms = ms;
-	st.min = ext[0];
-	st.max = ext[1];
-	st.crossings = (long long)cnt[0];
-	st.dropped = (long long)cnt[1];
+	st.min = m.lo;
+	st.max = m.hi;
+	st.crossings = (long long)m.made;
+	st.dropped = (long long)m.dropped;
 }
 
 void NCCDevice::histogram(int vmin, int vmax, long long* hist)
@@ -561,7 +756,9 @@ void NCCDevice::histogram(int vmin, int vmax, long long* hist)
 	if (hist_.count < size_t(len)) hist_.alloc(size_t(len));
 	k_ncc_zero<<<unsigned((len + 255) / 256), 256, 0, stream_>>>(hist_.ptr, int(len));
 	MLENS_HIP_CHECK(hipGetLastError());
-	if (len <= NCC_LDS_BINS)
+	if (len <= NCC_FEW_BINS)
+		k_ncc_histogram_few<<<grid_for(map_pixels_, 2048, 512), 256, 0, stream_>>>(map_.ptr, map_pixels_, vmin, int(len), hist_.ptr);
+	else if (len <= NCC_LDS_BINS)
 		k_ncc_histogram<true><<<grid_for(map_pixels_, 256, NCC_REDUCE_GRID), 256, 0, stream_>>>(map_.ptr, map_pixels_, vmin,
 			int(len), hist_.ptr);
 	else

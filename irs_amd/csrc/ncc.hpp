@@ -47,8 +47,10 @@ private:
 	hipStream_t stream_ = nullptr;
 	hipEvent_t ev0_ = nullptr, ev1_ = nullptr, ev2_ = nullptr;
 	DeviceBuffer<double> caustics_;
-	DeviceBuffer<int> fine_, map_, extremes_, row_ext_;
-	DeviceBuffer<unsigned long long> counters_, hist_;
+	DeviceBuffer<int> fine_, map_, row_ext_;
+	DeviceBuffer<int> lists_;    // the crossings of each sub-pixel row: counts, then entries
+	DeviceBuffer<char> meta_;    // what the host reads back
+	DeviceBuffer<unsigned long long> hist_;
 	long long map_pixels_ = 0;
 };
 

@@ -326,3 +326,36 @@ def test_deflections_of_mixed_waves(oracle, tmp_path, rect):
     ref = ref[0] if isinstance(ref, tuple) else ref
     assert np.max(np.abs(w[:256] - ref)) < 1e-10
     m.close()
+
+
+@pytest.mark.parametrize("npx,over_sample,curves", [((1, 1), 0, 3), ((7, 5), 0, 40), ((301, 9), 0, 40), ((64, 33), 1, 40),
+                                                    ((4095, 3), 0, 20), ((2048, 3), 1, 20), ((2049, 3), 1, 20), ((1025, 3), 3, 20),
+                                                    ((4100, 2), 2, 20), ((8193, 2), 1, 20), ((8193, 2), 2, 10), ((20, 6), 8, 8),
+                                                    ((40, 30), 1, 4000)])
+def test_crossing_lists(tmp_path, npx, over_sample, curves):
+    """Crossings go to a list per sub-pixel row, and one, two or four waves sum a row in
+    LDS: odd and even widths, one to 256 sub-pixels a pixel, the first and last width of
+    each variant, grids too wide for lists, and rows that overflow theirs (4000 curves over
+    60 rows), against the oracle: identical counts and histogram."""
+    from irs_amd.microlensing.NCC.ncc import NCC
+    from oracle import ncc as ON
+    rng = np.random.default_rng(curves + over_sample)
+    t = -np.linspace(0, 2 * np.pi, 60)
+    t[-1] = t[0]
+    size = np.exp(rng.normal(0.0, 0.5, (curves, 1)))
+    rows = (rng.uniform(-4, 4, (curves, 1)) + 1j * rng.uniform(-4, 4, (curves, 1)) +
+            size * np.exp(2j * np.pi * rng.random((curves, 1))) * (np.cos(t) ** 3 + 1j * np.sin(t) ** 3))
+    with open(tmp_path / "ccf_caustics.bin", "wb") as fh:
+        np.array(rows.shape, dtype=np.int32).tofile(fh)
+        np.ascontiguousarray(rows, dtype=np.complex128).tofile(fh)
+    say(f"[ncc lists] {npx}, over_sample {over_sample}, {curves} curves")
+    prefix = str(tmp_path) + "/"
+    n = NCC(infile_prefix=prefix, outfile_prefix=prefix, num_pixels_y1=npx[0], num_pixels_y2=npx[1], over_sample=over_sample,
+            write_maps=False)
+    n.run()
+    want = ON.ncc_map(rows, (0.0, 0.0), (5.0, 5.0), npx, over_sample)
+    np.testing.assert_array_equal(n.num_caustic_crossings, want)
+    n.save()
+    u, c = np.unique(want, return_counts=True)
+    np.testing.assert_array_equal(np.loadtxt(prefix + "ncc_ncc_numpixels.txt", dtype=np.int64, ndmin=2), np.column_stack([u, c]))
+    n.close()
