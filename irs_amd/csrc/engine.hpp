@@ -215,7 +215,7 @@ private:
 	int m2l_ready_p_ = -1;
 	bool m2l_ready_f32_ = false;
 	DeviceBuffer<float> m2l_af_;
-	DeviceBuffer<double> m2l_ad_;
+	DeviceBuffer<double> m2l_ad_, m2l_powers_;
 	DeviceBuffer<unsigned long long> m2l_count_;
 	hipEvent_t m2l_ev0_ = nullptr, m2l_ev1_ = nullptr;
 

@@ -258,60 +258,100 @@ void launch_m2l(int kp, bool wide, hipStream_t st, const T* At, const double* mu
 
 }  // namespace
 
-// the 40 offset matrices for order p, real-stacked, transposed and padded
+namespace
+{
+
+// per offset: log(-dz), then (-dz)^-k and dz^-k, k < P
+constexpr int M2L_POWERS = 1 + 2 * (MAX_EXPANSION_ORDER + 1);
+
+/* The 40 offset matrices for order p (blockIdx.x = offset), stacked [Mr -Mi; Mi Mr], stored transposed At[col][row]
+   and zero-padded to kp. The host sends the powers of the offsets (60 KB) and the binomials; building the matrices
+   there and copying them took 0.4 ms of a small field's build. Contraction is off: the entries are those that the
+   host's complex products give. */
+template <typename T>
+__global__ void k_m2l_matrices(const double* __restrict__ powers, const double* __restrict__ B, int p, int kp, T* __restrict__ A)
+{
+#pragma clang fp contract(off)
+	const int o = blockIdx.x, P = p + 1;
+	const double* w = powers + o * M2L_POWERS * 2;
+	const double *ip = w + 2, *dzi = ip + 2 * P;
+	T* Ao = A + (long long)o * kp * kp;
+	for (int i = blockIdx.y * blockDim.x + threadIdx.x; i < kp * kp; i += gridDim.y * blockDim.x)
+	{
+		const int col = i / kp, row = i - col * kp;
+		double v = 0;
+		if (col < 2 * P && row < 2 * P)
+		{
+			const int k = col % P, l = row % P;
+			double re, im;
+			if (l == 0)
+			{
+				re = k == 0 ? w[0] : ip[2 * k];
+				im = k == 0 ? w[1] : ip[2 * k + 1];
+			}
+			else if (k == 0)
+			{
+				re = -dzi[2 * l] / double(l);
+				im = -dzi[2 * l + 1] / double(l);
+			}
+			else
+			{
+				const int n = l + k - 1;
+				const double c = B[n * (n + 1) / 2 + k - 1];
+				const double a = c * ip[2 * k], b = c * ip[2 * k + 1], d = dzi[2 * l], e = dzi[2 * l + 1];
+				re = a * d - b * e;
+				im = a * e + b * d;
+			}
+			v = (col < P) == (row < P) ? re : (col < P ? im : -im);
+		}
+		Ao[i] = T(v);
+	}
+}
+
+}  // namespace
+
 void Engine::m2l_prepare(int p, bool f32)
 {
 	if (m2l_ready_p_ == p && m2l_ready_f32_ == f32) return;
 	const int P = p + 1, kp = m2l_kp(p);
-	// exact binomials C(n, k), n <= 2p
-	std::vector<std::vector<unsigned long long>> C(2 * P + 1);
-	for (int nr = 0; nr <= 2 * P; nr++)
-	{
-		C[nr].assign(nr + 1, 1ull);
-		for (int k = 1; k < nr; k++) C[nr][k] = C[nr - 1][k - 1] + C[nr - 1][k];
-	}
-	std::vector<double> A(size_t(M2L_OFFSETS) * kp * kp, 0.0);
+	std::vector<double> w(size_t(M2L_OFFSETS) * M2L_POWERS * 2, 0.0);
 	for (int b = -3; b <= 3; b++)
 		for (int a = -3; a <= 3; a++)
 		{
 			const int o = m2l_offset_index(a, b);
 			if (o < 0) continue;
 			const std::complex<double> dz(2.0 * a, 2.0 * b), mdz = -dz, imdz = 1.0 / mdz;
-			std::vector<std::complex<double>> ipow(P), dzinv(P);
-			ipow[0] = 1.0;
-			dzinv[0] = 1.0;
-			for (int k = 1; k < P; k++)
-			{
-				ipow[k] = ipow[k - 1] * imdz;
-				dzinv[k] = dzinv[k - 1] / dz;
-			}
-			double* Ao = A.data() + size_t(o) * kp * kp;
-			auto put = [&](int l, int k, std::complex<double> m) {
-				// stacked [Mr -Mi; Mi Mr], stored transposed: At[col][row]
-				Ao[size_t(k) * kp + l] = m.real();
-				Ao[size_t(P + k) * kp + l] = -m.imag();
-				Ao[size_t(k) * kp + P + l] = m.imag();
-				Ao[size_t(P + k) * kp + P + l] = m.real();
+			double* q = w.data() + size_t(o) * M2L_POWERS * 2;
+			auto put = [&](int at, std::complex<double> v) {
+				q[2 * at] = v.real();
+				q[2 * at + 1] = v.imag();
 			};
-			put(0, 0, std::log(mdz));
-			for (int k = 1; k < P; k++) put(0, k, ipow[k]);
-			for (int l = 1; l < P; l++)
+			put(0, std::log(mdz));
+			std::complex<double> ipow = 1.0, dzinv = 1.0;
+			for (int k = 0; k < P; k++)
 			{
-				put(l, 0, -dzinv[l] / double(l));
-				for (int k = 1; k < P; k++) put(l, k, double(C[l + k - 1][k - 1]) * ipow[k] * dzinv[l]);
+				put(1 + k, ipow);
+				put(1 + P + k, dzinv);
+				ipow = ipow * imdz;
+				dzinv = dzinv / dz;
 			}
 		}
+	m2l_powers_.alloc(w.size());
+	MLENS_HIP_CHECK(hipMemcpyAsync(m2l_powers_.ptr, w.data(), w.size() * sizeof(double), hipMemcpyHostToDevice, stream_));
+	const size_t n = size_t(M2L_OFFSETS) * kp * kp;
+	const dim3 grid(M2L_OFFSETS, 4);
 	if (f32)
 	{
-		std::vector<float> Af(A.begin(), A.end());
-		m2l_af_.alloc(Af.size());
-		MLENS_HIP_CHECK(hipMemcpy(m2l_af_.ptr, Af.data(), Af.size() * sizeof(float), hipMemcpyHostToDevice));
+		m2l_af_.alloc(n);
+		k_m2l_matrices<float><<<grid, 256, 0, stream_>>>(m2l_powers_.ptr, binom_.ptr, p, kp, m2l_af_.ptr);
 	}
 	else
 	{
-		m2l_ad_.alloc(A.size());
-		MLENS_HIP_CHECK(hipMemcpy(m2l_ad_.ptr, A.data(), A.size() * sizeof(double), hipMemcpyHostToDevice));
+		m2l_ad_.alloc(n);
+		k_m2l_matrices<double><<<grid, 256, 0, stream_>>>(m2l_powers_.ptr, binom_.ptr, p, kp, m2l_ad_.ptr);
 	}
+	MLENS_HIP_CHECK(hipGetLastError());
+	// w is read before the copy returns (pageable memory), so it may go
 	m2l_ready_p_ = p;
 	m2l_ready_f32_ = f32;
 }

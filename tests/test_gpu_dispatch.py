@@ -136,6 +136,24 @@ def test_trees_of_every_split_path(oracle, tmp_path, n, cluster):
     m.close()
 
 
+@pytest.mark.parametrize("n", [1, 15, 255, 256, 257, 4096, 4097, 70000])
+def test_star_moments_of_every_count(tmp_path, n):
+    """A block sums 16 of 256 interleaved chains, 16 stars of each at a time: fields with
+    fewer stars than chains, at a round's edges and of many rounds, masses over five
+    decades. The terms of a sum add in n / 256 + 8 steps of an ulp and log is good to
+    one, so 1e-12 of the sum of the terms' magnitudes holds for every n here."""
+    rng = np.random.default_rng(n)
+    mass = 10.0 ** rng.uniform(-4, 1, n)
+    mass *= 16.0 / mass.sum()
+    m = built(tmp_path / "stars.bin", np.column_stack([disk(rng, n, 39.0), mass]), 8)
+    logs = mass * mass * np.log(mass)
+    for got, terms in ((m.lib.get_mean_mass_actual(m.obj), mass), (m.lib.get_mean_mass2_actual(m.obj), mass * mass),
+                       (m.lib.get_mean_mass2_ln_mass_actual(m.obj), logs)):
+        assert abs(got - terms.mean()) <= 1e-12 * np.abs(terms).mean()
+    assert m.lib.get_m_lower_actual(m.obj) == mass.min() and m.lib.get_m_upper_actual(m.obj) == mass.max()
+    m.close()
+
+
 @pytest.mark.parametrize("order", [1, 3, 7, 8, 15, 16, 23, 24, 31])
 def test_fmm_at_the_edges_of_its_matrix_sizes(oracle, tmp_path, order):
     """The stacked M2L matrices are padded to 16, 32, 48 or 64: the first and last order
