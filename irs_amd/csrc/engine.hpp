@@ -238,6 +238,7 @@ private:
 	DeviceBuffer<char> tmap_, tmap_min_, tmap_sad_;
 	// FP64 span maps beside them: span_ for the map, span_min_ / span_sad_ with parities
 	DeviceBuffer<char> span_, span_min_, span_sad_;
+	DeviceBuffer<char> wide_;   // WideList; its counts are zero between shots
 	int tiles_x_ = 0;
 	size_t tmap_bytes_ = 0;
 	void ensure_tiled_maps();

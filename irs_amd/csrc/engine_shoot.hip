@@ -555,10 +555,10 @@ their exact areas in full passes of 64. A lane finds its entry (or row) as the
 last one that starts at or before its own index: every entry (row) starting in
 the current pass marks its first slot in LDS, and a max-scan over the slots
 carries each mark forward, starting from the entry (row) the previous pass
-ended in. rh / rt: next ring slot to process / to fill.
+ended in. rh / rt: next ring slot to process / to fill. Returns the passes it took, of rows and of pixels.
 */
 template <typename MapT, bool PARITY, bool TILED, class Q>
-__device__ __forceinline__ void tri_queue_flush(const ShootArgs& a, Q& q, int qn)
+__device__ __forceinline__ int tri_queue_flush(const ShootArgs& a, Q& q, int qn)
 {
 	const double factor = a.factor;
 	const int lane = threadIdx.x & 63;
@@ -721,6 +721,7 @@ __device__ __forceinline__ void tri_queue_flush(const ShootArgs& a, Q& q, int qn
 		tri_queue_exact<MapT, PARITY, TILED>(a, q, rh, rt - rh);
 	}
 	wave_lds_sync();
+	return (total >> 6) + (rt >> 6) + 2;
 }
 
 // wave-wide: lanes with gen set append g to the queue
@@ -749,6 +750,130 @@ __device__ __forceinline__ void tri_queue_push(Q& q, int& qn, bool gen, const Ge
 	qn += __popcll(m);
 }
 
+/*
+Work left for later launches. The demagnified images around a star are spread
+over the whole source plane, thousands of triangles of up to 1e4 pixels each in
+one or two tiles, and a launch used to end with the waves that hold them: on a
+1000^2 map all other tiles were done after 0.9 of the kernel's 3.4 ms.
+
+A triangle whose box has WIDE_SPAN or more rows and columns together goes to a
+list in memory instead of the wave's queue, and a launch of its own rasterises
+the list with the whole device. After a row that took more than ROW_BUDGET
+passes of the rasteriser the tile leaves its next ROW_RUN rows on another list;
+the launch after it shoots them in parts of ROW_PART cells, each deflecting its
+corners again. Where a list is full, the work stays with its wave.
+
+The three launches together (1000^2 map, the same in FP64 with parities, 256^2
+map): 1.74, 9.0 and 0.61 ms, against 3.4, 11.9 and 0.65 with neither list. With
+wide triangles from 48 on 1.99, 10.3 and 0.71 (parts of 16 cells, after 24
+passes); parts of whole rows 1.76, 9.2 and 0.68; after 96 passes 2.2, 10.1 and
+0.70. A 10000^2 map, 1.12 s, gains 0.1%. A batch keeps its waves busy to the
+end by itself, and the lists only cost there (6.7 ms without, 7.1 with wide
+triangles, 7.8 with both).
+*/
+constexpr int WIDE_SPAN = 96;
+constexpr unsigned WIDE_CAP = 1 << 16;
+constexpr int WIDE_GROUP = 8;   // triangles that a wave rasterises together, at most
+constexpr int ROW_BUDGET = 32;
+constexpr int ROW_RUN = 8;
+constexpr int ROW_PART = 32;
+constexpr int ROW_PARTS = 2;   // 63 cells
+constexpr unsigned ROW_CAP = 1 << 15;
+
+struct WideTri
+{
+	double x[3], y[3];
+	int X0, Y0, wb, h;
+};
+
+struct LateRow
+{
+	long long J;   // the row of the cells' upper corners
+	long long tile_x;
+};
+
+struct WideList
+{
+	unsigned count;   // triangles offered: may exceed WIDE_CAP
+	unsigned rows;    // rows offered: may exceed ROW_CAP
+	unsigned taken;   // parts of rows that the second launch has handed out
+	unsigned unused[13];
+	LateRow row[ROW_CAP];
+	WideTri tri[WIDE_CAP];
+};
+
+// wave-wide: leaves rows J .. J + n - 1 of the tile for later; how many of them the list had room for
+__device__ __forceinline__ int rows_push(const ShootArgs* cold, long long tile_x, long long J, int n)
+{
+	WideList* list = cold->wide;
+	const int lane = threadIdx.x & 63;
+	unsigned base = __builtin_amdgcn_readfirstlane(__hip_atomic_load(&list->rows, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+	if (base >= ROW_CAP) return 0;
+	if (lane == 0) base = atomicAdd(&list->rows, unsigned(n));
+	base = __builtin_amdgcn_readfirstlane(base);
+	if (base >= ROW_CAP) return 0;
+	n = min(n, int(ROW_CAP - base));
+	if (lane < n) list->row[base + lane] = LateRow{J + lane, tile_x};
+	return n;
+}
+
+// wave-wide: lanes with gen set and a wide triangle append it to the list; false in gen where they did
+__device__ __forceinline__ bool wide_push(const ShootArgs* cold, bool gen, const GenTri& g)
+{
+	const bool wide = gen && g.w + g.h >= WIDE_SPAN;
+	const unsigned long long m = __ballot(wide);
+	if (m == 0) return gen;
+	WideList* list = cold->wide;
+	unsigned base = __builtin_amdgcn_readfirstlane(__hip_atomic_load(&list->count, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+	if (base >= WIDE_CAP) return gen;   // full: no more waiting in line for its counter
+	if ((threadIdx.x & 63) == 0) base = atomicAdd(&list->count, unsigned(__popcll(m)));
+	base = __builtin_amdgcn_readfirstlane(base);
+	if (!wide) return gen;
+	const unsigned pos = base + __builtin_amdgcn_mbcnt_hi(unsigned(m >> 32), __builtin_amdgcn_mbcnt_lo(unsigned(m), 0u));
+	if (pos >= WIDE_CAP) return gen;
+	WideTri& t = list->tri[pos];
+#pragma unroll
+	for (int i = 0; i < 3; i++)
+	{
+		t.x[i] = g.x[i];
+		t.y[i] = g.y[i];
+	}
+	t.X0 = g.X0;
+	t.Y0 = g.Y0;
+	t.wb = (g.w << 1) | g.bit;
+	t.h = g.h;
+	return false;
+}
+
+// Rasterises the list: a wave takes WIDE_GROUP neighbouring triangles at a time, fewer when that leaves waves without any.
+template <typename MapT, bool PARITY, class Q>
+__device__ __forceinline__ void wide_flush(const ShootArgs& a, Q& q)
+{
+	const WideList* list = a.wide;
+	const unsigned n = min(list->count, WIDE_CAP);
+	const unsigned group = min(max(n / gridDim.x, 1u), unsigned(WIDE_GROUP));
+	const int lane = threadIdx.x & 63;
+	for (unsigned g0 = blockIdx.x * group; g0 < n; g0 += gridDim.x * group)
+	{
+		const int qn = int(min(group, n - g0));
+		if (lane < qn)
+		{
+			const WideTri& t = list->tri[g0 + lane];
+#pragma unroll
+			for (int k = 0; k < 3; k++)
+			{
+				q.x[k][lane] = t.x[k];
+				q.y[k][lane] = t.y[k];
+			}
+			q.X0[lane] = t.X0;
+			q.Y0[lane] = t.Y0;
+			q.wb[lane] = t.wb;
+			q.end[lane] = t.h;
+		}
+		tri_queue_flush<MapT, PARITY, true>(a, q, qn);
+	}
+}
+
 // waves per block: one for the single-map kernel (2.39 s on the 10000^2 map,
 // 2.409 s with two, 2.428 s with four) and for the persistent batch kernel, so
 // that no wave waits for the slowest wave of its block
@@ -760,16 +885,17 @@ constexpr int IPM_RESIDENT_WAVES_PER_CU = 16;   // four per SIMD: up to 128 VGPR
 constexpr int IPM_TILE_H = 8;         // lattice rows a wave walks: the shortest tile
 constexpr int IPM_TILE_H_MAX = 1024;  // and the tallest
 
+static inline unsigned wide_blocks(int num_cus) { return unsigned(IPM_RESIDENT_WAVES_PER_CU * (num_cus > 0 ? num_cus : 256)); }
+
 /* Rows per tile for a launch of ntx tile columns over `rows` lattice rows: the
    tallest power of two in [IPM_TILE_H, IPM_TILE_H_MAX] that still gives at
    least eight blocks per resident block slot. A tall tile deflects
    its first row once per 1024 rows instead of once per 64 and flushes its
    queue less often (10000^2 map: 2.475 s at 64 rows, 2.428 s at 1024). A short
    one keeps a small lattice spread over the whole device and its longest tile
-   short: the demagnified images around one star are the work of thousands of
-   other cells, and the launch ends with the tile that holds them. A 256^2 map
-   (2048 x 6144 cells) took 2.24 ms at 64 rows, 1.08 ms at 16, 0.64 ms at 8 and
-   the same at 4 or 2; a 1000^2 map (4288 x 10716) 6.1, 3.4, 3.3 and 3.3 ms. */
+   short. A 256^2 map (2048 x 6144 cells) took 0.61 ms at 8 rows and 0.76 at 16;
+   a 1000^2 map (4288 x 10716) 1.74 ms at either and 2.1 ms where four blocks a
+   slot were enough. */
 static inline int ipm_tile_rows(long long ntx, long long rows, int num_cus)
 {
 	const long long want = 8LL * (IPM_RESIDENT_WAVES_PER_CU / IPM_WAVES) * (num_cus > 0 ? num_cus : 256);
@@ -778,21 +904,27 @@ static inline int ipm_tile_rows(long long ntx, long long rows, int num_cus)
 	return h;
 }
 
-// One tile: this wave's 63 cells of lattice columns tile_x * 63 WAVES + wave * 63 + [0, 63),
-// cell rows [J0, J1). Every lane of the wave must call it.
-template <int PREC, bool PARITY, bool TILED, int WAVES, bool LIN, class Q>
-__device__ __forceinline__ void ipm_tile(const ShootArgs& a, const ShootArgs* cold, Q& q, long long tile_x, long long J0, long long J1)
+// What a wave shoots: a tile whose heavy rows and triangles are left for later launches, a tile and
+// all that is in it, or the part of one row of a tile that an earlier launch left.
+enum TileWork { TILE_LATE, TILE_WHOLE, TILE_PART };
+
+// One tile: this wave's 63 cells of lattice columns tile_x * 63 WAVES + wave * 63 + [0, 63), of a
+// part the cells [c0, c1) of them, cell rows [J0, J1). Every lane of the wave must call it.
+template <int PREC, bool PARITY, bool TILED, int WAVES, bool LIN, TileWork WORK, class Q>
+__device__ __forceinline__ void ipm_tile(const ShootArgs& a, const ShootArgs* cold, Q& q, long long tile_x, long long J0, long long J1,
+	int c0 = 0, int c1 = 63)
 {
+	constexpr bool PART = WORK == TILE_PART;
 	const int lane = threadIdx.x & 63;
 	const int wave = threadIdx.x >> 6;
 	const long long I = tile_x * (63 * WAVES) + wave * 63 + lane;
 	const long long Ic = I < a.N1 ? I : a.N1;
 	const double zx = lattice_at(a.x0, a.stepx, Ic);
-	const bool cell_ok = lane < 63 && I < a.N1;
+	const bool cell_ok = (PART ? lane >= c0 && lane < c1 : lane < 63) && I < a.N1;
 	LeafCache cache;
 	using MapT = typename std::conditional<PREC == PREC_MIXED, float, double>::type;
 	PixelAcc<MapT> acc;
-	int qn = 0;
+	int qn = 0, passes = 0;
 
 	auto corner = [&](long long J, double& px, double& py) {
 		double zy = lattice_at(a.y0, a.stepy, J);
@@ -802,11 +934,17 @@ __device__ __forceinline__ void ipm_tile(const ShootArgs& a, const ShootArgs* co
 		py = double(a.n2) - ((d.wy - a.cyy) + a.h2) * a.s2;
 	};
 
-	double bx, by;
-	corner(J0, bx, by);
-	double brx = __shfl_down(bx, 1), bry = __shfl_down(by, 1);
-	for (long long J = J0 + 1; J <= J1; J++)
+	double bx = 0, by = 0, brx = 0, bry = 0;
+	bool below = false;   // the corners below are at hand
+	for (long long J = J0; J <= J1; J++)
 	{
+		if (WORK == TILE_LATE && passes > ROW_BUDGET)
+		{
+			const int n = rows_push(cold, tile_x, J, int(min((long long)ROW_RUN, J1 - J + 1)));
+			below = below && n == 0;
+			if (n > 0) J += n - 1;
+		}
+		passes = 0;
 		double tx, ty;
 		corner(J, tx, ty);
 		double trx = __shfl_down(tx, 1), try_ = __shfl_down(ty, 1);
@@ -820,20 +958,37 @@ __device__ __forceinline__ void ipm_tile(const ShootArgs& a, const ShootArgs* co
 			const double bxx = t ? brx : tx, byy = t ? bry : ty;
 			const double cx = t ? trx : bx, cy = t ? try_ : by;
 			GenTri g;
-			const bool gen = cell_ok && ipm_triangle<PREC, PARITY, MapT, TILED>(a, acc, ax, ay, bxx, byy, cx, cy, g);
-			tri_queue_push(q, qn, gen, g);
-			if (qn > Q::FLUSH || (qn > 0 && t == 1 && J == J1))
+			const bool gen = below && cell_ok && ipm_triangle<PREC, PARITY, MapT, TILED>(a, acc, ax, ay, bxx, byy, cx, cy, g);
+			tri_queue_push(q, qn, WORK == TILE_WHOLE ? gen : wide_push(cold, gen, g), g);
+			if (qn > (PART ? Q::FLUSH + 64 - ROW_PART : Q::FLUSH) || (qn > 0 && t == 1 && J == J1))
 			{
-				tri_queue_flush<MapT, PARITY, TILED>(a, q, qn);
+				passes += tri_queue_flush<MapT, PARITY, TILED>(a, q, qn);
 				qn = 0;
 			}
 		}
+		below = true;
 		bx = tx;
 		by = ty;
 		brx = trx;
 		bry = try_;
 	}
 	acc_flush<MapT, PARITY>(a, acc);
+}
+
+// the parts of the listed rows, handed out one at a time; take(row, c0, c1) shoots one
+template <class F>
+__device__ __forceinline__ void late_rows(WideList* list, F take)
+{
+	const unsigned parts = min(list->rows, ROW_CAP) * ROW_PARTS;
+	for (;;)
+	{
+		unsigned u = 0;
+		if ((threadIdx.x & 63) == 0) u = atomicAdd(&list->taken, 1u);
+		u = __builtin_amdgcn_readfirstlane(u);
+		if (u >= parts) break;
+		const int c0 = int(u % ROW_PARTS) * ROW_PART;
+		take(load_const(&list->row[u / ROW_PARTS]), c0, min(c0 + ROW_PART, 63));
+	}
 }
 
 // Compiled for linear smooth matter (LIN) the kernel needs 114 VGPRs and spills no scalar
@@ -854,7 +1009,32 @@ __global__ __launch_bounds__(64 * IPM_WAVES, LIN ? 4 : 3) void k_ipm_fast(ShootA
 	if (J0 >= row1) return;
 	const long long J1 = min(J0 + tile_h, row1);
 	__shared__ TriQueue<IPM_QCAP> queues[IPM_WAVES];
-	ipm_tile<PREC, PARITY, true, IPM_WAVES, LIN>(a, kernarg_block(), queues[threadIdx.x >> 6], blockIdx.x, J0, J1);
+	ipm_tile<PREC, PARITY, true, IPM_WAVES, LIN, TILE_LATE>(a, kernarg_block(), queues[threadIdx.x >> 6], blockIdx.x, J0, J1);
+}
+
+// the rows that a launch of k_ipm_fast left
+template <int PREC, bool PARITY, bool LIN>
+__global__ __launch_bounds__(64, LIN ? 4 : 3) void k_ipm_rows(ShootArgs a, MLENS_TABLE_PARAMS, void* __restrict__ map,
+	void* __restrict__ mmin, void* __restrict__ msad, void* __restrict__ span, void* __restrict__ span_sad)
+{
+	MLENS_TABLE_REBIND(a)
+	a.map = map;
+	a.mmin = mmin;
+	a.msad = msad;
+	a.span = span;
+	a.span_sad = span_sad;
+	__shared__ TriQueue<IPM_QCAP> q;
+	late_rows(a.wide, [&](const LateRow& r, int c0, int c1) {
+		ipm_tile<PREC, PARITY, true, 1, LIN, TILE_PART>(a, kernarg_block(), q, r.tile_x, r.J - 1, r.J, c0, c1);
+	});
+}
+
+// the triangles that the two launches before it left
+template <typename MapT, bool PARITY>
+__global__ __launch_bounds__(64, 4) void k_ipm_wide(ShootArgs a)
+{
+	__shared__ TriQueue<WIDE_GROUP> q;
+	wide_flush<MapT, PARITY>(a, q);
 }
 
 /*
@@ -1016,7 +1196,7 @@ __global__ __launch_bounds__(64 * IPM_BATCH_WAVES, LIN ? 4 : 3) void k_ipm_batch
 		const long long J0 = ty * tile_h + piece * BATCH_PIECE_H;
 		const long long J1 = min(min(J0 + (long long)rows, (ty + 1) * tile_h), a.N2);
 		if (J0 >= J1) continue;
-		ipm_tile<PREC_MIXED, false, true, IPM_BATCH_WAVES, LIN>(a, args + lo, queues[threadIdx.x >> 6], tx, J0, J1);
+		ipm_tile<PREC_MIXED, false, true, IPM_BATCH_WAVES, LIN, TILE_WHOLE>(a, args + lo, queues[threadIdx.x >> 6], tx, J0, J1);
 	}
 }
 
@@ -1607,6 +1787,11 @@ void Engine::ensure_tiled_maps()
 	const int tx = (npix_[0] + W - 1) / W;
 	const size_t bytes = size_t(tx) * size_t((npix_[1] + H - 1) / H) * 128;
 	const size_t sbytes = bytes;
+	if (!wide_.ptr)
+	{
+		wide_.alloc(sizeof(WideList));
+		MLENS_HIP_CHECK(hipMemsetAsync(wide_.ptr, 0, offsetof(WideList, row), stream_));
+	}
 	const bool have = parities_ ? (tmap_min_.ptr && span_min_.ptr && span_sad_.ptr) : span_.ptr != nullptr;
 	if (tmap_.ptr && tiles_x_ == tx && tmap_bytes_ == bytes && have) return;
 	tiles_x_ = tx;
@@ -1636,11 +1821,12 @@ void Engine::ensure_tiled_maps()
 	}
 }
 
-// the fold of a whole map: a block of 4 waves takes 4 rows, one wave per row
+// the fold of a whole map: a block of 4 waves takes 4 rows, one wave per row. The list's triangles are in the maps by now.
 template <typename MapT>
 __global__ __launch_bounds__(256) void k_fold_rows(MapT* __restrict__ map, MapT* __restrict__ tiled, MapT* __restrict__ span,
-	int n1, int n2, int tiles_x)
+	int n1, int n2, int tiles_x, WideList* __restrict__ list)
 {
+	if (blockIdx.x == 0 && threadIdx.x == 0) list->count = list->rows = list->taken = 0;
 	const int y = blockIdx.x * 4 + (threadIdx.x >> 6);
 	if (y >= n2) return;
 	fold_row<MapT, false>(map + (long long)n1 * y, tiled, span, n1, tiles_x, y);
@@ -1650,6 +1836,7 @@ void Engine::fold_tiled_maps()
 {
 	if (!tmap_.ptr) return;
 	const unsigned grid = unsigned((npix_[1] + 3) / 4);
+	WideList* list = reinterpret_cast<WideList*>(wide_.ptr);
 	for (int k = 0; k < (parities_ ? 3 : 1); k++)
 	{
 		char* m = k == 0 ? map_.ptr : (k == 1 ? map_min_.ptr : map_sad_.ptr);
@@ -1657,9 +1844,9 @@ void Engine::fold_tiled_maps()
 		// with parities the kernel writes minima and saddles only, so the total has no spans
 		char* sp = k == 0 ? (parities_ ? nullptr : span_.ptr) : (k == 1 ? span_min_.ptr : span_sad_.ptr);
 		if (map_fp32_)
-			k_fold_rows<float><<<grid, 256, 0, stream_>>>((float*)m, (float*)t, (float*)sp, npix_[0], npix_[1], tiles_x_);
+			k_fold_rows<float><<<grid, 256, 0, stream_>>>((float*)m, (float*)t, (float*)sp, npix_[0], npix_[1], tiles_x_, list);
 		else
-			k_fold_rows<double><<<grid, 256, 0, stream_>>>((double*)m, (double*)t, (double*)sp, npix_[0], npix_[1], tiles_x_);
+			k_fold_rows<double><<<grid, 256, 0, stream_>>>((double*)m, (double*)t, (double*)sp, npix_[0], npix_[1], tiles_x_, list);
 	}
 	MLENS_HIP_CHECK(hipGetLastError());
 }
@@ -1674,7 +1861,8 @@ void Engine::zero_maps()
 		MLENS_HIP_CHECK(hipMemsetAsync(map_min_.ptr, 0, bytes, stream_));
 		MLENS_HIP_CHECK(hipMemsetAsync(map_sad_.ptr, 0, bytes, stream_));
 	}
-	// tiled and span maps are zero between shots unless a shot was cut short
+	// tiled and span maps and the list of wide triangles are empty between shots unless a shot was cut short
+	if (wide_.ptr) MLENS_HIP_CHECK(hipMemsetAsync(wide_.ptr, 0, offsetof(WideList, row), stream_));
 	for (DeviceBuffer<char>* t : {&tmap_, &tmap_min_, &tmap_sad_, &span_, &span_min_, &span_sad_})
 		if (t->ptr) MLENS_HIP_CHECK(hipMemsetAsync(t->ptr, 0, std::min(tmap_bytes_, t->count), stream_));
 }
@@ -1715,27 +1903,31 @@ ShootStats Engine::shoot_ipm(const LensParams& lens, const GridParams& g, Precis
 		a.msad = parities_ ? tmap_sad_.ptr : nullptr;
 		a.span = parities_ ? span_min_.ptr : span_.ptr;
 		a.span_sad = parities_ ? span_sad_.ptr : nullptr;
+		a.wide = reinterpret_cast<WideList*>(wide_.ptr);
 		const long long ntx = (a.N1 + IPM_TILE_W - 1) / IPM_TILE_W;
 		const int th = tile_rows_ > 0 ? tile_rows_ : ipm_tile_rows(ntx, row1 - row0, num_cus_);
 		last_tile_rows_ = th;
 		if ((row1 - row0 + th - 1) / th > 65535) throw HipError("too many tiles of this height for one launch", __FILE__, __LINE__);
 		dim3 grid(unsigned(ntx), unsigned((row1 - row0 + th - 1) / th));
 		dim3 block(64 * IPM_WAVES);
-		// the instantiation for this precision, with or without parities, linear or general smooth matter
-		auto launch = [&](auto kernel) {
-			kernel<<<grid, block, 0, stream_>>>(a, row0, row1, MLENS_TABLE_ARGS(a), a.map, a.mmin, a.msad, a.span, a.span_sad, th);
+		// the instantiations for this precision, with or without parities, linear or general smooth matter
+		const unsigned resident = wide_blocks(num_cus_);
+		auto launch = [&]<int P, bool PARITY, bool LIN>() {
+			k_ipm_fast<P, PARITY, LIN><<<grid, block, 0, stream_>>>(a, row0, row1, MLENS_TABLE_ARGS(a), a.map, a.mmin, a.msad, a.span,
+				a.span_sad, th);
+			k_ipm_rows<P, PARITY, LIN><<<resident, 64, 0, stream_>>>(a, MLENS_TABLE_ARGS(a), a.map, a.mmin, a.msad, a.span, a.span_sad);
 		};
-		const bool lin = a.smooth_linear != 0;
+		auto launch_lin = [&]<int P, bool PARITY>() {
+			a.smooth_linear ? launch.template operator()<P, PARITY, true>() : launch.template operator()<P, PARITY, false>();
+		};
 		if (prec == PREC_FP64)
-		{
-			if (parities_) launch(lin ? k_ipm_fast<PREC_FP64, true, true> : k_ipm_fast<PREC_FP64, true, false>);
-			else launch(lin ? k_ipm_fast<PREC_FP64, false, true> : k_ipm_fast<PREC_FP64, false, false>);
-		}
+			parities_ ? launch_lin.template operator()<PREC_FP64, true>() : launch_lin.template operator()<PREC_FP64, false>();
 		else
-		{
-			if (parities_) launch(lin ? k_ipm_fast<PREC_MIXED, true, true> : k_ipm_fast<PREC_MIXED, true, false>);
-			else launch(lin ? k_ipm_fast<PREC_MIXED, false, true> : k_ipm_fast<PREC_MIXED, false, false>);
-		}
+			parities_ ? launch_lin.template operator()<PREC_MIXED, true>() : launch_lin.template operator()<PREC_MIXED, false>();
+		MLENS_HIP_CHECK(hipGetLastError());
+		auto wide = prec == PREC_FP64 ? (parities_ ? k_ipm_wide<double, true> : k_ipm_wide<double, false>)
+			: (parities_ ? k_ipm_wide<float, true> : k_ipm_wide<float, false>);
+		wide<<<resident, 64, 0, stream_>>>(a);
 		MLENS_HIP_CHECK(hipGetLastError());
 		fold_tiled_maps();
 	}

@@ -49,6 +49,8 @@ struct ShootArgs
 	// row (tiled maps of the map's type): span (the map, or minima with
 	// parities), span_sad
 	void *span, *span_sad;
+	// where the IPM kernel leaves work for the next launches
+	struct WideList* wide;
 };
 
 // The hot read-only tables travel as separate __restrict__ kernel parameters:

@@ -83,6 +83,34 @@ def test_batch_tiles_and_pieces(general):
         m.close()
 
 
+@pytest.mark.parametrize("parities", [False, True])
+@pytest.mark.parametrize("pixels,rays", [(40, 2), (301, 1), (700, 4), (2500, 1)])
+def test_work_left_for_later_launches(parities, pixels, rays):
+    """A single map leaves wide triangles and rows of many triangles for two launches
+    of their own, up to the lists' lengths; a batch shoots every tile whole. Small and
+    odd maps, and one whose stars fill the lists, by rays few and many: the same map
+    from both. Each pixel is two FP32 sums of at most some 300 terms in another order,
+    300 * 2^-24 < 2e-5 of the pixel (of the mean, below it, for the residue of the runs)."""
+    from irs_amd.microlensing.IPM.batch import IPMBatch
+    from irs_amd.microlensing.IPM.ipm import IPM
+    params = dict(C1_SMALL, half_length_y1=6.0, half_length_y2=6.0, num_pixels_y1=pixels, num_pixels_y2=pixels,
+                  num_rays_y=rays)
+    whole = IPM(**params)
+    whole.prepare()
+    whole.build()
+    batch = IPMBatch()
+    batch.set_tuning(64, 16)
+    batch.add(whole)
+    batch.run()
+    m = make(params, write_parities=parities)
+    ref = whole.magnifications.astype(np.float64)
+    err = np.abs(m.magnifications - ref) / np.maximum(ref, ref.mean())
+    say(f"[later] {pixels} pixels, {rays} rays, parities {parities}: {err.max():.1e}")
+    assert ref.mean() > 0 and err.max() < 2e-5
+    m.close()
+    whole.close()
+
+
 def write_field(path, stars, radius):
     with open(path, "wb") as fh:
         np.array([len(stars), 0], dtype=np.int32).tofile(fh)
