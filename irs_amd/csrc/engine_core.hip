@@ -152,7 +152,7 @@ star.cuh:124-161: totals in FP64 over STAT_CHAINS interleaved chains (star i bel
 i % STAT_CHAINS), each summed in order, then the chains by a tree. A block takes STAT_GROUP
 chains, a lane per chain and sixteenth of a row of stars: the lanes fetch and take logarithms
 side by side, then each chain's own lane adds its terms in order. One block walking all the chains
-took 2.2 ms for 1.28e6 stars.
+took 2.2 ms for 1.28e6 stars, the 16 blocks take 0.48.
 */
 constexpr int STAT_CHAINS = 256;
 constexpr int STAT_GROUP = 16;   // chains of a block: 128 bytes of consecutive stars

@@ -265,7 +265,7 @@ namespace
 constexpr int M2L_POWERS = 1 + 2 * (MAX_EXPANSION_ORDER + 1);
 
 /* The 40 offset matrices for order p (blockIdx.x = offset), stacked [Mr -Mi; Mi Mr], stored transposed At[col][row]
-   and zero-padded to kp. The host sends the powers of the offsets (60 KB) and the binomials; building the matrices
+   and zero-padded to kp. The host sends the powers of the offsets (42 KB) and the binomials; building the matrices
    there and copying them took 0.4 ms of a small field's build. Contraction is off: the entries are those that the
    host's complex products give. */
 template <typename T>
