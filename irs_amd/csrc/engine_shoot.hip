@@ -42,7 +42,10 @@ struct LeafCache
 
 /* cold: the argument block in memory, read only for points outside the root
    box. Read from `a` instead, its tree pointers (16 scalar registers) would be
-   loaded ahead of the shooting loop and spilled. SHARED > 0: scattered points;
+   loaded ahead of the shooting loop and spilled. With general smooth matter the
+   loop holds a call to alpha_smooth, which spills them either way, and the block's
+   own address costs more than it saves: 1.04e9 rays through the exact circular sheet
+   take 13.3 ms without it and 13.8 with. SHARED > 0: scattered points;
    after that many shared leaves the wave's remaining lanes each read their own
    leaf's tables, all at once, where leaf after leaf would take up to 64 passes
    of scalar loads. */
@@ -98,8 +101,13 @@ __device__ __forceinline__ Deflection deflect(const ShootArgs& a, const ShootArg
 	}
 	else
 	{
-		asm volatile("" : "+s"(cold));   // keeps the loads here
-		d = deflect_node<MU, LIN>(*cold, c.node, zx, zy);
+		if (!LIN && !MU)
+			d = deflect_node<MU, LIN>(a, c.node, zx, zy);
+		else
+		{
+			asm volatile("" : "+s"(cold));   // keeps the loads here
+			d = deflect_node<MU, LIN>(*cold, c.node, zx, zy);
+		}
 	}
 	return d;
 }
