@@ -294,7 +294,11 @@ pixels).
 // A larger queue fills the passes of a flush better but costs waves: the 10000^2 map at four
 // rays a pixel took 1.145 s with 100 entries (12 blocks), 1.130 s with 88 (14) and 1.126 s
 // with 74; 24 batched maps 8.1 ms with 79 entries at 12 blocks, 7.2 ms with 74 at 16.
+// General smooth matter runs at three waves per SIMD, which leaves room for 100 entries (12.7 KB):
+// 2000^2 maps at four rays a pixel, rectangular and exact circular sheet, 25.8 and 10.9 ms against
+// 26.1 and 11.1 with 74. The batch kernel keeps 74 for either.
 constexpr int IPM_QCAP = 74;
+constexpr int IPM_QCAP_GENERAL = 100;
 
 template <int CAP>
 struct TriQueue
@@ -1016,7 +1020,7 @@ __global__ __launch_bounds__(64 * IPM_WAVES, LIN ? 4 : 3) void k_ipm_fast(ShootA
 	const long long J0 = row0 + (long long)blockIdx.y * tile_h;
 	if (J0 >= row1) return;
 	const long long J1 = min(J0 + tile_h, row1);
-	__shared__ TriQueue<IPM_QCAP> queues[IPM_WAVES];
+	__shared__ TriQueue<LIN ? IPM_QCAP : IPM_QCAP_GENERAL> queues[IPM_WAVES];
 	ipm_tile<PREC, PARITY, true, IPM_WAVES, LIN, TILE_LATE>(a, kernarg_block(), queues[threadIdx.x >> 6], blockIdx.x, J0, J1);
 }
 
@@ -1031,7 +1035,7 @@ __global__ __launch_bounds__(64, LIN ? 4 : 3) void k_ipm_rows(ShootArgs a, MLENS
 	a.msad = msad;
 	a.span = span;
 	a.span_sad = span_sad;
-	__shared__ TriQueue<IPM_QCAP> q;
+	__shared__ TriQueue<LIN ? IPM_QCAP : IPM_QCAP_GENERAL> q;
 	late_rows(a.wide, [&](const LateRow& r, int c0, int c1) {
 		ipm_tile<PREC, PARITY, true, 1, LIN, TILE_PART>(a, kernarg_block(), q, r.tile_x, r.J - 1, r.J, c0, c1);
 	});
