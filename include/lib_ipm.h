@@ -118,6 +118,10 @@ int get_m2l_mode(IPMHandle* self);
 void set_tile_rows(IPMHandle* self, int val);
 int get_tile_rows(IPMHandle* self);
 int get_last_tile_rows(IPMHandle* self);                  /* the height the last shoot used */
+/* extension: wide triangles and heavy rows that the last shoot left for launches of their own (their lists hold 65536 and
+   32768; what a full list turned away was done at once and is not counted) */
+long long get_late_triangles(IPMHandle* self);
+long long get_late_rows(IPMHandle* self);
 double get_t_m2l(IPMHandle* self);          /* seconds in the M2L kernels of the last build (MFMA modes) */
 long long get_m2l_pairs(IPMHandle* self);   /* M2L (target, source) pairs of the last build (MFMA modes) */
 int get_m2l_fp32(IPMHandle* self);          /* 1 if the last build's M2L ran on FP32 MFMA */

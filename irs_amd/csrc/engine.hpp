@@ -77,6 +77,13 @@ struct MapExtremes
 	double positive_min;   // smallest positive value, +infinity if there is none
 };
 
+/* what an IPM shot offered to the launches after its first: triangles (the list holds 65536) and rows of
+   tiles (32768); work that a full list turned away was done at once and is not counted */
+struct LateWork
+{
+	long long triangles = 0, rows = 0;
+};
+
 struct ShootStats
 {
 	double ms = 0;                 // kernel time (HIP events)
@@ -134,6 +141,7 @@ public:
 	void set_tile_rows(int rows) { tile_rows_ = rows; }
 	int tile_rows() const { return tile_rows_; }
 	int last_tile_rows() const { return last_tile_rows_; }   // the height of the last shooting launch
+	LateWork late_work() const;                               // of the last IPM shot
 	void add_parity_maps();
 	void download_map(int which, void* host) const;   // 0 = total, 1 = minima, 2 = saddles
 	/* of the first nmaps of total, minima, saddles (which must exist) */

@@ -809,7 +809,8 @@ struct WideList
 	unsigned count;   // triangles offered: may exceed WIDE_CAP
 	unsigned rows;    // rows offered: may exceed ROW_CAP
 	unsigned taken;   // parts of rows that the second launch has handed out
-	unsigned unused[13];
+	unsigned last_count, last_rows;   // count and rows of the last shot
+	unsigned unused[11];
 	LateRow row[ROW_CAP];
 	WideTri tri[WIDE_CAP];
 };
@@ -1833,12 +1834,18 @@ void Engine::ensure_tiled_maps()
 	}
 }
 
-// the fold of a whole map: a block of 4 waves takes 4 rows, one wave per row. The list's triangles are in the maps by now.
+// the fold of a whole map: a block of 4 waves takes 4 rows, one wave per row. The list's triangles are in the maps by now:
+// the launch that is given the list keeps its counts for the caller and clears it.
 template <typename MapT>
 __global__ __launch_bounds__(256) void k_fold_rows(MapT* __restrict__ map, MapT* __restrict__ tiled, MapT* __restrict__ span,
 	int n1, int n2, int tiles_x, WideList* __restrict__ list)
 {
-	if (blockIdx.x == 0 && threadIdx.x == 0) list->count = list->rows = list->taken = 0;
+	if (list && blockIdx.x == 0 && threadIdx.x == 0)
+	{
+		list->last_count = list->count;
+		list->last_rows = list->rows;
+		list->count = list->rows = list->taken = 0;
+	}
 	const int y = blockIdx.x * 4 + (threadIdx.x >> 6);
 	if (y >= n2) return;
 	fold_row<MapT, false>(map + (long long)n1 * y, tiled, span, n1, tiles_x, y);
@@ -1848,19 +1855,31 @@ void Engine::fold_tiled_maps()
 {
 	if (!tmap_.ptr) return;
 	const unsigned grid = unsigned((npix_[1] + 3) / 4);
-	WideList* list = reinterpret_cast<WideList*>(wide_.ptr);
 	for (int k = 0; k < (parities_ ? 3 : 1); k++)
 	{
 		char* m = k == 0 ? map_.ptr : (k == 1 ? map_min_.ptr : map_sad_.ptr);
 		char* t = k == 0 ? tmap_.ptr : (k == 1 ? tmap_min_.ptr : tmap_sad_.ptr);
 		// with parities the kernel writes minima and saddles only, so the total has no spans
 		char* sp = k == 0 ? (parities_ ? nullptr : span_.ptr) : (k == 1 ? span_min_.ptr : span_sad_.ptr);
+		WideList* list = k == 0 ? reinterpret_cast<WideList*>(wide_.ptr) : nullptr;
 		if (map_fp32_)
 			k_fold_rows<float><<<grid, 256, 0, stream_>>>((float*)m, (float*)t, (float*)sp, npix_[0], npix_[1], tiles_x_, list);
 		else
 			k_fold_rows<double><<<grid, 256, 0, stream_>>>((double*)m, (double*)t, (double*)sp, npix_[0], npix_[1], tiles_x_, list);
 	}
 	MLENS_HIP_CHECK(hipGetLastError());
+}
+
+LateWork Engine::late_work() const
+{
+	LateWork w;
+	if (!wide_.ptr) return w;
+	unsigned n[2];
+	static_assert(offsetof(WideList, last_rows) == offsetof(WideList, last_count) + sizeof(unsigned), "read together");
+	MLENS_HIP_CHECK(hipMemcpy(n, wide_.ptr + offsetof(WideList, last_count), sizeof(n), hipMemcpyDeviceToHost));
+	w.triangles = n[0];
+	w.rows = n[1];
+	return w;
 }
 
 void Engine::zero_maps()

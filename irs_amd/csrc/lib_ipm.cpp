@@ -28,6 +28,8 @@ ipm_dtype* get_pixels(IPMHandle* self) { return self->m.get_pixels(); }
 ipm_dtype* get_pixels_minima(IPMHandle* self) { return self->m.get_pixels_minima(); }
 ipm_dtype* get_pixels_saddles(IPMHandle* self) { return self->m.get_pixels_saddles(); }
 double get_t_shoot_cells(IPMHandle* self) { return self->m.get_t_shoot(); }
+long long get_late_triangles(IPMHandle* self) { MLENS_GUARD(return self->m.get_late_work().triangles, return -1) }
+long long get_late_rows(IPMHandle* self) { MLENS_GUARD(return self->m.get_late_work().rows, return -1) }
 
 bool ipm_prepare(IPMHandle* self, int verbose) { MLENS_GUARD(return self->m.prepare(verbose), return false) }
 bool ipm_derive(IPMHandle* self, int verbose) { MLENS_GUARD(return self->m.derive(verbose), return false) }

@@ -257,6 +257,7 @@ public:
 	T get_m_lower_actual() const { return m_lower_actual_; }
 	T get_m_upper_actual() const { return m_upper_actual_; }
 	int get_last_tile_rows() const { return engine_ ? engine_->last_tile_rows() : 0; }
+	LateWork get_late_work() const { return engine_ ? engine_->late_work() : LateWork(); }
 	Engine* engine() { return engine_.get(); }
 	bool is_built() const { return built_; }
 	double mean_near_stars() const { return engine_ ? engine_->mean_near_stars(grid()) : 0; }

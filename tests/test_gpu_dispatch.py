@@ -83,17 +83,23 @@ def test_batch_tiles_and_pieces(general):
         m.close()
 
 
+def late_work(m):
+    """Wide triangles and rows that the last shot left for later launches."""
+    return m.lib.get_late_triangles(m.obj), m.lib.get_late_rows(m.obj)
+
+
 @pytest.mark.parametrize("parities", [False, True])
-@pytest.mark.parametrize("pixels,rays", [(40, 2), (301, 1), (700, 4), (2500, 1)])
-def test_work_left_for_later_launches(parities, pixels, rays):
+@pytest.mark.parametrize("pixels,rays,half,least", [(40, 2, 6.0, (0, 1)), (301, 1, 6.0, (1, 1)), (700, 4, 6.0, (1, 1)),
+                                                    (2500, 1, 6.0, (65536, 1)), (3000, 4, 10.0, (65536, 32768))])
+def test_work_left_for_later_launches(parities, pixels, rays, half, least):
     """A single map leaves wide triangles and rows of many triangles for two launches
     of their own, up to the lists' lengths; a batch shoots every tile whole. Small and
-    odd maps, and one whose stars fill the lists, by rays few and many: the same map
+    odd maps, one that fills the list of triangles and one that fills both: the same map
     from both. Each pixel is two FP32 sums of at most some 300 terms in another order,
     300 * 2^-24 < 2e-5 of the pixel (of the mean, below it, for the residue of the runs)."""
     from irs_amd.microlensing.IPM.batch import IPMBatch
     from irs_amd.microlensing.IPM.ipm import IPM
-    params = dict(C1_SMALL, half_length_y1=6.0, half_length_y2=6.0, num_pixels_y1=pixels, num_pixels_y2=pixels,
+    params = dict(C1_SMALL, half_length_y1=half, half_length_y2=half, num_pixels_y1=pixels, num_pixels_y2=pixels,
                   num_rays_y=rays)
     whole = IPM(**params)
     whole.prepare()
@@ -105,10 +111,43 @@ def test_work_left_for_later_launches(parities, pixels, rays):
     m = make(params, write_parities=parities)
     ref = whole.magnifications.astype(np.float64)
     err = np.abs(m.magnifications - ref) / np.maximum(ref, ref.mean())
-    say(f"[later] {pixels} pixels, {rays} rays, parities {parities}: {err.max():.1e}")
+    say(f"[later] {pixels} pixels, {rays} rays, parities {parities}: {err.max():.1e}, {late_work(m)} left")
+    assert all(got >= n for got, n in zip(late_work(m), least))
     assert ref.mean() > 0 and err.max() < 2e-5
     m.close()
     whole.close()
+
+
+@pytest.mark.parametrize("double", [True, False])
+@pytest.mark.parametrize("pixels,rays,rect", [(301, 1, False), (301, 1, True), (700, 4, False)])
+def test_later_launches_keep_the_parities(oracle, tmp_path, double, pixels, rays, rect):
+    """Triangles and rows shot by the later launches land in the map of their parity: total,
+    minima and saddles each against the oracle's, for both value types, linear and general
+    smooth matter, with and without parity maps. FP64 corners differ by rounding, which moves
+    a pixel by 1e-8 at most over 3e8 cells (whole-map parity tests); mixed ones to the bounds
+    of the mixed parity test, and the flux of a map by the few triangles whose area is zero to
+    FP32 (less than 1e-6 of all; half of the wide ones would be 1e-5 or more)."""
+    field = dict(C1_SMALL, half_length_y1=6.0, half_length_y2=6.0, num_pixels_y1=pixels, num_pixels_y2=pixels, num_rays_y=rays,
+                 rectangular=rect)
+    stars = write_starfile(oracle, tmp_path / "stars.bin", field, seed=11, margin=1.2)
+    params = dict(from_starfile(field, tmp_path / "stars.bin"), expansion_order=16, is_double=double)
+    m = make(params, write_parities=True)
+    assert all(n > 0 for n in late_work(m))
+    ref = Mirror(oracle, m, stars=stars).ipm_map(parities=True)[:3]
+    plain = make(params)
+    mean = ref[0].mean()
+    for what, got, want in zip(("total", "minima", "saddles", "plain"), (m.magnifications, m.magnifications_minima,
+                               m.magnifications_saddles, plain.magnifications), (*ref, ref[0])):
+        e = np.abs(got - want) / np.maximum(want, mean)
+        flux = abs(got.sum(dtype=np.float64) - want.sum()) / ref[0].sum()
+        say(f"[later {what}] {pixels} pixels, rect {rect}, double {double}: max {e.max():.1e}, p99 {np.percentile(e, 99):.1e}, "
+            f"flux {flux:.1e}")
+        if double:
+            assert e.max() < 1e-7 and flux < 1e-10
+        else:
+            assert np.median(e) < 1e-4 and np.percentile(e, 99) < 1e-2 and flux < 1e-5
+    m.close()
+    plain.close()
 
 
 def write_field(path, stars, radius):
