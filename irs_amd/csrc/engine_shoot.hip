@@ -782,6 +782,14 @@ passes); parts of whole rows 1.76, 9.2 and 0.68; after 96 passes 2.2, 10.1 and
 0.70. A 10000^2 map, 1.12 s, gains 0.1%. A batch keeps its waves busy to the
 end by itself, and the lists only cost there (6.7 ms without, 7.1 with wide
 triangles, 7.8 with both).
+
+A row that is left deflects 128 corners for its 63 cells where its tile would
+deflect 64. That pays except with the rectangular sheet, whose deflection (four
+logarithms, or four series of up to 101 terms) costs several times the rest: a
+2000^2 map at four rays a pixel takes 25.3 ms without late rows and 25.9 with,
+a 1000^2 one in FP64 with parities 15.0 and 15.4, a 256^2 one 1.33 and 1.42;
+a 1000^2 map takes 4.4 either way. The exact circular sheet keeps them: 11.0
+against 17.3, 6.4 against 9.3, 0.57 against 0.81 and 1.85 against 2.7 ms.
 */
 constexpr int WIDE_SPAN = 96;
 constexpr unsigned WIDE_CAP = 1 << 16;
@@ -938,6 +946,7 @@ __device__ __forceinline__ void ipm_tile(const ShootArgs& a, const ShootArgs* co
 	using MapT = typename std::conditional<PREC == PREC_MIXED, float, double>::type;
 	PixelAcc<MapT> acc;
 	int qn = 0, passes = 0;
+	const bool late = WORK == TILE_LATE && (LIN || !a.rectangular);
 
 	auto corner = [&](long long J, double& px, double& py) {
 		double zy = lattice_at(a.y0, a.stepy, J);
@@ -951,7 +960,7 @@ __device__ __forceinline__ void ipm_tile(const ShootArgs& a, const ShootArgs* co
 	bool below = false;   // the corners below are at hand
 	for (long long J = J0; J <= J1; J++)
 	{
-		if (WORK == TILE_LATE && passes > ROW_BUDGET)
+		if (late && passes > ROW_BUDGET)
 		{
 			const int n = rows_push(cold, tile_x, J, int(min((long long)ROW_RUN, J1 - J + 1)));
 			below = below && n == 0;

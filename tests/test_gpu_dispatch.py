@@ -132,7 +132,8 @@ def test_later_launches_keep_the_parities(oracle, tmp_path, double, pixels, rays
     stars = write_starfile(oracle, tmp_path / "stars.bin", field, seed=11, margin=1.2)
     params = dict(from_starfile(field, tmp_path / "stars.bin"), expansion_order=16, is_double=double)
     m = make(params, write_parities=True)
-    assert all(n > 0 for n in late_work(m))
+    triangles, rows = late_work(m)
+    assert triangles > 0 and (rows == 0 if rect else rows > 0)   # a rectangular sheet's rows stay with their tile
     ref = Mirror(oracle, m, stars=stars).ipm_map(parities=True)[:3]
     plain = make(params)
     mean = ref[0].mean()
