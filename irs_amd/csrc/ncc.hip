@@ -366,24 +366,26 @@ __global__ __launch_bounds__(256) void k_ncc_rows_to_map(const int* __restrict__
 }
 
 /*
-The final map from the rows' lists. A workgroup of WAVES waves owns WAVES / s final rows (at least one); a wave takes
+The final map from the rows' lists. A workgroup of four waves owns 4 / s final rows (at least one); a wave takes
 one sub-pixel row at a time: it clears the row's columns in LDS, adds the row's crossings to them, and sums from
 the right in tiles of 64 words, two columns a word in halves (an upward crossing's -1 borrows from the upper half,
 which reading the lower half as signed gives back; |difference| <= cap < 2^15). The s columns of a final pixel are
 s / 2 words of consecutive lanes, which take their maximum by DPP; one of them merges it into the final row in LDS.
 The over-sampled grid used to be zeroed, added to and read back in memory (64 MB at the defaults: 16 + 24 + 26 us,
-and 350 us to allocate and free); this takes no grid. Four waves share a workgroup up to 8192 columns, two up to
-16384 and one up to 32768, so that their rows fit in LDS.
+and 350 us to allocate and free); this takes no grid. CMAX: room for the final rows, COLS for s = 2, and a quarter
+of that for s >= 4, which lets four workgroups of 4096 columns share a CU, or two of 8192. Wider rows leave so few
+waves on a CU that the grid in memory is faster: with one wave of 20000 columns a CU a 2500^2 map over-sampled
+by 8 took 6.1 ms, with the grid 4.5.
 */
-constexpr int NCC_LIST_COLS = 32768;
+constexpr int NCC_LIST_COLS = 8192;
 
-template <int COLS, int WAVES>
-__global__ __launch_bounds__(64 * WAVES) void k_ncc_map_from_lists(NCCLists lists, int* __restrict__ map, int np1, int np2, int s,
+template <int COLS, int CMAX>
+__global__ __launch_bounds__(256) void k_ncc_map_from_lists(NCCLists lists, int* __restrict__ map, int np1, int np2, int s,
 	int* __restrict__ row_ext)
 {
-	constexpr int THREADS = 64 * WAVES;
+	constexpr int WAVES = 4, THREADS = 64 * WAVES;
 	__shared__ unsigned words[WAVES][COLS / 2];
-	__shared__ int cmax[WAVES > 2 ? COLS : COLS / 2];   // the workgroup's final rows, s > 1
+	__shared__ int cmax[CMAX];   // the workgroup's final rows, s > 1
 	__shared__ int part[2][WAVES];
 	const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
 	const int width = np1 * s, nw = (width + 1) / 2;
@@ -697,15 +699,13 @@ void NCCDevice::count(const double* caustics, int nrows, int ncols, const NCCGri
 		k_ncc_crossings<true><<<seg_blocks, 64, 0, stream_>>>(caustics_.ptr, nrows, ncols, a, nullptr, l, meta);
 		MLENS_HIP_CHECK(hipEventRecord(ev1_, stream_));
 		unsigned blocks = 0;
-		auto rows_to_map = [&](auto kernel, int waves) {
-			const int per = s >= waves ? 1 : int(waves / s);
+		auto rows_to_map = [&](auto kernel) {
+			const int per = s >= 4 ? 1 : int(4 / s);
 			blocks = unsigned((g.num_pixels_im + per - 1) / per);
-			kernel<<<blocks, 64 * waves, 0, stream_>>>(l, map_.ptr, g.num_pixels_re, g.num_pixels_im, int(s), row_ext_.ptr);
+			kernel<<<blocks, 256, 0, stream_>>>(l, map_.ptr, g.num_pixels_re, g.num_pixels_im, int(s), row_ext_.ptr);
 		};
-		if (npx <= 4096) rows_to_map(k_ncc_map_from_lists<4096, 4>, 4);
-		else if (npx <= 8192) rows_to_map(k_ncc_map_from_lists<8192, 4>, 4);
-		else if (npx <= 16384) rows_to_map(k_ncc_map_from_lists<16384, 2>, 2);
-		else rows_to_map(k_ncc_map_from_lists<32768, 1>, 1);
+		if (npx <= 4096) rows_to_map(s >= 4 ? k_ncc_map_from_lists<4096, 1024> : k_ncc_map_from_lists<4096, 4096>);
+		else rows_to_map(s >= 4 ? k_ncc_map_from_lists<8192, 2048> : k_ncc_map_from_lists<8192, 8192>);
 		MLENS_HIP_CHECK(hipEventRecord(ev2_, stream_));
 		k_ncc_row_extremes<<<1, 256, 0, stream_>>>(row_ext_.ptr, int(blocks), meta);
 		finish();

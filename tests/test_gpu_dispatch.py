@@ -416,11 +416,13 @@ def test_deflections_of_mixed_waves(oracle, tmp_path, rect):
 
 @pytest.mark.parametrize("npx,over_sample,curves", [((1, 1), 0, 3), ((7, 5), 0, 40), ((301, 9), 0, 40), ((64, 33), 1, 40),
                                                     ((4095, 3), 0, 20), ((2048, 3), 1, 20), ((2049, 3), 1, 20), ((1025, 3), 3, 20),
+                                                    ((1024, 3), 2, 20), ((8192, 2), 0, 20), ((8193, 2), 0, 20), ((4096, 3), 1, 20),
+                                                    ((2048, 3), 2, 20), ((1024, 3), 3, 20),
                                                     ((4100, 2), 2, 20), ((8193, 2), 1, 20), ((8193, 2), 2, 10), ((20, 6), 8, 8),
                                                     ((40, 30), 1, 4000)])
 def test_crossing_lists(tmp_path, npx, over_sample, curves):
-    """Crossings go to a list per sub-pixel row, and one, two or four waves sum a row in
-    LDS: odd and even widths, one to 256 sub-pixels a pixel, the first and last width of
+    """Crossings go to a list per sub-pixel row, and the waves of a workgroup sum a row each
+    in LDS: odd and even widths, one to 256 sub-pixels a pixel, the first and last width of
     each variant, grids too wide for lists, and rows that overflow theirs (4000 curves over
     60 rows), against the oracle: identical counts and histogram."""
     from irs_amd.microlensing.NCC.ncc import NCC
