@@ -76,6 +76,7 @@ bool save(NCCHandle* self, int verbose);
 void ncc_free(NCCHandle* self);            /* the reference leaks its objects */
 double get_t_ncc(NCCHandle* self);         /* seconds counting the crossings */
 double get_t_reduce(NCCHandle* self);      /* seconds reducing the over-sampled grid */
+int get_crossing_path(NCCHandle* self);    /* of the last run: 0 a grid in memory, 1 a list per row, 2 a list overflowed, then a grid */
 
 #ifdef __cplusplus
 }

@@ -33,6 +33,7 @@ MLENS_STRING_FIELD(outfile_prefix, outfile_prefix)
 int* get_num_crossings(NCCHandle* self) { return self->m.get_num_crossings(); }
 double get_t_ncc(NCCHandle* self) { return self->m.get_t_ncc(); }
 double get_t_reduce(NCCHandle* self) { return self->m.get_t_reduce(); }
+int get_crossing_path(NCCHandle* self) { return self->m.get_crossing_path(); }
 
 bool run(NCCHandle* self, int verbose) { MLENS_GUARD(return self->m.run(verbose), return false) }
 bool save(NCCHandle* self, int verbose) { MLENS_GUARD(return self->m.save(verbose), return false) }

@@ -12,8 +12,8 @@ over-sampled grid is reduced to the final one by the maximum over each
 2^over_sample x 2^over_sample block, which is what the reference's repeated
 2 x 2 reductions and shifts (ncc_functions.cuh:345-411) leave behind. The
 over-sampled counts never exist in memory. Grids of more than NCC_LIST_COLS
-columns, and maps with a row whose list overflows, keep a row-difference grid
-in memory instead, to which a crossing adds its +1 or -1.
+columns, dense networks and maps with a row whose list overflows keep a
+row-difference grid in memory instead, to which a crossing adds its +1 or -1.
 
 Segment clipping and crossing positions follow ncc_functions.cuh:43-301 step
 by step in FP64. The reference evaluates the line intersection as
@@ -130,7 +130,8 @@ out to its lanes, 64 at a time, so that a long segment near a cusp (hundreds
 of rows) does not hold up the wave: a lane finds the segment of crossing c by
 a binary search over the lanes' first crossing indices. meta counts the
 crossings and those whose row is outside the grid (dropped, as the
-reference's bounds check drops them). One wave per workgroup.
+reference's bounds check drops them). Waves that find a list overflowed leave
+theirs undealt: the caller starts again without lists. One wave per workgroup.
 */
 template <bool LISTS>
 __global__ __launch_bounds__(64) void k_ncc_crossings(const double* __restrict__ caus, int nrows, int ncols, NCCArgs g,
@@ -146,6 +147,8 @@ __global__ __launch_bounds__(64) void k_ncc_crossings(const double* __restrict__
 		long long n = 0, k0 = 0;
 		double px0 = 0, py0 = 0, px1 = 0, py1 = 0;
 		int up = 0;
+		// asked for here and looked at below, so that the answer comes with the segments
+		const int overflow = LISTS ? __hip_atomic_load(&meta->overflow, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0;
 		if (sg < nseg)
 		{
 			const long long i = sg / (ncols - 1), j = sg - i * (ncols - 1);
@@ -179,6 +182,7 @@ __global__ __launch_bounds__(64) void k_ncc_crossings(const double* __restrict__
 				}
 			}
 		}
+		if (LISTS && overflow) return;
 		// crossings of lanes 0..lane, and the wave's total
 		long long incl = n;
 		for (int d = 1; d < 64; d <<= 1)
@@ -381,9 +385,10 @@ constexpr int NCC_LIST_COLS = 8192;
 
 template <int COLS, int CMAX>
 __global__ __launch_bounds__(256) void k_ncc_map_from_lists(NCCLists lists, int* __restrict__ map, int np1, int np2, int s,
-	int* __restrict__ row_ext)
+	int* __restrict__ row_ext, const NCCMeta* __restrict__ meta)
 {
 	constexpr int WAVES = 4, THREADS = 64 * WAVES;
+	if (meta->overflow) return;
 	__shared__ unsigned words[WAVES][COLS / 2];
 	__shared__ int cmax[CMAX];   // the workgroup's final rows, s > 1
 	__shared__ int part[2][WAVES];
@@ -647,6 +652,26 @@ NCCDevice::~NCCDevice()
 	if (stream_) (void)hipStreamDestroy(stream_);
 }
 
+/* Crossings of a sub-pixel row, on average over the rows, from up to 128 segments: the rows that the parts of them
+   beside and right of the map span. The samples follow the golden ratio, since a fixed stride could meet the same
+   place of every curve. Not a number if a sampled point is not one. */
+static double crossings_per_row(const double* caus, int nrows, int ncols, const NCCGrid& g)
+{
+	const long long nseg = (long long)nrows * (ncols - 1);
+	const int n = int(std::min<long long>(nseg, 128));
+	double sum = 0;
+	for (int k = 0; k < n; k++)
+	{
+		const double at = k * 0.6180339887498949;
+		const long long sg = std::min<long long>(nseg - 1, (long long)((at - std::floor(at)) * double(nseg)));
+		const double* p = caus + 2 * (sg / (ncols - 1) * ncols + sg % (ncols - 1));
+		const double y0 = std::clamp(p[1] - g.center_im, -g.half_length_im, g.half_length_im);
+		const double y1 = std::clamp(p[3] - g.center_im, -g.half_length_im, g.half_length_im);
+		if (!(std::max(p[0], p[2]) - g.center_re <= -g.half_length_re)) sum += std::fabs(y1 - y0);
+	}
+	return sum / (2 * g.half_length_im) * double(nseg) / n;
+}
+
 void NCCDevice::count(const double* caustics, int nrows, int ncols, const NCCGrid& g, int* out, NCCStats& st)
 {
 	if (nrows < 1 || ncols < 2) throw std::runtime_error("the caustics need at least one row of two points");
@@ -679,18 +704,26 @@ void NCCDevice::count(const double* caustics, int nrows, int ncols, const NCCGri
 	// one wave per workgroup: a few tens of thousands of segments still reach every CU
 	const unsigned seg_blocks = grid_for(nseg, 64, 1 << 16);
 	NCCMeta m;
+	// what the kernels left, and the map unless a list overflowed
 	auto finish = [&]() {
 		MLENS_HIP_CHECK(hipGetLastError());
 		MLENS_HIP_CHECK(hipMemcpyAsync(&m, meta, sizeof(m), hipMemcpyDeviceToHost, stream_));
+		MLENS_HIP_CHECK(hipStreamSynchronize(stream_));
+		if (m.overflow) return;
 		MLENS_HIP_CHECK(hipMemcpyAsync(out, map_.ptr, size_t(npix) * sizeof(int), hipMemcpyDeviceToHost, stream_));
 		MLENS_HIP_CHECK(hipStreamSynchronize(stream_));
 	};
-	bool lists = npx <= NCC_LIST_COLS;
+	// room for 512 crossings a row, more where rows are few; never more than the grid would take, or 4 MB
+	NCCLists l;
+	l.cap = int(std::min<long long>(8192, std::max<long long>(std::min<long long>(npx - 1, 512), (1 << 20) / npy)));
+	// Lists that a row would overflow are not begun, nor long ones: up to some 600 crossings a row they are as
+	// fast as the grid or faster (1000^2 pixels over-sampled by 4, kept object, 600 a row: 0.93 against 0.96 ms),
+	// and slower from there on (1000 a row 1.31 against 1.20 ms; 300^2 pixels, 2000 a row: 1.69 against 1.41). Rows
+	// differ, so the mean may be half of either bound.
+	bool lists = npx <= NCC_LIST_COLS && 2 * crossings_per_row(caustics, nrows, ncols, g) <= std::min(l.cap, 1024);
+	st.path = lists ? NCC_LISTS : NCC_GRID;
 	if (lists)
 	{
-		// room for 512 crossings a row, more where rows are few; never more than the grid would take
-		NCCLists l;
-		l.cap = int(std::min<long long>(std::min<long long>(npx, 8192), std::max<long long>(512, (1 << 20) / npy)));
 		if (lists_.count < size_t(npy) * size_t(l.cap + 1)) lists_.alloc(size_t(npy) * size_t(l.cap + 1));
 		l.count = lists_.ptr;
 		l.entry = reinterpret_cast<unsigned*>(lists_.ptr + npy);
@@ -702,7 +735,7 @@ void NCCDevice::count(const double* caustics, int nrows, int ncols, const NCCGri
 		auto rows_to_map = [&](auto kernel) {
 			const int per = s >= 4 ? 1 : int(4 / s);
 			blocks = unsigned((g.num_pixels_im + per - 1) / per);
-			kernel<<<blocks, 256, 0, stream_>>>(l, map_.ptr, g.num_pixels_re, g.num_pixels_im, int(s), row_ext_.ptr);
+			kernel<<<blocks, 256, 0, stream_>>>(l, map_.ptr, g.num_pixels_re, g.num_pixels_im, int(s), row_ext_.ptr, meta);
 		};
 		if (npx <= 4096) rows_to_map(s >= 4 ? k_ncc_map_from_lists<4096, 1024> : k_ncc_map_from_lists<4096, 4096>);
 		else rows_to_map(s >= 4 ? k_ncc_map_from_lists<8192, 2048> : k_ncc_map_from_lists<8192, 8192>);
@@ -710,6 +743,7 @@ void NCCDevice::count(const double* caustics, int nrows, int ncols, const NCCGri
 		k_ncc_row_extremes<<<1, 256, 0, stream_>>>(row_ext_.ptr, int(blocks), meta);
 		finish();
 		lists = !m.overflow;
+		if (!lists) st.path = NCC_OVERFLOW;
 	}
 	if (!lists)
 	{

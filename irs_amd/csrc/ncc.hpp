@@ -20,8 +20,17 @@ struct NCCGrid
 	int over_sample = 2;                            // log2 of the sub-pixels per pixel and axis
 };
 
+// how the crossings of the last map were kept: a grid in memory, a list per row, or lists of which one overflowed and then a grid
+enum NCCPath
+{
+	NCC_GRID = 0,
+	NCC_LISTS = 1,
+	NCC_OVERFLOW = 2
+};
+
 struct NCCStats
 {
+	NCCPath path = NCC_GRID;
 	double t_ncc_ms = 0;      // the crossings (HIP events)
 	double t_reduce_ms = 0;   // row sums and block maxima onto the final grid (HIP events)
 	long long crossings = 0;  // crossings recorded over the fine grid

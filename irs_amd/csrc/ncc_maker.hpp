@@ -66,6 +66,7 @@ public:
 	double get_t_ncc() const { return t_ncc_; }
 	double get_t_reduce() const { return t_reduce_; }
 	long long get_num_crossings_recorded() const { return stats_.crossings; }
+	int get_crossing_path() const { return stats_.path; }
 
 private:
 	const std::string caustics_file = "ccf_caustics.bin";

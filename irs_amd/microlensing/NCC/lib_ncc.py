@@ -31,6 +31,8 @@ def load(path=_PATH):
     for name in ("get_t_ncc", "get_t_reduce"):
         getattr(lib, name).argtypes = [v]
         getattr(lib, name).restype = d
+    lib.get_crossing_path.argtypes = [v]
+    lib.get_crossing_path.restype = i
     lib.run.argtypes = [v, i]
     lib.run.restype = ctypes.c_bool
     lib.save.argtypes = [v, i]

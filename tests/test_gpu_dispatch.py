@@ -414,36 +414,58 @@ def test_deflections_of_mixed_waves(oracle, tmp_path, rect):
     m.close()
 
 
-@pytest.mark.parametrize("npx,over_sample,curves", [((1, 1), 0, 3), ((7, 5), 0, 40), ((301, 9), 0, 40), ((64, 33), 1, 40),
-                                                    ((4095, 3), 0, 20), ((2048, 3), 1, 20), ((2049, 3), 1, 20), ((1025, 3), 3, 20),
-                                                    ((1024, 3), 2, 20), ((8192, 2), 0, 20), ((8193, 2), 0, 20), ((4096, 3), 1, 20),
-                                                    ((2048, 3), 2, 20), ((1024, 3), 3, 20),
-                                                    ((4100, 2), 2, 20), ((8193, 2), 1, 20), ((8193, 2), 2, 10), ((20, 6), 8, 8),
-                                                    ((40, 30), 1, 4000)])
-def test_crossing_lists(tmp_path, npx, over_sample, curves):
-    """Crossings go to a list per sub-pixel row, and the waves of a workgroup sum a row each
-    in LDS: odd and even widths, one to 256 sub-pixels a pixel, the first and last width of
-    each variant, grids too wide for lists, and rows that overflow theirs (4000 curves over
-    60 rows), against the oracle: identical counts and histogram."""
-    from irs_amd.microlensing.NCC.ncc import NCC
-    from oracle import ncc as ON
-    rng = np.random.default_rng(curves + over_sample)
+def astroids(rng, curves, spread, size):
+    """Closed clockwise curves around centres uniform in a box of half-lengths `spread`."""
     t = -np.linspace(0, 2 * np.pi, 60)
     t[-1] = t[0]
-    size = np.exp(rng.normal(0.0, 0.5, (curves, 1)))
-    rows = (rng.uniform(-4, 4, (curves, 1)) + 1j * rng.uniform(-4, 4, (curves, 1)) +
+    return (rng.uniform(-spread[0], spread[0], (curves, 1)) + 1j * rng.uniform(-spread[1], spread[1], (curves, 1)) +
             size * np.exp(2j * np.pi * rng.random((curves, 1))) * (np.cos(t) ** 3 + 1j * np.sin(t) ** 3))
+
+
+def check_crossings(tmp_path, rows, npx, over_sample, path):
+    """A run over the curves `rows` takes the given path (0 grid, 1 lists, 2 lists that overflow)
+    and gives the oracle's counts and histogram."""
+    from irs_amd.microlensing.NCC.ncc import NCC
+    from oracle import ncc as ON
     with open(tmp_path / "ccf_caustics.bin", "wb") as fh:
         np.array(rows.shape, dtype=np.int32).tofile(fh)
         np.ascontiguousarray(rows, dtype=np.complex128).tofile(fh)
-    say(f"[ncc lists] {npx}, over_sample {over_sample}, {curves} curves")
     prefix = str(tmp_path) + "/"
     n = NCC(infile_prefix=prefix, outfile_prefix=prefix, num_pixels_y1=npx[0], num_pixels_y2=npx[1], over_sample=over_sample,
             write_maps=False)
     n.run()
+    say(f"[ncc lists] {npx}, over_sample {over_sample}, {len(rows)} curves: path {n.lib.get_crossing_path(n.obj)}")
     want = ON.ncc_map(rows, (0.0, 0.0), (5.0, 5.0), npx, over_sample)
     np.testing.assert_array_equal(n.num_caustic_crossings, want)
     n.save()
     u, c = np.unique(want, return_counts=True)
     np.testing.assert_array_equal(np.loadtxt(prefix + "ncc_ncc_numpixels.txt", dtype=np.int64, ndmin=2), np.column_stack([u, c]))
+    assert n.lib.get_crossing_path(n.obj) == path
     n.close()
+
+
+@pytest.mark.parametrize("npx,over_sample,curves", [((1, 1), 0, 3), ((7, 5), 0, 40), ((301, 9), 0, 40), ((64, 33), 1, 40),
+                                                    ((4095, 3), 0, 20), ((2048, 3), 1, 20), ((2049, 3), 1, 20), ((1025, 3), 3, 20),
+                                                    ((1024, 3), 2, 20), ((8192, 2), 0, 20), ((8193, 2), 0, 20), ((4096, 3), 1, 20),
+                                                    ((2048, 3), 2, 20), ((1024, 3), 3, 20),
+                                                    ((4100, 2), 2, 20), ((8193, 2), 1, 20), ((8193, 2), 2, 10), ((20, 6), 8, 8)])
+def test_crossing_lists(tmp_path, npx, over_sample, curves):
+    """Crossings go to a list per sub-pixel row, and the waves of a workgroup sum a row each
+    in LDS: odd and even widths, one to 256 sub-pixels a pixel, the first and last width of
+    each variant, and grids too wide for lists, against the oracle: identical counts and
+    histogram."""
+    rng = np.random.default_rng(curves + over_sample)
+    rows = astroids(rng, curves, (4, 4), np.exp(rng.normal(0.0, 0.5, (curves, 1))))
+    check_crossings(tmp_path, rows, npx, over_sample, 1 if npx[0] << over_sample <= 8192 else 0)
+
+
+@pytest.mark.parametrize("npx,over_sample,curves,height,size,path", [((40, 30), 1, 4000, 4, 1.0, 0), ((100, 100), 0, 900, 4, 1.0, 1),
+                                                                     ((600, 2100), 0, 3000, 0.005, 0.05, 2),
+                                                                     ((64, 700), 2, 3000, 0.005, 0.05, 2), ((1, 3000), 0, 30, 4, 1.0, 1)])
+def test_crossings_of_dense_networks(tmp_path, npx, over_sample, curves, height, size, path):
+    """Networks with more crossings a row than lists are good for go to the grid at once, narrow
+    maps have room for many, curves heaped on a few rows overflow lists that the mean allowed (all
+    waves then stop and the grid takes over), and one column: the oracle's counts and histogram on
+    each path."""
+    rng = np.random.default_rng(curves)
+    check_crossings(tmp_path, astroids(rng, curves, (4, height), size), npx, over_sample, path)
