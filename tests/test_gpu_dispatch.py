@@ -469,3 +469,14 @@ def test_crossings_of_dense_networks(tmp_path, npx, over_sample, curves, height,
     each path."""
     rng = np.random.default_rng(curves)
     check_crossings(tmp_path, astroids(rng, curves, (4, height), size), npx, over_sample, path)
+
+
+@pytest.mark.parametrize("heaped", [False, True])
+@pytest.mark.parametrize("npx", [(1023, 512), (1024, 512), (1025, 513), (1500, 1201)])
+def test_crossing_histograms(tmp_path, npx, heaped):
+    """Maps of 2^19 pixels or more with at most 64 values are counted in a column per lane, all
+    others in shared bins: below, at and above that size, with pixels left over in a block, of few
+    values and (curves heaped on one place) of more than 64: the oracle's counts and histogram."""
+    rng = np.random.default_rng(npx[0])
+    curves = astroids(rng, 200 if heaped else 30, (0.3, 0.3) if heaped else (4, 4), 1.0)
+    check_crossings(tmp_path, curves, npx, 0, 1)
