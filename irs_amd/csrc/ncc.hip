@@ -756,6 +756,8 @@ void NCCDevice::count(const double* caustics, int nrows, int ncols, const NCCGri
 	if (!lists)
 	{
 		const size_t nfine = size_t(npx) * size_t(npy);
+		// the memory check above counted the grid alone: lists that overflowed make room for it
+		if (st.path == NCC_OVERFLOW && fine_.count < nfine) lists_.free();
 		if (fine_.count < nfine) fine_.alloc(nfine);
 		MLENS_HIP_CHECK(hipMemsetAsync(fine_.ptr, 0, nfine * sizeof(int), stream_));
 		k_ncc_init<<<1, 64, 0, stream_>>>(meta, nullptr, 0);

@@ -1,6 +1,7 @@
 """The kernel variants that a call's sizes and options choose, each at the edges of
 its range, against the FP64 oracle or the general path."""
 
+import ctypes
 import os
 
 import numpy as np
@@ -81,6 +82,13 @@ def test_batch_tiles_and_pieces(general):
         batch.close()
     for m in objs:
         m.close()
+
+
+def free_memory(lib):
+    """Bytes of device memory left, through the HIP runtime that the engine library is linked with."""
+    free, total = ctypes.c_size_t(), ctypes.c_size_t()
+    assert lib.hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)) == 0
+    return free.value
 
 
 def late_work(m):
@@ -480,3 +488,24 @@ def test_crossing_histograms(tmp_path, npx, heaped):
     rng = np.random.default_rng(npx[0])
     curves = astroids(rng, 200 if heaped else 30, (0.3, 0.3) if heaped else (4, 4), 1.0)
     check_crossings(tmp_path, curves, npx, 0, 1)
+
+
+def test_overflowed_lists_make_room(tmp_path):
+    """The memory check counts the grid: lists that overflowed are freed before it is allocated,
+    so that a map which passes the check fits. 512 x 131072 sub-pixels, 256 MB either way."""
+    from irs_amd.microlensing.NCC.ncc import NCC
+    rows = astroids(np.random.default_rng(1), 3000, (4, 0.005), 0.01)
+    with open(tmp_path / "ccf_caustics.bin", "wb") as fh:
+        np.array(rows.shape, dtype=np.int32).tofile(fh)
+        np.ascontiguousarray(rows, dtype=np.complex128).tofile(fh)
+    n = NCC(infile_prefix=str(tmp_path) + "/", num_pixels_y1=32, num_pixels_y2=8192, over_sample=4, write_maps=False)
+    warm = NCC(infile_prefix=str(tmp_path) + "/", num_pixels_y1=32, num_pixels_y2=32, write_maps=False)
+    warm.run()
+    before = free_memory(n.lib)
+    n.run()
+    held = before - free_memory(n.lib)
+    warm.close()
+    say(f"[ncc memory] path {n.lib.get_crossing_path(n.obj)}, {held >> 20} MB held")
+    assert n.lib.get_crossing_path(n.obj) == 2 and n.num_caustic_crossings.max() > 0
+    assert held < 384 << 20
+    n.close()
