@@ -7,6 +7,7 @@
 #include <sys/mman.h>
 
 #include <cstdlib>
+#include <cstring>
 #include <new>
 #include <utility>
 
@@ -40,6 +41,21 @@ public:
 			ptr_ = static_cast<T*>(std::malloc(bytes));
 		if (!ptr_) throw std::bad_alloc();
 		size_ = n;
+	}
+	// n elements that fill(data) writes; zeros if it throws
+	template <typename F>
+	void fill(size_t n, F fill)
+	{
+		resize(n);
+		try
+		{
+			fill(ptr_);
+		}
+		catch (...)
+		{
+			if (ptr_) std::memset(static_cast<void*>(ptr_), 0, n * sizeof(T));
+			throw;
+		}
 	}
 	void clear()
 	{

@@ -787,8 +787,7 @@ private:
 	// the star field in tree order, as get_stars returns it
 	void download_stars()
 	{
-		stars_host_.resize(size_t(num_stars_) * 3);
-		engine_->download_stars(stars_host_.data());
+		stars_host_.fill(size_t(num_stars_) * 3, [&](T* to) { engine_->download_stars(to); });
 		stars_stale_ = false;
 	}
 
@@ -796,29 +795,30 @@ private:
 	{
 		size_t n = size_t(num_pixels_y.re) * num_pixels_y.im;
 		auto fetch = [&](int which, HostArray<T>& dst) {
-			dst.resize(n);
-			if (engine_->maps_are_fp32())
-			{
-				if (std::is_same<T, float>::value)
-					engine_->download_map(which, dst.data());
+			dst.fill(n, [&](T* to) {
+				if (engine_->maps_are_fp32())
+				{
+					if (std::is_same<T, float>::value)
+						engine_->download_map(which, to);
+					else
+					{
+						std::vector<float> f(n);
+						engine_->download_map(which, f.data());
+						for (size_t i = 0; i < n; i++) to[i] = T(f[i]);
+					}
+				}
 				else
 				{
-					std::vector<float> f(n);
-					engine_->download_map(which, f.data());
-					for (size_t i = 0; i < n; i++) dst[i] = T(f[i]);
+					if (std::is_same<T, double>::value)
+						engine_->download_map(which, to);
+					else
+					{
+						std::vector<double> d(n);
+						engine_->download_map(which, d.data());
+						for (size_t i = 0; i < n; i++) to[i] = T(d[i]);
+					}
 				}
-			}
-			else
-			{
-				if (std::is_same<T, double>::value)
-					engine_->download_map(which, dst.data());
-				else
-				{
-					std::vector<double> d(n);
-					engine_->download_map(which, d.data());
-					for (size_t i = 0; i < n; i++) dst[i] = T(d[i]);
-				}
-			}
+			});
 		};
 		if (IS_IPM)
 		{
@@ -836,14 +836,11 @@ private:
 		}
 		else
 		{
-			ipix_.resize(n);
-			engine_->download_map(0, ipix_.data());
+			ipix_.fill(n, [&](int* to) { engine_->download_map(0, to); });
 			if (write_parities)
 			{
-				ipix_min_.resize(n);
-				ipix_sad_.resize(n);
-				engine_->download_map(1, ipix_min_.data());
-				engine_->download_map(2, ipix_sad_.data());
+				ipix_min_.fill(n, [&](int* to) { engine_->download_map(1, to); });
+				ipix_sad_.fill(n, [&](int* to) { engine_->download_map(2, to); });
 			}
 			else
 			{

@@ -160,8 +160,8 @@ private:
 		g.num_pixels_re = num_pixels_y.re;
 		g.num_pixels_im = num_pixels_y.im;
 		g.over_sample = over_sample;
-		num_.resize(size_t(num_pixels_y.re) * size_t(num_pixels_y.im));
-		device_->count(caustics_.data(), num_rows_, num_cols_, g, num_.data(), stats_);
+		num_.fill(size_t(num_pixels_y.re) * size_t(num_pixels_y.im),
+			[&](int* num) { device_->count(caustics_.data(), num_rows_, num_cols_, g, num, stats_); });
 		t_ncc_ = stats_.t_ncc_ms / 1000;
 		t_reduce_ = stats_.t_reduce_ms / 1000;
 		if (stats_.dropped > 0)

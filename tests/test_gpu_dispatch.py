@@ -509,3 +509,24 @@ def test_overflowed_lists_make_room(tmp_path):
     assert n.lib.get_crossing_path(n.obj) == 2 and n.num_caustic_crossings.max() > 0
     assert held < 384 << 20
     n.close()
+
+
+def test_failed_crossings_leave_zeros(tmp_path):
+    """A run that fails on the device (an over-sampled grid past its memory) leaves a map of zeros,
+    the first time and after a run that held counts, never what memory happened to hold."""
+    from irs_amd.microlensing.NCC.ncc import NCC
+    rows = astroids(np.random.default_rng(1), 50, (1, 1), 1.0)
+    with open(tmp_path / "ccf_caustics.bin", "wb") as fh:
+        np.array(rows.shape, dtype=np.int32).tofile(fh)
+        np.ascontiguousarray(rows, dtype=np.complex128).tofile(fh)
+    for first in (True, False):
+        n = NCC(infile_prefix=str(tmp_path) + "/", num_pixels_y1=300, num_pixels_y2=200, over_sample=0, write_maps=False)
+        if not first:
+            n.run()
+            assert n.num_caustic_crossings.max() > 0
+        n.over_sample = 12
+        with pytest.raises(Exception, match="Error running NCC"):
+            n.run()
+        counts = np.ctypeslib.as_array(n.lib.get_num_crossings(n.obj), shape=(200, 300))
+        assert not counts.any()
+        n.close()
