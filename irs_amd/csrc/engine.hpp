@@ -224,6 +224,7 @@ private:
 	bool m2l_ready_f32_ = false;
 	DeviceBuffer<float> m2l_af_;
 	DeviceBuffer<double> m2l_ad_, m2l_powers_;
+	std::vector<double> m2l_host_;   // what m2l_powers_ is copied from
 	DeviceBuffer<unsigned long long> m2l_count_;
 	hipEvent_t m2l_ev0_ = nullptr, m2l_ev1_ = nullptr;
 

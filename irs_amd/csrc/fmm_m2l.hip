@@ -314,7 +314,8 @@ void Engine::m2l_prepare(int p, bool f32)
 {
 	if (m2l_ready_p_ == p && m2l_ready_f32_ == f32) return;
 	const int P = p + 1, kp = m2l_kp(p);
-	std::vector<double> w(size_t(M2L_OFFSETS) * M2L_POWERS * 2, 0.0);
+	std::vector<double>& w = m2l_host_;   // outlives the copy
+	w.assign(size_t(M2L_OFFSETS) * M2L_POWERS * 2, 0.0);
 	for (int b = -3; b <= 3; b++)
 		for (int a = -3; a <= 3; a++)
 		{
@@ -351,7 +352,6 @@ void Engine::m2l_prepare(int p, bool f32)
 		k_m2l_matrices<double><<<grid, 256, 0, stream_>>>(m2l_powers_.ptr, binom_.ptr, p, kp, m2l_ad_.ptr);
 	}
 	MLENS_HIP_CHECK(hipGetLastError());
-	// w is read before the copy returns (pageable memory), so it may go
 	m2l_ready_p_ = p;
 	m2l_ready_f32_ = f32;
 }
