@@ -177,6 +177,7 @@ long long ipm_window_cells(IPMHandle* self, int x0, int y0, int width, int heigh
                            long long capacity);
 /* the tree as the oracle exports it: geom[3n], info[9n], lists[40n] */
 int get_num_nodes(IPMHandle* self);
+int get_num_leaves(IPMHandle* self);   /* of the nodes; the leaf tables hold one entry each */
 bool ipm_export_tree(IPMHandle* self, double* geom, int* info, int* lists);
 bool ipm_export_coeffs(IPMHandle* self, int which, double* out);   /* 0 multipole, 1 local; 2(p+1) doubles per node */
 /* validation and derived geometry only (no device work): num_stars, the

@@ -115,6 +115,7 @@ public:
 	void build_tree(double root_half_length);
 	int tree_levels() const { return levels_; }
 	int num_nodes() const { return num_nodes_; }
+	int num_leaves() const { return num_leaves_; }   // of the tree, and entries of the leaf tables
 	const std::vector<int>& level_start() const { return level_start_; }
 	void export_tree(double* geom, int* info, int* lists) const;   // same layout as the oracle's export
 
@@ -228,7 +229,8 @@ private:
 	DeviceBuffer<unsigned long long> m2l_count_;
 	hipEvent_t m2l_ev0_ = nullptr, m2l_ev1_ = nullptr;
 
-	int num_leaves_ = 0;   // entries of the leaf tables: one per node, those of inner nodes empty
+	int num_leaves_ = 0;   // entries of the leaf tables
+	int last_level_leaf0_ = 0;   // of them on the levels before the last
 	DeviceBuffer<int> leaf_of_node_;
 	DeviceBuffer<double> leaf_geom_;      // cx, cy, hl, 1/hl per leaf
 	DeviceBuffer<int> leaf_near_n_;       // padded to a multiple of 4; FP32 polynomial entries to skip << 16

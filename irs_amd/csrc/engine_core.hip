@@ -423,13 +423,18 @@ SPLIT_MAX stars, whose passes a single block would walk alone.
 */
 constexpr int SPLIT_MAX = 16384;
 
+// A node of a level that splits further: its place in the leaf tables, -1 for one that splits itself. leaf0 leaves stand
+// on earlier levels; build_leaf_tables numbers the last level, whose nodes are all leaves.
+__device__ __forceinline__ int leaf_index(const int* flags, const int* rank, int k, int leaf0) { return flags[k] ? -1 : leaf0 + k - rank[k]; }
+
 template <int THREADS>
 __global__ __launch_bounds__(THREADS) void k_split_nodes(TreeView t, int l0, const int* __restrict__ flags, const int* __restrict__ rank,
-	int base, double* sx, double* sy, double* sm, double* tx, double* ty, double* tm)
+	int base, int leaf0, int* __restrict__ leaf_of_node, double* sx, double* sy, double* sm, double* tx, double* ty, double* tm)
 {
 	constexpr int WAVES = THREADS / 64;
 	__shared__ int part[4][WAVES];
 	const int i = l0 + blockIdx.x;
+	if (threadIdx.x == 0) leaf_of_node[i] = leaf_index(flags, rank, blockIdx.x, leaf0);
 	if (!flags[blockIdx.x]) return;
 	const int c0 = base + 4 * rank[blockIdx.x];
 	const int b = t.begin[i], n = t.count[i];
@@ -520,10 +525,12 @@ __global__ __launch_bounds__(THREADS) void k_split_nodes(TreeView t, int l0, con
 }
 
 // the device-wide partition of a level (k_split_nodes takes the levels whose nodes are small)
-__global__ void k_make_children(TreeView t, int l0, int l1, const int* flags, const int* rank, int base)
+__global__ void k_make_children(TreeView t, int l0, int l1, const int* flags, const int* rank, int base, int leaf0, int* leaf_of_node)
 {
 	int i = l0 + blockIdx.x * blockDim.x + threadIdx.x;
-	if (i >= l1 || !flags[i - l0]) return;
+	if (i >= l1) return;
+	leaf_of_node[i] = leaf_index(flags, rank, i - l0, leaf0);
+	if (!flags[i - l0]) return;
 	int c0 = base + 4 * rank[i - l0];
 	t.child0[i] = c0;
 	for (int q = 0; q < 4; q++) make_child(t, i, c0, q);
@@ -688,6 +695,7 @@ void Engine::ensure_node_capacity(int n)
 	grow(nnbr_, u * 8, size_t(cap) * 8);
 	grow(nm2l_, u * 27, size_t(cap) * 27);
 	grow(np2l_, u * 5, size_t(cap) * 5);
+	grow(leaf_of_node_, u, cap);
 	node_cap_ = cap;
 }
 
@@ -706,6 +714,7 @@ void Engine::build_tree(double root_half_length)
 	ensure_node_capacity(std::max(1024, n + n / 8));
 	level_start_.assign({0, 1});
 	levels_ = 0;
+	num_leaves_ = 0;   // on the levels before this one
 
 	num_nodes_ = 1;
 	const size_t ns = size_t(std::max(n, 1));
@@ -743,7 +752,12 @@ void Engine::build_tree(double root_half_length)
 		LevelCount lc;
 		MLENS_HIP_CHECK(hipMemcpyAsync(&lc, counts, sizeof(lc), hipMemcpyDeviceToHost, stream_));
 		MLENS_HIP_CHECK(hipStreamSynchronize(stream_));
-		if (lc.split == 0) break;
+		if (lc.split == 0)
+		{
+			last_level_leaf0_ = num_leaves_;
+			num_leaves_ += nl;
+			break;
+		}
 		const int base = l1;
 		ensure_node_capacity(base + 4 * lc.split);
 		const TreeView t = tree();
@@ -757,7 +771,8 @@ void Engine::build_tree(double root_half_length)
 			star_node_tmp_.alloc(ns);
 			if (!star_nodes) MLENS_HIP_CHECK(hipMemsetAsync(star_node_.ptr, 0, ns * sizeof(int), stream_));
 			star_nodes = true;
-			k_make_children<<<blocks_for(nl, 256), 256, 0, stream_>>>(t, l0, l1, node_flag_.ptr, node_rank_.ptr, base);
+			k_make_children<<<blocks_for(nl, 256), 256, 0, stream_>>>(t, l0, l1, node_flag_.ptr, node_rank_.ptr, base,
+				num_leaves_, leaf_of_node_.ptr);
 			k_star_onehot<<<blocks_for(n, 256), 256, 0, stream_>>>(t, sx_.ptr, sy_.ptr, star_node_.ptr, l0, node_flag_.ptr, onehot, n);
 			MLENS_HIP_CHECK(hipGetLastError());
 			scan_i4(onehot, pre, tiles, n, stream_);
@@ -779,14 +794,15 @@ void Engine::build_tree(double root_half_length)
 			// a block per node, as wide as its largest node can use (children never hold more stars than
 			// their parent, so the device-wide partition is not needed again)
 			auto split = [&](auto kernel, int threads) {
-				kernel<<<nl, threads, 0, stream_>>>(t, l0, node_flag_.ptr, node_rank_.ptr, base, sx_.ptr, sy_.ptr, sm_.ptr, tx_.ptr,
-					ty_.ptr, tm_.ptr);
+				kernel<<<nl, threads, 0, stream_>>>(t, l0, node_flag_.ptr, node_rank_.ptr, base, num_leaves_, leaf_of_node_.ptr, sx_.ptr,
+					sy_.ptr, sm_.ptr, tx_.ptr, ty_.ptr, tm_.ptr);
 			};
 			if (lc.largest <= 256) split(k_split_nodes<64>, 64);
 			else if (lc.largest <= 2048) split(k_split_nodes<256>, 256);
 			else split(k_split_nodes<1024>, 1024);
 			MLENS_HIP_CHECK(hipGetLastError());
 		}
+		num_leaves_ += nl - lc.split;
 		num_nodes_ = base + 4 * lc.split;
 		levels_++;
 		level_start_.push_back(num_nodes_);
@@ -1025,12 +1041,12 @@ Leaf tables for shooting: geometry, the near-field star list (own stars then
 each neighbour's, alpha_star.cuh:26-37) and the deflection polynomial
 A_i = (theta^2/h) i c_i of alpha_local.cuh:18-36, so that
 alpha_local(z) = conj( sum_{i=1..p} A_i dz^(i-1) ), dz = (z - c)/h.
-A leaf's tables stand at its node's index (inner nodes leave theirs unused, a
-quarter of them): no scan over the nodes and no wait for its total. 32 lanes per
-leaf, a near star and a polynomial entry each: one lane per leaf wrote 2 KB in
-24-byte steps (2.0 ms for the 1.28e6-star tree).
+Leaves are numbered as the levels are split (leaf_index), the last level's nodes,
+from `last` on, here: no scan over the nodes. 32 lanes per node, a near star and a
+polynomial entry each: one lane per leaf wrote 2 KB in 24-byte steps (2.0 ms for
+the 1.28e6-star tree).
 */
-__global__ __launch_bounds__(256) void k_leaf_tables(TreeView t, int nn, int p, double theta2, const double* __restrict__ sx,
+__global__ __launch_bounds__(256) void k_leaf_tables(TreeView t, int nn, int last, int last_leaf0, int p, double theta2, const double* __restrict__ sx,
 	const double* __restrict__ sy, const double* __restrict__ sm, const double* __restrict__ local, int* leaf_of_node, double* geom,
 	int* near_n, int* near_true, double* near_d, float* near_f, double* poly_d, float* poly_f)
 {
@@ -1040,16 +1056,9 @@ __global__ __launch_bounds__(256) void k_leaf_tables(TreeView t, int nn, int p, 
 	__shared__ double lead_s[256 / LANES][LANES];
 	const int lane = threadIdx.x % LANES, slot = threadIdx.x / LANES;
 	const int i = blockIdx.x * (256 / LANES) + slot;
-	const bool node = i < nn, leaf = node && t.child0[i] < 0;
-	if (node && lane == 0) leaf_of_node[i] = leaf ? i : -1;
-	const long long L = i;
-	if (node && !leaf && lane == 0)
-	{
-		// an inner node's entry: no area and no stars
-		for (int k = 0; k < 4; k++) geom[4 * L + k] = 0;
-		near_n[L] = 0;
-		near_true[L] = 0;
-	}
+	const long long L = i >= nn ? -1 : (i >= last ? last_leaf0 + (i - last) : leaf_of_node[i]);
+	const bool leaf = L >= 0;
+	if (leaf && i >= last && lane == 0) leaf_of_node[i] = int(L);
 	double cx = 0, cy = 0, h = 1, scale_l1 = 0, lead = 0;
 	int total = 0, padded = 0;
 	const int SD = poly_stride_d(p), SF = poly_stride_f(p);
@@ -1203,9 +1212,7 @@ void Engine::fmm(int p, const LensParams& lens)
 void Engine::build_leaf_tables(const LensParams& lens)
 {
 	const int nn = num_nodes_;
-	num_leaves_ = nn;   // entries: one per node
 	const int SD = poly_stride_d(p_), SF = poly_stride_f(p_);
-	leaf_of_node_.alloc(nn);
 	leaf_geom_.alloc(size_t(num_leaves_) * 4);
 	leaf_near_n_.alloc(num_leaves_);
 	leaf_near_true_.alloc(num_leaves_);
@@ -1214,7 +1221,7 @@ void Engine::build_leaf_tables(const LensParams& lens)
 	leaf_poly_d_.alloc(size_t(std::max(num_leaves_, 1)) * SD * 2);
 	leaf_poly_f_.alloc(size_t(std::max(num_leaves_, 1)) * std::max(SF, 1) * 2);
 	TreeView t = view(ncx_, ncy_, nhl_, nlevel_, nparent_, nchild0_, nbegin_, ncount_, nnnbr_, nnm2l_, nnp2l_, nnbr_, nm2l_, np2l_);
-	k_leaf_tables<<<blocks_for(nn, 8), 256, 0, stream_>>>(t, nn, p_, lens.theta * lens.theta, sx_.ptr, sy_.ptr,
+	k_leaf_tables<<<blocks_for(nn, 8), 256, 0, stream_>>>(t, nn, level_start_[levels_], last_level_leaf0_, p_, lens.theta * lens.theta, sx_.ptr, sy_.ptr,
 		sm_.ptr, local_.ptr, leaf_of_node_.ptr, leaf_geom_.ptr, leaf_near_n_.ptr, leaf_near_true_.ptr, leaf_near_d_.ptr,
 		leaf_near_f_.ptr,
 		leaf_poly_d_.ptr, leaf_poly_f_.ptr);

@@ -28,6 +28,7 @@ ipm_dtype* get_pixels(IPMHandle* self) { return self->m.get_pixels(); }
 ipm_dtype* get_pixels_minima(IPMHandle* self) { return self->m.get_pixels_minima(); }
 ipm_dtype* get_pixels_saddles(IPMHandle* self) { return self->m.get_pixels_saddles(); }
 double get_t_shoot_cells(IPMHandle* self) { return self->m.get_t_shoot(); }
+int get_num_leaves(IPMHandle* self) { return self->m.engine() ? self->m.engine()->num_leaves() : 0; }
 long long get_late_triangles(IPMHandle* self) { MLENS_GUARD(return self->m.get_late_work().triangles, return -1) }
 long long get_late_rows(IPMHandle* self) { MLENS_GUARD(return self->m.get_late_work().rows, return -1) }
 

@@ -92,6 +92,7 @@ def load(path, dtype, irs=False):
         sig("get_t_shoot_cells", [v], ctypes.c_double)
         sig("get_late_triangles", [v], ll)
         sig("get_late_rows", [v], ll)
+        sig("get_num_leaves", [v], i)
         sig("ipm_prepare", [v, i], b)
         sig("ipm_build", [v, i], b)
         sig("ipm_shoot", [v, i, ll, ll], b)
@@ -132,7 +133,7 @@ IPM_SYMBOLS = (["init"] + [f"set_{n}" for n, _ in _FIELDS[:26]] + [f"get_{n}" fo
                 "ipm_export_coeffs", "ipm_derive", "ipm_batch_create", "ipm_batch_free", "ipm_batch_add",
                 "ipm_batch_shoot", "get_batch_t_shoot", "get_batch_cells", "get_batch_size", "ipm_batch_histograms",
                 "get_batch_tile_h", "get_batch_blocks_per_cu", "get_batch_t_tune", "ipm_batch_set_tuning",
-                "get_late_triangles", "get_late_rows"] + _M2L_SYMBOLS)
+                "get_late_triangles", "get_late_rows", "get_num_leaves"] + _M2L_SYMBOLS)
 
 IRS_SYMBOLS = (["init", "irs_free"] + [f"set_{n}" for n, _ in _FIELDS[:26]] + [f"get_{n}" for n, _ in _FIELDS[:26]] +
                ["get_num_stars", "get_corner_x1", "get_corner_x2", "get_stars", "get_pixels", "get_pixels_minima",

@@ -193,7 +193,9 @@ def coefficient_errors(m, tree):
 def test_trees_of_every_split_path(oracle, tmp_path, n, cluster):
     """A level is split by one block per node of 64, 256 or 1024 threads, or device-wide
     above 16384 stars in a node, its nodes ranked by one block or, above 32768 of them,
-    by a device-wide scan; M2L runs one or two column tiles per block. Even fields and
+    by a device-wide scan; M2L runs one or two column tiles per block. The leaf tables hold
+    an entry per leaf, numbered as the levels are split: points in the first leaf, the last and
+    a few thousand others deflect as in the oracle's tree (the parity tests' bound). Even fields and
     fields with a cluster a few thousandths wide: the oracle's tree bit for bit, its
     coefficients to FP64 rounding (the bound of the parity tests)."""
     rng = np.random.default_rng(n + cluster)
@@ -209,6 +211,16 @@ def test_trees_of_every_split_path(oracle, tmp_path, n, cluster):
     for which, err in coefficient_errors(m, tree):
         say(f"[tree] {which}: {err:.1e}")
         assert err < 1e-11, which
+    geom, info, _ = m.export_tree()
+    leaves = geom[info[:, 2] < 0]
+    assert m.lib.get_num_leaves(m.obj) == len(leaves)
+    some = leaves[np.unique(np.linspace(0, len(leaves) - 1, 4000).astype(int))]
+    z = some[:, 0] + 0.3 * some[:, 2] + 1j * (some[:, 1] - 0.4 * some[:, 2])
+    lens = oracle.make_lens(m.kappa_tot, m.shear, m.theta_star, m.kappa_star, (40.0, 0.0), 0, 1, m.lib.get_taylor_smooth(m.obj))
+    want, _ = tree.deflect(lens, z)
+    err = np.abs(m.deflect(z) - want)
+    say(f"[tree] {len(leaves)} leaves, deflections of {len(z)}: {err.max():.1e}")
+    assert err.max() < 1e-10
     m.close()
 
 
