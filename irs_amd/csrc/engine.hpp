@@ -148,9 +148,9 @@ public:
 	/* of the first nmaps of total, minima, saddles (which must exist) */
 	void map_extremes(int nmaps, MapExtremes* out);
 	/* counts of round(value * factor - hist_min) in [0, length) and, with log_length > 0, of log10(value)
-	   likewise over the positive pixels: length + log_length counts per map */
+	   likewise over the positive pixels, into lin[map] and log[map] */
 	void map_histograms(int nmaps, int factor, long long hist_min, long long length, long long log_min,
-		long long log_length, long long* host_hist);
+		long long log_length, long long* const* lin, long long* const* log);
 
 	/* critical curves (ccf_functions.cuh, ccf.cuh): refine nroots roots per phase for
 	   nphi + nb phases (nb branches of nphi / nb + 1 phases), starting from init_roots

@@ -2325,21 +2325,46 @@ void Engine::map_extremes(int nmaps, MapExtremes* out)
 	MLENS_HIP_CHECK(hipStreamSynchronize(stream_));
 }
 
+/* All maps in one pass while their histograms are small (the usual few thousand bins): one copy brings them. Ranges of
+   millions of bins (a bright caustic) are counted map by map, copied straight to the caller's arrays, and their
+   memory is given back. */
 void Engine::map_histograms(int nmaps, int factor, long long hmin, long long len, long long log_min, long long log_len,
-	long long* host_hist)
+	long long* const* lin, long long* const* log)
 {
+	constexpr size_t TOGETHER = size_t(1) << 20;   // bins: 8 MB
 	const long long n = (long long)npix_[0] * npix_[1];
-	const size_t total = size_t(nmaps) * size_t(len + log_len);
-	hist_.alloc(total);
-	MLENS_HIP_CHECK(hipMemsetAsync(hist_.ptr, 0, sizeof(long long) * total, stream_));
+	const size_t each = size_t(len + log_len);
+	const bool together = size_t(nmaps) * each <= TOGETHER;
+	const int step = together ? nmaps : 1;
+	hist_.alloc(size_t(step) * each);
 	unsigned long long* hp = reinterpret_cast<unsigned long long*>(hist_.ptr);
 	const unsigned nb = unsigned(std::min<long long>(HIST_BLOCKS_MAX, (n + HIST_PIXELS - 1) / HIST_PIXELS));
-	with_maps([&](auto maps) {
-		k_histograms<<<dim3(nb, nmaps), HIST_THREADS, 0, stream_>>>(maps, n, factor, hmin, len, log_min, log_len, hp);
-	});
-	MLENS_HIP_CHECK(hipGetLastError());
-	MLENS_HIP_CHECK(hipMemcpyAsync(host_hist, hist_.ptr, sizeof(long long) * total, hipMemcpyDeviceToHost, stream_));
-	MLENS_HIP_CHECK(hipStreamSynchronize(stream_));
+	std::vector<long long> counts(together ? size_t(nmaps) * each : 0);
+	for (int first = 0; first < nmaps; first += step)
+	{
+		MLENS_HIP_CHECK(hipMemsetAsync(hist_.ptr, 0, sizeof(long long) * size_t(step) * each, stream_));
+		with_maps([&](auto maps) {
+			maps.map[0] = maps.map[first];
+			k_histograms<<<dim3(nb, step), HIST_THREADS, 0, stream_>>>(maps, n, factor, hmin, len, log_min, log_len, hp);
+		});
+		MLENS_HIP_CHECK(hipGetLastError());
+		if (together)
+			MLENS_HIP_CHECK(hipMemcpyAsync(counts.data(), hist_.ptr, sizeof(long long) * counts.size(), hipMemcpyDeviceToHost, stream_));
+		else
+		{
+			MLENS_HIP_CHECK(hipMemcpyAsync(lin[first], hist_.ptr, sizeof(long long) * size_t(len), hipMemcpyDeviceToHost, stream_));
+			if (log_len > 0)
+				MLENS_HIP_CHECK(hipMemcpyAsync(log[first], hist_.ptr + len, sizeof(long long) * size_t(log_len), hipMemcpyDeviceToHost, stream_));
+		}
+		MLENS_HIP_CHECK(hipStreamSynchronize(stream_));
+	}
+	for (int k = 0; k < nmaps && together; k++)
+	{
+		const long long* c = counts.data() + size_t(k) * each;
+		std::copy(c, c + len, lin[k]);
+		std::copy(c + len, c + each, log[k]);
+	}
+	if (!together) hist_.free();
 }
 
 }  // namespace mlens

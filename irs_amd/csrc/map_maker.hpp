@@ -773,14 +773,15 @@ private:
 			min_log_mag_ = llo;
 			max_log_mag_ = lhi;
 		}
-		std::vector<long long> counts(size_t(nmaps) * size_t(len + log_len));
-		engine_->map_histograms(nmaps, factor, lo, len, llo, log_len, counts.data());
+		long long *lin[3], *log[3];
 		for (int k = 0; k < nmaps; k++)
 		{
-			const auto first = counts.begin() + k * (len + log_len);
-			hist_[k].assign(first, first + len);
-			if (log_len > 0) log_hist_[k].assign(first + len, first + len + log_len);
+			hist_[k].assign(size_t(len), 0);
+			if (log_len > 0) log_hist_[k].assign(size_t(log_len), 0);
+			lin[k] = hist_[k].data();
+			log[k] = log_hist_[k].data();
 		}
+		engine_->map_histograms(nmaps, factor, lo, len, llo, log_len, lin, log);
 		return true;
 	}
 

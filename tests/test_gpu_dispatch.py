@@ -273,6 +273,12 @@ def test_histograms_inside_and_past_the_window(tmp_path, irs, double, n1, n2):
              half_length_y2=0.02 * n2, num_pixels_y1=n1, num_pixels_y2=n2, num_rays_y=900 if irs else 4, light_loss=0.01,
              random_seed=5, expansion_order=12, write_parities=True, write_histograms=True, outfile_prefix=prefix,
              **({"is_double": double} if not irs else {}))
+    check_histograms(m, prefix, irs)
+    m.close()
+
+
+def check_histograms(m, prefix, irs):
+    """Every bin of the saved histograms against numpy's count of the returned maps."""
     m.save()
     maps = (m.num_rays, m.num_rays_minima, m.num_rays_saddles) if irs else (
         m.magnifications, m.magnifications_minima, m.magnifications_saddles)
@@ -287,6 +293,31 @@ def test_histograms_inside_and_past_the_window(tmp_path, irs, double, n1, n2):
             got = np.loadtxt(prefix + ("irs_" if irs else "ipm_") + kind + suffix + ".txt", dtype=np.int64, ndmin=2)
             np.testing.assert_array_equal(got, np.column_stack([u, c]), err_msg=kind + suffix)
             say(f"[hist] {kind}{suffix}: {len(u)} bins up to {u[-1]}")
+
+
+@pytest.mark.parametrize("irs", [False, True])
+def test_histograms_of_wide_ranges(tmp_path, irs):
+    """One star images the pixel behind it into a ring, thousands of times the others: histograms
+    of millions of bins, counted map by map; and the memory they took is given back."""
+    from irs_amd.microlensing.IPM.ipm import IPM
+    from irs_amd.microlensing.IRS.irs import IRS
+    path = tmp_path / "stars.bin"
+    write_field(path, np.array([[0.0, 0.0, 1.0]]), 40.0)
+    prefix = str(tmp_path) + "/"
+    kw = dict(kappa_tot=1.0 / 1600, shear=0.0, starfile=str(path), light_loss=4e-4, half_length_y1=0.3, half_length_y2=0.3,
+              num_pixels_y1=501, num_pixels_y2=501, num_rays_y=1000 if irs else 30, expansion_order=8, write_parities=True,
+              outfile_prefix=prefix)
+    m = (IRS if irs else IPM)(**kw, write_stars=False, write_maps=False, write_histograms=True)
+    m.prepare()
+    m.build()
+    m.shoot()
+    before = free_memory(m.lib)
+    m.finish()
+    held = before - free_memory(m.lib)
+    bins = float((m.num_rays if irs else 1000 * m.magnifications).max())
+    say(f"[hist wide] irs {irs}: {bins:.3g} bins, {held >> 20} MB held")
+    assert bins > 1 << 20 and held < 8 << 20
+    check_histograms(m, prefix, irs)
     m.close()
 
 
