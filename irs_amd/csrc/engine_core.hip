@@ -134,13 +134,17 @@ __global__ void k_stars_aos(const double* sx, const double* sy, const double* sm
 template <typename F>
 void Engine::download_stars_as(F* aos)
 {
-	const int n = nstars_;
-	if (n <= 0) return;
-	stars_aos_.alloc(3 * sizeof(F) * size_t(n));
+	// in pieces, so that the rows' buffer stays small beside a large field (6 MB)
+	constexpr int PIECE = 1 << 18;
+	stars_aos_.alloc(3 * sizeof(F) * size_t(std::min(std::max(nstars_, 0), PIECE)));
 	F* d = reinterpret_cast<F*>(stars_aos_.ptr);
-	k_stars_aos<F><<<blocks_for(n, 256), 256, 0, stream_>>>(sx_.ptr, sy_.ptr, sm_.ptr, n, d);
-	MLENS_HIP_CHECK(hipGetLastError());
-	MLENS_HIP_CHECK(hipMemcpyAsync(aos, d, 3 * sizeof(F) * size_t(n), hipMemcpyDeviceToHost, stream_));
+	for (int i = 0; i < nstars_; i += std::min(PIECE, nstars_ - i))
+	{
+		const int n = std::min(PIECE, nstars_ - i);
+		k_stars_aos<F><<<blocks_for(n, 256), 256, 0, stream_>>>(sx_.ptr + i, sy_.ptr + i, sm_.ptr + i, n, d);
+		MLENS_HIP_CHECK(hipGetLastError());
+		MLENS_HIP_CHECK(hipMemcpyAsync(aos + 3 * size_t(i), d, 3 * sizeof(F) * size_t(n), hipMemcpyDeviceToHost, stream_));
+	}
 	MLENS_HIP_CHECK(hipStreamSynchronize(stream_));
 }
 

@@ -573,3 +573,24 @@ def test_failed_crossings_leave_zeros(tmp_path):
         counts = np.ctypeslib.as_array(n.lib.get_num_crossings(n.obj), shape=(200, 300))
         assert not counts.any()
         n.close()
+
+
+@pytest.mark.parametrize("n", [262143, 262144, 262145, 600001])
+def test_star_fields_come_back_in_pieces(tmp_path, n):
+    """Stars return through a buffer of 2^18 rows: fields of less than one piece, one, and
+    several with a remainder come back whole, and what the device keeps for it stays small."""
+    from irs_amd.microlensing.IPM.ipm import IPM
+    rng = np.random.default_rng(n)
+    stars = np.column_stack([disk(rng, n, 39.0), rng.uniform(0.5, 1.5, n) * 16.0 / n])
+    write_field(tmp_path / "stars.bin", stars, 40.0)
+    m = IPM(kappa_tot=0.3, shear=0.3, light_loss=0.01, starfile=str(tmp_path / "stars.bin"), half_length_y1=0.5, half_length_y2=0.5,
+            num_pixels_y1=16, num_pixels_y2=16, is_double=True, expansion_order=3)
+    m.prepare()
+    assert m.lib.ipm_build(m.obj, 0)
+    before = free_memory(m.lib)
+    got = np.ctypeslib.as_array(m.lib.get_stars(m.obj), shape=(n, 3)).copy()
+    held = before - free_memory(m.lib)
+    say(f"[stars] {n}: {held >> 20} MB held")
+    np.testing.assert_array_equal(got[np.lexsort(got.T)], stars[np.lexsort(stars.T)])
+    assert held <= 8 << 20
+    m.close()
