@@ -2044,6 +2044,9 @@ void Engine::deflect_points(const LensParams& lens, const double* z, int n, Prec
 	MLENS_HIP_CHECK(hipMemcpyAsync(w, dw, sizeof(double) * 2 * n, hipMemcpyDeviceToHost, stream_));
 	if (mu) MLENS_HIP_CHECK(hipMemcpyAsync(mu, dmu, sizeof(double) * n, hipMemcpyDeviceToHost, stream_));
 	MLENS_HIP_CHECK(hipStreamSynchronize(stream_));
+	// kept for the next call up to 84 MB; a call of more points spends longer on its copies than on an allocation
+	constexpr int POINTS_KEPT = 1 << 21;
+	if (n > POINTS_KEPT) points_.free();
 }
 
 /*

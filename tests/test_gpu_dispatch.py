@@ -594,3 +594,17 @@ def test_star_fields_come_back_in_pieces(tmp_path, n):
     np.testing.assert_array_equal(got[np.lexsort(got.T)], stars[np.lexsort(stars.T)])
     assert held <= 8 << 20
     m.close()
+
+
+def test_large_deflection_calls_give_their_memory_back(tmp_path):
+    """The points of a call stay on the device for the next one up to 2^21 of them; a call of more
+    frees them, and both give the same deflections."""
+    rng = np.random.default_rng(5)
+    m = built(tmp_path / "stars.bin", np.column_stack([disk(rng, 500, 39.0), np.full(500, 16.0 / 500)]), 8)
+    z = 20 * (rng.random((1 << 21) + 1) - 0.5) + 1j * (rng.random((1 << 21) + 1) - 0.5)
+    m.deflect(z[:10])
+    before = free_memory(m.lib)
+    w = m.deflect(z)
+    assert before - free_memory(m.lib) < 8 << 20
+    np.testing.assert_array_equal(m.deflect(z[:-1]), w[:-1])
+    m.close()
