@@ -87,6 +87,10 @@ const char* get_outfile_prefix(CCFHandle* self);
    solver does so by itself where other work keeps them from being there at once); the results are the same */
 void set_resident_chains(CCFHandle* self, int val);
 int get_resident_chains(CCFHandle* self);
+/* extension: how often a block that stays on the device looks for the others after an iteration, about 1.5 us each, before
+   the solver starts again with a launch per iteration (default 2^24) */
+void set_chain_polls(CCFHandle* self, int val);
+int get_chain_polls(CCFHandle* self);
 
 /* derived values and results, lib_ccf.cu:62-69 */
 int get_num_roots(CCFHandle* self);

@@ -223,12 +223,12 @@ __device__ __forceinline__ void store_shared(double* p, double v) { __hip_atomic
 /*
 The barrier after iteration `slot` of a chain of `blocks` blocks: each adds one to the low half of the slot's word
 and its count of unconverged roots to the high half. Returns the chain's total (final, and so the same in every
-block, once all have arrived), or -1 if some block waited CCF_SPINS polls in vain and set *failed. Every slot is
-used once and starts at zero.
+block, once all have arrived), or -1 if some block polled `polls` times in vain and set *failed: an iteration of
+millions of roots can take longer than the others wait, and the caller then starts the chain again without waiting.
+Every slot is used once and starts at zero.
 */
 constexpr int CCF_THREADS = 512;
 constexpr int CCF_TILE = 2048;   // roots and stars staged in LDS at a time (32 KB each)
-constexpr long long CCF_SPINS = 1ll << 24;
 constexpr long long CCF_MEET_TICKS = 500000;   // 5 ms of the 100 MHz clock
 
 /*
@@ -266,7 +266,7 @@ __device__ bool all_resident(unsigned long long* state)
 	return go;
 }
 
-__device__ int chain_barrier(unsigned long long* slot, int blocks, int active, int* failed)
+__device__ int chain_barrier(unsigned long long* slot, int blocks, int active, int* failed, int polls)
 {
 	__shared__ int result;
 	// this wave's stores have reached the coherence point; then every wave's have
@@ -276,13 +276,13 @@ __device__ int chain_barrier(unsigned long long* slot, int blocks, int active, i
 	{
 		unsigned long long v = __hip_atomic_fetch_add(slot, 1ull + ((unsigned long long)active << 32), __ATOMIC_RELAXED,
 			__HIP_MEMORY_SCOPE_AGENT);
-		long long spins = 0;
+		int polled = 0;
 		result = 0;
 		do
 		{
 			v = __hip_atomic_load(slot, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 			if (int(v & 0xffffffffu) == blocks) break;
-			if (++spins > CCF_SPINS || __hip_atomic_load(failed, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+			if (polled++ >= polls || __hip_atomic_load(failed, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
 			{
 				__hip_atomic_store(failed, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 				result = -1;
@@ -309,13 +309,14 @@ iterations of 5 us, most of which is the round trip through the barrier and the 
 1024 threads took 1.74 and 2.37 ms, and 4.1 and 2.7 ms on the larger field. rows: (nphi + nb) rows of nroots roots, the result; work: two copies of each chain's
 roots; slots: one word for the launch, then iters words per step of each chain, zeroed. The blocks meet first:
 if they are not all resident at once, the launch does nothing and failed[1] says so. (A cooperative launch would
-promise that they are, but the device grants those to one process at a time.) The same work then goes out one
-iteration per launch, `only` = its number (j0 = j1, flip: which copy is current), with no waiting.
+promise that they are, but the device grants those to one process at a time.) If a block waits in vain at a
+barrier, failed[0] says so and all leave. The same work then goes out one iteration per launch, `only` = its
+number (j0 = j1, flip: which copy is current), with no waiting.
 */
 template <bool LIN>
 __global__ __launch_bounds__(CCF_THREADS) void k_ccf_chain(ShootArgs a, dcx* __restrict__ rows, double* work, char* __restrict__ fin,
 	int* __restrict__ leaf_cache, unsigned long long* slots, int* failed, int nroots, int nstars, int circle_pole, int j0, int j1,
-	int nphi, int nb, int sides, int iters, int first_chain, int only, int flip)
+	int nphi, int nb, int sides, int iters, int first_chain, int only, int flip, int polls)
 {
 	__shared__ double rx_s[CCF_TILE], ry_s[CCF_TILE], px_s[CCF_TILE], py_s[CCF_TILE];
 	__shared__ int active_s;
@@ -501,7 +502,7 @@ __global__ __launch_bounds__(CCF_THREADS) void k_ccf_chain(ShootArgs a, dcx* __r
 			__syncthreads();
 			if (together)
 			{
-				const int left = chain_barrier(slot + (long long)(j - j0) * iters + it, int(gridDim.x), active_s, failed);
+				const int left = chain_barrier(slot + (long long)(j - j0) * iters + it, int(gridDim.x), active_s, failed, polls);
 				if (left < 0) return;
 				turn_over();
 				if (left == 0) break;
@@ -519,14 +520,14 @@ __global__ __launch_bounds__(CCF_THREADS) void k_ccf_chain(ShootArgs a, dcx* __r
 	}
 }
 
-// every chain's working copy from the rows its first step starts from (step j)
-__global__ void k_ccf_start(const dcx* __restrict__ rows, dcx* work, int nroots, int j, int nphi, int nb, int sides)
+// the working copies of chains first_chain + [0, gridDim.y) from the rows their first step starts from (step j)
+__global__ void k_ccf_start(const dcx* __restrict__ rows, dcx* work, int nroots, int j, int nphi, int nb, int sides, int first_chain)
 {
 	const int k = blockIdx.x * blockDim.x + threadIdx.x;
 	if (k >= nroots) return;
-	const int c = blockIdx.y / sides, b = blockIdx.y % sides;
+	const int chain = first_chain + blockIdx.y, c = chain / sides, b = chain % sides;
 	const CCRow from = cc_row(c, (sides == 1 || b == 1) ? 1 : -1, j, nphi, nb);
-	work[2ll * blockIdx.y * nroots + k] = rows[(long long)from.row * nroots + k];
+	work[2ll * chain * nroots + k] = rows[(long long)from.row * nroots + k];
 }
 
 /*
@@ -614,9 +615,12 @@ CCFResult Engine::ccf_solve(const LensParams& lens, const double* init_roots, in
 	MLENS_HIP_CHECK(hipMemsetAsync(err.ptr, 0, sizeof(unsigned long long), stream_));
 	MLENS_HIP_CHECK(hipMemsetAsync(flags.ptr, 0, 3 * sizeof(int), stream_));
 	// starting roots at the centre row of each branch
-	for (int c = 0; c < nb; c++)
-		MLENS_HIP_CHECK(hipMemcpyAsync(A.ptr + (long long)(c * (2 * J + 1) + J) * nroots, init_roots + 2 * (long long)c * nroots,
-			nroots * sizeof(dcx), hipMemcpyHostToDevice, stream_));
+	auto upload_start = [&](int first, int branches) {
+		for (int c = first; c < first + branches; c++)
+			MLENS_HIP_CHECK(hipMemcpyAsync(A.ptr + (long long)(c * (2 * J + 1) + J) * nroots, init_roots + 2 * (long long)c * nroots,
+				nroots * sizeof(dcx), hipMemcpyHostToDevice, stream_));
+	};
+	upload_start(0, nb);
 	// Steps j0 .. j1 of every chain. The blocks of a chain wait for each other, so all blocks of a launch must be
 	// resident: they share out evenly over the chains what the device holds, no more than a chain has roots for;
 	// chains beyond that go into further launches.
@@ -624,6 +628,7 @@ CCFResult Engine::ccf_solve(const LensParams& lens, const double* init_roots, in
 	int per_cu = 0;
 	MLENS_HIP_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, CCF_THREADS, 0));
 	const int resident = num_cus_ * std::max(1, per_cu);
+	bool together = ccf_together_;   // until a block has waited in vain
 	auto sweep = [&](int from, int j0, int j1, int sides, int iters) {
 		if (j1 < j0 || iters < 1) return;
 		const int chains = nb * sides, waves = CCF_THREADS / 64;
@@ -635,26 +640,35 @@ CCFResult Engine::ccf_solve(const LensParams& lens, const double* init_roots, in
 			const int blocks = std::max(1, std::min((nroots + waves - 1) / waves, resident / here));
 			auto kernel = a.smooth_linear ? k_ccf_chain<true> : k_ccf_chain<false>;
 			kernel<<<dim3(unsigned(blocks), unsigned(here)), CCF_THREADS, 0, stream_>>>(a, A.ptr, Bb.ptr, fin.ptr, leaf_cache.ptr,
-				slots.ptr, bad, nroots, ns, pole, ja, jb, nphi, nb, sides, iters, first, only, flip);
+				slots.ptr, bad, nroots, ns, pole, ja, jb, nphi, nb, sides, iters, first, only, flip, ccf_polls_);
 			MLENS_HIP_CHECK(hipGetLastError());
 		};
-		k_ccf_start<<<dim3(row_blocks, unsigned(chains)), 256, 0, stream_>>>(A.ptr, work, nroots, from, nphi, nb, sides);
-		MLENS_HIP_CHECK(hipGetLastError());
+		auto start = [&](int first, int here) {
+			k_ccf_start<<<dim3(row_blocks, unsigned(here)), 256, 0, stream_>>>(A.ptr, work, nroots, from, nphi, nb, sides, first);
+			MLENS_HIP_CHECK(hipGetLastError());
+		};
+		start(0, chains);
 		MLENS_HIP_CHECK(hipMemsetAsync(slots.ptr, 0, (chains + (size_t)chains * (j1 - j0 + 1) * iters) * sizeof(unsigned long long), stream_));
 		const int group = std::min(chains, resident);
 		for (int first = 0; first < chains; first += group)
 		{
 			const int here = std::min(group, chains - first);
 			int nf[2] = {0, 1};
-			if (ccf_together_)
+			if (together)
 			{
 				MLENS_HIP_CHECK(hipMemsetAsync(bad, 0, sizeof(nf), stream_));
 				launch(first, here, j0, j1, -1, 0);
 				MLENS_HIP_CHECK(hipMemcpyAsync(nf, bad, sizeof(nf), hipMemcpyDeviceToHost, stream_));
 				MLENS_HIP_CHECK(hipStreamSynchronize(stream_));
 			}
-			if (nf[0]) throw HipError("the blocks of a critical-curve chain lost each other", __FILE__, __LINE__);
-			if (!nf[1]) continue;
+			if (!nf[0] && !nf[1]) continue;
+			if (nf[0])
+			{
+				// some blocks have gone on: again from where the chains started (the first sweep writes that row)
+				together = false;
+				if (j0 == from) upload_start(first, here);
+				start(first, here);
+			}
 			for (int j = j0, n = 0; j <= j1; j++)
 				for (int it = 0; it < iters; it++, n++) launch(first, here, j, j, it, n & 1);
 		}

@@ -54,6 +54,7 @@ public:
 
 	/* extension: 0 sends every iteration out as a launch of its own (Engine::set_ccf_together) */
 	int resident_chains = 1;
+	int chain_polls = 1 << 24;   // Engine::set_ccf_polls
 
 	/* ccf.cuh:1263-1280 */
 	bool run(int verbose)
@@ -429,6 +430,7 @@ private:
 		std::vector<double> ccs(2 * total), caust(write_caustics ? 2 * total : 0), mu(write_mu_length_scales ? total : 0);
 		MLENS_VERBOSE("Finding critical curve positions...\n", verbose, 1);
 		engine_->set_ccf_together(resident_chains != 0);
+		engine_->set_ccf_polls(chain_polls);
 		CCFResult r = engine_->ccf_solve(lens(), init.data(), num_roots_, num_phi, num_branches, !rectangular && !approx, ccs.data(),
 			write_caustics ? caust.data() : nullptr, write_mu_length_scales ? mu.data() : nullptr);
 		t_init_roots_ = r.t_init_ms / 1000.0;

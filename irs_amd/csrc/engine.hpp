@@ -162,6 +162,8 @@ public:
 
 	/* false: one iteration per launch, as when other work keeps the blocks of a chain from being resident at once */
 	void set_ccf_together(bool on) { ccf_together_ = on; }
+	// how often a block looks for the others before it gives up (about 1.5 us each)
+	void set_ccf_polls(int polls) { ccf_polls_ = polls; }
 
 	/* thin test entry: lens equation at arbitrary points through the tree */
 	void deflect_points(const LensParams& lens, const double* z, int n, Precision prec, double* w, double* mu);
@@ -265,6 +267,7 @@ private:
 	DeviceBuffer<char> stars_aos_;
 	DeviceBuffer<double> scratch_d_;
 	bool ccf_together_ = true;
+	int ccf_polls_ = 1 << 24;
 	DeviceBuffer<double> points_;   // deflect_points: points, deflections, magnifications
 	DeviceBuffer<long long> scratch_ll_, hist_;
 };

@@ -40,6 +40,7 @@ MLENS_FIELD(write_caustics, int, write_caustics)
 MLENS_FIELD(write_mu_length_scales, int, write_mu_length_scales)
 MLENS_STRING_FIELD(outfile_prefix, outfile_prefix)
 MLENS_FIELD(resident_chains, int, resident_chains)
+MLENS_FIELD(chain_polls, int, chain_polls)
 
 int get_num_roots(CCFHandle* self) { return self->m.get_num_roots(); }
 ccf_dtype get_corner_x1(CCFHandle* self) { return self->m.get_corner().re; }

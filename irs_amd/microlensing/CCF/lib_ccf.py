@@ -12,7 +12,7 @@ _FIELDS = [
     ("safety_scale", "d"), ("num_stars", "i"), ("starfile", "s"), ("num_phi", "i"), ("num_branches", "i"),
     ("random_seed", "i"), ("write_stars", "i"), ("write_critical_curves", "i"), ("write_caustics", "i"),
     ("write_mu_length_scales", "i"), ("outfile_prefix", "s"),
-    ("resident_chains", "i"),
+    ("resident_chains", "i"), ("chain_polls", "i"),
 ]
 
 

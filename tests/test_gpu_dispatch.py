@@ -385,6 +385,13 @@ def test_critical_curve_chains(stars, phases, branches, exact):
     single.run()
     np.testing.assert_array_equal(single.critical_curves, c.critical_curves)
     single.close()
+    # blocks that give up on each other after one look, which starts the chains again: the same
+    for polls in (0, 1, 20):
+        impatient = CCF(**kw)
+        impatient.lib.set_chain_polls(impatient.obj, polls)
+        impatient.run()
+        np.testing.assert_array_equal(impatient.critical_curves, c.critical_curves)
+        impatient.close()
     prob = OC.Problem(c.stars, 0.3, 0.3, 1.0, 0.27, c.corner, approx=int(not exact))
     z = c.critical_curves[..., 0] + 1j * c.critical_curves[..., 1]
     half = phases // (2 * branches)
