@@ -15,7 +15,8 @@
 // the result does not depend on the order in which blocks run. Each branch and
 // side is a chain of steps and iterations that only its own roots link; the
 // blocks of a chain stay resident and meet at a barrier after each iteration,
-// and leave a step as soon as every root has converged.
+// and leave a step as soon as every root has converged. Fields of more than
+// 1024 stars, and a busy device, take a launch per iteration.
 #include "shoot_common.hpp"
 
 #include <algorithm>
@@ -228,7 +229,7 @@ millions of roots can take longer than the others wait, and the caller then star
 Every slot is used once and starts at zero.
 */
 constexpr int CCF_THREADS = 512;
-constexpr int CCF_TILE = 2048;   // roots and stars staged in LDS at a time (32 KB each)
+constexpr int CCF_FIT = 2048;   // roots and stars of a chain that a block holds in LDS (32 KB each)
 constexpr long long CCF_MEET_TICKS = 500000;   // 5 ms of the 100 MHz clock
 
 /*
@@ -299,29 +300,112 @@ __device__ int chain_barrier(unsigned long long* slot, int blocks, int active, i
 }
 
 /*
+What an update of the root at z needs beside the sums over roots and stars: its leaf, from the previous iteration
+while the root stays strictly inside it (there the tree descent would end in the same leaf), else by a fresh descent.
+*/
+struct CCPlace
+{
+	int node;
+	bool leaf;
+	CCLeaf f;
+};
+
+__device__ __forceinline__ void cc_find_place(const ShootArgs& a, dcx z, int* cache, CCPlace& p)
+{
+	const int cached = __builtin_amdgcn_readfirstlane(*cache);
+	bool inside = false;
+	if (cached >= 0)
+	{
+		const double h = a.nhl[cached] * (1 - 1e-12);
+		inside = fabs(z.re - a.ncx[cached]) < h && fabs(z.im - a.ncy[cached]) < h;
+	}
+	p.node = __builtin_amdgcn_readfirstlane(inside ? cached : find_node(a, z.re, z.im));
+	p.leaf = a.nchild0[p.node] < 0;
+	if (!inside && (threadIdx.x & 63) == 0) *cache = p.leaf ? p.node : -1;
+	if (p.leaf) p.f = cc_load_leaf(a, p.node);
+}
+
+// this lane's share of the sum of 1 / (z - x_q) over points q < n of a tile, leaving out point `skip`
+__device__ __forceinline__ void cc_pair_sum(const double* x, const double* y, int n, int skip, dcx z, double& re, double& im)
+{
+	for (int q = threadIdx.x & 63; q < n; q += 64)
+	{
+		if (q == skip) continue;
+		const double dx = z.re - x[q], dy = z.im - y[q];
+		const double ir2 = dev::rcp64(dx * dx + dy * dy);
+		re += dx * ir2;
+		im -= dy * ir2;
+	}
+}
+
+// The Aberth update of z from its lanes' shares of the sums over the other roots (r) and the poles (p): the new root
+// (in lane 0), and whether it is final.
+template <bool LIN>
+__device__ __forceinline__ dcx cc_update(const ShootArgs& a, const CCPlace& place, dcx z, dcx r, dcx p, double phi, int circle_pole, bool& fin)
+{
+	CCTerms t;
+	if (place.leaf)
+		t = cc_terms_leaf<LIN>(a, place.f, z);
+	else
+	{
+		// outside the root box; the tree's pointers are read here only
+		const ShootArgs* cold = reinterpret_cast<const ShootArgs*>((const void*)__builtin_amdgcn_kernarg_segment_ptr());
+		asm volatile("" : "+s"(cold));
+		t = cc_terms<LIN>(*cold, place.node, z, true, threadIdx.x & 63, 64);
+	}
+	r.re = wave_sum(r.re);
+	r.im = wave_sum(r.im);
+	p.re = wave_sum(p.re);
+	p.im = wave_sum(p.im);
+	t.S1.re = wave_sum(t.S1.re);
+	t.S1.im = wave_sum(t.S1.im);
+	t.S2.re = wave_sum(t.S2.re);
+	t.S2.im = wave_sum(t.S2.im);
+	dcx zn = z;
+	if ((threadIdx.x & 63) == 0)
+	{
+		const dcx f0 = cc_f0(a, t, phi);
+		// 1/mu below 1e-9 (both bounds of ccf_functions.cuh:207-211): the root stays
+		fin = cc_inv_mu_error(a, t, f0) < 1e-9;
+		if (!fin)
+		{
+			const dcx f1 = dcx{-2 * a.theta2 * t.S2.re - t.L2.re - t.d2s.re, -2 * a.theta2 * t.S2.im - t.L2.im + t.d2s.im};
+			dcx psum = dcx{2 * p.re, 2 * p.im};
+			if (circle_pole)
+			{
+				const dcx iz = dev::cdiv(dcx{1, 0}, z);
+				psum = dev::add(psum, dev::scale(iz, 2));
+			}
+			const dcx den = dev::add(f1, dev::mul(f0, dcx{psum.re - r.re, psum.im - r.im}));
+			zn = dev::sub(z, dev::cdiv(f0, den));
+			fin = dev::cabs(dev::sub(zn, z)) / sqrt(a.theta2) < 1e-9;
+		}
+	}
+	return zn;
+}
+
+/*
 Steps j0 .. j1 of chains first_chain + [0, gridDim.y) (ccf_functions.cuh:171-240, 309-386): chain c * sides + b is
 branch c, side b (side 0 steps phi down, side 1 up; at j = 0 there is one side). A step starts from the roots of
 the one before it and runs at most `iters` Aberth iterations; once every root of the chain has converged the rest
 would change nothing and is left out. Blocks of eight waves, a wave per root at a time, root by root round the
-chain's gridDim.x blocks. 137 stars (274 roots, 100 phases): 1.78 ms, against 5.20 ms with one launch per
-iteration and all 20 of them at every step; 1500 stars, 20 phases: 3.0 against 4.9 ms. A step takes about seven
-iterations of 5 us, most of which is the round trip through the barrier and the shared roots. Blocks of 256 or
-1024 threads took 1.74 and 2.37 ms, and 4.1 and 2.7 ms on the larger field. rows: (nphi + nb) rows of nroots roots, the result; work: two copies of each chain's
-roots; slots: one word for the launch, then iters words per step of each chain, zeroed. The blocks meet first:
-if they are not all resident at once, the launch does nothing and failed[1] says so. (A cooperative launch would
-promise that they are, but the device grants those to one process at a time.) If a block waits in vain at a
-barrier, failed[0] says so and all leave. The same work then goes out one iteration per launch, `only` = its
-number (j0 = j1, flip: which copy is current), with no waiting.
+chain's gridDim.x blocks; each holds all roots and stars in LDS, at most CCF_FIT of either. 137 stars (274 roots,
+100 phases): 1.8 ms, against 4.5 ms with one launch per iteration. A step takes about seven iterations of 5 us, most
+of which is the round trip through the barrier and the shared roots. Blocks of 256 or 1024 threads took 1.74 and
+2.37 ms. rows: (nphi + nb) rows of nroots roots, the result; work: two copies of each chain's roots; slots: one word
+for the launch, then iters words per step of each chain, zeroed. The blocks meet first: if they are not all resident
+at once, the launch does nothing and failed[1] says so. (A cooperative launch would promise that they are, but the
+device grants those to one process at a time.) If a block waits in vain at a barrier, failed[0] says so and all
+leave. The work then goes out through k_ccf_iterate, with no waiting.
 */
 template <bool LIN>
 __global__ __launch_bounds__(CCF_THREADS) void k_ccf_chain(ShootArgs a, dcx* __restrict__ rows, double* work, char* __restrict__ fin,
 	int* __restrict__ leaf_cache, unsigned long long* slots, int* failed, int nroots, int nstars, int circle_pole, int j0, int j1,
-	int nphi, int nb, int sides, int iters, int first_chain, int only, int flip, int polls)
+	int nphi, int nb, int sides, int iters, int first_chain, int polls)
 {
-	__shared__ double rx_s[CCF_TILE], ry_s[CCF_TILE], px_s[CCF_TILE], py_s[CCF_TILE];
+	__shared__ double rx_s[CCF_FIT], ry_s[CCF_FIT], px_s[CCF_FIT], py_s[CCF_FIT];
 	__shared__ int active_s;
-	const bool together = only < 0;
-	if (together && !all_resident(slots + first_chain))
+	if (!all_resident(slots + first_chain))
 	{
 		if (threadIdx.x == 0) __hip_atomic_store(failed + 1, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 		return;
@@ -334,163 +418,44 @@ __global__ __launch_bounds__(CCF_THREADS) void k_ccf_chain(ShootArgs a, dcx* __r
 	const int waves = int(gridDim.x) * (CCF_THREADS / 64);
 	double* cur = work + 4ll * chain * nroots;   // (re, im) of every root, twice
 	double* nxt = cur + 2ll * nroots;
-	auto turn_over = [&]() {
-		double* t = cur;
-		cur = nxt;
-		nxt = t;
-	};
-	if (flip) turn_over();
-	const bool stars_fit = nstars <= CCF_TILE;
-	if (stars_fit)
-		for (int i = threadIdx.x; i < nstars; i += CCF_THREADS)
-		{
-			px_s[i] = a.sx[i];
-			py_s[i] = a.sy[i];
-		}
+	for (int i = threadIdx.x; i < nstars; i += CCF_THREADS)
+	{
+		px_s[i] = a.sx[i];
+		py_s[i] = a.sy[i];
+	}
 	unsigned long long* slot = slots + nb * sides + (long long)chain * (j1 - j0 + 1) * iters;
 	char* done = fin + ((long long)c * 2 + b) * nroots;
 	int* leaves = leaf_cache + ((long long)c * 2 + b) * nroots;
 	for (int j = j0; j <= j1; j++)
 	{
 		const CCRow R = cc_row(c, sgn, j, nphi, nb);
-		const int it0 = together ? 0 : only, it1 = together ? iters : only + 1;
-		if (it0 == 0)
-			for (int k = wave; k < nroots; k += waves)
-				if (lane == 0) done[k] = 0;
-		for (int it = it0; it < it1; it++)
+		for (int k = wave; k < nroots; k += waves)
+			if (lane == 0) done[k] = 0;
+		for (int it = 0; it < iters; it++)
 		{
 			if (threadIdx.x == 0) active_s = 0;
-			// the loop runs once if the roots fit one tile; a wave then updates its roots in turn
-			const bool roots_fit = nroots <= CCF_TILE;
-			if (roots_fit)
-				for (int i = threadIdx.x; i < nroots; i += CCF_THREADS)
-				{
-					rx_s[i] = load_shared(cur + 2 * i);
-					ry_s[i] = load_shared(cur + 2 * i + 1);
-				}
-			__syncthreads();
-			// every wave takes as many turns as the first, since the tiles are shared by the block
-			const int turns = (nroots - (wave & ~(CCF_THREADS / 64 - 1)) + waves - 1) / waves;
-			for (int turn = 0; turn < turns; turn++)
+			for (int i = threadIdx.x; i < nroots; i += CCF_THREADS)
 			{
-				const int k = wave + turn * waves;
-				const bool mine = k < nroots;
-				const bool active = mine && !done[k];
-				dcx z = {0, 0};
-				if (mine) z = roots_fit ? dcx{rx_s[k], ry_s[k]} : dcx{load_shared(cur + 2 * k), load_shared(cur + 2 * k + 1)};
-				// the root's leaf from the previous iteration while the root stays strictly inside
-				// it (there the tree descent would end in the same leaf), else a fresh descent
-				int node = 0;
-				bool leaf = false;
-				CCLeaf f;
-				if (active)
+				rx_s[i] = load_shared(cur + 2 * i);
+				ry_s[i] = load_shared(cur + 2 * i + 1);
+			}
+			__syncthreads();
+			for (int k = wave; k < nroots; k += waves)
+			{
+				const dcx z = dcx{rx_s[k], ry_s[k]};
+				dcx zn = z;
+				bool fin_now = true;
+				if (!done[k])
 				{
-					const int cached = __builtin_amdgcn_readfirstlane(leaves[k]);
-					bool inside = false;
-					if (cached >= 0)
-					{
-						const double h = a.nhl[cached] * (1 - 1e-12);
-						inside = fabs(z.re - a.ncx[cached]) < h && fabs(z.im - a.ncy[cached]) < h;
-					}
-					node = __builtin_amdgcn_readfirstlane(inside ? cached : find_node(a, z.re, z.im));
-					leaf = a.nchild0[node] < 0;
-					if (!inside && lane == 0) leaves[k] = leaf ? node : -1;
-					if (leaf) f = cc_load_leaf(a, node);
+					CCPlace place;
+					cc_find_place(a, z, leaves + k, place);
+					dcx r = {0, 0}, p = {0, 0};
+					cc_pair_sum(rx_s, ry_s, nroots, k, z, r.re, r.im);
+					cc_pair_sum(px_s, py_s, nstars, -1, z, p.re, p.im);
+					zn = cc_update<LIN>(a, place, z, r, p, R.phi, circle_pole, fin_now);
 				}
-				// this lane's share of the sums over the other roots and over the poles (stars)
-				double rx = 0, ry = 0, px = 0, py = 0;
-				for (int t0 = 0; t0 < nroots; t0 += CCF_TILE)
-				{
-					const int n = min(CCF_TILE, nroots - t0);
-					if (!roots_fit)
-					{
-						__syncthreads();
-						for (int i = threadIdx.x; i < n; i += CCF_THREADS)
-						{
-							rx_s[i] = load_shared(cur + 2 * (t0 + i));
-							ry_s[i] = load_shared(cur + 2 * (t0 + i) + 1);
-						}
-						__syncthreads();
-					}
-					if (active)
-						for (int q = lane; q < n; q += 64)
-						{
-							if (t0 + q == k) continue;
-							const double dx = z.re - rx_s[q], dy = z.im - ry_s[q];
-							const double ir2 = dev::rcp64(dx * dx + dy * dy);
-							rx += dx * ir2;
-							ry -= dy * ir2;
-						}
-				}
-				for (int t0 = 0; t0 < nstars; t0 += CCF_TILE)
-				{
-					const int n = min(CCF_TILE, nstars - t0);
-					if (!stars_fit)
-					{
-						__syncthreads();
-						for (int i = threadIdx.x; i < n; i += CCF_THREADS)
-						{
-							px_s[i] = a.sx[t0 + i];
-							py_s[i] = a.sy[t0 + i];
-						}
-						__syncthreads();
-					}
-					if (active)
-						for (int q = lane; q < n; q += 64)
-						{
-							const double dx = z.re - px_s[q], dy = z.im - py_s[q];
-							const double ir2 = dev::rcp64(dx * dx + dy * dy);
-							px += dx * ir2;
-							py -= dy * ir2;
-						}
-				}
-				if (!mine) continue;
-				if (!active)
-				{
-					if (lane == 0)
-					{
-						store_shared(nxt + 2 * k, z.re);
-						store_shared(nxt + 2 * k + 1, z.im);
-					}
-					continue;
-				}
-				CCTerms t;
-				if (leaf)
-					t = cc_terms_leaf<LIN>(a, f, z);
-				else
-				{
-					// outside the root box; the tree's pointers are read here only
-					const ShootArgs* cold = reinterpret_cast<const ShootArgs*>((const void*)__builtin_amdgcn_kernarg_segment_ptr());
-					asm volatile("" : "+s"(cold));
-					t = cc_terms<LIN>(*cold, node, z, true, lane, 64);
-				}
-				rx = wave_sum(rx);
-				ry = wave_sum(ry);
-				px = wave_sum(px);
-				py = wave_sum(py);
-				t.S1.re = wave_sum(t.S1.re);
-				t.S1.im = wave_sum(t.S1.im);
-				t.S2.re = wave_sum(t.S2.re);
-				t.S2.im = wave_sum(t.S2.im);
 				if (lane == 0)
 				{
-					const dcx f0 = cc_f0(a, t, R.phi);
-					dcx zn = z;
-					// 1/mu below 1e-9 (both bounds of ccf_functions.cuh:207-211): the root stays
-					bool fin_now = cc_inv_mu_error(a, t, f0) < 1e-9;
-					if (!fin_now)
-					{
-						const dcx f1 = dcx{-2 * a.theta2 * t.S2.re - t.L2.re - t.d2s.re, -2 * a.theta2 * t.S2.im - t.L2.im + t.d2s.im};
-						dcx psum = dcx{2 * px, 2 * py};
-						if (circle_pole)
-						{
-							const dcx iz = dev::cdiv(dcx{1, 0}, z);
-							psum = dev::add(psum, dev::scale(iz, 2));
-						}
-						const dcx den = dev::add(f1, dev::mul(f0, dcx{psum.re - rx, psum.im - ry}));
-						zn = dev::sub(z, dev::cdiv(f0, den));
-						fin_now = dev::cabs(dev::sub(zn, z)) / sqrt(a.theta2) < 1e-9;
-					}
 					store_shared(nxt + 2 * k, zn.re);
 					store_shared(nxt + 2 * k + 1, zn.im);
 					if (fin_now)
@@ -500,25 +465,84 @@ __global__ __launch_bounds__(CCF_THREADS) void k_ccf_chain(ShootArgs a, dcx* __r
 				}
 			}
 			__syncthreads();
-			if (together)
-			{
-				const int left = chain_barrier(slot + (long long)(j - j0) * iters + it, int(gridDim.x), active_s, failed, polls);
-				if (left < 0) return;
-				turn_over();
-				if (left == 0) break;
-			}
-			else
-			{
-				// the roots this wave has just written are the ones it stores below
-				asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-				turn_over();
-			}
+			const int left = chain_barrier(slot + (long long)(j - j0) * iters + it, int(gridDim.x), active_s, failed, polls);
+			if (left < 0) return;
+			double* t = cur;
+			cur = nxt;
+			nxt = t;
+			if (left == 0) break;
 		}
-		if (!together && it1 < iters) continue;
 		for (int k = wave; k < nroots; k += waves)
 			if (lane < 2) reinterpret_cast<double*>(rows + (long long)R.row * nroots + k)[lane] = load_shared(cur + 2 * k + lane);
 	}
 }
+
+/*
+One iteration of step j of chains first_chain + [0, gridDim.y) by itself: four roots a block, a wave each, the same
+sums in the same order. flip: which working copy is current; first, last: of the step's iterations. A block whose
+roots are final copies them and leaves, so the iterations after the last change cost a launch each. Seven waves per
+SIMD (70 VGPRs), which the sums over many roots need: 20000 stars, two phases, take 59 ms in all, 118 ms where
+resident blocks of eight waves, one to a CU, read the roots past the caches once for every root of a wave.
+*/
+constexpr int CCF_ROOTS = 4;
+constexpr int CCF_TILE = 256;
+
+template <bool LIN>
+__global__ __launch_bounds__(64 * CCF_ROOTS) void k_ccf_iterate(ShootArgs a, dcx* __restrict__ rows, dcx* work, char* __restrict__ fin,
+	int* __restrict__ leaf_cache, int nroots, int nstars, int circle_pole, int j, int nphi, int nb, int sides, int first_chain, int flip,
+	int first, int last)
+{
+	__shared__ double x_s[CCF_TILE], y_s[CCF_TILE];
+	const int chain = first_chain + blockIdx.y;
+	const int c = chain / sides, b = chain % sides;
+	const CCRow R = cc_row(c, (sides == 1 || b == 1) ? 1 : -1, j, nphi, nb);
+	const int lane = threadIdx.x & 63, k = __builtin_amdgcn_readfirstlane(int(blockIdx.x) * CCF_ROOTS + int(threadIdx.x >> 6));
+	const dcx* cur = work + (2ll * chain + flip) * nroots;
+	dcx* nxt = work + (2ll * chain + (1 - flip)) * nroots;
+	char* done = fin + ((long long)c * 2 + b) * nroots;
+	int* leaves = leaf_cache + ((long long)c * 2 + b) * nroots;
+	const bool mine = k < nroots, active = mine && (first || !done[k]);
+	const dcx z = mine ? cur[k] : dcx{0, 0};
+	dcx zn = z;
+	if (__syncthreads_or(active))
+	{
+		CCPlace place;
+		if (active) cc_find_place(a, z, leaves + k, place);
+		dcx r = {0, 0}, p = {0, 0};
+		for (int t0 = 0; t0 < nroots; t0 += CCF_TILE)
+		{
+			const int i = t0 + threadIdx.x;
+			const dcx v = i < nroots ? cur[i] : dcx{0, 0};
+			__syncthreads();
+			x_s[threadIdx.x] = v.re;
+			y_s[threadIdx.x] = v.im;
+			__syncthreads();
+			if (active) cc_pair_sum(x_s, y_s, min(CCF_TILE, nroots - t0), k - t0, z, r.re, r.im);
+		}
+		for (int t0 = 0; t0 < nstars; t0 += CCF_TILE)
+		{
+			const int i = t0 + threadIdx.x;
+			const dcx v = i < nstars ? dcx{a.sx[i], a.sy[i]} : dcx{0, 0};
+			__syncthreads();
+			x_s[threadIdx.x] = v.re;
+			y_s[threadIdx.x] = v.im;
+			__syncthreads();
+			if (active) cc_pair_sum(x_s, y_s, min(CCF_TILE, nstars - t0), -1, z, p.re, p.im);
+		}
+		if (active)
+		{
+			bool fin_now = false;
+			zn = cc_update<LIN>(a, place, z, r, p, R.phi, circle_pole, fin_now);
+			if (lane == 0) done[k] = fin_now;
+		}
+	}
+	if (mine && lane == 0)
+	{
+		nxt[k] = zn;
+		if (last) rows[(long long)R.row * nroots + k] = zn;
+	}
+}
+static_assert(CCF_TILE == 64 * CCF_ROOTS, "a thread stages a point");
 
 // the working copies of chains first_chain + [0, gridDim.y) from the rows their first step starts from (step j)
 __global__ void k_ccf_start(const dcx* __restrict__ rows, dcx* work, int nroots, int j, int nphi, int nb, int sides, int first_chain)
@@ -628,7 +652,9 @@ CCFResult Engine::ccf_solve(const LensParams& lens, const double* init_roots, in
 	int per_cu = 0;
 	MLENS_HIP_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, CCF_THREADS, 0));
 	const int resident = num_cus_ * std::max(1, per_cu);
-	bool together = ccf_together_;   // until a block has waited in vain
+	// resident chains for fields that fit a block's LDS: 20 stars 1.5 against 2.9 ms, 500 stars 3.6 against 5.0, 1000
+	// stars 3.0 against 3.4; from there on the pair sums count, not the launches. Until a block has waited in vain.
+	bool together = ccf_together_ && nroots <= CCF_FIT && nstars_ <= CCF_FIT;
 	auto sweep = [&](int from, int j0, int j1, int sides, int iters) {
 		if (j1 < j0 || iters < 1) return;
 		const int chains = nb * sides, waves = CCF_THREADS / 64;
@@ -636,11 +662,20 @@ CCFResult Engine::ccf_solve(const LensParams& lens, const double* init_roots, in
 		dcx* work = reinterpret_cast<dcx*>(Bb.ptr);
 		int* bad = flags.ptr + 1;
 		const int ns = nstars_, pole = circle_pole ? 1 : 0;
-		auto launch = [&](int first, int here, int ja, int jb, int only, int flip) {
+		auto chain_steps = [&](int first, int here) {
 			const int blocks = std::max(1, std::min((nroots + waves - 1) / waves, resident / here));
 			auto kernel = a.smooth_linear ? k_ccf_chain<true> : k_ccf_chain<false>;
 			kernel<<<dim3(unsigned(blocks), unsigned(here)), CCF_THREADS, 0, stream_>>>(a, A.ptr, Bb.ptr, fin.ptr, leaf_cache.ptr,
-				slots.ptr, bad, nroots, ns, pole, ja, jb, nphi, nb, sides, iters, first, only, flip, ccf_polls_);
+				slots.ptr, bad, nroots, ns, pole, j0, j1, nphi, nb, sides, iters, first, ccf_polls_);
+			MLENS_HIP_CHECK(hipGetLastError());
+		};
+		auto iterations = [&](int first, int here) {
+			auto kernel = a.smooth_linear ? k_ccf_iterate<true> : k_ccf_iterate<false>;
+			const dim3 grid(unsigned((nroots + CCF_ROOTS - 1) / CCF_ROOTS), unsigned(here));
+			for (int j = j0, n = 0; j <= j1; j++)
+				for (int it = 0; it < iters; it++, n++)
+					kernel<<<grid, 64 * CCF_ROOTS, 0, stream_>>>(a, A.ptr, work, fin.ptr, leaf_cache.ptr, nroots, ns, pole, j, nphi, nb,
+						sides, first, n & 1, it == 0, it == iters - 1);
 			MLENS_HIP_CHECK(hipGetLastError());
 		};
 		auto start = [&](int first, int here) {
@@ -657,7 +692,7 @@ CCFResult Engine::ccf_solve(const LensParams& lens, const double* init_roots, in
 			if (together)
 			{
 				MLENS_HIP_CHECK(hipMemsetAsync(bad, 0, sizeof(nf), stream_));
-				launch(first, here, j0, j1, -1, 0);
+				chain_steps(first, here);
 				MLENS_HIP_CHECK(hipMemcpyAsync(nf, bad, sizeof(nf), hipMemcpyDeviceToHost, stream_));
 				MLENS_HIP_CHECK(hipStreamSynchronize(stream_));
 			}
@@ -669,8 +704,7 @@ CCFResult Engine::ccf_solve(const LensParams& lens, const double* init_roots, in
 				if (j0 == from) upload_start(first, here);
 				start(first, here);
 			}
-			for (int j = j0, n = 0; j <= j1; j++)
-				for (int it = 0; it < iters; it++, n++) launch(first, here, j, j, it, n & 1);
+			iterations(first, here);
 		}
 	};
 	CCFResult r;

@@ -364,10 +364,12 @@ def test_critical_curves_beside_other_work(tmp_path):
 
 
 @pytest.mark.parametrize("stars,phases,branches,exact", [(1, 4, 1, False), (2, 4, 2, True), (5, 600, 300, False),
-                                                         (1100, 2, 1, False), (2100, 2, 1, False)])
+                                                         (1024, 2, 1, False), (1025, 2, 1, False), (1100, 2, 1, False),
+                                                         (2100, 2, 1, False), (1300, 2, 1, True)])
 def test_critical_curve_chains(stars, phases, branches, exact):
     """Chains of one block and of many, more chains than the device holds at once (600),
-    roots past one LDS tile (2048) and stars past it, linear and general smooth matter:
+    the last field that a block holds (1024 stars, 2048 roots) and larger ones, which take
+    a launch per iteration, linear and general smooth matter:
     every root solves the critical-curve equation by direct sums (1/mu below 1e-6, as in
     the oracle tests) and the roots of a phase are distinct."""
     from irs_amd.microlensing.CCF.ccf import CCF
