@@ -551,6 +551,7 @@ void Surrogate::predict(const float* x, int n, float* probs)
 
 double Surrogate::time_predict(const float* x, int n, int reps)
 {
+	if (n < 1) throw HipError("a timed surrogate request needs at least one row", __FILE__, __LINE__);
 	const int rows = std::min(n, max_batch_), M = (rows + 15) / 16 * 16;
 	std::vector<unsigned short> xp(size_t(M) * SURR_PIN);
 	pad_inputs(x, rows, xp.data());

@@ -413,7 +413,6 @@ def test_surrogate_batches_and_requests(batch, n):
     leave rows over, against an epoch made of single steps (the same kernels in the same
     order: equal); and requests through pinned memory (up to 256 rows) and through device
     buffers, padded or not, against the FP64 network (the bound of the gradient test)."""
-    import ctypes
     from irs_amd.microlensing.Surrogate import surrogate as S
     from oracle import mlp
     rng = np.random.default_rng(batch)
@@ -617,3 +616,14 @@ def test_large_deflection_calls_give_their_memory_back(tmp_path):
     assert before - free_memory(m.lib) < 8 << 20
     np.testing.assert_array_equal(m.deflect(z[:-1]), w[:-1])
     m.close()
+
+
+@pytest.mark.parametrize("n", [0, -1, -16, -20, -31, -40])
+def test_timed_request_without_rows_is_refused(n):
+    """No rows to time, and counts below none, give the error value."""
+    from irs_amd.microlensing.Surrogate import surrogate as S
+    s = S.HistogramSurrogate(max_batch=64, seed=1)
+    x = np.zeros((1, 6), dtype=np.float32)
+    assert S.lib.surrogate_time_predict(s.obj, x.ctypes.data_as(ctypes.POINTER(ctypes.c_float)), n, 3) == -1.0
+    assert s.seconds_per_histogram(x) > 0
+    s.close()
