@@ -714,7 +714,7 @@ void Engine::build_tree(double root_half_length)
 {
 	const int n = nstars_;
 	num_nodes_ = 0;
-	// an even field ends with 0.9 nodes per star; growing copies every node array (0.15 ms each time at 7e3 stars)
+	// an even field ends with 0.6 to 0.9 nodes per star; growing copies every node array (0.15 ms each time at 7e3 stars)
 	ensure_node_capacity(std::max(1024, n + n / 8));
 	level_start_.assign({0, 1});
 	levels_ = 0;

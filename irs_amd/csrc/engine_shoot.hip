@@ -1013,9 +1013,9 @@ __device__ __forceinline__ void late_rows(WideList* list, F take)
 	}
 }
 
-// Compiled for linear smooth matter (LIN) the kernel needs 114 VGPRs and spills no scalar
-// register: four waves per SIMD. With the general sheet's code in it, 136 VGPRs hold 130
-// spilled scalars as well, and it runs at three.
+// Compiled for linear smooth matter (LIN) the kernel needs 113 to 117 VGPRs and spills at most
+// six scalar registers: four waves per SIMD. With the general sheet's code in it, 137 to 139 VGPRs
+// hold some 120 spilled scalars as well, and it runs at three.
 template <int PREC, bool PARITY, bool LIN>
 __global__ __launch_bounds__(64 * IPM_WAVES, LIN ? 4 : 3) void k_ipm_fast(ShootArgs a, long long row0, long long row1,
 	MLENS_TABLE_PARAMS, void* __restrict__ map, void* __restrict__ mmin, void* __restrict__ msad,
@@ -1613,11 +1613,11 @@ __device__ __forceinline__ void irs_count(const ShootArgs& a, const IrsWindow& w
 		atomicAdd(reinterpret_cast<int*>(PARITY ? ((key_y & 1) ? a.msad : a.mmin) : a.map) + ((long long)py * a.n1 + px), v);
 }
 
-// LIN (linear smooth matter) takes the mixed kernel from 116 to 85 VGPRs and its 90 spilled scalar
-// registers to 2, hence from four waves per SIMD to five: 1.04e9 rays in 8.2 ms against 9.5 ms.
+// LIN (linear smooth matter) takes the mixed kernel from 116 to 85 VGPRs and its 92 spilled scalar
+// registers to 4, hence from four waves per SIMD to five: 1.04e9 rays in 7.4 ms against 9.5 ms.
 // With parities (FP64 positions and magnifications; 1.6e9 rays) the shot took 118 ms with a second
 // pass over the leaf's tables for the magnification and parity counts sent straight to the maps,
-// and takes 40 ms.
+// and takes 32 ms.
 template <int PREC, bool PARITY, bool LIN>
 __global__ __launch_bounds__(IRS_THREADS) void k_irs_fast(ShootArgs a, long long row0, long long row1,
 	unsigned long long* __restrict__ received, MLENS_TABLE_PARAMS, void* __restrict__ map, void* __restrict__ mmin,
