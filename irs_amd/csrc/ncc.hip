@@ -693,7 +693,8 @@ void NCCDevice::count(const double* caustics, int nrows, int ncols, const NCCGri
 	size_t free_b = 0, total_b = 0;
 	MLENS_HIP_CHECK(hipMemGetInfo(&free_b, &total_b));
 	const double need = double(npx) * double(npy) * sizeof(int);
-	if (need > 0.9 * double(free_b))
+	// lists of an earlier run make room for a grid (below)
+	if (need > 0.9 * (double(free_b) + double(lists_.count) * sizeof(int)))
 		throw std::runtime_error("the over-sampled pixel grid (" + std::to_string((long long)(need / 1048576)) +
 			" MiB) does not fit in device memory");
 
@@ -756,9 +757,12 @@ void NCCDevice::count(const double* caustics, int nrows, int ncols, const NCCGri
 	if (!lists)
 	{
 		const size_t nfine = size_t(npx) * size_t(npy);
-		// the memory check above counted the grid alone: lists that overflowed make room for it
-		if (st.path == NCC_OVERFLOW && fine_.count < nfine) lists_.free();
-		if (fine_.count < nfine) fine_.alloc(nfine);
+		// the memory check above counted the grid alone: lists, overflowed or of an earlier run, make room for it
+		if (fine_.count < nfine)
+		{
+			lists_.free();
+			fine_.alloc(nfine);
+		}
 		MLENS_HIP_CHECK(hipMemsetAsync(fine_.ptr, 0, nfine * sizeof(int), stream_));
 		k_ncc_init<<<1, 64, 0, stream_>>>(meta, nullptr, 0);
 		MLENS_HIP_CHECK(hipEventRecord(ev0_, stream_));

@@ -560,6 +560,22 @@ def test_overflowed_lists_make_room(tmp_path):
     assert n.lib.get_crossing_path(n.obj) == 2 and n.num_caustic_crossings.max() > 0
     assert held < 384 << 20
     n.close()
+    # the same of an object whose lists sufficed for its first run
+    with open(tmp_path / "ccf_caustics.bin", "wb") as fh:
+        np.array([1, rows.shape[1]], dtype=np.int32).tofile(fh)
+        np.ascontiguousarray(rows[:1], dtype=np.complex128).tofile(fh)
+    n = NCC(infile_prefix=str(tmp_path) + "/", num_pixels_y1=32, num_pixels_y2=8192, over_sample=4, write_maps=False)
+    before = free_memory(n.lib)
+    n.run()
+    assert n.lib.get_crossing_path(n.obj) == 1
+    with open(tmp_path / "ccf_caustics.bin", "wb") as fh:
+        np.array(rows.shape, dtype=np.int32).tofile(fh)
+        np.ascontiguousarray(rows, dtype=np.complex128).tofile(fh)
+    n.run()
+    held = before - free_memory(n.lib)
+    say(f"[ncc memory] second run: path {n.lib.get_crossing_path(n.obj)}, {held >> 20} MB held")
+    assert held < 384 << 20
+    n.close()
 
 
 def test_failed_crossings_leave_zeros(tmp_path):
